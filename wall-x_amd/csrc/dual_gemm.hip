@@ -7,7 +7,7 @@
 // (thousands of VL rows next to tens of action rows, or an empty group) is just a longer or shorter tile list.
 //
 // Workgroup tile 256 x 256, K step 32, one workgroup per CU: eight wavefronts (two per SIMD) as 2 x 4, wave tile
-// 128 x 64 = 4 x 2 MFMA 32x32x16 accumulator blocks (128 accumulator registers per lane), of which one per SIMD
+// 128 x 64 = 8 x 4 MFMA 16x16x32 accumulator blocks (128 accumulator registers per lane), of which one per SIMD
 // issues the global -> LDS loads; the projection that rotates heads in its epilogue runs the same tile with the
 // wavefronts as 4 x 2 (wave tile 64 x 128: a wavefront holds whole heads).  Problems whose 256 x 256
 // tiles would leave most CUs idle (a denoise step of a few thousand action tokens) run the same kernel with a
@@ -47,7 +47,8 @@ namespace {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
 constexpr int BK = 32;
 constexpr int kStages = 4;                     // ring slots per operand
@@ -63,29 +64,27 @@ struct TileShape {
   static constexpr int kWaves = kWavesM * kWavesN;
   static constexpr int kLoadWaves = LW_ > 0 ? LW_ : kWaves;
   static constexpr int kThreads = kWaves * 64;
-  static constexpr int FM = BM / kWavesM / 32;        // 32x32 accumulator blocks per wave along M
-  static constexpr int FN = BN / kWavesN / 32;        // ... and along N
+  static constexpr int FM = BM / kWavesM / 16;        // 16x16 accumulator blocks per wave along M
+  static constexpr int FN = BN / kWavesN / 16;        // ... and along N
   static constexpr int kLoadRowsA = BM / kLoadWaves;  // LDS rows of A one loading wave loads per K step
   static constexpr int kLoadRowsB = BN / kLoadWaves;  // ... and of B
   static constexpr int kLoadsA = kLoadRowsA / 16;     // 16-row load instructions per wave per K step: A
   static constexpr int kLoadsB = kLoadRowsB / 16;     // ... and B
   static constexpr int kSlotBytesA = BM * kRowBytes;  // bytes of A per K step
   static constexpr int kSlotBytesB = BN * kRowBytes;
-  static constexpr int kStageBytes = FN >= 4 ? (kWaves > 4 || BM <= 128 ? 4096 : 8192) : 2048;  // per-wave staging for the epilogue
+  static constexpr int kStageBytes = FN * 512;        // per-wave staging for the epilogue: 16 rows of the wave tile
   static constexpr int kLdsBytes = kStages * (kSlotBytesA + kSlotBytesB) + kWaves * kStageBytes;
-  static constexpr int kWgPerCu = kLdsBytes <= 80 * 1024 && FM * FN * 16 <= 128 ? 2 : 1;
+  static constexpr int kWgPerCu = kLdsBytes <= 80 * 1024 && FM * FN * 4 <= 128 ? 2 : 1;
   static_assert(kLdsBytes <= 160 * 1024, "LDS budget");
-  static_assert(FM >= 1 && FN >= 2 && FN % 2 == 0 && kLoadsA >= 1 && kLoadsB >= 1 && kLoadsB <= kLoadsA, "tile shape");
+  static_assert(FM >= 2 && FN >= 4 && FM % 2 == 0 && FN % 4 == 0 && kLoadsA >= 1 && kLoadsB >= 1 && kLoadsB <= kLoadsA, "tile shape");
 };
-// four wavefronts (one per SIMD) as 2 x 2: wave tile 128 x 128, 256 accumulator registers per lane
-using BigTile = TileShape<256, 256, 2, 2>;
 // eight wavefronts (two per SIMD) as 2 x 4: wave tile 128 x 64, 128 accumulator registers per lane, and only the
 // first four (one per SIMD) issue the global -> LDS loads.  A wavefront that issues a load stalls while the CU's load
 // path takes the instruction in; here its partner on the same SIMD issues no loads and keeps the MFMA pipe fed
-// meanwhile.  Against BigTile, on the config 3 shapes: gate/up 4-7 % faster, down 3 %, the row-major op 2-6 %.
-// (With all eight loading on one schedule, both partners stall together: that form was 2 % ahead of BigTile on
-// gate/up and behind it elsewhere.)
-using BigTile8 = TileShape<256, 256, 2, 4, 4>;
+// meanwhile.  Against four wavefronts of 128 x 128, on the config 3 shapes: gate/up 4-7 % faster, down 3 %, the
+// row-major op 2-6 %.  (With all eight loading on one schedule, both partners stall together: that form was 2 % ahead
+// of the four wavefronts on gate/up and behind them elsewhere.)
+using BigTile = TileShape<256, 256, 2, 4, 4>;
 // The small tile, for problems with too few large tiles to fill the chip: two workgroups per CU, each eight
 // wavefronts as 4 x 2 (wave tile 32 x 64), four of them loading, like the large tile.  (Four wavefronts of 64 x 64
 // measure 6 % slower on a denoise step; timestamps inside that kernel put 254 ns on a K step whose 8 MFMAs per
@@ -93,10 +92,10 @@ using BigTile8 = TileShape<256, 256, 2, 4, 4>;
 using SmallTile = TileShape<128, 128, 4, 2, 4>;
 // the same eight wavefronts as 4 x 2: wave tile 64 x 128, for the epilogue that needs a wavefront to hold whole
 // 128-column heads (the rotation partner of a channel is 64 columns away)
-using BigTile8Q = TileShape<256, 256, 4, 2, 4>;
+using BigTileQ = TileShape<256, 256, 4, 2, 4>;
 // The large tile of a launch.
 template <int MODE>
-using BigTileFor = std::conditional_t<MODE == 3 || MODE == 4 /* kQkvRope, kQkvRopeFull */, BigTile8Q, BigTile8>;
+using BigTileFor = std::conditional_t<MODE == 3 || MODE == 4 /* kQkvRope, kQkvRopeFull */, BigTileQ, BigTile>;
 // the shape that runs the ragged last round of a launch (see tail_split_point): BigTile cut in four.  (Cut in two,
 // 256 x 128 with one workgroup per CU, measures the same.)
 using TailTile = SmallTile;
@@ -377,7 +376,11 @@ __device__ __forceinline__ void dual_gemm_body(const Params& p, const int wg, co
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform: keeps descriptors and LDS bases scalar
   const int wm = wave / kWavesN, wn = wave % kWavesN;
-  const int l32 = lane & 31, lhi = lane >> 5;
+  // MFMA fragment: row (column) l16, 16-byte K chunk lq of the step's four.  Any order of the chunks over the four lane
+  // groups will do as long as both operands use it; in this one a ds_read_b128 of 16 swizzled rows, which is served 16
+  // lanes at a time -- 0-3, 12-15, 20-27, then 4-11, 16-19, 28-31, and the same above -- touches every bank once each
+  // time (in the plain order 0, 1, 2, 3 every read takes twice as long).
+  const int l16 = lane & 15, lq = (0x9c >> (2 * (lane >> 4))) & 3;  // 0, 3, 1, 2
   // With more wavefronts than SIMDs only the first kLoadWaves (one per SIMD) issue the global -> LDS loads.  A
   // wavefront that issues a load is held while the CU's load path takes the instruction in; its partner on the same
   // SIMD, which issues none, keeps the MFMA pipe fed meanwhile.  When both partners load on the same schedule they
@@ -464,15 +467,13 @@ __device__ __forceinline__ void dual_gemm_body(const Params& p, const int wg, co
   // Instruction i of this wave covers rows [wave*64 + 16i, +16) of A.  Chunk c of row r lives in slot c ^ ((r >> 2) & 3).
   const int ld_row0 = wave * kLoadRowsA + (lane >> 2);
   const int ld_chunk = (lane & 3) ^ ((lane >> 4) & 3);
-  // fragment reads: row = base + l32, chunk kc = 2*kk + lhi
-  const int sw = (l32 >> 2) & 3;
-  int frag_off[2];
-#pragma unroll
-  for (int kk = 0; kk < 2; ++kk) frag_off[kk] = ((2 * kk + lhi) ^ sw) << 4;
-  const int a_row_off = (wm * (FM * 32) + l32) * kRowBytes;
+  // fragment reads: row = base + l16, K chunk lq; 16 rows x 64 bytes, i.e. one whole KiB per read
+  const int sw = (l16 >> 2) & 3;
+  const int frag_off = (lq ^ sw) << 4;
+  const int a_row_off = (wm * (FM * 16) + l16) * kRowBytes + frag_off;
   // paired slots: row r of a step's half sits at block r / 8 (1 KiB each), row r % 8 inside it
-  const int pair_lane_off = ((l32 >> 3) << 10) + ((l32 & 7) << 6);
-  const int a_pair_off = wm * (FM * 32) * 128 + pair_lane_off;
+  const int pair_lane_off = ((l16 >> 3) << 10) + ((l16 & 7) << 6) + frag_off;
+  const int a_pair_off = wm * (FM * 16) * 128 + pair_lane_off;
   // paired loader: lane -> (row lane / 4 % 8 of the instruction's 8 rows, step half lane / 32, slot lane % 4)
   constexpr int kPairLoadsA = kLoadRowsA / 8, kPairLoadsB = kLoadRowsB / 8;
   const int pl_row = (lane >> 2) & 7, pl_half = lane >> 5, pl_slot = lane & 3;
@@ -485,31 +486,46 @@ __device__ __forceinline__ void dual_gemm_body(const Params& p, const int wg, co
   // B fragment j of this wave starts at LDS row b_row(j): plain tiles hold 256 weight rows; SwiGLU tiles hold 128
   // gate rows then the 128 up rows of the same output columns, and fragments [0, FN/2) are gate, [FN/2, FN) up
   auto b_row = [&](int j) {
-    if constexpr (SWIGLU) return (j < FN / 2 ? 0 : BN / 2) + wn * (FN / 2 * 32) + (j % (FN / 2)) * 32;
-    else return wn * (FN * 32) + j * 32;
+    if constexpr (SWIGLU) return (j < FN / 2 ? 0 : BN / 2) + wn * (FN / 2 * 16) + (j % (FN / 2)) * 16;
+    else return wn * (FN * 16) + j * 16;
   };
-  const int b_lane_off = l32 * kRowBytes;
-  // K-major operand (KA / KB): a slot holds BK rows of K, each a run of BM (BN) columns, as whole 16-byte chunks;
-  // the 64-byte segment s of row k sits at segment position s ^ (k & 3), so that the four rows one transposing
-  // read touches fall into different banks.  ds_read_b64_tr_b16 works on groups of 16 lanes: lane j of a group
-  // supplies the address of 4 consecutive columns of row (j >> 2), and receives column j of the 4 rows.  A group
-  // covers 16 columns; the two groups of a half-wave cover a 32-column block, the half-waves rows k and k + 8.
-  const int tr_j = lane & 15, tr_grp = (lane >> 4) & 1;
-  const int tr_in = (2 * tr_grp + ((tr_j >> 1) & 1)) * 16 + 8 * (tr_j & 1);  // bytes inside the 64-byte segment
-  auto tr_lane_base = [&](int row_bytes, int first_block) {  // first_block: this wave's first 32-column block
-    return (8 * lhi + (tr_j >> 2)) * row_bytes + ((first_block ^ (tr_j >> 2)) << 6) + tr_in;
+  const int b_lane_off = l16 * kRowBytes + frag_off;
+  // K-major operand (KA / KB): a slot holds BK rows of K, each a run of BM (BN) columns, as whole 16-byte chunks.
+  // ds_read_b64_tr_b16 works on groups of 16 lanes: lane j of a group supplies the address of 4 consecutive columns of
+  // row (j >> 2), and receives column j of the 4 rows.  A group covers one 16-column block (32 bytes of a row); group
+  // lq takes K rows [8 lq, +8) in two reads of four.  The 32-byte unit u of row k sits at position
+  // u ^ (2 (k & 3)) ^ ((k >> 3) & 1): the four rows of one group and the two groups that are served together (rows
+  // 8 apart) fall into different banks.
+  const int tr_row = l16 >> 2;
+  auto tr_lane_base = [&](int row_bytes, int first_block) {  // first_block: this wave's first 16-column block
+    return (8 * lq + tr_row) * row_bytes + ((first_block ^ (2 * tr_row) ^ (lq & 1)) << 5) + (l16 & 3) * 8;
   };
   const int tr_base_a = KA ? tr_lane_base(BM * 2, wm * FM) : 0;
   const int tr_base_b = KB ? tr_lane_base(BN * 2, wn * FN) : 0;
 
+  // K-major loads: a loading wavefront fills K rows [8 wave, +8) of the slot, instruction i rows [kRows i, +kRows) of
+  // those (kRows = 1024 / row bytes).  The 16-byte LDS position lane is chunk lane % chunks of row lane / chunks, which
+  // takes the matrix chunk whose 32-byte unit index is XORed as described at tr_lane_base.  Columns past the matrix
+  // edge read whatever follows (the next row, or zero past the end): they only reach output rows / columns that are
+  // never stored.  Rows past K are out of the descriptor's range and read as zero.  (The offset is worked out at each
+  // use -- `step` keeps it from being held in registers across the loop, which has none to spare.)
+  static_assert((!KA || kLoadsA * 1024 == 8 * BM * 2) && (!KB || kLoadsB * 1024 == 8 * BN * 2), "8 rows of K per wave");
+  auto k_major_voff = [&](int i, int cols, uint32_t row_bytes, int step) {
+    int l = lane;
+    asm("" : "+v"(l) : "s"(step));
+    const int chunks = cols / 8, rows = 1024 / (cols * 2);
+    const int row = l / chunks, chunk = (l % chunks) ^ (row << 2) ^ (((rows * i) & 3) << 2) ^ ((wave & 1) << 1);
+    return __umul24(row, row_bytes) + static_cast<uint32_t>(chunk) * 16u + static_cast<uint32_t>(8 * wave + rows * i) * row_bytes;
+  };
   // ---- per-tile state ------------------------------------------------------------------------------
   struct Loader {   // where this wave's kLoadsA + kLoadsB loads per K step come from
     const __bf16 *a_base, *b_base;
     uint32_t a_bytes, b_bytes;        // readable bytes from the base (row-major) / from the current block (tiled)
     uint32_t voff_a[kPA ? 2 : kLoadsA], voff_b[kPB ? 2 : kLoadsB];  // paired slots: [even i, odd i] of instruction 0
-    uint32_t pitch8_a, pitch8_b;      // paired slots: bytes between the rows of consecutive load instructions
-    int64_t a_step, b_step;           // tiled: bytes between consecutive K steps
-    // tiled: the load stream walks a tile's K steps in order, so the step's base and the bytes readable from it are
+    uint32_t pitch_a, pitch_b;        // paired slots: bytes between the rows of consecutive load instructions; K-major:
+                                      // bytes of a row
+    int64_t a_step, b_step;           // tiled, K-major: bytes between consecutive K steps
+    // tiled, K-major: the load stream walks a tile's K steps in order, so the step's base and the bytes readable from it are
     // kept as running values (one add and one saturating subtract per step) instead of products with the step index
     const char *a_cur, *b_cur;
     uint32_t a_left, b_left, a_dec, b_dec;
@@ -613,24 +629,15 @@ __device__ __forceinline__ void dual_gemm_body(const Params& p, const int wg, co
       const int rows_a = G.m - row0 < BM ? G.m - row0 : BM;
       const int rows_b = G.n - col0 < kTileN ? G.n - col0 : kTileN;
       L.a_step = L.b_step = 0;
-      // K-major operand: load instruction q of the slot (1 KiB of LDS) holds 1024 / row_bytes rows of K; the lane's
-      // 16-byte LDS position p = 64 q + lane is chunk p % chunks of row p / chunks, which takes the matrix chunk
-      // whose 64-byte segment index is XORed with (row & 3).  Columns past the matrix edge read whatever follows
-      // (the next row, or zero past the end): they only reach output rows / columns that are never stored.
-      // Rows past K are out of the descriptor's range and read as zero.
-      auto k_major_voff = [&](int q, int chunks, int ld) {
-        const int pos = 64 * q + lane;
-        const int krow = pos / chunks, c = pos % chunks;
-        const int src_chunk = ((((c >> 2) ^ (krow & 3)) << 2) | (c & 3));
-        return static_cast<uint32_t>(krow) * static_cast<uint32_t>(ld) * 2u + static_cast<uint32_t>(src_chunk) * 16u;
-      };
       if constexpr (KA) {
         L.a_base = G.a + row0;
         const int64_t left = (static_cast<int64_t>(G.k) * G.lda - row0) * 2;
         L.a_bytes = static_cast<uint32_t>(left < 0 ? 0 : left);
-        L.a_step = static_cast<int64_t>(G.lda) * 2;  // bytes per K row
-#pragma unroll
-        for (int i = 0; i < kLoadsA; ++i) L.voff_a[i] = k_major_voff(wave * kLoadsA + i, BM / 8, G.lda);
+        L.a_step = static_cast<int64_t>(G.lda) * (2 * BK);
+        L.a_cur = reinterpret_cast<const char*>(L.a_base);
+        L.a_left = L.a_bytes;
+        L.a_dec = static_cast<uint32_t>(L.a_step);
+        L.pitch_a = 2u * static_cast<uint32_t>(G.lda);
       } else {
         L.a_base = G.a + static_cast<int64_t>(row0) * G.lda;
         L.a_bytes = static_cast<uint32_t>(rows_a) * G.lda * 2u;
@@ -638,7 +645,7 @@ __device__ __forceinline__ void dual_gemm_body(const Params& p, const int wg, co
           const uint32_t row_off = static_cast<uint32_t>(wave * kLoadRowsA + pl_row) * G.lda * 2u;
           L.voff_a[0] = row_off + pair_chunk_even * 16u;
           L.voff_a[1] = row_off + pair_chunk_odd * 16u;
-          L.pitch8_a = 16u * static_cast<uint32_t>(G.lda);
+          L.pitch_a = 16u * static_cast<uint32_t>(G.lda);
         } else {
 #pragma unroll
           for (int i = 0; i < kLoadsA; ++i) L.voff_a[i] = static_cast<uint32_t>(ld_row0 + 16 * i) * G.lda * 2u + ld_chunk * 16u;
@@ -648,9 +655,11 @@ __device__ __forceinline__ void dual_gemm_body(const Params& p, const int wg, co
         L.b_base = b_src + col0;
         const int64_t left = (static_cast<int64_t>(G.k) * G.ldb - col0) * 2;
         L.b_bytes = static_cast<uint32_t>(left < 0 ? 0 : left);
-        L.b_step = static_cast<int64_t>(G.ldb) * 2;
-#pragma unroll
-        for (int i = 0; i < kLoadsB; ++i) L.voff_b[i] = k_major_voff(b_wave * kLoadsB + i, BN / 8, G.ldb);
+        L.b_step = static_cast<int64_t>(G.ldb) * (2 * BK);
+        L.b_cur = reinterpret_cast<const char*>(L.b_base);
+        L.b_left = L.b_bytes;
+        L.b_dec = static_cast<uint32_t>(L.b_step);
+        L.pitch_b = 2u * static_cast<uint32_t>(G.ldb);
       } else {
         L.b_base = b_src + static_cast<int64_t>(col0) * G.ldb;
         L.b_bytes = static_cast<uint32_t>(rows_b) * G.ldb * 2u;
@@ -658,7 +667,7 @@ __device__ __forceinline__ void dual_gemm_body(const Params& p, const int wg, co
           const uint32_t row_off = static_cast<uint32_t>(b_wave * kLoadRowsB + pl_row) * G.ldb * 2u;
           L.voff_b[0] = row_off + pair_chunk_even * 16u;
           L.voff_b[1] = row_off + pair_chunk_odd * 16u;
-          L.pitch8_b = 16u * static_cast<uint32_t>(G.ldb);
+          L.pitch_b = 16u * static_cast<uint32_t>(G.ldb);
         } else {
           const int b_ld_row0 = b_wave * kLoadRowsB + (lane >> 2);
 #pragma unroll
@@ -675,7 +684,7 @@ __device__ __forceinline__ void dual_gemm_body(const Params& p, const int wg, co
   struct Pending {
     __amdgpu_buffer_rsrc_t rb;
     uint32_t voff_b[kPB ? 2 : kLoadsB];
-    uint32_t pitch8_b;  // paired slots
+    uint32_t pitch_b;  // paired slots, K-major
   };
   // Paired slots: the loads of K steps ks and ks + 1 (ks even) of this wave's rows, A here and B through `Pending`.
   auto issue_pair_a = [&](Loader& L, int ks, unsigned char* pa, Pending& P) {
@@ -691,19 +700,19 @@ __device__ __forceinline__ void dual_gemm_body(const Params& p, const int wg, co
       P.rb = make_rsrc(L.b_base + k0, L.b_bytes > adv ? L.b_bytes - adv : 0u);
       P.voff_b[0] = L.voff_b[0] | oob_even;
       P.voff_b[1] = L.voff_b[1] | oob_odd;
-      P.pitch8_b = L.pitch8_b;
+      P.pitch_b = L.pitch_b;
     }
     const uint32_t va_even = L.voff_a[0] | oob_even, va_odd = L.voff_a[1] | oob_odd;
 #pragma unroll
     for (int i = 0; i < kPairLoadsA; ++i)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, LDS_PTR(pa + (wave * kPairLoadsA + i) * 1024), 16,
-                                               ((i & 1) ? va_odd : va_even) + static_cast<uint32_t>(i) * L.pitch8_a, 0, 0, 0);
+                                               ((i & 1) ? va_odd : va_even) + static_cast<uint32_t>(i) * L.pitch_a, 0, 0, 0);
   };
   auto issue_pair_b = [&](const Pending& P, unsigned char* pb) {
 #pragma unroll
     for (int i = 0; i < kPairLoadsB; ++i)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(P.rb, LDS_PTR(pb + (wave * kPairLoadsB + i) * 1024), 16,
-                                               P.voff_b[i & 1] + static_cast<uint32_t>(i) * P.pitch8_b, 0, 0, 0);
+                                               P.voff_b[i & 1] + static_cast<uint32_t>(i) * P.pitch_b, 0, 0, 0);
   };
   auto issue_a = [&](Loader& L, int ks, unsigned char* sa, Pending& P) {
     __amdgpu_buffer_rsrc_t ra;
@@ -731,37 +740,39 @@ __device__ __forceinline__ void dual_gemm_body(const Params& p, const int wg, co
       // A K-major operand advances by whole rows of K instead, and its rows past K are past the end by themselves.
       const uint32_t adv = 2u * static_cast<uint32_t>(k0);
       if constexpr (KA) {
-        const int64_t da = L.a_step * k0;
-        ra = make_rsrc(reinterpret_cast<const char*>(L.a_base) + da, L.a_bytes > da ? static_cast<uint32_t>(L.a_bytes - da) : 0u);
+        ra = make_rsrc(L.a_cur, L.a_left);
+        L.a_cur += L.a_step;
+        L.a_left = L.a_left > L.a_dec ? L.a_left - L.a_dec : 0u;
       } else {
         ra = make_rsrc(L.a_base + k0, L.a_bytes > adv ? L.a_bytes - adv : 0u);
       }
       if constexpr (KB) {
-        const int64_t db = L.b_step * k0;
-        P.rb = make_rsrc(reinterpret_cast<const char*>(L.b_base) + db, L.b_bytes > db ? static_cast<uint32_t>(L.b_bytes - db) : 0u);
+        P.rb = make_rsrc(L.b_cur, L.b_left);
+        L.b_cur += L.b_step;
+        L.b_left = L.b_left > L.b_dec ? L.b_left - L.b_dec : 0u;
+        P.pitch_b = L.pitch_b;
       } else {
         P.rb = make_rsrc(L.b_base + k0, L.b_bytes > adv ? L.b_bytes - adv : 0u);
       }
       const bool k_tail = k0 + BK > L.K;
       oob = (k_tail && k0 + ld_chunk * 8 >= L.K) ? 0x80000000u : 0u;
     }
-    const uint32_t oob_a = KA ? 0u : oob, oob_b = KB ? 0u : oob;
-    if constexpr (!kPB) {
+    if constexpr (!kPB && !KB) {
 #pragma unroll
-      for (int i = 0; i < kLoadsB; ++i) P.voff_b[i] = L.voff_b[i] | oob_b;
+      for (int i = 0; i < kLoadsB; ++i) P.voff_b[i] = L.voff_b[i] | oob;
     }
     if constexpr (!kPA) {  // (A in pairs: this call only prepares the step's B descriptor)
 #pragma unroll
       for (int i = 0; i < kLoadsA; ++i)
         __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, LDS_PTR(sa + (wave * kLoadRowsA + 16 * i) * kRowBytes), 16,
-                                                 L.voff_a[i] | oob_a, 0, 0, 0);
+                                                 KA ? k_major_voff(i, BM, L.pitch_a, ks) : L.voff_a[i] | oob, 0, 0, 0);
     }
   };
-  auto issue_b = [&](const Pending& P, unsigned char* sb) {
+  auto issue_b = [&](const Pending& P, unsigned char* sb, int step = 0) {
 #pragma unroll
     for (int i = 0; i < kLoadsB; ++i)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(P.rb, LDS_PTR(sb + (wave * kLoadRowsB + 16 * i) * kRowBytes), 16,
-                                               P.voff_b[i], 0, 0, 0);
+                                               KB ? k_major_voff(i, BN, P.pitch_b, step) : P.voff_b[i], 0, 0, 0);
   };
 
   // Fused launch, consumer: the B half of K step `s` of a tile that has not started yet (s < kStages), leaving the
@@ -855,155 +866,161 @@ __device__ __forceinline__ void dual_gemm_body(const Params& p, const int wg, co
   };
   int passed_before = 0;
 
-  f32x16 acc[FM][FN];
-  bf16x8 fa[2][FM], fb[2][FN];  // two fragment sets: one feeds the MFMAs while the other is being read from LDS
+  // A K step is one MFMA deep (16x16x32) and its FM x FN products go out in two halves around the step's barrier.
+  // The operand with more blocks is the one that is cut: its first half and all of the other operand are needed for the
+  // first half of the products, its second half only for the second.  So the cut operand has one register set (each
+  // half is refilled while the other half's products run) and the other one has two, by the step's parity.
+  // Why 16x16x32 and not 32x32x16 (the same operations per cycle): on normally distributed operands the chip holds a
+  // clock that depends on what the instructions switch, and back-to-back MFMAs reach 2.04 PFLOP/s in this shape
+  // against 1.81 in the other; 2.09 when each differs from the one before in one operand only (the serpentine below).
+  // 28160 + 1024 rows, before and after on one chip: gate/up 1.892 -> 1.757 ms (1.35 -> 1.45 PFLOP/s), down 0.950 ->
+  // 0.887 ms; the row-major op at 28160 x 11008 x 2048: forward 0.967 -> 0.900 ms, dX 0.967 -> 0.917, dW (half the
+  // tokens) 0.540 -> 0.511.  On all-zero operands, where the clock is the same for both shapes, neither is faster.
+  // The operands go in as (B, A), so a lane's four accumulator registers are four consecutive COLUMNS of one row of C:
+  // the epilogue packs them into 8 bytes without exchanging anything between lanes.
+  constexpr bool kCutA = FM >= FN;
+  constexpr int kFirstReads = (kCutA ? FM / 2 : FM) * (KA ? 2 : 1) + (kCutA ? FN : FN / 2) * (KB ? 2 : 1);
+  constexpr int kSecondReads = kCutA ? FM / 2 * (KA ? 2 : 1) : FN / 2 * (KB ? 2 : 1);
+  f32x4 acc[FM][FN];
+  bf16x8 fa[kCutA ? 1 : 2][FM], fb[kCutA ? 2 : 1][FN];
 
-  // Fragments are read in the order the MFMAs (A-major: all B blocks for A block 0, then A block 1, ...) first
-  // need them: A0, every B, then the other A blocks.
-  // K-major slot: K values [8 lhi, +8) of step half kk for the lane's column of 32-column block `blk` (counted
-  // from the wave's first block): two transposing reads of four rows each.
-  auto read_k_major = [&](const unsigned char* slot, int lane_base, int row_bytes, int blk, int kk) {
-    const unsigned char* at = slot + (lane_base ^ (blk << 6)) + 16 * kk * row_bytes;
+  // K-major slot: K values [8 lq, +8) for the lane's column of 16-column block `blk` (counted from the wave's first
+  // block): two transposing reads of four rows each.
+  // (`step` keeps the compiler from holding the FM + FN addresses in registers across the loop, which it does not have:
+  // one exclusive-or per read instead)
+  auto read_k_major = [&](const unsigned char* slot, int lane_base, int row_bytes, int blk, int step) {
+    asm("" : "+v"(lane_base) : "s"(step));
+    const unsigned char* at = slot + (lane_base ^ (blk << 5));
     const bf16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4bf16(LDS_TR_PTR(at));
     const bf16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4bf16(LDS_TR_PTR(at + 4 * row_bytes));
     return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
   };
-  auto read_a = [&](const unsigned char* sa, int i, int kk) {
-    if constexpr (KA) return read_k_major(sa, tr_base_a, BM * 2, i, kk);
-    else if constexpr (kPA) return *reinterpret_cast<const bf16x8*>(sa + a_pair_off + i * 32 * 128 + frag_off[kk]);
-    else return *reinterpret_cast<const bf16x8*>(sa + a_row_off + i * 32 * kRowBytes + frag_off[kk]);
+  auto read_a = [&](const unsigned char* sa, int i, int step) {
+    if constexpr (KA) return read_k_major(sa, tr_base_a, BM * 2, i, step);
+    else if constexpr (kPA) return *reinterpret_cast<const bf16x8*>(sa + a_pair_off + i * 16 * 128);
+    else return *reinterpret_cast<const bf16x8*>(sa + a_row_off + i * 16 * kRowBytes);
   };
-  auto read_b = [&](const unsigned char* sb, int j, int kk) {
-    if constexpr (KB) return read_k_major(sb, tr_base_b, BN * 2, j, kk);
-    else if constexpr (kPB) return *reinterpret_cast<const bf16x8*>(sb + b_row(j) * 128 + pair_lane_off + frag_off[kk]);
-    else return *reinterpret_cast<const bf16x8*>(sb + b_row(j) * kRowBytes + b_lane_off + frag_off[kk]);
+  auto read_b = [&](const unsigned char* sb, int j, int step) {
+    if constexpr (KB) return read_k_major(sb, tr_base_b, BN * 2, j, step);
+    else if constexpr (kPB) return *reinterpret_cast<const bf16x8*>(sb + b_row(j) * 128 + pair_lane_off);
+    else return *reinterpret_cast<const bf16x8*>(sb + b_row(j) * kRowBytes + b_lane_off);
   };
-  auto read_frags = [&](const unsigned char* sa, const unsigned char* sb, int kk, int set) {
-    fa[set][0] = read_a(sa, 0, kk);
+  // What the first half of the products of the step in slot (sa, sb), of parity `par`, needs, in first-use order ...
+  auto read_first = [&](const unsigned char* sa, const unsigned char* sb, int par, int step) {
+    if constexpr (kCutA) {
+      fa[0][0] = read_a(sa, 0, step);
 #pragma unroll
-    for (int j = 0; j < FN; ++j) fb[set][j] = read_b(sb, j, kk);
+      for (int j = 0; j < FN; ++j) fb[par][j] = read_b(sb, j, step);
 #pragma unroll
-    for (int i = 1; i < FM; ++i) fa[set][i] = read_a(sa, i, kk);
-  };
-  auto mma = [&](int set) {
+      for (int i = 1; i < FM / 2; ++i) fa[0][i] = read_a(sa, i, step);
+    } else {
+      fb[0][0] = read_b(sb, 0, step);
 #pragma unroll
-    for (int i = 0; i < FM; ++i)
+      for (int i = 0; i < FM; ++i) fa[par][i] = read_a(sa, i, step);
 #pragma unroll
-      for (int jj = 0; jj < FN; ++jj) {
-        const int j = jj;
-        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[set][i], fb[set][j], acc[i][j], 0, 0, 0);
-      }
-  };
-  // Scheduling hints.  Before the barrier: the LDS reads of the other fragment set and the B half of the previous
-  // slot's refill go out among the first half of this group's MFMAs; the second half covers the read latency, so
-  // the wait in front of the barrier finds the reads done.
-  auto schedule_before_barrier = [&](auto with_loads) {
-    constexpr int kB = decltype(with_loads)::value ? kLoadsB : 0;
-    constexpr int kMfma = FM * FN, kReads = FM * (KA ? 2 : 1) + FN * (KB ? 2 : 1);
-    constexpr int kCarry = kMfma / 2;                              // MFMAs that carry other instructions
-    constexpr int kReadsPer = (kReads + kCarry - 1) / kCarry;      // LDS reads per carrying MFMA
-    constexpr int kLoadEvery = kB > 0 && kCarry / kB > 0 ? kCarry / kB : 1;
-#pragma unroll
-    for (int m = 0; m < kCarry; ++m) {
-      __builtin_amdgcn_sched_group_barrier(0x100, kReadsPer, 0);
-      if (m % kLoadEvery == 0 && m / kLoadEvery < kB) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      for (int j = 1; j < FN / 2; ++j) fb[0][j] = read_b(sb, j, step);
     }
-    __builtin_amdgcn_sched_group_barrier(0x008, kMfma - kCarry, 0);
-    __builtin_amdgcn_sched_barrier(0);
   };
-  // After the barrier: the A half of the refill and the next slot's fragment reads are spread over the whole group.
-  auto schedule_after_barrier = [&](auto with_loads) {
-    constexpr int kA = decltype(with_loads)::value ? kLoadsA : 0;
-    constexpr int kMfma = FM * FN, kReads = FM * (KA ? 2 : 1) + FN * (KB ? 2 : 1);
-    constexpr int kReadEvery = kMfma / kReads > 0 ? kMfma / kReads : 1;
-    constexpr int kReadsPer = kReads * kReadEvery > kMfma ? (kReads + kMfma - 1) / kMfma : 1;
-    constexpr int kLoadEvery = kA > 0 && kMfma / kA > 0 ? kMfma / kA : 1;
+  // ... and the second half's rest
+  auto read_second = [&](const unsigned char* sa, const unsigned char* sb, int step) {
+    if constexpr (kCutA) {
+#pragma unroll
+      for (int i = FM / 2; i < FM; ++i) fa[0][i] = read_a(sa, i, step);
+    } else {
+#pragma unroll
+      for (int j = FN / 2; j < FN; ++j) fb[0][j] = read_b(sb, j, step);
+    }
+  };
+  auto mma = [&](int half, int par) {
+    if constexpr (kCutA) {
+#pragma unroll
+      for (int ii = 0; ii < FM / 2; ++ii)
+#pragma unroll
+        for (int jj = 0; jj < FN; ++jj) {
+          const int i = half * (FM / 2) + ii, j = (ii & 1) ? FN - 1 - jj : jj;
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[par][j], fa[0][i], acc[i][j], 0, 0, 0);
+        }
+    } else {
+#pragma unroll
+      for (int jj = 0; jj < FN / 2; ++jj)
+#pragma unroll
+        for (int ii = 0; ii < FM; ++ii) {
+          const int j = half * (FN / 2) + jj, i = (jj & 1) ? FM - 1 - ii : ii;
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[0][j], fa[par][i], acc[i][j], 0, 0, 0);
+        }
+    }
+  };
+  // Scheduling hints.  Before the barrier: the LDS reads of the step's second half and the B half of the previous
+  // slot's refill go out among the first MFMAs of this half; the rest of them cover the read latency, so the wait in
+  // front of the barrier finds the reads done.  After it: the loads of the refill are spread over the whole half, the
+  // next slot's fragment reads over three quarters of it.  (Other shares of the MFMAs, a quarter to all of them, measure
+  // within 1 % of these.)
+  auto schedule_half = [&](auto n_reads, auto n_loads, auto n_read_carry, auto n_carry) {
+    constexpr int kReads = decltype(n_reads)::value, kLoads = decltype(n_loads)::value;
+    constexpr int kMfma = FM * FN / 2, kReadCarry = decltype(n_read_carry)::value, kCarry = decltype(n_carry)::value;  // MFMAs that carry reads / loads
 #pragma unroll
     for (int m = 0; m < kMfma; ++m) {
-      if (m % kLoadEvery == 0 && m / kLoadEvery < kA) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
-      if (m % kReadEvery == 0 && m / kReadEvery * kReadsPer < kReads) __builtin_amdgcn_sched_group_barrier(0x100, kReadsPer, 0);
+      // the m-th MFMA is preceded by an even share of the reads and of the loads
+      const int reads = m < kReadCarry ? (m + 1) * kReads / kReadCarry - m * kReads / kReadCarry : 0;
+      const int loads = m < kCarry ? (m + 1) * kLoads / kCarry - m * kLoads / kCarry : 0;
+#pragma unroll
+      for (int q = 0; q < reads; ++q) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+#pragma unroll
+      for (int q = 0; q < loads; ++q) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
       __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
     }
     __builtin_amdgcn_sched_barrier(0);
   };
+  constexpr int kHalfMfma = FM * FN / 2;
+  auto schedule_before = [&](auto n_loads) {
+    schedule_half(std::integral_constant<int, kSecondReads>{}, n_loads, std::integral_constant<int, kHalfMfma / 2>{}, std::integral_constant<int, kHalfMfma / 2>{});
+  };
+  auto schedule_after = [&](auto n_loads) {
+    schedule_half(std::integral_constant<int, kFirstReads>{}, n_loads, std::integral_constant<int, kHalfMfma * 3 / 4>{}, std::integral_constant<int, kHalfMfma>{});
+  };
 
-  // One K step on slot (sa, sb); (sa_n, sb_n) is the next slot of the ring and sb_p the previous one.  On entry
-  // fragment set 0 holds kk = 0 of this slot.  After the barrier every wave has finished reading this slot, so its
-  // refill with the K step kStages ahead in the load stream (step `ld_ks` of tile `L`) starts at once: the A half
-  // here, the B half in the next step's first group.  The next slot's data was issued kStages - 1 steps ago.
+  // One K step on slot S of the ring (step S of a ring round).  On entry the registers hold what the first half of its
+  // products needs.  After the barrier every wave has finished reading this slot, so its refill with the K step kStages
+  // ahead in the load stream (step `ld_ks` + S of tile `L`) starts at once: the A half here, the B half in the next
+  // step's first half.  The next slot's data was issued kStages - 1 steps ago.
   // A wavefront that does not load runs the same step without the load instructions (and its counted wait passes
   // at once: it has no loads in flight).
   Pending pend;
-  auto k_step_as = [&](auto with_loads, Loader& L, int ld_ks, unsigned char* sa, unsigned char* sb, unsigned char* sa_n,
-                       unsigned char* sb_n, unsigned char* sb_p) {
+  auto k_step_as = [&](auto with_loads, auto step_c, Loader& L, int ld_ks) {
     constexpr bool LD = decltype(with_loads)::value;
-    read_frags(sa, sb, 1, 1);
-    if constexpr (LD) issue_b(pend, sb_p);
-    mma(0);
-    schedule_before_barrier(with_loads);
+    constexpr int S = decltype(step_c)::value;
+    read_second(slot_a(S), slot_b(S), ld_ks);
+    if constexpr (LD) issue_b(pend, slot_b((S + kStages - 1) % kStages), ld_ks);
+    mma(0, S & 1);
+    schedule_before(std::integral_constant<int, LD ? kLoadsB : 0>{});
     // my LDS reads have returned; of my loads at most the kStages - 2 youngest K steps' worth are still in flight,
     // i.e. the next slot is complete
     __builtin_amdgcn_s_waitcnt(waitcnt_imm(LD ? (kStages - 2) * kLoadsPerStep : 63, 0));
     barrier_no_fence();
-    if constexpr (LD) issue_a(L, ld_ks, sa, pend);
-    read_frags(sa_n, sb_n, 0, 0);
-    mma(1);
-    schedule_after_barrier(with_loads);
+    if constexpr (LD) issue_a(L, ld_ks + S, slot_a(S), pend);
+    read_first(slot_a((S + 1) % kStages), slot_b((S + 1) % kStages), (S + 1) & 1, ld_ks);
+    mma(1, S & 1);
+    schedule_after(std::integral_constant<int, LD ? kLoadsA : 0>{});
   };
-  // The same step on paired slots (step S of a ring round; slots 0, 1 are pair 0, slots 2, 3 pair 1).  A pair is
+  // The same step on paired slots (slots 0, 1 are pair 0, slots 2, 3 pair 1).  A pair is
   // free once its odd slot has been read, i.e. after the barrier of steps 1 and 3: its A refill (the K steps one ring
   // round ahead) goes out there, its B refill at the start of the following step, and everything must have landed
   // by the barrier two steps on, which is the only load still in flight then -- the counted wait becomes vmcnt(0) on
   // odd steps and none on even ones.
-  auto schedule_pair = [&](auto n_before, auto n_after) {
-    constexpr int kB = decltype(n_before)::value, kA = decltype(n_after)::value;
-    constexpr int kMfma = FM * FN, kReads = FM + FN;
-    (void)kA;
-    constexpr int kCarry = kMfma / 2;
-    constexpr int kReadsPer = (kReads + kCarry - 1) / kCarry;
-    constexpr int kBd = kB > 0 ? kB : 1;
-    constexpr int kLoadEvery = kCarry / kBd > 0 ? kCarry / kBd : 1;
-    constexpr int kLoadsPer = kB > kCarry ? (kB + kCarry - 1) / kCarry : 1;
-#pragma unroll
-    for (int m = 0; m < kCarry; ++m) {
-      __builtin_amdgcn_sched_group_barrier(0x100, kReadsPer, 0);
-      if (kB > 0 && m % kLoadEvery == 0 && m / kLoadEvery * kLoadsPer < kB) __builtin_amdgcn_sched_group_barrier(0x020, kLoadsPer, 0);
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-    }
-    __builtin_amdgcn_sched_group_barrier(0x008, kMfma - kCarry, 0);
-    __builtin_amdgcn_sched_barrier(0);
-  };
-  auto schedule_pair_after = [&](auto n_after) {
-    constexpr int kA = decltype(n_after)::value;
-    constexpr int kMfma = FM * FN, kReads = FM * (KA ? 2 : 1) + FN * (KB ? 2 : 1);
-    constexpr int kReadEvery = kMfma / kReads > 0 ? kMfma / kReads : 1;
-    constexpr int kReadsPer = kReads * kReadEvery > kMfma ? (kReads + kMfma - 1) / kMfma : 1;
-    constexpr int kAd = kA > 0 ? kA : 1;
-    constexpr int kLoadEvery = kMfma / kAd > 0 ? kMfma / kAd : 1;
-    constexpr int kLoadsPer = kA > kMfma ? (kA + kMfma - 1) / kMfma : 1;
-#pragma unroll
-    for (int m = 0; m < kMfma; ++m) {
-      if (kA > 0 && m % kLoadEvery == 0 && m / kLoadEvery * kLoadsPer < kA) __builtin_amdgcn_sched_group_barrier(0x020, kLoadsPer, 0);
-      if (m % kReadEvery == 0 && m / kReadEvery * kReadsPer < kReads) __builtin_amdgcn_sched_group_barrier(0x100, kReadsPer, 0);
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-    }
-    __builtin_amdgcn_sched_barrier(0);
-  };
   auto k_step_pair = [&](auto with_loads, auto step_c, Loader& L, int ld_ks) {
     constexpr bool LD = decltype(with_loads)::value;
     constexpr int S = decltype(step_c)::value;
     constexpr bool kOdd = (S & 1) != 0;
-    read_frags(slot_a(S), slot_b(S), 1, 1);
+    read_second(slot_a(S), slot_b(S), ld_ks);
     if constexpr (LD && !kOdd) issue_pair_b(pend, S == 0 ? s_pb1 : s_pb0);
-    mma(0);
-    schedule_pair(std::integral_constant<int, (LD && !kOdd) ? kPairLoadsB : 0>{}, std::integral_constant<int, 0>{});
+    mma(0, S & 1);
+    schedule_before(std::integral_constant<int, (LD && !kOdd) ? kPairLoadsB : 0>{});
     __builtin_amdgcn_s_waitcnt(waitcnt_imm((LD && kOdd) ? 0 : 63, 0));
     barrier_no_fence();
     if constexpr (LD && kOdd) issue_pair_a(L, ld_ks + (S == 1 ? 0 : 2), S == 1 ? s_pa0 : s_pa1, pend);
-    read_frags(slot_a((S + 1) % kStages), slot_b((S + 1) % kStages), 0, 0);
-    mma(1);
-    schedule_pair_after(std::integral_constant<int, (LD && kOdd) ? kPairLoadsA : 0>{});
+    read_first(slot_a((S + 1) % kStages), slot_b((S + 1) % kStages), (S + 1) & 1, ld_ks);
+    mma(1, S & 1);
+    schedule_after(std::integral_constant<int, (LD && kOdd) ? kPairLoadsA : 0>{});
   };
   // ... and with A alone in pairs (NN).  B keeps the slot-by-slot schedule of k_step_as (the refill of slot S - 1 at
   // the start of step S, its descriptor prepared after the barrier of step S - 1), A the pairs' (after the barrier of
@@ -1013,37 +1030,89 @@ __device__ __forceinline__ void dual_gemm_body(const Params& p, const int wg, co
     constexpr bool LD = decltype(with_loads)::value;
     constexpr int S = decltype(step_c)::value;
     constexpr bool kOdd = (S & 1) != 0;
-    read_frags(slot_a(S), slot_b(S), 1, 1);
-    if constexpr (LD) issue_b(pend, slot_b((S + kStages - 1) % kStages));
-    mma(0);
-    schedule_before_barrier(with_loads);
+    read_second(slot_a(S), slot_b(S), ld_ks);
+    if constexpr (LD) issue_b(pend, slot_b((S + kStages - 1) % kStages), ld_ks);
+    mma(0, S & 1);
+    schedule_before(std::integral_constant<int, LD ? kLoadsB : 0>{});
     __builtin_amdgcn_s_waitcnt(waitcnt_imm(LD ? (kOdd ? 2 * kLoadsB : 2 * kLoadsB + kPairLoadsA) : 63, 0));
     barrier_no_fence();
     if constexpr (LD) {
       issue_a(L, ld_ks + S, nullptr, pend);
       if constexpr (kOdd) issue_pair_a(L, ld_ks + S - 1, S == 1 ? s_pa0 : s_pa1, pend);
     }
-    read_frags(slot_a((S + 1) % kStages), slot_b((S + 1) % kStages), 0, 0);
-    mma(1);
-    schedule_pair_after(std::integral_constant<int, (LD && kOdd) ? kPairLoadsA : 0>{});
+    read_first(slot_a((S + 1) % kStages), slot_b((S + 1) % kStages), (S + 1) & 1, ld_ks);
+    mma(1, S & 1);
+    schedule_after(std::integral_constant<int, (LD && kOdd) ? kPairLoadsA : 0>{});
   };
   // ---- epilogue ------------------------------------------------------------------------------------------
-  // Accumulator register r of lane l holds row 8*(r/4) + 4*(l/32) + r%4, column l%32 of its 32x32 block.  Values
-  // are rounded to bf16, paired with the neighbouring column through a lane swap (even lanes keep the even
-  // register's row, odd lanes the odd register's row), written to this wave's staging area as dwords, and read
-  // back as 16-byte lanes laid out the way the destination wants them.
+  // Lane l of a 16x16 block holds row l % 16, columns 4 (l / 16) .. + 3.  Values are rounded to bf16, written to this
+  // wave's staging area 8 bytes at a time, and read back as 16-byte lanes laid out the way the destination wants them.
   unsigned char* stage = s_out + wave * kStageBytes;
-  // Stores register pair (r, r+1) of one 32x32 block -- rows srow and srow + 1, column scol of this lane -- into
-  // the staging area with row pitch `pitch` bytes.
-  auto stage_pair = [&](float v0, float v1, int srow, int scol, int pitch, int odd) {
-    // both values are converted at once (low half v0, high half v1) and the pair is swapped with the neighbour;
-    // even lane keeps (own v0, neighbour's v0) -> row srow; odd lane (neighbour's v1, own v1) -> row srow + 1.
-    // One byte permute picks the two halves: selector bytes 0-3 address `theirs`, 4-7 address `mine`.
-    const uint32_t mine = pack_bf16x2(v0, v1);
-    const uint32_t theirs = static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(mine), 0xB1, 0xF, 0xF, true));
-    const uint32_t sel = odd ? 0x07060302u : 0x01000504u;
-    const uint32_t packed = __builtin_amdgcn_perm(mine, theirs, sel);
-    *reinterpret_cast<uint32_t*>(stage + (srow + odd) * pitch + (scol & ~1) * 2) = packed;
+
+  // The row-major half of the epilogue.  `with_res`: the addend's form is one of its own, chosen once per tile -- with a
+  // test at each of the addend's loads and uses the compiler sees the loads still in flight on paths around their use
+  // and makes every wavefront wait for ALL of its loads at the head of the K loop, once per ring round.
+  auto store_rows = [&](const Store& S, const int lane_e, auto with_res) {
+    constexpr bool RES = decltype(with_res)::value;
+    const int e16 = lane_e & 15, eq = lane_e >> 4;
+    // wave output: FM row blocks of 16 rows x kOutCols columns, row-major, staged one row block at a time.  Row r of
+    // the staging area keeps 16-byte chunk c in slot c ^ swz(r): both the 8-byte writes (16 rows x one chunk) and the
+    // 16-byte reads (whole rows) then touch every bank once.
+    constexpr int kOutCols = FN * 16;
+    constexpr int kPitch = kOutCols * 2;
+    static_assert(kStageBytes == 16 * kPitch && (kPitch == 128 || kPitch == 256), "staging holds one row block");
+    constexpr int kLanesPerRow = kPitch / 16, kRowsPerStore = 64 / kLanesPerRow, kStores = 16 / kRowsPerStore;
+    auto swz = [](int r) { return kPitch == 128 ? (r >> 1) & 7 : r & 15; };
+    // a row is kPitch bytes = kLanesPerRow lanes; one store instruction writes kRowsPerStore rows
+    const int rl = lane_e / kLanesPerRow, cc = lane_e % kLanesPerRow;
+    const int col = wn * kOutCols + cc * 8;
+#pragma unroll
+    for (int i = 0; i < FM; ++i) {
+      int out_row[kStores];
+      u32x4 resv[kStores];
+#pragma unroll
+      for (int q = 0; q < kStores; ++q) {
+        const int row = (wm * FM + i) * 16 + q * kRowsPerStore + rl;
+        out_row[q] = row;
+        if constexpr (MODE == kDown) {
+          // scatter: the row ids of the round (and the residual's chunks) are fetched together, ahead of the
+          // staging writes and reads
+          if (S.row_id != nullptr && row < S.rows) out_row[q] = S.row_id[row];
+        }
+      }
+      if constexpr (RES) {
+#pragma unroll
+        for (int q = 0; q < kStores; ++q) {
+          const int row = (wm * FM + i) * 16 + q * kRowsPerStore + rl;
+          resv[q] = u32x4{0u, 0u, 0u, 0u};
+          if (row < S.rows && col < S.cols_left)
+            resv[q] = *reinterpret_cast<const u32x4*>(S.res + static_cast<int64_t>(out_row[q]) * S.ldc + col);
+        }
+      }
+#pragma unroll
+      for (int j = 0; j < FN; ++j)
+        *reinterpret_cast<u32x2*>(stage + e16 * kPitch + (((2 * j + (eq >> 1)) ^ swz(e16)) << 4) + (eq & 1) * 8) =
+            u32x2{pack_bf16x2(acc[i][j][0], acc[i][j][1]), pack_bf16x2(acc[i][j][2], acc[i][j][3])};
+      __builtin_amdgcn_s_waitcnt(waitcnt_imm(63, 0));
+#pragma unroll
+      for (int q = 0; q < kStores; ++q) {
+        const int srow = q * kRowsPerStore + rl;
+        u32x4 v = *reinterpret_cast<const u32x4*>(stage + srow * kPitch + ((cc ^ swz(srow)) << 4));
+        const int row = (wm * FM + i) * 16 + srow;
+        if constexpr (RES) {  // bf16(y) + bf16(residual), summed in fp32 and rounded once, like the eager add
+#pragma unroll
+          for (int w = 0; w < 4; ++w) {
+            const float lo = __builtin_bit_cast(float, v[w] << 16) + __builtin_bit_cast(float, resv[q][w] << 16);
+            const float hi = __builtin_bit_cast(float, v[w] & 0xFFFF0000u) +
+                             __builtin_bit_cast(float, resv[q][w] & 0xFFFF0000u);
+            v[w] = pack_bf16x2(lo, hi);
+          }
+        }
+        if (row < S.rows && col < S.cols_left)
+          *reinterpret_cast<u32x4*>(S.c_base + static_cast<int64_t>(out_row[q]) * S.ldc + col) = v;
+      }
+      __builtin_amdgcn_s_waitcnt(waitcnt_imm(63, 0));
+    }
   };
 
   auto epilogue = [&](const Store& S) {
@@ -1051,61 +1120,55 @@ __device__ __forceinline__ void dual_gemm_body(const Params& p, const int wg, co
     // of being hoisted out of the persistent loop and held in registers across the K loop.
     int lane_e = lane;
     asm volatile("" : "+v"(lane_e));
-    const int el32 = lane_e & 31, elhi = lane_e >> 5, odd = lane_e & 1;
+    const int e16 = lane_e & 15, eq = lane_e >> 4;
     if constexpr (SWIGLU) {
-      // wave output: 128 rows x kOutCols intermediate columns, staged kRound rows at a time
-      constexpr int kOutCols = FN / 2 * 32;
-      constexpr int kPitch = kOutCols * 2;
-      constexpr int kRound = kStageBytes / kPitch;  // rows per round (64 / 32)
-      constexpr int kIPerRound = kRound / 32;       // 32-row accumulator blocks per round
-      static_assert(kIPerRound >= 1 && FM % kIPerRound == 0, "staging holds whole accumulator blocks");
+      // wave output: FM row blocks x kColBlocks column blocks of the tiled intermediate (16 x 32, 1 KiB each).  The
+      // staging area holds blocks in their final layout (16-byte chunk c of row r in slot c ^ ((r >> 2) & 3)), so a
+      // block is read back and stored as it lies; kRound row blocks go through it at a time.
+      constexpr int kColBlocks = FN / 4;
+      constexpr int kRound = kStageBytes / (kColBlocks * kBlkBytes);
+      static_assert(FN % 4 == 0 && kRound >= 1 && FM % kRound == 0, "staging holds whole rounds of blocks");
       // what == 0: the intermediate h; 1 / 2: the gate / up projections themselves, when the caller keeps them
       const int n_what = p.keep_gate != nullptr ? 3 : 1;
       const int64_t keep_off[3] = {0, reinterpret_cast<unsigned char*>(p.keep_gate) - reinterpret_cast<unsigned char*>(p.g[0].c),
                                    reinterpret_cast<unsigned char*>(p.keep_up) - reinterpret_cast<unsigned char*>(p.g[0].c)};
 #pragma unroll
-      for (int round = 0; round < FM / kIPerRound; ++round) {
+      for (int round = 0; round < FM / kRound; ++round) {
         for (int what = 0; what < n_what; ++what) {
 #pragma unroll
-          for (int ii = 0; ii < kIPerRound; ++ii) {
-            const int i = round * kIPerRound + ii;
+          for (int ii = 0; ii < kRound; ++ii) {
+            const int i = round * kRound + ii;
 #pragma unroll
             for (int j = 0; j < FN / 2; ++j) {
+              float h[4];
 #pragma unroll
-              for (int r = 0; r < 16; r += 2) {
-                float h[2];
-#pragma unroll
-                for (int q = 0; q < 2; ++q) {
-                  // eager bf16 evaluation of act_fn(gate) * up (act.py:80-82): gate, up, silu(gate) and the
-                  // product are each rounded to bf16
-                  const uint32_t gu = pack_bf16x2(acc[i][j][r + q], acc[i][j + FN / 2][r + q]);  // one convert for both
-                  const float g = __uint_as_float(gu << 16);
-                  const float u = __uint_as_float(gu & 0xffff0000u);
-                  if (what == 0) {
-                    const float sg = round_bf16(g * __builtin_amdgcn_rcpf(1.0f + __expf(-g)));
-                    h[q] = sg * u;
-                  } else {
-                    h[q] = what == 1 ? g : u;
-                  }
+              for (int r = 0; r < 4; ++r) {
+                // eager bf16 evaluation of act_fn(gate) * up (act.py:80-82): gate, up, silu(gate) and the
+                // product are each rounded to bf16
+                const uint32_t gu = pack_bf16x2(acc[i][j][r], acc[i][j + FN / 2][r]);  // one convert for both
+                const float g = __uint_as_float(gu << 16);
+                const float u = __uint_as_float(gu & 0xffff0000u);
+                if (what == 0) {
+                  const float sg = round_bf16(g * __builtin_amdgcn_rcpf(1.0f + __expf(-g)));
+                  h[r] = sg * u;
+                } else {
+                  h[r] = what == 1 ? g : u;
                 }
-                const int srow = ii * 32 + 8 * (r >> 2) + 4 * elhi + (r & 3);
-                stage_pair(h[0], h[1], srow, j * 32 + el32, kPitch, odd);
               }
+              const int chunk = 2 * (j & 1) + (eq >> 1);  // of the 32-column block j / 2
+              *reinterpret_cast<u32x2*>(stage + (ii * kColBlocks + j / 2) * kBlkBytes + e16 * 64 +
+                                        ((chunk ^ ((e16 >> 2) & 3)) << 4) + (eq & 1) * 8) =
+                  u32x2{pack_bf16x2(h[0], h[1]), pack_bf16x2(h[2], h[3])};
             }
           }
           __builtin_amdgcn_s_waitcnt(waitcnt_imm(63, 0));
-          // kRound rows x kOutCols columns = (kRound / 16) row blocks x (kOutCols / 32) column blocks of the tiled
-          // intermediate, 1 KiB each; one store instruction per block: lane -> (row lane/4, slot lane%4) holding
-          // chunk slot ^ ((row >> 2) & 3)
-          const int r16 = lane_e >> 2, slot = lane_e & 3, chunk = slot ^ ((r16 >> 2) & 3);
 #pragma unroll
-          for (int rbl = 0; rbl < kRound / 16; ++rbl) {
+          for (int rbl = 0; rbl < kRound; ++rbl) {
 #pragma unroll
-            for (int kbl = 0; kbl < kOutCols / 32; ++kbl) {
-              const u32x4 v =
-                  *reinterpret_cast<const u32x4*>(stage + (rbl * 16 + r16) * kPitch + (kbl * 32 + chunk * 8) * 2);
-              const int row = wm * (FM * 32) + round * kRound + rbl * 16;  // first row of the block inside the tile
-              const int col = wn * kOutCols + kbl * 32;                     // first column of the block inside the tile
+            for (int kbl = 0; kbl < kColBlocks; ++kbl) {
+              const u32x4 v = *reinterpret_cast<const u32x4*>(stage + (rbl * kColBlocks + kbl) * kBlkBytes + lane_e * 16);
+              const int row = (wm * FM + round * kRound + rbl) * 16;     // first row of the block inside the tile
+              const int col = (wn * kColBlocks + kbl) * 32;              // first column of the block inside the tile
               // rows past the expert's last row are padding of the tiled matrix: harmless to write, never read
               if (col < S.cols_left) {
                 unsigned char* dst = reinterpret_cast<unsigned char*>(S.c_base) + keep_off[what] +
@@ -1126,157 +1189,69 @@ __device__ __forceinline__ void dual_gemm_body(const Params& p, const int wg, co
     } else {
       if constexpr (MODE == kQkvRope || MODE == kQkvRopeFull) {
         // Bias and rotary embedding on the accumulators, before they are staged.  A wavefront's 128 columns are one
-        // head; channel d of the head sits in block d / 32 at lane d % 32, so its rotation partner d +/- 64 is two
-        // blocks away in the same lane.  Evaluated like eager bf16 code: the projection (with its bias) rounded once,
+        // head; channel d of the head sits in block d / 16, so its rotation partner d +/- 64 is four blocks away in
+        // the same lane and register.  Evaluated like eager bf16 code: the projection (with its bias) rounded once,
         // then q * cos + rotate_half(q) * sin with each product and the sum rounded (vl.py:771-772).
-        static_assert(FN == 4, "a wavefront covers whole heads of 128 channels");
+        static_assert(FN == 8, "a wavefront covers whole heads of 128 channels");
         const int col_w = S.col0 + wn * 128;  // first output column of this wavefront's head
         const bool live = wn * 128 < S.cols_left;
-        float bias_v[4] = {0.f, 0.f, 0.f, 0.f};
+        u32x2 bias_v[FN];  // this lane's four columns of each block, bf16
+#pragma unroll
+        for (int j = 0; j < FN; ++j) bias_v[j] = u32x2{0u, 0u};
         if (p.bias != nullptr && live) {
+          const uint16_t* b = reinterpret_cast<const uint16_t*>(p.bias) + col_w + 4 * eq;
+          if ((reinterpret_cast<uintptr_t>(p.bias) & 7) == 0) {
 #pragma unroll
-          for (int j = 0; j < 4; ++j) bias_v[j] = static_cast<float>(p.bias[col_w + j * 32 + el32]);
+            for (int j = 0; j < FN; ++j) bias_v[j] = *reinterpret_cast<const u32x2*>(b + j * 16);
+          } else {
+#pragma unroll
+            for (int j = 0; j < FN; ++j)
+              bias_v[j] = u32x2{b[j * 16] | static_cast<uint32_t>(b[j * 16 + 1]) << 16,
+                                b[j * 16 + 2] | static_cast<uint32_t>(b[j * 16 + 3]) << 16};
+          }
         }
+        auto bias_of = [&](int j, int r) {
+          return __uint_as_float((r & 1) ? (bias_v[j][r >> 1] & 0xffff0000u) : (bias_v[j][r >> 1] << 16));
+        };
         const bool rotate = live && col_w < p.rope_cols;  // wave-uniform: q and k heads rotate, v heads do not
-        if constexpr (MODE == kQkvRope) {  // channels d and d + 64 share a table entry (64 per token)
+        constexpr int kWidth = MODE == kQkvRope ? 64 : 128;  // table entries per token: shared by d and d + 64, or one each
 #pragma unroll
-          for (int i = 0; i < FM; ++i) {
-            // cos | sin of this lane's channels 32 jp + lane % 32 (shared with the channel 64 further) for its 16 rows:
-            // all 32 loads go out before the first is used
-            uint32_t cs[16][2];
-            if (rotate) {
+        for (int i = 0; i < FM; ++i) {
+          // cos | sin of this lane's channels, four per load, all loads ahead of their first use
+          u32x4 cs[kWidth / 16];
+          if (rotate) {
+            const int row = (wm * FM + i) * 16 + e16;
+            const uint32_t* t = p.rope_table + static_cast<int64_t>(S.row0 + (row < S.rows ? row : 0)) * kWidth + 4 * eq;
 #pragma unroll
-              for (int r = 0; r < 16; ++r) {
-                const int row = wm * (FM * 32) + i * 32 + 8 * (r >> 2) + 4 * elhi + (r & 3);
-                const bool in = row < S.rows;
-                const uint32_t* t = p.rope_table + static_cast<int64_t>(S.row0 + (in ? row : 0)) * 64 + el32;
-                cs[r][0] = t[0];
-                cs[r][1] = t[32];
-              }
-            }
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-#pragma unroll
-              for (int jp = 0; jp < 2; ++jp) {
-                const float lo = round_bf16(acc[i][jp][r] + bias_v[jp]);
-                const float hi = round_bf16(acc[i][jp + 2][r] + bias_v[jp + 2]);
-                if (rotate) {
-                  const float c = __uint_as_float(cs[r][jp] << 16), sn = __uint_as_float(cs[r][jp] & 0xffff0000u);
-                  acc[i][jp][r] = round_bf16(lo * c) - round_bf16(hi * sn);
-                  acc[i][jp + 2][r] = round_bf16(hi * c) + round_bf16(lo * sn);
-                } else {
-                  acc[i][jp][r] = lo;
-                  acc[i][jp + 2][r] = hi;
-                }
-              }
-            }
+            for (int j = 0; j < kWidth / 16; ++j) cs[j] = *reinterpret_cast<const u32x4*>(t + j * 16);
           }
-        } else {
-          // one table entry per channel (128 per token): the same walk, one half of the channel pairs at a time (32
-          // entries in flight)
 #pragma unroll
-          for (int i = 0; i < FM; ++i) {
+          for (int j = 0; j < 4; ++j) {
 #pragma unroll
-            for (int jp = 0; jp < 2; ++jp) {
-              uint32_t cs[16][2];  // [row][0]: channel 32 jp + lane % 32, [1]: the channel 64 further
+            for (int r = 0; r < 4; ++r) {
+              const float lo = round_bf16(acc[i][j][r] + bias_of(j, r));
+              const float hi = round_bf16(acc[i][j + 4][r] + bias_of(j + 4, r));
               if (rotate) {
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                  const int row = wm * (FM * 32) + i * 32 + 8 * (r >> 2) + 4 * elhi + (r & 3);
-                  const bool in = row < S.rows;
-                  const uint32_t* t = p.rope_table + static_cast<int64_t>(S.row0 + (in ? row : 0)) * 128 + jp * 32 + el32;
-                  cs[r][0] = t[0];
-                  cs[r][1] = t[64];
-                }
-              }
-#pragma unroll
-              for (int r = 0; r < 16; ++r) {
-                const float lo = round_bf16(acc[i][jp][r] + bias_v[jp]);
-                const float hi = round_bf16(acc[i][jp + 2][r] + bias_v[jp + 2]);
-                if (rotate) {
-                  const float c_lo = __uint_as_float(cs[r][0] << 16), s_lo = __uint_as_float(cs[r][0] & 0xffff0000u);
-                  const float c_hi = __uint_as_float(cs[r][1] << 16), s_hi = __uint_as_float(cs[r][1] & 0xffff0000u);
-                  acc[i][jp][r] = round_bf16(lo * c_lo) - round_bf16(hi * s_lo);
-                  acc[i][jp + 2][r] = round_bf16(hi * c_hi) + round_bf16(lo * s_hi);
-                } else {
-                  acc[i][jp][r] = lo;
-                  acc[i][jp + 2][r] = hi;
-                }
+                const uint32_t t_lo = cs[j][r], t_hi = cs[MODE == kQkvRope ? j : j + 4][r];
+                const float c_lo = __uint_as_float(t_lo << 16), s_lo = __uint_as_float(t_lo & 0xffff0000u);
+                const float c_hi = __uint_as_float(t_hi << 16), s_hi = __uint_as_float(t_hi & 0xffff0000u);
+                acc[i][j][r] = round_bf16(lo * c_lo) - round_bf16(hi * s_lo);
+                acc[i][j + 4][r] = round_bf16(hi * c_hi) + round_bf16(lo * s_hi);
+              } else {
+                acc[i][j][r] = lo;
+                acc[i][j + 4][r] = hi;
               }
             }
           }
         }
       }
-      // wave output: 128 rows x kOutCols columns row-major, staged kRound rows at a time
-      constexpr int kOutCols = FN * 32;
-      constexpr int kPitch = kOutCols * 2;
-      constexpr int kRound = kStageBytes / kPitch;  // 32 / 16 rows
-      constexpr int kParts = 32 / kRound;           // rounds per 32-row accumulator block
-      static_assert(kParts == 1 || kParts == 2, "a round is a whole or half accumulator block");
-      constexpr int kLanesPerRow = kPitch / 16, kRowsPerStore = 64 / kLanesPerRow;
-#pragma unroll
-      for (int i = 0; i < FM; ++i) {
-#pragma unroll
-        for (int part = 0; part < kParts; ++part) {
-          // a row is kPitch bytes = kLanesPerRow lanes; one store instruction writes kRowsPerStore rows
-          const int rl = lane_e / kLanesPerRow, cc = (lane_e % kLanesPerRow) * 8;
-          const int col = wn * kOutCols + cc;
-          constexpr int kStores = kRound / kRowsPerStore;
-          int out_row[kStores];
-          u32x4 resv[kStores];
-#pragma unroll
-          for (int q = 0; q < kStores; ++q) {
-            const int row = wm * (FM * 32) + i * 32 + part * kRound + q * kRowsPerStore + rl;
-            out_row[q] = row;
-            if constexpr (MODE == kDown) {
-              // scatter: the row ids of the round (and the residual's chunks) are fetched together, ahead of the
-              // staging writes and reads
-              if (S.row_id != nullptr && row < S.rows) out_row[q] = S.row_id[row];
-            }
-          }
-          if constexpr (MODE == kDown || MODE == kGeneric) {
-            if (S.res != nullptr) {
-#pragma unroll
-              for (int q = 0; q < kStores; ++q) {
-                const int row = wm * (FM * 32) + i * 32 + part * kRound + q * kRowsPerStore + rl;
-                resv[q] = u32x4{0u, 0u, 0u, 0u};
-                if (row < S.rows && col < S.cols_left)
-                  resv[q] = *reinterpret_cast<const u32x4*>(S.res + static_cast<int64_t>(out_row[q]) * S.ldc + col);
-              }
-            }
-          }
-#pragma unroll
-          for (int j = 0; j < FN; ++j) {
-#pragma unroll
-            for (int rr = 0; rr < 16 / kParts; rr += 2) {
-              const int r = part * (16 / kParts) + rr;  // half blocks: registers 0..7 are rows 0..15, 8..15 rows 16..31
-              const int srow = 8 * (r >> 2) + 4 * elhi + (r & 3) - part * kRound;
-              stage_pair(acc[i][j][r], acc[i][j][r + 1], srow, j * 32 + el32, kPitch, odd);
-            }
-          }
-          __builtin_amdgcn_s_waitcnt(waitcnt_imm(63, 0));
-#pragma unroll
-          for (int q = 0; q < kStores; ++q) {
-            const int srow = q * kRowsPerStore + rl;
-            u32x4 v = *reinterpret_cast<const u32x4*>(stage + srow * kPitch + cc * 2);
-            const int row = wm * (FM * 32) + i * 32 + part * kRound + srow;
-            if constexpr (MODE == kDown || MODE == kGeneric) {
-              if (S.res != nullptr) {  // bf16(y) + bf16(residual), summed in fp32 and rounded once, like the eager add
-#pragma unroll
-                for (int w = 0; w < 4; ++w) {
-                  const float lo = __builtin_bit_cast(float, v[w] << 16) + __builtin_bit_cast(float, resv[q][w] << 16);
-                  const float hi = __builtin_bit_cast(float, v[w] & 0xFFFF0000u) +
-                                   __builtin_bit_cast(float, resv[q][w] & 0xFFFF0000u);
-                  v[w] = pack_bf16x2(lo, hi);
-                }
-              }
-            }
-            if (row < S.rows && col < S.cols_left)
-              *reinterpret_cast<u32x4*>(S.c_base + static_cast<int64_t>(out_row[q]) * S.ldc + col) = v;
-          }
-          __builtin_amdgcn_s_waitcnt(waitcnt_imm(63, 0));
+      if constexpr (MODE == kDown || MODE == kGeneric) {
+        if (S.res != nullptr) {
+          store_rows(S, lane_e, std::true_type{});
+          return;
         }
       }
+      store_rows(S, lane_e, std::false_type{});
     }
   };
 
@@ -1368,7 +1343,7 @@ __device__ __forceinline__ void dual_gemm_body(const Params& p, const int wg, co
       __builtin_amdgcn_s_waitcnt(waitcnt_imm((kStages - 2) * kLoadsPerStep + kLoadsA, 15));
     }
     __syncthreads();
-    read_frags(slot_a(0), slot_b(0), 0, 0);
+    read_first(slot_a(0), slot_b(0), 0, 0);
 
     while (have) {
 #pragma unroll
@@ -1376,7 +1351,7 @@ __device__ __forceinline__ void dual_gemm_body(const Params& p, const int wg, co
 #pragma unroll
         for (int j = 0; j < FN; ++j)
 #pragma unroll
-          for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+          for (int r = 0; r < 4; ++r) acc[i][j][r] = 0.f;
 
       const Store done = S;
       const int nk = S.nk;
@@ -1406,10 +1381,10 @@ __device__ __forceinline__ void dual_gemm_body(const Params& p, const int wg, co
           k_step_pair(with_loads, std::integral_constant<int, 2>{}, L, ld_ks);
           k_step_pair(with_loads, std::integral_constant<int, 3>{}, L, ld_ks);
         } else {
-#pragma unroll
-          for (int s = 0; s < kStages; ++s)
-            k_step_as(with_loads, L, ld_ks + s, slot_a(s), slot_b(s), slot_a((s + 1) % kStages), slot_b((s + 1) % kStages),
-                      slot_b((s + kStages - 1) % kStages));
+          k_step_as(with_loads, std::integral_constant<int, 0>{}, L, ld_ks);
+          k_step_as(with_loads, std::integral_constant<int, 1>{}, L, ld_ks);
+          k_step_as(with_loads, std::integral_constant<int, 2>{}, L, ld_ks);
+          k_step_as(with_loads, std::integral_constant<int, 3>{}, L, ld_ks);
         }
       }
       epilogue(done);
@@ -1422,7 +1397,7 @@ __device__ __forceinline__ void dual_gemm_body(const Params& p, const int wg, co
           setup_store(tc, S);
           consumer_prologue();
           __syncthreads();
-          read_frags(slot_a(0), slot_b(0), 0, 0);
+          read_first(slot_a(0), slot_b(0), 0, 0);
         }
       }
     }
