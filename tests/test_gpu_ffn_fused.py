@@ -230,3 +230,41 @@ def test_one_launch_ffn_on_two_streams_at_once(dev):
         for i, ln in enumerate(lanes):
             assert torch.equal(ln["out"][0], ln["out"][1]) and torch.equal(ln["hm"][0], ln["hm"][1]), f"rep {rep} stream {i}"
             assert int(ln["work"].abs().sum()) == 0, f"rep {rep} stream {i}: counters or the error flag left set"
+
+
+# Few rows (a denoise step of one robot, or a few): tiles of 16 or 32 rows whose contraction is cut over a workgroup's
+# wavefronts.  The edges of its row blocks, both tile heights, the last row count it takes at these widths (256) and the
+# first it does not, both experts, and a hidden size whose last column tile is half empty.
+@pytest.mark.parametrize("T,m0,H,I0,I1", [
+    (1, 0, 2048, 1536, 1024), (15, 0, 2048, 1536, 1024), (16, 0, 2048, 1536, 1024), (17, 0, 2048, 1536, 1024),
+    (32, 0, 2048, 1536, 1024), (128, 0, 2048, 1536, 1024), (129, 0, 2048, 1536, 1024), (217, 0, 2048, 1536, 1024),
+    (256, 0, 2048, 1536, 1024), (257, 0, 2048, 1536, 1024), (40, 23, 512, 448, 96), (33, 33, 288, 64, 32),
+    (50, 1, 1280, 320, 1024), (1024, 700, 256, 64, 32),
+])
+def test_few_rows(dev, T, m0, H, I0, I1):
+    ws_, packed, types, x, res, off, inv, xt = _case(dev, T, m0, H, I0, I1, T + H)
+    p = [t.data_ptr() for t in packed]
+    stream = torch.cuda.current_stream().cuda_stream
+    pad = native.padded_sorted_rows(T)
+    rows = _lib.i64x2((m0, T - m0))
+    work = _workspace(dev)
+    got = []
+    for form in range(5):  # one launch and two, with and without the row counts on the host, and with the permute inside
+        hm = torch.zeros(pad * max(I0, I1), dtype=torch.bfloat16, device=dev)
+        out = torch.full((T, H), 7.0, dtype=torch.bfloat16, device=dev)
+        known = rows if form % 2 == 0 else None
+        if form < 2:
+            _two_launches(p, xt, hm, out, res, off, inv, T, H, I0, I1, known, stream)
+        else:
+            _one_launch(p, xt, hm, out, res, off, inv, T, H, I0, I1, known, work, stream, x_rows=x if form == 4 else None)
+        torch.cuda.synchronize()
+        assert int(work.abs().sum()) == 0, f"form {form}"
+        got.append((out, hm))
+    for form, (out, hm) in enumerate(got):
+        assert torch.equal(out, got[0][0]) and torch.equal(hm, got[0][1]), f"form {form}"
+    wc = [tuple(w.cpu() for w in ws_[:3]), tuple(w.cpu() for w in ws_[3:])]
+    ref = oracle.sparse_moe_block_ref(x.cpu()[None], types.cpu()[None], wc)[0].float()
+    ref = (res.cpu().float() + ref).to(torch.bfloat16).float()
+    err = (got[0][0].cpu().float() - ref).abs()
+    # (the bound of the other tests of this FFN: bf16 steps of the intermediate and of the result)
+    assert not (err > 2e-2 + 1e-2 * ref.abs()).any(), float(err.max())

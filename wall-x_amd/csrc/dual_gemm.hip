@@ -13,7 +13,7 @@
 // tiles would leave most CUs idle (a denoise step of a few thousand action tokens) run the same kernel with a
 // 128 x 128 tile, two workgroups per CU.  A ragged last round of the fused FFN launches (tiles left over after the
 // whole rounds of one tile per CU) runs in that small shape too, in a second launch, when it then fits the chip in
-// one go.
+// one go.  The FFN of few rows (a denoise step of one robot) has tiles of its own, see few_rows_body.
 // Operands are K-contiguous, so both MFMA fragments are 16-byte LDS reads.
 // Global -> LDS uses buffer loads that write LDS directly (no register staging) into a ring of four K-step slots
 // per operand; the load stream runs four K steps ahead of the MFMAs and crosses tile boundaries, with one
@@ -131,6 +131,8 @@ struct Params {
   // number of 256 x 256 tiles is on its side of `gate_tiles`.  0 = always run, 1 = run if at most gate_tiles,
   // 2 = run if more.
   int gate, gate_tiles;
+  // CUs that the few-rows form may fill (see few_rows_fm); 0 = this launch does not take that form.
+  int few_rows_cus;
   // Tail split (see tail_split_point): 0 = off; 1 = this launch does the whole rounds of 256 x 256 tiles and leaves
   // the ragged last round to a second launch; 2 = this is that second launch, with 128 x 128 tiles.
   // split_cus = workgroups of the first launch (one per CU).
@@ -310,6 +312,259 @@ struct FusedSync {
   const int32_t* gather;
 };
 
+// Fused launch: what this workgroup wrote for row block `rb` is in memory (its stores are write-through and every
+// wavefront has waited for its own before the barrier); one lane counts it.
+__device__ __forceinline__ void count_done(const FusedSync& fs, int tid, int rb) {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+  __builtin_amdgcn_s_waitcnt(waitcnt_imm(0, 0));
+  __syncthreads();
+  if (tid == 0)
+    __hip_atomic_fetch_add(fs.ready + rb * kFusedCounterStride, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// Fused launch: wait (bounded) until ready[rb] has reached `need`, and take a number among the workgroups that
+// get past this wait (`before`: how many were past it already; the answer travels while the tile is computed).
+// No cache is invalidated afterwards: the launch began with clean caches, and no line of what the wait is for is
+// read anywhere before it is complete (whole cache lines belong to one writer), so no cache can hold an older
+// version of it.
+__device__ __forceinline__ void wait_for_count(const FusedSync& fs, int tid, int rb, int need, int& before) {
+  if (tid == 0) {
+    const int* flag = fs.ready + rb * kFusedCounterStride;
+    const long long start = __builtin_amdgcn_s_memrealtime();
+    while (__hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < need) {
+      if (static_cast<long long>(__builtin_amdgcn_s_memrealtime()) - start > kFusedWaitTicks) {
+        __hip_atomic_store(fs.error, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        break;
+      }
+      __builtin_amdgcn_s_sleep(2);
+    }
+    before = __hip_atomic_fetch_add(fs.passed + rb * kFusedCounterStride, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  barrier_no_fence();  // (no wait for the counter's answer here)
+}
+// ... and once the tile is done: the workgroup that was the last of its row block to get past the wait (everything
+// the wait was for is done, and every other waiter is past its wait as well) leaves the two counters at zero for
+// the next launch
+__device__ __forceinline__ void clear_if_last(const FusedSync& fs, int tid, int rb, int before, int waiters) {
+  if (tid == 0 && before == waiters - 1) {
+    __hip_atomic_store(fs.ready + rb * kFusedCounterStride, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(fs.passed + rb * kFusedCounterStride, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+}
+
+// SwiGLU of a gate and an up accumulator like eager bf16 code (act.py:80-82): gate, up and silu(gate) are each rounded
+// to bf16 here, the product by the caller's pack.
+__device__ __forceinline__ float swiglu_bf16(float gate, float up) {
+  const uint32_t gu = pack_bf16x2(gate, up);  // one convert for both
+  const float g = __uint_as_float(gu << 16);
+  return round_bf16(g * __builtin_amdgcn_rcpf(1.0f + __expf(-g))) * __uint_as_float(gu & 0xffff0000u);
+}
+
+// ---- few rows ------------------------------------------------------------------------------------------------
+// A denoise step of one robot is 32 rows.  As 128 x 128 tiles its two GEMMs occupy 16 CUs each, and every K step of those
+// waits for the one before it (~250 ns, 96 of them).  This form makes the tiles small and cuts the contraction instead:
+// a workgroup computes 16 FM rows x 64 operand rows of B (32 gate + 32 up, or 64 output columns), its eight wavefronts
+// take an eighth of the K steps each, and the partial sums meet in LDS.  Fragments go from memory to registers (a block
+// of a K-tiled matrix is one fragment of a 16x16x32 MFMA), a ring of them in flight per wavefront, so a tile costs a few
+// memory latencies in place of K / 32 barriers.  Each row block reads the weights again (through L2: the tiles of a
+// column are on one XCD where the column tiles are a multiple of eight), which is why many rows keep the large tiles.
+// Measured (hidden 2048, experts 11008 / 1024, per layer): 32 rows 17 us where the 128 x 128 tiles take 35, 217 rows 22 where
+// they take 34.  The line lies where the tiles of a round of their own run out (256 rows at these widths): beyond it a second
+// round of small tiles re-reads the weights as often as the larger tiles' K loop takes.
+constexpr int kFewCols = 64;       // rows of B per tile
+constexpr int kFewMaxFm = 2;       // row blocks of 16 per tile: 1 or 2
+constexpr int kFewWavesPerSimd = 4;  // two workgroups per CU, which the fused launch counts on (128 registers)
+constexpr int kFewMaxRows = 1024;  // (a bound for the host; few_rows_fm decides)
+
+// Row blocks per tile of the few-rows form, or 0 where the problem keeps the 128 x 128 (256 x 256) tiles: the smaller
+// tile whose gate/up and down tiles each fit the CUs in one round.  Evaluated identically by the host (when it knows the
+// row counts) and on the device, by every launch form, so that they all add up in one order.
+__host__ __device__ inline int few_rows_fm(int64_t m0, int64_t m1, int64_t inter0, int64_t inter1, int64_t hidden, int cus) {
+  if (cus <= 0 || m0 + m1 > kFewMaxRows) return 0;
+  for (int fm = 1; fm <= kFewMaxFm; ++fm) {
+    const int64_t r0 = (m0 + 16 * fm - 1) / (16 * fm), r1 = (m1 + 16 * fm - 1) / (16 * fm);
+    if (r0 * (inter0 / 32) + r1 * (inter1 / 32) <= cus && (r0 + r1) * ((hidden + kFewCols - 1) / kFewCols) <= cus) return fm;
+  }
+  return 0;
+}
+
+// MODE, ROLE, AROWS as in dual_gemm_body.  512 threads.
+template <int MODE, int FM, int ROLE, bool AROWS>
+__device__ __forceinline__ void few_rows_body(const Params& p, const int wg, const int n_wg, const FusedSync& fs) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  static_assert(MODE == kGateUp || MODE == kDown, "the FFN's two GEMMs");
+  constexpr bool SWIGLU = MODE == kGateUp;
+  constexpr int kRows = 16 * FM;
+  constexpr int kRing = FM == 1 ? 4 : 3;  // K steps in flight per wavefront: what 128 registers hold
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l16 = lane & 15, lq = lane >> 4;
+  // the partial sums of wavefront w, one KiB per 16 x 16 block: in the LDS of the 128 x 128 tile's ring
+  unsigned char* const part[8] = {lds_array<8192, 1024, 0>(), lds_array<8192, 1024, 1>(), lds_array<8192, 1024, 2>(),
+                                  lds_array<8192, 1024, 3>(), lds_array<8192, 1024, 4>(), lds_array<8192, 1024, 5>(),
+                                  lds_array<8192, 1024, 6>(), lds_array<8192, 1024, 7>()};
+  unsigned char* const stage = lds_array<SmallTile::kWaves * SmallTile::kStageBytes, 1024, 12>();
+  static_assert(SmallTile::kSlotBytesA == 8192 && SmallTile::kSlotBytesB == 8192 && FM * 4 * 1024 <= 8192, "ring slots hold the partial sums");
+  unsigned char* mine = part[0];
+#pragma unroll
+  for (int w = 1; w < 8; ++w) mine = wave == w ? part[w] : mine;
+
+  const int o0 = p.offsets[0], o1 = p.offsets[1], o2 = p.offsets[2];
+  const int m[2] = {o1 - o0, o2 - o1};
+  const int pad0 = static_cast<int>(round_up_256(m[0])), pad1 = static_cast<int>(round_up_256(m[1]));
+  constexpr int kTileN = SWIGLU ? kFewCols / 2 : kFewCols;  // output columns per tile
+  const int blocks[2] = {(m[0] + kRows - 1) / kRows, (m[1] + kRows - 1) / kRows};
+  const int cols[2] = {(p.g[0].n + kTileN - 1) / kTileN, (p.g[1].n + kTileN - 1) / kTileN};
+  const int total0 = blocks[0] * cols[0], total = total0 + blocks[1] * cols[1];
+  const int frag = (l16 << 6) + ((lq ^ ((l16 >> 2) & 3)) << 4);  // this lane's 16 bytes of a K-tiled block
+
+  for (int t = wg; t < total; t += n_wg) {
+    const int e = t >= total0 ? 1 : 0;
+    const Group G = e ? p.g[1] : p.g[0];
+    const int nct = e ? cols[1] : cols[0], me = e ? m[1] : m[0], pad_e = e ? pad1 : pad0;
+    const int te = e ? t - total0 : t;
+    const int rb = __builtin_amdgcn_readfirstlane(te / nct), ct = te - rb * nct;
+    const int row0 = rb * kRows, col0 = ct * kTileN;
+    const int counter = e * kFusedMaxRowBlocks + rb;
+    const int steps = G.k / 32, share = (steps + 7) / 8;
+    const int k_first = wave * share, k_last = k_first + share < steps ? k_first + share : steps;
+
+    // A: K-tiled rows (the activations, or the intermediate of this expert), or the token rows themselves.  A K step's
+    // descriptor begins at that step (scalar work) and ends with it, so the lanes' offsets are the same in every step;
+    // steps past this wavefront's share have an empty descriptor and read as zeros.
+    const char* a_base;
+    uint32_t a_off[FM], a_step, a_bytes;
+    if constexpr (AROWS) {
+      a_base = reinterpret_cast<const char*>(fs.x);
+      a_step = 64;
+      a_bytes = static_cast<uint32_t>(o2) * static_cast<uint32_t>(G.k) * 2u;
+#pragma unroll
+      for (int i = 0; i < FM; ++i) {
+        const int r = row0 + 16 * i + l16;
+        a_off[i] = r < me ? static_cast<uint32_t>(fs.gather[(e ? o1 : o0) + r]) * static_cast<uint32_t>(G.k) * 2u + lq * 16u : 0x80000000u;
+      }
+    } else {
+      const int a_blocks = SWIGLU ? G.lda : pad_e / kBlkRows;
+      const int first = (SWIGLU && e ? pad0 : 0) / kBlkRows + row0 / kBlkRows;
+      a_base = reinterpret_cast<const char*>(SWIGLU ? G.a : G.a + (e ? static_cast<int64_t>(pad0) * p.g[0].k : 0));
+      a_step = a_bytes = static_cast<uint32_t>(a_blocks) << 10;
+#pragma unroll
+      for (int i = 0; i < FM; ++i) a_off[i] = (static_cast<uint32_t>(first + i) << 10) + frag;
+    }
+    const uint32_t b_step = static_cast<uint32_t>(G.ldb) << 10;  // (blocks past the matrix's last row of B are past it)
+    const uint32_t b_off = (static_cast<uint32_t>(col0 / kBlkRows) << 10) + frag;
+    u32x4 fa[kRing][FM], fb[kRing][4];
+    auto load_a = [&](int slot, int ks) {
+      const int64_t adv = static_cast<int64_t>(ks) * a_step;
+      const __amdgpu_buffer_rsrc_t r = make_rsrc(a_base + adv, ks >= k_last ? 0u : (AROWS ? a_bytes - static_cast<uint32_t>(adv) : a_bytes));
+#pragma unroll
+      for (int i = 0; i < FM; ++i) fa[slot][i] = __builtin_amdgcn_raw_buffer_load_b128(r, a_off[i], 0, 0);
+    };
+    auto load_b = [&](int slot, int ks) {
+      const int64_t adv = static_cast<int64_t>(ks) * b_step;
+      const uint32_t bytes = ks < k_last ? b_step : 0u;
+      const __amdgpu_buffer_rsrc_t r0 = make_rsrc(reinterpret_cast<const char*>(G.b0) + adv, bytes);
+      const __amdgpu_buffer_rsrc_t r1 = SWIGLU ? make_rsrc(reinterpret_cast<const char*>(G.b1) + adv, bytes) : r0;
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        fb[slot][j] = __builtin_amdgcn_raw_buffer_load_b128(SWIGLU && j >= 2 ? r1 : r0, b_off + (SWIGLU ? j & 1 : j) * kBlkBytes, 0, 0);
+    };
+    f32x4 acc[FM][4];
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+    // where the finished blocks go: block q of the tile (row block q / 4, column block q % 4) is summed by wavefront q
+    const bool sums = wave < FM * (SWIGLU ? 2 : 4);
+    int out_row = -1;
+    u32x2 res = {0u, 0u};
+#pragma unroll
+    for (int s = 0; s < kRing; ++s) load_b(s, k_first + s);
+    if constexpr (!SWIGLU) {
+      const int r = row0 + (wave >> 2) * 16 + l16, c = col0 + (wave & 3) * 16 + 4 * lq;
+      if (sums && r < me && c < G.n) {
+        const int sorted = (e ? o1 : o0) + r;
+        out_row = p.scatter != nullptr ? p.scatter[sorted] : sorted;
+        if (p.residual != nullptr) res = *reinterpret_cast<const u32x2*>(p.residual + static_cast<int64_t>(out_row) * G.ldc + c);
+      }
+    }
+    int before = 0;
+    if constexpr (ROLE == 2) wait_for_count(fs, tid, counter, (e ? p.g[1].k : p.g[0].k) / 32, before);
+#pragma unroll
+    for (int s = 0; s < kRing; ++s) load_a(s, k_first + s);
+    for (int ks = 0; ks < share; ks += kRing) {
+#pragma unroll
+      for (int s = 0; s < kRing; ++s) {
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, fb[s][j]), __builtin_bit_cast(bf16x8, fa[s][i]), acc[i][j], 0, 0, 0);
+        load_b(s, k_first + ks + s + kRing);
+        load_a(s, k_first + ks + s + kRing);
+      }
+    }
+    // partial sums: lane l of a block holds row l % 16, columns 4 (l / 16) .. + 3
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) *reinterpret_cast<f32x4*>(mine + (i * 4 + j) * 1024 + lane * 16) = acc[i][j];
+    __syncthreads();
+    auto sum_of = [&](int block) {
+      f32x4 v = *reinterpret_cast<const f32x4*>(part[0] + block * 1024 + lane * 16);
+#pragma unroll
+      for (int w = 1; w < 8; ++w) v += *reinterpret_cast<const f32x4*>(part[w] + block * 1024 + lane * 16);
+      return v;
+    };
+    if constexpr (SWIGLU) {
+      if (sums) {  // wavefront 2 i + j: row block i, columns 16 j .. of the tile's 32
+        const int i = wave >> 1, j = wave & 1;
+        const f32x4 g = sum_of(i * 4 + j), u = sum_of(i * 4 + j + 2);
+        float h[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) h[r] = swiglu_bf16(g[r], u[r]);
+        const int chunk = 2 * j + (lq >> 1);
+        *reinterpret_cast<u32x2*>(stage + i * kBlkBytes + l16 * 64 + ((chunk ^ ((l16 >> 2) & 3)) << 4) + (lq & 1) * 8) =
+            u32x2{pack_bf16x2(h[0], h[1]), pack_bf16x2(h[2], h[3])};
+      }
+      __syncthreads();
+      if (wave < FM) {  // whole blocks of the K-tiled intermediate, written through where another XCD waits for them
+        const u32x4 v = *reinterpret_cast<const u32x4*>(stage + wave * kBlkBytes + lane * 16);
+        unsigned char* dst = reinterpret_cast<unsigned char*>(p.g[0].c + (e ? static_cast<int64_t>(pad0) * p.g[0].n : 0)) +
+                             ((static_cast<int64_t>(ct) * (pad_e / kBlkRows) + row0 / kBlkRows + wave) << 10);
+        if constexpr (ROLE == 1) __builtin_amdgcn_raw_buffer_store_b128(v, make_rsrc(dst, kBlkBytes), lane * 16, 0, 16 /* sc1 */);
+        else *reinterpret_cast<u32x4*>(dst + lane * 16) = v;
+      }
+      if constexpr (ROLE == 1) count_done(fs, tid, counter);
+    } else {
+      if (sums && out_row >= 0) {
+        const f32x4 y = sum_of(wave);
+        u32x2 v = {pack_bf16x2(y[0], y[1]), pack_bf16x2(y[2], y[3])};
+        if (p.residual != nullptr) {
+#pragma unroll
+          for (int q = 0; q < 2; ++q)
+            v[q] = pack_bf16x2(__uint_as_float(v[q] << 16) + __uint_as_float(res[q] << 16),
+                               __uint_as_float(v[q] & 0xffff0000u) + __uint_as_float(res[q] & 0xffff0000u));
+        }
+        *reinterpret_cast<u32x2*>(p.g[0].c + static_cast<int64_t>(out_row) * G.ldc + col0 + (wave & 3) * 16 + 4 * lq) = v;
+      }
+      if constexpr (ROLE == 2) clear_if_last(fs, tid, counter, before, nct);
+    }
+    __syncthreads();  // the partial sums' LDS is written by the next tile
+  }
+#endif
+}
+// The form for the row counts in p.offsets; false: the caller runs the tiles.
+template <int MODE, int ROLE, bool AROWS = false>
+__device__ __forceinline__ bool few_rows(const Params& p, const int wg, const int n_wg, const FusedSync& fs) {
+  const int inter0 = MODE == kGateUp ? p.g[0].n : p.g[0].k, inter1 = MODE == kGateUp ? p.g[1].n : p.g[1].k;
+  const int hidden = MODE == kGateUp ? p.g[0].k : p.g[0].n;
+  const int fm = few_rows_fm(p.offsets[1] - p.offsets[0], p.offsets[2] - p.offsets[1], inter0, inter1, hidden, p.few_rows_cus);
+  if (fm == 0) return false;
+  if (fm == 1) few_rows_body<MODE, 1, ROLE, AROWS>(p, wg, n_wg, fs);
+  else few_rows_body<MODE, 2, ROLE, AROWS>(p, wg, n_wg, fs);
+  return true;
+}
+
 // KA / KB (generic mode only): the operand is stored with K as its slow dimension -- A as [k, m], B as [k, n] --
 // and is transposed on the way from LDS to the MFMA registers.
 //
@@ -431,6 +686,12 @@ __device__ __forceinline__ void dual_gemm_body(const Params& p, const int wg, co
   tiles_m[1] = (g1.m + BM - 1) / BM;
   tiles_n[1] = (g1.n + kTileN - 1) / kTileN;
   if (g1.m <= 0 || g1.n <= 0) tiles_m[1] = tiles_n[1] = 0;
+  if constexpr (TILED_IN && std::is_same_v<TS, BigTileFor<MODE>>) {
+    // (a launch of large tiles beside one that runs the few-rows form)
+    if (p.few_rows_cus != 0 && few_rows_fm(g0.m, g1.m, MODE == kGateUp ? g0.n : g0.k, MODE == kGateUp ? g1.n : g1.k,
+                                           MODE == kGateUp ? g0.k : g0.n, p.few_rows_cus) != 0)
+      return;
+  }
   if (p.gate != 0) {
     constexpr int kBigN = SWIGLU ? BigTile::BN / 2 : BigTile::BN;
     auto big = [](int m, int n) { return (m <= 0 || n <= 0) ? 0 : ((m + BigTile::BM - 1) / BigTile::BM) * ((n + kBigN - 1) / kBigN); };
@@ -787,44 +1048,6 @@ __device__ __forceinline__ void dual_gemm_body(const Params& p, const int wg, co
     for (int i = 0; i < kLoadsB; ++i) P.voff_b[i] = L.voff_b[i];
     issue_b(P, sb);
   };
-  // Fused launch: what this workgroup wrote for row block `rb` is in memory (its stores are write-through and every
-  // wavefront has waited for its own before the barrier); one lane counts it.
-  auto count_done = [&](int* counters, int rb) {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-    __builtin_amdgcn_s_waitcnt(waitcnt_imm(0, 0));
-    __syncthreads();
-    if (tid == 0)
-      __hip_atomic_fetch_add(counters + rb * kFusedCounterStride, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  };
-  // Fused launch: wait (bounded) until counters[rb] has reached `need`, and take a number among the workgroups that
-  // get past this wait (`before`: how many were past it already; the answer travels while the tile is computed).
-  // No cache is invalidated afterwards: the launch began with clean caches, and no line of what the wait is for is
-  // read anywhere before it is complete (whole cache lines belong to one writer), so no cache can hold an older
-  // version of it.
-  auto wait_for_count = [&](const int* counters, int* passed, int rb, int need, int& before) {
-    if (tid == 0) {
-      const int* flag = counters + rb * kFusedCounterStride;
-      const long long start = __builtin_amdgcn_s_memrealtime();
-      while (__hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < need) {
-        if (static_cast<long long>(__builtin_amdgcn_s_memrealtime()) - start > kFusedWaitTicks) {
-          __hip_atomic_store(fs.error, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          break;
-        }
-        __builtin_amdgcn_s_sleep(2);
-      }
-      before = __hip_atomic_fetch_add(passed + rb * kFusedCounterStride, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-    barrier_no_fence();  // (no wait for the counter's answer here)
-  };
-  // ... and once the tile is done: the workgroup that was the last of its row block to get past the wait (everything
-  // the wait was for is done, and every other waiter is past its wait as well) leaves the two counters at zero for
-  // the next launch
-  auto clear_if_last = [&](int* counters, int* passed, int rb, int before, int waiters) {
-    if (tid == 0 && before == waiters - 1) {
-      __hip_atomic_store(counters + rb * kFusedCounterStride, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      __hip_atomic_store(passed + rb * kFusedCounterStride, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-  };
   // Fused launch, consumer, wavefronts that issue no loads: while the workgroup waits for its row block they pull
   // a share of the PRODUCERS' weights through this XCD's L2, so that weights which come from HBM (every layer of a
   // model has its own) are on their way before the producers' ring, four K steps deep, asks for them.  Workgroup c
@@ -1143,17 +1366,8 @@ __device__ __forceinline__ void dual_gemm_body(const Params& p, const int wg, co
               float h[4];
 #pragma unroll
               for (int r = 0; r < 4; ++r) {
-                // eager bf16 evaluation of act_fn(gate) * up (act.py:80-82): gate, up, silu(gate) and the
-                // product are each rounded to bf16
-                const uint32_t gu = pack_bf16x2(acc[i][j][r], acc[i][j + FN / 2][r]);  // one convert for both
-                const float g = __uint_as_float(gu << 16);
-                const float u = __uint_as_float(gu & 0xffff0000u);
-                if (what == 0) {
-                  const float sg = round_bf16(g * __builtin_amdgcn_rcpf(1.0f + __expf(-g)));
-                  h[r] = sg * u;
-                } else {
-                  h[r] = what == 1 ? g : u;
-                }
+                const float gate = acc[i][j][r], up = acc[i][j + FN / 2][r];
+                h[r] = what == 0 ? swiglu_bf16(gate, up) : (what == 1 ? gate : up);  // (rounded by the pack)
               }
               const int chunk = 2 * (j & 1) + (eq >> 1);  // of the 32-column block j / 2
               *reinterpret_cast<u32x2*>(stage + (ii * kColBlocks + j / 2) * kBlkBytes + e16 * 64 +
@@ -1304,7 +1518,7 @@ __device__ __forceinline__ void dual_gemm_body(const Params& p, const int wg, co
           warm_producer_weights();
         }
       }
-      wait_for_count(fs.ready, fs.passed, S.row_block, fs.need[tc.group], passed_before);
+      wait_for_count(fs, tid, S.row_block, fs.need[tc.group], passed_before);
       if constexpr (LD) {
 #pragma unroll
         for (int s = 0; s < kStages; ++s) issue_a(L, s, slot_a(s), pend);
@@ -1388,9 +1602,9 @@ __device__ __forceinline__ void dual_gemm_body(const Params& p, const int wg, co
         }
       }
       epilogue(done);
-      if constexpr (ROLE == 1) count_done(fs.ready, done.row_block);
+      if constexpr (ROLE == 1) count_done(fs, tid, done.row_block);
       if constexpr (ROLE == 2) {
-        clear_if_last(fs.ready, fs.passed, done.row_block, passed_before, fs.consumers);
+        clear_if_last(fs, tid, done.row_block, passed_before, fs.consumers);
         have = next_tile(tc);
         if (have) {  // (one tile per consumer unless the host's row counts were not the device's)
           if constexpr (LD) setup_loader(tc, L);
@@ -1416,19 +1630,34 @@ __global__ __launch_bounds__(TS::kThreads, TS::kWgPerCu) void dual_gemm_kernel(P
   dual_gemm_body<MODE, TS, KA, KB, 0>(p, blockIdx.x, gridDim.x, FusedSync{});
 }
 
+// The same launch where the row counts may call for the few-rows form (MODE: gate/up or down).
+template <int MODE>
+__global__ __launch_bounds__(SmallTile::kThreads, kFewWavesPerSimd) void dual_gemm_few_rows_kernel(Params p) {
+  if (!few_rows<MODE, 0>(p, blockIdx.x, gridDim.x, FusedSync{}))
+    dual_gemm_body<MODE, SmallTile, false, false, 0>(p, blockIdx.x, gridDim.x, FusedSync{});
+}
+
 // The fused FFN launch (see FusedSync): workgroups [0, producers) run the gate/up form on `pg`, the rest the down
 // form on `pd`, both in the small tile shape.  `producers` is a multiple of 8, so a workgroup's index among its
 // form's workgroups names the same XCD as its index in the grid.  (A workgroup that waits is a consumer, and what
 // it waits for belongs to workgroups with lower indices, which never wait: whatever part of the grid is resident,
 // the launch makes progress.)
 // AROWS: the producers read the token rows (fs.x through fs.gather) in place of the K-tiled activations.
-template <bool AROWS>
-__global__ __launch_bounds__(SmallTile::kThreads, SmallTile::kWgPerCu) void ffn_fused_kernel(Params pg, Params pd,
+// FEW: the row counts may call for the few-rows form (a kernel of its own, so that the other's registers are its own).
+template <bool AROWS, bool FEW>
+__global__ __launch_bounds__(SmallTile::kThreads, FEW ? kFewWavesPerSimd : SmallTile::kWgPerCu) void ffn_fused_kernel(Params pg, Params pd,
                                                                                              FusedSync fs,
                                                                                              int producers) {
-  const int wg = blockIdx.x;
-  if (wg < producers) dual_gemm_body<kGateUp, SmallTile, false, false, 1, AROWS>(pg, wg, producers, fs);
-  else dual_gemm_body<kDown, SmallTile, false, false, 2>(pd, wg - producers, static_cast<int>(gridDim.x) - producers, fs);
+  const int wg = blockIdx.x, consumers = static_cast<int>(gridDim.x) - producers;
+  if (wg < producers) {
+    if constexpr (FEW)
+      if (few_rows<kGateUp, 1, AROWS>(pg, wg, producers, fs)) return;
+    dual_gemm_body<kGateUp, SmallTile, false, false, 1, AROWS>(pg, wg, producers, fs);
+  } else {
+    if constexpr (FEW)
+      if (few_rows<kDown, 2>(pd, wg - producers, consumers, fs)) return;
+    dual_gemm_body<kDown, SmallTile, false, false, 2>(pd, wg - producers, consumers, fs);
+  }
 }
 
 // ---- plain FMA tiles: any transpose combination, any k --------------------------------------------------------
@@ -1524,12 +1753,22 @@ int check_dims(const char* who, int64_t m, int64_t n, int64_t k, bool k_in_rows 
 // second launch with 128 x 128 tiles takes the ragged last round when that pays (the row-major op, whose sizes the
 // host knows, decides it on the host); when the host cannot tell, both launches are made and the device decides (the
 // second returns at once if there is nothing to split).
+// few: whether the few-rows form (few_rows_fm) takes the problem; kFewMaybe = the device finds out.
+enum Few { kFewNever, kFewMaybe, kFewAlways };
 template <int MODE, bool KA = false, bool KB = false>
 int launch_mfma(Params p, int64_t tiles_lo, int64_t tiles_hi, hipStream_t s, const char* who,
-                const int64_t* tiles_by_expert = nullptr) {
+                const int64_t* tiles_by_expert = nullptr, Few few = kFewNever) {
   const int cus = device_cu_count();
   const int threshold = cus / 2;
-  bool small = tiles_lo <= threshold, big = tiles_hi > threshold;
+  p.few_rows_cus = few == kFewNever ? 0 : cus;
+  if constexpr (MODE == kGateUp || MODE == kDown) {
+    if (few == kFewAlways) {
+      p.gate = p.split = 0;
+      hipLaunchKernelGGL((dual_gemm_few_rows_kernel<MODE>), dim3(cus), dim3(SmallTile::kThreads), 0, s, p);
+      return check_launch(who);
+    }
+  }
+  bool small = tiles_lo <= threshold || few == kFewMaybe, big = tiles_hi > threshold;
   if (tiles_by_expert != nullptr) {  // the host knows the split: the count that decides is shape_deciding_tiles'
     small = shape_deciding_tiles(tiles_by_expert[0], tiles_by_expert[1], p.g[0].k, p.g[1].k) <= threshold;
     big = !small;
@@ -1542,7 +1781,11 @@ int launch_mfma(Params p, int64_t tiles_lo, int64_t tiles_hi, hipStream_t s, con
   p.split_cus = cus;
   if (small) {
     p.gate = big ? 1 : 0;
-    hipLaunchKernelGGL((dual_gemm_kernel<MODE, SmallTile, KA, KB>), dim3(cus * SmallTile::kWgPerCu),
+    if constexpr (MODE == kGateUp || MODE == kDown) {
+      if (few == kFewMaybe)
+        hipLaunchKernelGGL((dual_gemm_few_rows_kernel<MODE>), dim3(cus * SmallTile::kWgPerCu), dim3(SmallTile::kThreads), 0, s, p);
+    }
+    if (few != kFewMaybe) hipLaunchKernelGGL((dual_gemm_kernel<MODE, SmallTile, KA, KB>), dim3(cus * SmallTile::kWgPerCu),
                        dim3(SmallTile::kThreads), 0, s, p);
   }
   if (big) {
@@ -1816,18 +2059,33 @@ Params gate_up_params(const FfnArgs& a) {
   return p;
 }
 
+// Whether the few-rows form takes this FFN.  Not where the projections are kept for a backward pass, and not with
+// matrices beyond 31-bit byte offsets.
+Few few_rows_of(const FfnArgs& a) {
+  const int cus = device_cu_count();
+  const int64_t max_inter = a.inter[0] > a.inter[1] ? a.inter[0] : a.inter[1];
+  if (a.keep_gate != nullptr || a.rows > kFewMaxRows || (max_inter + 16) * (a.hidden + 32) * 2 >= (1ll << 31) ||
+      padded_sorted_rows(a.rows) * (a.hidden > max_inter ? a.hidden : max_inter) * 2 >= (1ll << 31))
+    return kFewNever;
+  if (a.host_rows != nullptr)
+    return few_rows_fm(a.host_rows[0], a.host_rows[1], a.inter[0], a.inter[1], a.hidden, cus) ? kFewAlways : kFewNever;
+  // the split lies with the device: possible if it is with every row on the narrower expert
+  const int64_t i0 = a.inter[0], i1 = a.inter[1];
+  return few_rows_fm(i0 <= i1 ? a.rows : 0, i0 <= i1 ? 0 : a.rows, i0, i1, a.hidden, cus) ? kFewMaybe : kFewNever;
+}
+
 int launch_gate_up(const FfnArgs& a, hipStream_t s) {
   const Params p = gate_up_params(a);
   const int64_t t0 = ceil_div(a.inter[0], BigTile::BN / 2), t1 = ceil_div(a.inter[1], BigTile::BN / 2);
   if (a.host_rows != nullptr) {  // the caller knows the split: one launch of the right tile shape
     const int64_t by_expert[2] = {ceil_div(a.host_rows[0], BigTile::BM) * t0, ceil_div(a.host_rows[1], BigTile::BM) * t1};
     const int64_t tiles = by_expert[0] + by_expert[1];
-    return launch_mfma<kGateUp>(p, tiles, tiles, s, "dual_gemm_kernel<gate_up>", by_expert);
+    return launch_mfma<kGateUp>(p, tiles, tiles, s, "dual_gemm_kernel<gate_up>", by_expert, few_rows_of(a));
   }
   // the split of the rows between the experts is only known on the device: bound the tile count from the total
   const int64_t row_tiles = ceil_div(a.rows, BigTile::BM);
   return launch_mfma<kGateUp>(p, row_tiles * (t0 < t1 ? t0 : t1), (row_tiles + 1) * (t0 > t1 ? t0 : t1), s,
-                              "dual_gemm_kernel<gate_up>");
+                              "dual_gemm_kernel<gate_up>", nullptr, few_rows_of(a));
 }
 
 // out_e = hmid_e @ down_e^T, row-major, expert e's rows start at offsets[e]
@@ -1857,10 +2115,11 @@ int launch_down(const FfnArgs& a, hipStream_t s) {
   if (a.host_rows != nullptr) {
     const int64_t by_expert[2] = {ceil_div(a.host_rows[0], BigTile::BM) * col_tiles, ceil_div(a.host_rows[1], BigTile::BM) * col_tiles};
     const int64_t tiles = by_expert[0] + by_expert[1];
-    return launch_mfma<kDown>(p, tiles, tiles, s, "dual_gemm_kernel<down>", by_expert);
+    return launch_mfma<kDown>(p, tiles, tiles, s, "dual_gemm_kernel<down>", by_expert, few_rows_of(a));
   }
   const int64_t row_tiles = ceil_div(a.rows, BigTile::BM);
-  return launch_mfma<kDown>(p, row_tiles * col_tiles, (row_tiles + 1) * col_tiles, s, "dual_gemm_kernel<down>");
+  return launch_mfma<kDown>(p, row_tiles * col_tiles, (row_tiles + 1) * col_tiles, s, "dual_gemm_kernel<down>", nullptr,
+                            few_rows_of(a));
 }
 
 // Both launches as one (ffn_fused_kernel), for the shapes where each is a single round of small tiles with the row
@@ -1909,7 +2168,13 @@ int launch_ffn_fused(const FfnArgs& a, int* ws, hipStream_t s) {
     }
   }
   const bool rows_known = a.host_rows != nullptr;
-  if (!rows_known) {
+  const Few few = few_rows_of(a);
+  if (few == kFewAlways) {  // tiles of the few-rows form (at most one per CU)
+    const int rows = 16 * few_rows_fm(a.host_rows[0], a.host_rows[1], a.inter[0], a.inter[1], a.hidden, cus);
+    const int64_t r0 = ceil_div(a.host_rows[0], rows), r1 = ceil_div(a.host_rows[1], rows);
+    gate_tiles = r0 * (a.inter[0] / 32) + r1 * (a.inter[1] / 32);
+    down_tiles = (r0 + r1) * ceil_div(a.hidden, kFewCols);
+  } else if (!rows_known) {
     // The split of the rows is only known on the device.  The launch is right for any split (workgroups take as
     // many tiles as there are), so what the host has to settle is whether it is the faster form whatever the split.
     // Up to two rows per CU it is: 24-27 against 29-34 us with every row on the narrow expert, 2-9 % ahead with a
@@ -1925,6 +2190,7 @@ int launch_ffn_fused(const FfnArgs& a, int* ws, hipStream_t s) {
   Params pg = gate_up_params(a), pd = down_params(a);
   pg.gate = pd.gate = 0;
   pg.split = pd.split = 0;
+  pg.few_rows_cus = pd.few_rows_cus = few == kFewNever ? 0 : cus;
   FusedSync fs{};
   fs.ready = ws;
   fs.passed = ws + kFusedCounters;
@@ -1944,10 +2210,9 @@ int launch_ffn_fused(const FfnArgs& a, int* ws, hipStream_t s) {
   fs.gather = a.out_row_id;
   const int producers = static_cast<int>((gate_tiles + kXcds - 1) / kXcds * kXcds);
   const int consumers = static_cast<int>((down_tiles + kXcds - 1) / kXcds * kXcds);
-  if (a.x_rows != nullptr)
-    hipLaunchKernelGGL(ffn_fused_kernel<true>, dim3(producers + consumers), dim3(SmallTile::kThreads), 0, s, pg, pd, fs, producers);
-  else
-    hipLaunchKernelGGL(ffn_fused_kernel<false>, dim3(producers + consumers), dim3(SmallTile::kThreads), 0, s, pg, pd, fs, producers);
+  const auto kernel = a.x_rows != nullptr ? (few != kFewNever ? ffn_fused_kernel<true, true> : ffn_fused_kernel<true, false>)
+                                          : (few != kFewNever ? ffn_fused_kernel<false, true> : ffn_fused_kernel<false, false>);
+  hipLaunchKernelGGL(kernel, dim3(producers + consumers), dim3(SmallTile::kThreads), 0, s, pg, pd, fs, producers);
   return check_launch("ffn_fused_kernel");
 }
 
