@@ -268,3 +268,30 @@ def test_few_rows(dev, T, m0, H, I0, I1):
     err = (got[0][0].cpu().float() - ref).abs()
     # (the bound of the other tests of this FFN: bf16 steps of the intermediate and of the result)
     assert not (err > 2e-2 + 1e-2 * ref.abs()).any(), float(err.max())
+
+
+@pytest.mark.parametrize("T,m0,H,I0,I1", [(32, 0, 2048, 1536, 1024), (217, 0, 2048, 1536, 1024), (19, 0, 768, 512, 1024),
+                                          (40, 23, 512, 448, 96), (1, 0, 256, 64, 32)])
+def test_few_rows_with_the_norm_inside(dev, T, m0, H, I0, I1):
+    """The RMSNorm inside the few-rows launch gives what the norm's own launch gives, bit for bit; row counts on the host
+    that are not the device's change neither the launch's result nor its workspace.  (217 rows have tiles of 32 rows and a norm
+    of their own again.)"""
+    _, packed, types, x, _, off, inv, _ = _case(dev, T, m0, H, I0, I1, T + H + 1)
+    rmap = native.partition(types, 2, 0, None, want_sorted=True)[0]
+    experts = native.PackedExperts(packed, (H, I0, I1))
+    norm = (torch.randn(H, generator=torch.Generator().manual_seed(3)) * 0.1 + 1).to(torch.bfloat16).to(dev)
+
+    def run(rows, one):
+        old = native.set_one_launch_ffn(one)
+        try:
+            return native.packed_block_forward(experts, x, rmap, inv, off, rows, (norm, 1e-6), True)
+        finally:
+            native.set_one_launch_ffn(old)
+
+    want = run(_lib.i64x2((m0, T - m0)), False)
+    assert torch.equal(run(_lib.i64x2((m0, T - m0)), True), want)
+    assert torch.equal(run(_lib.i64x2((m0, T - m0)), True), want)  # on the workspace the call before it left
+    assert torch.equal(run(None, True), want)
+    if m0 == 0:
+        assert torch.allclose(run(_lib.i64x2((T, 0)), True).float(), want.float(), rtol=1e-2, atol=2e-2)
+    torch.cuda.synchronize()

@@ -310,6 +310,9 @@ struct FusedSync {
   // (sorted position -> token)
   const __bf16* x;
   const int32_t* gather;
+  // few-rows form with the norm folded in: the token rows pass through an RMSNorm on their way to the MFMAs
+  const __bf16* norm_weight;
+  float norm_eps;
 };
 
 // Fused launch: what this workgroup wrote for row block `rb` is in memory (its stores are write-through and every
@@ -387,14 +390,25 @@ __host__ __device__ inline int few_rows_fm(int64_t m0, int64_t m1, int64_t inter
   return 0;
 }
 
+// One row's bf16 pair through the RMSNorm: w * bf16(x * inv), rounded, as the norm's own kernel has it.
+__device__ __forceinline__ uint32_t rms_scale(uint32_t x, uint32_t w, float inv) {
+  return pack_bf16x2(__uint_as_float(w << 16) * round_bf16(__uint_as_float(x << 16) * inv),
+                     __uint_as_float(w & 0xffff0000u) * round_bf16(__uint_as_float(x & 0xffff0000u) * inv));
+}
+
 // MODE, ROLE, AROWS as in dual_gemm_body.  512 threads.
-template <int MODE, int FM, int ROLE, bool AROWS>
+// NORM (with AROWS; k a multiple of 256): the rows are normalised here.  Every tile sums the squares of its own rows while
+// its first weights are on their way from memory, which takes the norm's launch (6 us at 32 rows, all of it latency) out
+// of the layer.  The sums are formed in the order of rmsnorm_permute_tiled128_kernel, so the values are the same.
+template <int MODE, int FM, int ROLE, bool AROWS, bool NORM = false>
 __device__ __forceinline__ void few_rows_body(const Params& p, const int wg, const int n_wg, const FusedSync& fs) {
 #if defined(__HIP_DEVICE_COMPILE__)
   static_assert(MODE == kGateUp || MODE == kDown, "the FFN's two GEMMs");
   constexpr bool SWIGLU = MODE == kGateUp;
   constexpr int kRows = 16 * FM;
-  constexpr int kRing = FM == 1 ? 4 : 3;  // K steps in flight per wavefront: what 128 registers hold
+  // K steps in flight per wavefront: what 128 registers hold.  (Eight of them, a wavefront's whole share of 2048, at one
+  // workgroup per CU: 21.5 us in place of 20.4 for a layer of 32 rows.)
+  constexpr int kRing = FM == 1 ? 4 : 3;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l16 = lane & 15, lq = lane >> 4;
   // the partial sums of wavefront w, one KiB per 16 x 16 block: in the LDS of the 128 x 128 tile's ring
@@ -451,12 +465,14 @@ __device__ __forceinline__ void few_rows_body(const Params& p, const int wg, con
     }
     const uint32_t b_step = static_cast<uint32_t>(G.ldb) << 10;  // (blocks past the matrix's last row of B are past it)
     const uint32_t b_off = (static_cast<uint32_t>(col0 / kBlkRows) << 10) + frag;
-    u32x4 fa[kRing][FM], fb[kRing][4];
+    u32x4 fa[kRing][FM], fb[kRing][4], fw[NORM ? kRing : 1];
     auto load_a = [&](int slot, int ks) {
       const int64_t adv = static_cast<int64_t>(ks) * a_step;
       const __amdgpu_buffer_rsrc_t r = make_rsrc(a_base + adv, ks >= k_last ? 0u : (AROWS ? a_bytes - static_cast<uint32_t>(adv) : a_bytes));
 #pragma unroll
       for (int i = 0; i < FM; ++i) fa[slot][i] = __builtin_amdgcn_raw_buffer_load_b128(r, a_off[i], 0, 0);
+      if constexpr (NORM)
+        fw[slot] = __builtin_amdgcn_raw_buffer_load_b128(make_rsrc(fs.norm_weight + ks * 32, ks < k_last ? 64u : 0u), lq * 16, 0, 0);
     };
     auto load_b = [&](int slot, int ks) {
       const int64_t adv = static_cast<int64_t>(ks) * b_step;
@@ -487,6 +503,47 @@ __device__ __forceinline__ void few_rows_body(const Params& p, const int wg, con
         if (p.residual != nullptr) res = *reinterpret_cast<const u32x2*>(p.residual + static_cast<int64_t>(out_row) * G.ldc + c);
       }
     }
+    float inv[FM];
+    if constexpr (NORM) {
+      // wavefront: quarter wave % 4 of the row, eight rows wave / 4; lane: row lane / 8, 16 bytes of each 128
+      float* const ss_of = reinterpret_cast<float*>(stage + 8192);  // [row][quarter]
+      const int quarter = wave & 3, r8 = 8 * (wave >> 2) + (lane >> 3), per_quarter = G.k / 256;
+      const __amdgpu_buffer_rsrc_t rx = make_rsrc(a_base, a_bytes);
+      constexpr int kAtOnce = 4;
+#pragma unroll
+      for (int i = 0; i < FM; ++i) {
+        const int r = row0 + 16 * i + r8;
+        uint32_t off = 0x80000000u;
+        if (r < me)
+          off = static_cast<uint32_t>(fs.gather[(e ? o1 : o0) + r]) * static_cast<uint32_t>(G.k) * 2u +
+                static_cast<uint32_t>(quarter * per_quarter * 8 + (lane & 7)) * 16u;
+        float ss = 0.f;
+        for (int u = 0; u < per_quarter; u += kAtOnce) {
+          u32x4 v[kAtOnce];
+#pragma unroll
+          for (int q = 0; q < kAtOnce; ++q)
+            v[q] = __builtin_amdgcn_raw_buffer_load_b128(rx, u + q < per_quarter ? off + (u + q) * 128 : 0x80000000u, 0, 0);
+#pragma unroll
+          for (int q = 0; q < kAtOnce; ++q)
+#pragma unroll
+            for (int w = 0; w < 4; ++w) {
+              const float lo = __uint_as_float(v[q][w] << 16), hi = __uint_as_float(v[q][w] & 0xffff0000u);
+              ss += lo * lo;
+              ss += hi * hi;
+            }
+        }
+        ss += __shfl_xor(ss, 1);
+        ss += __shfl_xor(ss, 2);
+        ss += __shfl_xor(ss, 4);
+        if ((lane & 7) == 0) ss_of[(16 * i + r8) * 4 + quarter] = ss;
+      }
+      __syncthreads();
+#pragma unroll
+      for (int i = 0; i < FM; ++i) {
+        const f32x4 q = *reinterpret_cast<const f32x4*>(ss_of + (16 * i + l16) * 4);
+        inv[i] = __frsqrt_rn((q[0] + q[1] + q[2] + q[3]) / static_cast<float>(G.k) + fs.norm_eps);
+      }
+    }
     int before = 0;
     if constexpr (ROLE == 2) wait_for_count(fs, tid, counter, (e ? p.g[1].k : p.g[0].k) / 32, before);
 #pragma unroll
@@ -494,6 +551,12 @@ __device__ __forceinline__ void few_rows_body(const Params& p, const int wg, con
     for (int ks = 0; ks < share; ks += kRing) {
 #pragma unroll
       for (int s = 0; s < kRing; ++s) {
+        if constexpr (NORM) {
+#pragma unroll
+          for (int i = 0; i < FM; ++i)
+#pragma unroll
+            for (int w = 0; w < 4; ++w) fa[s][i][w] = rms_scale(fa[s][i][w], fw[s][w], inv[i]);
+        }
 #pragma unroll
         for (int i = 0; i < FM; ++i)
 #pragma unroll
@@ -1660,6 +1723,17 @@ __global__ __launch_bounds__(SmallTile::kThreads, FEW ? kFewWavesPerSimd : Small
   }
 }
 
+// The one launch in the few-rows form alone, with the RMSNorm in front of the FFN folded in: the host knows the row
+// counts.  (Tiles of 16 rows, whatever the device's counts are: the tile list is right for any split.)  At 32 rows a layer
+// takes 20.7 us where the norm's launch and the FFN's take 24; with tiles of 32 rows (217 rows) the norm's registers spill
+// and it takes 30 in place of 29, so those keep the two launches.
+__global__ __launch_bounds__(SmallTile::kThreads, kFewWavesPerSimd) void ffn_few_rows_norm_kernel(Params pg, Params pd, FusedSync fs,
+                                                                                                  int producers) {
+  const int wg = blockIdx.x, consumers = static_cast<int>(gridDim.x) - producers;
+  if (wg < producers) few_rows_body<kGateUp, 1, 1, true, true>(pg, wg, producers, fs);
+  else few_rows_body<kDown, 1, 2, false>(pd, wg - producers, consumers, fs);
+}
+
 // ---- plain FMA tiles: any transpose combination, any k --------------------------------------------------------
 // Used for what the MFMA kernel does not take: K-major operands of 4 GiB or more.
 __global__ __launch_bounds__(256) void dual_gemm_reference_layout_kernel(Params p, int trans_a, int trans_b) {
@@ -2012,6 +2086,8 @@ struct FfnArgs {
   const int32_t* out_row_id = nullptr;  // optional: sorted row r of the result goes to row out_row_id[r] of `out`
   void *keep_gate = nullptr, *keep_up = nullptr;  // optional: the gate / up projections, K-tiled like hmid
   const void* residual = nullptr;  // optional (with out_row_id): rows added to the result, laid out like `out`
+  const void* norm_weight = nullptr;  // optional (with x_rows): the rows pass through an RMSNorm first; few rows only
+  float norm_eps = 0.f;
   const void* x_rows = nullptr;    // optional: the activations in token order; `x` is then built by the fused launch
 };
 
@@ -2169,8 +2245,10 @@ int launch_ffn_fused(const FfnArgs& a, int* ws, hipStream_t s) {
   }
   const bool rows_known = a.host_rows != nullptr;
   const Few few = few_rows_of(a);
+  const int few_fm = few == kFewAlways ? few_rows_fm(a.host_rows[0], a.host_rows[1], a.inter[0], a.inter[1], a.hidden, cus) : 0;
+  if (a.norm_weight != nullptr && few_fm != 1) return 1;
   if (few == kFewAlways) {  // tiles of the few-rows form (at most one per CU)
-    const int rows = 16 * few_rows_fm(a.host_rows[0], a.host_rows[1], a.inter[0], a.inter[1], a.hidden, cus);
+    const int rows = 16 * few_fm;
     const int64_t r0 = ceil_div(a.host_rows[0], rows), r1 = ceil_div(a.host_rows[1], rows);
     gate_tiles = r0 * (a.inter[0] / 32) + r1 * (a.inter[1] / 32);
     down_tiles = (r0 + r1) * ceil_div(a.hidden, kFewCols);
@@ -2210,6 +2288,12 @@ int launch_ffn_fused(const FfnArgs& a, int* ws, hipStream_t s) {
   fs.gather = a.out_row_id;
   const int producers = static_cast<int>((gate_tiles + kXcds - 1) / kXcds * kXcds);
   const int consumers = static_cast<int>((down_tiles + kXcds - 1) / kXcds * kXcds);
+  if (a.norm_weight != nullptr) {
+    fs.norm_weight = static_cast<const __bf16*>(a.norm_weight);
+    fs.norm_eps = a.norm_eps;
+    hipLaunchKernelGGL(ffn_few_rows_norm_kernel, dim3(producers + consumers), dim3(SmallTile::kThreads), 0, s, pg, pd, fs, producers);
+    return check_launch("ffn_few_rows_norm_kernel");
+  }
   const auto kernel = a.x_rows != nullptr ? (few != kFewNever ? ffn_fused_kernel<true, true> : ffn_fused_kernel<true, false>)
                                           : (few != kFewNever ? ffn_fused_kernel<false, true> : ffn_fused_kernel<false, false>);
   hipLaunchKernelGGL(kernel, dim3(producers + consumers), dim3(SmallTile::kThreads), 0, s, pg, pd, fs, producers);
@@ -2217,6 +2301,30 @@ int launch_ffn_fused(const FfnArgs& a, int* ws, hipStream_t s) {
 }
 
 }  // namespace
+
+namespace wx {
+int launch_norm_ffn_few_rows(const void* x, const void* x_tiled, void* out, const void* residual, const int32_t* sorted_row_id,
+                             const int32_t* expert_offsets, const void* const* weights0, const void* const* weights1, void* hmid,
+                             int64_t num_rows, int64_t hidden, int64_t inter0, int64_t inter1, const int64_t* host_rows,
+                             const void* norm_weight, float eps, void* workspace, hipStream_t stream) {
+  // (hidden: what the norm's kernel takes in its whole-line form)
+  if (!x || !x_tiled || !out || !sorted_row_id || !host_rows || !norm_weight || !workspace || !(eps >= 0.f) || num_rows <= 0 ||
+      num_rows > kFewMaxRows || hidden <= 0 || hidden % 256 != 0 || hidden > 2048)
+    return 1;
+  if ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(x_tiled) | reinterpret_cast<uintptr_t>(norm_weight) |
+       reinterpret_cast<uintptr_t>(residual) | reinterpret_cast<uintptr_t>(out)) & 15)
+    return 1;
+  if (reinterpret_cast<uintptr_t>(workspace) & 3) return 1;
+  FfnArgs a{x_tiled, {weights0[0], weights1[0]}, {weights0[1], weights1[1]}, {weights0[2], weights1[2]},
+            out, hmid, host_rows, expert_offsets, num_rows, hidden, {inter0, inter1}, sorted_row_id};
+  if (check_ffn("wx_moe_block_forward", a, true, true) != WX_OK) return 1;
+  a.residual = residual;
+  a.x_rows = x;
+  a.norm_weight = norm_weight;
+  a.norm_eps = eps;
+  return launch_ffn_fused(a, static_cast<int*>(workspace), stream);
+}
+}  // namespace wx
 
 extern "C" size_t wx_ffn_fused_workspace_bytes(void) { return kFusedWorkspaceInts * sizeof(int); }
 

@@ -600,6 +600,14 @@ extern "C" int wx_moe_block_forward(const void* x, void* out, const int32_t* row
     return wx_dual_swiglu_ffn_fused(x, x_tiled, out, add_residual ? x : nullptr, expert_offsets, gate0, up0, down0, gate1,
                                     up1, down1, hmid, num_rows, hidden, inter0, inter1, host_rows_per_expert,
                                     sorted_row_id, ffn_workspace, stream);
+  if (norm_weight != nullptr) {  // few rows: all of it in one launch
+    const void* w0[3] = {gate0, up0, down0};
+    const void* w1[3] = {gate1, up1, down1};
+    const int rc = launch_norm_ffn_few_rows(x, x_tiled, out, add_residual ? x : nullptr, sorted_row_id, expert_offsets, w0, w1, hmid,
+                                            num_rows, hidden, inter0, inter1, host_rows_per_expert, norm_weight, eps,
+                                            ffn_workspace, as_stream(stream));
+    if (rc <= 0) return rc;
+  }
   if (int rc = norm_weight != nullptr
                    ? wx_rmsnorm_permute_rows_tiled(x, norm_weight, eps, x_tiled, sorted_row_id, expert_offsets, num_rows,
                                                    hidden, stream)
