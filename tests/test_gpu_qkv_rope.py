@@ -164,3 +164,26 @@ def test_qkv_rope_projection_backward(dev, B, S, H, nq, nkv, with_bias, layout):
     with torch.no_grad():
         q0, k0, v0 = ops.qkv_projection_with_rope(x.to(dev), w.to(dev), None if b is None else b.to(dev), table, nq, nkv)
     assert torch.equal(q0, gq) and torch.equal(k0, gk) and torch.equal(v0, gv)
+
+
+@pytest.mark.parametrize("layout", ["hf", "csrc"])
+@pytest.mark.parametrize("rows", [1, 127, 129, 3072, 3073])  # 3072 rows are the last of the 128 x 128 tiles at this width
+def test_qkv_rope_projection_of_few_rows_is_a_slice_of_many(dev, rows, layout):
+    """The tile shape follows the row count and a row's result does not: every accumulator sums its K steps in order."""
+    T, H, nq, nkv = 3400, 256, 16, 2
+    g = torch.Generator().manual_seed(5)
+    n = (nq + 2 * nkv) * 128
+    x = torch.randn(1, T, H, generator=g).to(torch.bfloat16).to(dev)
+    w = (torch.randn(n, H, generator=g) * 0.05).to(torch.bfloat16).to(dev)
+    b = (torch.randn(n, generator=g) * 0.5).to(torch.bfloat16).to(dev)
+    pos = torch.randint(0, 300, (3, 1, T), generator=g)
+
+    def run(m):
+        table = ops.multimodal_rope_table(pos[:, :, :m].contiguous().to(dev), wl.text_inv_freq().to(dev), wl.MROPE_SECTION, layout)
+        return ops.qkv_projection_with_rope(x[:, :m].contiguous(), w, b, table, nq, nkv)
+
+    for got, want in zip(run(rows), run(T)):
+        assert torch.equal(got, want[:, :, :rows])
+    pick = torch.tensor(sorted({0, rows // 2, rows - 1}))
+    for got, ref in zip(run(rows), _reference(x.cpu(), w.cpu(), b.cpu(), pos, nq, nkv, rows=pick, layout=layout)):
+        _close(got[:, :, pick.to(dev)], ref, f"{rows} rows")

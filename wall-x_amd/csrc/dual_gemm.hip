@@ -2030,21 +2030,27 @@ extern "C" int wx_qkv_rope_proj(const void* x, const void* weight, const void* b
   using Tail = TailTileFor<kQkvRope>;
   const int cus = device_cu_count();
   const int64_t tiles = ceil_div(num_tokens, Tile::BM) * ceil_div(n, Tile::BN);
-  const bool split = tiles < INT32_MAX && tail_split_point(static_cast<int>(tiles), 0, g.k, 0, cus) != tiles;
+  // Too few large tiles for half of the CUs (a denoise step, a short prefill): 128 x 128 tiles alone, as in launch_mfma.
+  // The table, this launch and the o projection at n 2560, k 2048: 32 rows 66 -> 45 us, 1024 rows 70 -> 48, 2048 rows
+  // 73 -> 63, 3072 rows 83 -> 76; one more row of large tiles is past the line.
+  const bool small = tiles <= cus / 2;
+  const bool split = !small && tiles < INT32_MAX && tail_split_point(static_cast<int>(tiles), 0, g.k, 0, cus) != tiles;
   p.split = split ? 1 : 0;
   p.split_cus = cus;
   hipStream_t s = as_stream(stream);
   if (table_width == head_dim) {
-    hipLaunchKernelGGL((dual_gemm_kernel<kQkvRopeFull, Tile, false, false>), dim3(cus), dim3(Tile::kThreads), 0, s, p);
-    if (split) {
-      p.split = 2;
+    if (!small)
+      hipLaunchKernelGGL((dual_gemm_kernel<kQkvRopeFull, Tile, false, false>), dim3(cus), dim3(Tile::kThreads), 0, s, p);
+    if (split || small) {
+      p.split = split ? 2 : 0;
       hipLaunchKernelGGL((dual_gemm_kernel<kQkvRopeFull, Tail, false, false>), dim3(cus * Tail::kWgPerCu),
                          dim3(Tail::kThreads), 0, s, p);
     }
   } else {
-    hipLaunchKernelGGL((dual_gemm_kernel<kQkvRope, Tile, false, false>), dim3(cus), dim3(Tile::kThreads), 0, s, p);
-    if (split) {
-      p.split = 2;
+    if (!small)
+      hipLaunchKernelGGL((dual_gemm_kernel<kQkvRope, Tile, false, false>), dim3(cus), dim3(Tile::kThreads), 0, s, p);
+    if (split || small) {
+      p.split = split ? 2 : 0;
       hipLaunchKernelGGL((dual_gemm_kernel<kQkvRope, Tail, false, false>), dim3(cus * Tail::kWgPerCu),
                          dim3(Tail::kThreads), 0, s, p);
     }
