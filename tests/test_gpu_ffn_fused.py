@@ -295,3 +295,26 @@ def test_few_rows_with_the_norm_inside(dev, T, m0, H, I0, I1):
     if m0 == 0:
         assert torch.allclose(run(_lib.i64x2((T, 0)), True).float(), want.float(), rtol=1e-2, atol=2e-2)
     torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("T,m0,H,I0,I1", [(33, 0, 512, 448, 256), (40, 23, 512, 448, 96), (200, 90, 256, 384, 128)])
+def test_few_rows_keep_the_projections(dev, T, m0, H, I0, I1):
+    """With the gate and up projections kept for a backward pass the intermediate is the same, and it is their SwiGLU."""
+    _, packed, _, _, _, off, inv, xt = _case(dev, T, m0, H, I0, I1, T)
+    p = [t.data_ptr() for t in packed]
+    stream = torch.cuda.current_stream().cuda_stream
+    pad0, pad1 = (m0 + 255) // 256 * 256, (T - m0 + 255) // 256 * 256
+    n = native.padded_sorted_rows(T) * max(I0, I1)
+    hm, hk, gate, up = (torch.zeros(n, dtype=torch.bfloat16, device=dev) for _ in range(4))
+    for rows in (_lib.i64x2((m0, T - m0)), None):
+        _lib.call("wx_dual_swiglu_gate_up", xt.data_ptr(), hm.data_ptr(), off.data_ptr(), p[0], p[1], p[3], p[4], T, H, I0, I1,
+                  rows, stream)
+        _lib.call("wx_dual_swiglu_gate_up_keep", xt.data_ptr(), hk.data_ptr(), gate.data_ptr(), up.data_ptr(), off.data_ptr(),
+                  p[0], p[1], p[3], p[4], T, H, I0, I1, rows, stream)
+        torch.cuda.synchronize()
+        used = pad0 * I0 + pad1 * I1
+        assert torch.equal(hm, hk)
+        want = torch.nn.functional.silu(gate[:used].float()).to(torch.bfloat16).float() * up[:used].float()
+        # one bf16 step of silu(gate) and one of the product
+        assert torch.allclose(hk[:used].float(), want, rtol=2.0 ** -6, atol=1e-6)
+        assert float(gate.abs().max()) > 0 and float(up.abs().max()) > 0

@@ -586,8 +586,16 @@ __device__ __forceinline__ void few_rows_body(const Params& p, const int wg, con
 #pragma unroll
         for (int r = 0; r < 4; ++r) h[r] = swiglu_bf16(g[r], u[r]);
         const int chunk = 2 * j + (lq >> 1);
-        *reinterpret_cast<u32x2*>(stage + i * kBlkBytes + l16 * 64 + ((chunk ^ ((l16 >> 2) & 3)) << 4) + (lq & 1) * 8) =
-            u32x2{pack_bf16x2(h[0], h[1]), pack_bf16x2(h[2], h[3])};
+        const int in_block = l16 * 64 + ((chunk ^ ((l16 >> 2) & 3)) << 4) + (lq & 1) * 8;
+        *reinterpret_cast<u32x2*>(stage + i * kBlkBytes + in_block) = u32x2{pack_bf16x2(h[0], h[1]), pack_bf16x2(h[2], h[3])};
+        if constexpr (ROLE == 0) {  // the projections themselves, for a backward pass
+          if (p.keep_gate != nullptr) {
+            const int64_t off = (e ? static_cast<int64_t>(pad0) * p.g[0].n * 2 : 0) +
+                                ((static_cast<int64_t>(ct) * (pad_e / kBlkRows) + row0 / kBlkRows + i) << 10) + in_block;
+            *reinterpret_cast<u32x2*>(reinterpret_cast<unsigned char*>(p.keep_gate) + off) = u32x2{pack_bf16x2(g[0], g[1]), pack_bf16x2(g[2], g[3])};
+            *reinterpret_cast<u32x2*>(reinterpret_cast<unsigned char*>(p.keep_up) + off) = u32x2{pack_bf16x2(u[0], u[1]), pack_bf16x2(u[2], u[3])};
+          }
+        }
       }
       __syncthreads();
       if (wave < FM) {  // whole blocks of the K-tiled intermediate, written through where another XCD waits for them
@@ -2141,12 +2149,12 @@ Params gate_up_params(const FfnArgs& a) {
   return p;
 }
 
-// Whether the few-rows form takes this FFN.  Not where the projections are kept for a backward pass, and not with
-// matrices beyond 31-bit byte offsets.
+// Whether the few-rows form takes this FFN.  Not with matrices beyond 31-bit byte offsets.  (Where the projections are kept
+// for a backward pass it does, as everywhere: a block's forward is the same with and without gradients.)
 Few few_rows_of(const FfnArgs& a) {
   const int cus = device_cu_count();
   const int64_t max_inter = a.inter[0] > a.inter[1] ? a.inter[0] : a.inter[1];
-  if (a.keep_gate != nullptr || a.rows > kFewMaxRows || (max_inter + 16) * (a.hidden + 32) * 2 >= (1ll << 31) ||
+  if (a.rows > kFewMaxRows || (max_inter + 16) * (a.hidden + 32) * 2 >= (1ll << 31) ||
       padded_sorted_rows(a.rows) * (a.hidden > max_inter ? a.hidden : max_inter) * 2 >= (1ll << 31))
     return kFewNever;
   if (a.host_rows != nullptr)
