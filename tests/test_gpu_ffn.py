@@ -127,6 +127,24 @@ def test_dual_gemm_k_major_layouts_through_the_c_abi(dev, shape):
         _close(o1, r1, what=f"C ABI ta={ta} tb={tb}")
 
 
+# rows of A past 2^24 bytes: the last that the MFMA kernel's 32-bit byte counts hold (below 2^26 columns), and the first
+# that they do not
+@pytest.mark.parametrize("m,k,trans_b,mfma", [(2 ** 23 + 8, 16, False, True), (2 ** 23 + 8, 40, True, True), (2 ** 26 - 8, 9, False, True),
+                                              (2 ** 26, 9, False, False)])
+def test_dual_gemm_with_very_long_k_major_rows(dev, m, k, trans_b, mfma):
+    g = torch.Generator(device=dev).manual_seed(23)
+    a = torch.empty(k, m, dtype=torch.bfloat16, device=dev).normal_(generator=g)
+    w = torch.empty((8, k) if trans_b else (k, 8), dtype=torch.bfloat16, device=dev).normal_(generator=g)
+    out = torch.full((m, 8), 7.0, dtype=torch.bfloat16, device=dev)
+    none = [torch.empty(s, dtype=torch.bfloat16, device=dev) for s in ((k, 0), (8, k) if trans_b else (k, 8), (0, 8))]
+    native.asym_dual_gmm(a, none[0], w, none[1], out, none[2], True, trans_b)
+    assert bool(_lib.load().wx_last_gemm_path() & _lib.WX_GEMM_PATH_MFMA) == mfma
+    w = (w.t() if trans_b else w).float()
+    ref, size = a.t().float() @ w, a.t().float().abs() @ w.abs()
+    # one rounding to bf16, and k exact products summed in fp32 in two different orders
+    assert ((out.float() - ref).abs() <= 2.0 ** -8 * ref.abs() + 2 * k * 2.0 ** -24 * size).all()
+
+
 @pytest.mark.parametrize("trans_a,trans_b", [(False, False), (False, True), (True, False), (True, True)])
 def test_dual_gemm_add_accumulates_onto_an_addend(dev, trans_a, trans_b):
     """wx_dual_gemm_add: out_e = op(a_e) @ op(w_e) + add_e, bit-equal to the plain product followed by an eager bf16

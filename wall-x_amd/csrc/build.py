@@ -22,7 +22,7 @@ OBJ_DIR = os.path.join(HERE, "build")
 
 SOURCES = ["common.hip", "partition.hip", "dual_gemm.hip", "mrope.hip", "rope_index.hip", "vision_index.hip",
            "fused_movers.hip", "swiglu_bwd.hip"]
-HEADERS = ["common.h", "grid_prefix.h", "tiled_layout.h", os.path.join(INCLUDE, "wallx_mi355.h")]
+HEADERS = ["common.h", "grid_prefix.h", "k_major.h", "tiled_layout.h", os.path.join(INCLUDE, "wallx_mi355.h")]
 # benchmark-only MFMA rate probe: its own library, not part of the product library or its ABI
 PROBE_SOURCE = "probe.hip"
 PROBE_LIB = os.path.join(OUT_DIR, "libwallx_probe.so")

@@ -40,6 +40,7 @@
 #include <type_traits>
 
 #include "common.h"
+#include "k_major.h"
 #include "tiled_layout.h"
 
 namespace wx {
@@ -835,9 +836,7 @@ __device__ __forceinline__ void dual_gemm_body(const Params& p, const int wg, co
   const int tr_base_a = KA ? tr_lane_base(BM * 2, wm * FM) : 0;
   const int tr_base_b = KB ? tr_lane_base(BN * 2, wn * FN) : 0;
 
-  // K-major loads: a loading wavefront fills K rows [8 wave, +8) of the slot, instruction i rows [kRows i, +kRows) of
-  // those (kRows = 1024 / row bytes).  The 16-byte LDS position lane is chunk lane % chunks of row lane / chunks, which
-  // takes the matrix chunk whose 32-byte unit index is XORed as described at tr_lane_base.  Columns past the matrix
+  // K-major loads (k_major.h): a loading wavefront fills K rows [8 wave, +8) of the slot.  Columns past the matrix
   // edge read whatever follows (the next row, or zero past the end): they only reach output rows / columns that are
   // never stored.  Rows past K are out of the descriptor's range and read as zero.  (The offset is worked out at each
   // use -- `step` keeps it from being held in registers across the loop, which has none to spare.)
@@ -845,9 +844,7 @@ __device__ __forceinline__ void dual_gemm_body(const Params& p, const int wg, co
   auto k_major_voff = [&](int i, int cols, uint32_t row_bytes, int step) {
     int l = lane;
     asm("" : "+v"(l) : "s"(step));
-    const int chunks = cols / 8, rows = 1024 / (cols * 2);
-    const int row = l / chunks, chunk = (l % chunks) ^ (row << 2) ^ (((rows * i) & 3) << 2) ^ ((wave & 1) << 1);
-    return __umul24(row, row_bytes) + static_cast<uint32_t>(chunk) * 16u + static_cast<uint32_t>(8 * wave + rows * i) * row_bytes;
+    return k_major_offset(l, wave, i, cols, row_bytes);
   };
   // ---- per-tile state ------------------------------------------------------------------------------
   struct Loader {   // where this wave's kLoadsA + kLoadsB loads per K step come from
@@ -968,7 +965,7 @@ __device__ __forceinline__ void dual_gemm_body(const Params& p, const int wg, co
         L.a_step = static_cast<int64_t>(G.lda) * (2 * BK);
         L.a_cur = reinterpret_cast<const char*>(L.a_base);
         L.a_left = L.a_bytes;
-        L.a_dec = static_cast<uint32_t>(L.a_step);
+        L.a_dec = static_cast<uint32_t>(L.a_step);  // (below 2^32: k_major_fits)
         L.pitch_a = 2u * static_cast<uint32_t>(G.lda);
       } else {
         L.a_base = G.a + static_cast<int64_t>(row0) * G.lda;
@@ -1074,14 +1071,14 @@ __device__ __forceinline__ void dual_gemm_body(const Params& p, const int wg, co
       if constexpr (KA) {
         ra = make_rsrc(L.a_cur, L.a_left);
         L.a_cur += L.a_step;
-        L.a_left = L.a_left > L.a_dec ? L.a_left - L.a_dec : 0u;
+        L.a_left = k_major_left(L.a_left, L.a_dec);
       } else {
         ra = make_rsrc(L.a_base + k0, L.a_bytes > adv ? L.a_bytes - adv : 0u);
       }
       if constexpr (KB) {
         P.rb = make_rsrc(L.b_cur, L.b_left);
         L.b_cur += L.b_step;
-        L.b_left = L.b_left > L.b_dec ? L.b_left - L.b_dec : 0u;
+        L.b_left = k_major_left(L.b_left, L.b_dec);
         P.pitch_b = L.pitch_b;
       } else {
         P.rb = make_rsrc(L.b_base + k0, L.b_bytes > adv ? L.b_bytes - adv : 0u);
@@ -1751,7 +1748,7 @@ __global__ __launch_bounds__(256) void dual_gemm_reference_layout_kernel(Params 
   for (int e = 0; e < 2; ++e) {
     const Group& G = p.g[e];
     if (G.m <= 0 || G.n <= 0) continue;
-    const int tiles_n = (G.n + 31) / 32, tiles_m = (G.m + 31) / 32;
+    const int tiles_n = (G.n - 1) / 32 + 1, tiles_m = (G.m - 1) / 32 + 1;  // (m up to INT32_MAX)
     for (int64_t t = blockIdx.x; t < static_cast<int64_t>(tiles_m) * tiles_n; t += gridDim.x) {
       const int row0 = static_cast<int>(t / tiles_n) * 32, col0 = static_cast<int>(t % tiles_n) * 32;
       float acc[4] = {0.f, 0.f, 0.f, 0.f};
@@ -1977,11 +1974,12 @@ int dual_gemm_impl(const void* in0, const void* in1, const void* w0, const void*
   }
   if ((p.g[0].m == 0 || n0 == 0) && (p.g[1].m == 0 || n1 == 0)) return WX_OK;
   const int64_t mm0 = p.g[0].m, mm1 = p.g[1].m;  // row counts left after the empty contractions are done
-  // K-major operands (A stored [k, m], B stored [k, n]) advance by whole rows of K through a 32-bit byte count
+  // K-major operands (A stored [k, m], B stored [k, n]) advance by whole rows of K through 32-bit byte counts
   bool fits = true;
   for (int e = 0; e < 2; ++e) {
-    if (trans_a && dims[e][2] * dims[e][0] * 2 >= (1ll << 32)) fits = false;
-    if (!trans_b && dims[e][2] * dims[e][1] * 2 >= (1ll << 32)) fits = false;
+    if (p.g[e].m == 0 || p.g[e].n == 0) continue;
+    if (trans_a && !k_major_fits(dims[e][2], dims[e][0])) fits = false;
+    if (!trans_b && !k_major_fits(dims[e][2], dims[e][1])) fits = false;
   }
   if (fits) {
     const int64_t tiles = ceil_div(mm0, BigTile::BM) * ceil_div(n0, BigTile::BN) + ceil_div(mm1, BigTile::BM) * ceil_div(n1, BigTile::BN);
