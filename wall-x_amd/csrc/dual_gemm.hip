@@ -1371,6 +1371,15 @@ __device__ __forceinline__ void dual_gemm_body(const Params& p, const int wg, co
           if (S.row_id != nullptr && row < S.rows) out_row[q] = S.row_id[row];
         }
       }
+      if constexpr (MODE == kDown) {
+        // The ids are waited for here, whether or not this lane stores a row.  (A row block with nothing to store skips
+        // the stores and with them the wait; the compiler then keeps the registers of the ids from being written again
+        // before the loads are back, with a wait of its own in the first K step of every ring round, which drains the
+        // ring: the one-launch layer of 260 .. 2048 rows took 28.3 us in place of 26.4 at 512 rows, hidden 2048, expert
+        // 1024.)
+#pragma unroll
+        for (int q = 0; q < kStores; ++q) asm volatile("" : "+v"(out_row[q]));
+      }
       if constexpr (RES) {
 #pragma unroll
         for (int q = 0; q < kStores; ++q) {
