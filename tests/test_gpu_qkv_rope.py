@@ -187,3 +187,24 @@ def test_qkv_rope_projection_of_few_rows_is_a_slice_of_many(dev, rows, layout):
     pick = torch.tensor(sorted({0, rows // 2, rows - 1}))
     for got, ref in zip(run(rows), _reference(x.cpu(), w.cpu(), b.cpu(), pos, nq, nkv, rows=pick, layout=layout)):
         _close(got[:, :, pick.to(dev)], ref, f"{rows} rows")
+
+
+@pytest.mark.parametrize("layout", ["hf", "csrc"])
+@pytest.mark.parametrize("rows", [200, 3400])  # the 128 x 128 tiles alone, and the 256 x 256 tiles
+def test_qkv_rope_projection_with_table_and_bias_at_any_element(dev, rows, layout):
+    """The packed table at any word and the bias at any bf16 value: what the aligned buffers give, bit for bit."""
+    H, nq, nkv = 64, 16, 2
+    g = torch.Generator().manual_seed(11)
+    n = (nq + 2 * nkv) * 128
+    x = torch.randn(1, rows, H, generator=g).to(torch.bfloat16).to(dev)
+    w = (torch.randn(n, H, generator=g) * 0.05).to(torch.bfloat16).to(dev)
+    b = (torch.randn(n, generator=g) * 0.5).to(torch.bfloat16).to(dev)
+    pos = torch.randint(0, 300, (3, 1, rows), generator=g)
+    table = ops.multimodal_rope_table(pos.to(dev), wl.text_inv_freq().to(dev), wl.MROPE_SECTION, layout)
+    want = ops.qkv_projection_with_rope(x, w, b, table, nq, nkv)
+    for off in (1, 2, 3):
+        t2 = table.new_empty(table.numel() + 4)[off:off + table.numel()].view_as(table).copy_(table)
+        b2 = b.new_empty(n + 8)[off:off + n].copy_(b)
+        assert t2.data_ptr() % 16 == 4 * off and b2.data_ptr() % 8 == 2 * off
+        for got, ref in zip(ops.qkv_projection_with_rope(x, w, b2, t2, nq, nkv), want):
+            assert torch.equal(got, ref)

@@ -50,6 +50,7 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x4_word __attribute__((ext_vector_type(4), aligned(4)));  // four words at any word's address
 
 constexpr int BK = 32;
 constexpr int kStages = 4;                     // ring slots per operand
@@ -1508,13 +1509,14 @@ __device__ __forceinline__ void dual_gemm_body(const Params& p, const int wg, co
         constexpr int kWidth = MODE == kQkvRope ? 64 : 128;  // table entries per token: shared by d and d + 64, or one each
 #pragma unroll
         for (int i = 0; i < FM; ++i) {
-          // cos | sin of this lane's channels, four per load, all loads ahead of their first use
+          // cos | sin of this lane's channels, four per load (the table need only be word-aligned), all loads ahead of their
+          // first use
           u32x4 cs[kWidth / 16];
           if (rotate) {
             const int row = (wm * FM + i) * 16 + e16;
             const uint32_t* t = p.rope_table + static_cast<int64_t>(S.row0 + (row < S.rows ? row : 0)) * kWidth + 4 * eq;
 #pragma unroll
-            for (int j = 0; j < kWidth / 16; ++j) cs[j] = *reinterpret_cast<const u32x4*>(t + j * 16);
+            for (int j = 0; j < kWidth / 16; ++j) cs[j] = *reinterpret_cast<const u32x4_word*>(t + j * 16);
           }
 #pragma unroll
           for (int j = 0; j < 4; ++j) {
