@@ -79,3 +79,12 @@ def test_a_ring_is_never_drained_in_its_k_loop(loops):
 def test_no_k_loop_spills(loops):
     bad = [(k, [x for x in body if x.startswith("scratch_")]) for k, body in loops if any(x.startswith("scratch_") for x in body)]
     assert not bad, bad
+
+
+@pytest.mark.parametrize("kernel", ["dual_gemm_kernel", "dual_gemm_few_rows_kernel", "ffn_few_rows_norm_kernel", "ffn_fused_kernel"])
+def test_the_build_warns_of_a_spill_in_any_gemm_kernel(kernel, capsys):
+    remark = "f.hip:1:1: remark: Function Name: _ZN2wx{}E [-Rpass]\nf.hip:1:1: remark:     ScratchSize [bytes/lane]: {} [-Rpass]\n"
+    csrc_build._check_resources("dual_gemm.hip", remark.format(kernel, 96))
+    assert not capsys.readouterr().err
+    csrc_build._check_resources("dual_gemm.hip", remark.format(kernel, 100))
+    assert kernel in capsys.readouterr().err

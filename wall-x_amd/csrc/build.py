@@ -52,21 +52,21 @@ def _newer(target: str, deps) -> bool:
     return all(os.path.getmtime(d) <= t for d in deps)
 
 
-# The large-tile GEMM kernels use every register a wave can have; a small source change can push values of the K
-# loop into scratch memory, which costs a factor of three and shows in no test.  Their compile prints the
-# resource-usage remarks and this limit on "ScratchSize [bytes/lane]" turns a spill into a loud warning.
-# (Values that are only live outside the K loop do spill: up to 52 bytes in the tiled kernels and 88 in the
-# large-tile variants with K-major operands, all measured at full speed.)
-RESOURCE_CHECKED = {"dual_gemm.hip": ("dual_gemm_kernel", 96)}
+# The GEMM kernels use every register a wave can have; a small source change can push values of the K loop into scratch
+# memory, which costs a factor of three and shows in no test of results.  Their compile prints the resource-usage remarks
+# and this limit on "ScratchSize [bytes/lane]" of any kernel of the file turns a spill into a loud warning.
+# (Values that are only live outside the K loop do spill: 64 bytes in the few-rows gate/up kernel, 24 in the one with the
+# norm, 8 in the large tile with a K-major A; tests/test_k_loop_assembly.py shows that none is inside a loop.)
+RESOURCE_CHECKED = {"dual_gemm.hip": 96}
 
 
 def _check_resources(src, stderr):
-    name_part, limit = RESOURCE_CHECKED[src]
+    limit = RESOURCE_CHECKED[src]
     current = None
     for line in stderr.splitlines():
         if "Function Name:" in line:
             current = line.split("Function Name:")[1].split()[0]
-        elif "ScratchSize [bytes/lane]:" in line and current and name_part in current:
+        elif "ScratchSize [bytes/lane]:" in line and current:
             size = int(line.split("ScratchSize [bytes/lane]:")[1].split()[0])
             if size > limit:
                 sys.stderr.write(f"[wallx_mi355] WARNING: {current} spills {size} bytes per lane to scratch "
