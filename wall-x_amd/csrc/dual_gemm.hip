@@ -759,12 +759,6 @@ __device__ __forceinline__ void dual_gemm_body(const Params& p, const int wg, co
   tiles_m[1] = (g1.m + BM - 1) / BM;
   tiles_n[1] = (g1.n + kTileN - 1) / kTileN;
   if (g1.m <= 0 || g1.n <= 0) tiles_m[1] = tiles_n[1] = 0;
-  if constexpr (TILED_IN && std::is_same_v<TS, BigTileFor<MODE>>) {
-    // (a launch of large tiles beside one that runs the few-rows form)
-    if (p.few_rows_cus != 0 && few_rows_fm(g0.m, g1.m, MODE == kGateUp ? g0.n : g0.k, MODE == kGateUp ? g1.n : g1.k,
-                                           MODE == kGateUp ? g0.k : g0.n, p.few_rows_cus) != 0)
-      return;
-  }
   if (p.gate != 0) {
     constexpr int kBigN = SWIGLU ? BigTile::BN / 2 : BigTile::BN;
     auto big = [](int m, int n) { return (m <= 0 || n <= 0) ? 0 : ((m + BigTile::BM - 1) / BigTile::BM) * ((n + kBigN - 1) / kBigN); };
@@ -1879,6 +1873,8 @@ int launch_mfma(Params p, int64_t tiles_lo, int64_t tiles_hi, hipStream_t s, con
                        dim3(SmallTile::kThreads), 0, s, p);
   }
   if (big) {
+    // (a problem of the few-rows form has at most cus / 4 + 4 large tiles, a quarter of its own and one row block's
+    // remainder each: this launch leaves it alone)
     p.gate = small ? 2 : 0;
     using Big = BigTileFor<MODE>;
     static_assert(Big::kWgPerCu == 1, "the split counts one large tile per CU and round");
