@@ -240,6 +240,8 @@ def test_one_launch_ffn_on_two_streams_at_once(dev):
     (32, 0, 2048, 1536, 1024), (128, 0, 2048, 1536, 1024), (129, 0, 2048, 1536, 1024), (217, 0, 2048, 1536, 1024),
     (256, 0, 2048, 1536, 1024), (257, 0, 2048, 1536, 1024), (40, 23, 512, 448, 96), (33, 33, 288, 64, 32),
     (50, 1, 1280, 320, 1024), (1024, 700, 256, 64, 32),
+    # a wide expert: without row counts the large tiles are launched as well, and the device settles which form runs
+    (32, 0, 2048, 11008, 1024), (217, 3, 2048, 11008, 1024), (256, 0, 2048, 11008, 1024),
 ])
 def test_few_rows(dev, T, m0, H, I0, I1):
     ws_, packed, types, x, res, off, inv, xt = _case(dev, T, m0, H, I0, I1, T + H)
@@ -318,3 +320,59 @@ def test_few_rows_keep_the_projections(dev, T, m0, H, I0, I1):
         # one bf16 step of silu(gate) and one of the product
         assert torch.allclose(hk[:used].float(), want, rtol=2.0 ** -6, atol=1e-6)
         assert float(gate.abs().max()) > 0 and float(up.abs().max()) > 0
+
+
+def _norm_block(dev, T, seed):
+    """A few-rows block with the norm inside: (forward of x into out through the C ABI on a stream, x, row counts)."""
+    H, I0, I1 = 2048, 1536, 1024
+    _, packed, types, x, _, off, inv, _ = _case(dev, T, 0, H, I0, I1, seed)
+    rmap = native.partition(types, 2, 0, None, want_sorted=True)[0]
+    experts = native.PackedExperts(packed, (H, I0, I1))
+    norm = (torch.randn(H, generator=torch.Generator().manual_seed(seed)) * 0.1 + 1).to(torch.bfloat16).to(dev)
+    x_elems, h_elems = experts.sizes(T)
+    xt, hm = (torch.zeros(n, dtype=torch.bfloat16, device=dev) for n in (x_elems, h_elems))
+    work, rows = _workspace(dev), _lib.i64x2((0, T))
+
+    def run(x, out, stream, one=True):
+        _lib.call("wx_moe_block_forward", x.data_ptr(), out.data_ptr(), rmap.data_ptr(), inv.data_ptr(), off.data_ptr(),
+                  *experts.ptrs, xt.data_ptr(), hm.data_ptr(), T, H, I0, I1, rows, norm.data_ptr(), 1e-6, 1,
+                  work.data_ptr() if one else None, stream)
+
+    return run, x, work, (packed, norm, experts)
+
+
+def test_few_rows_with_the_norm_in_place_on_two_streams_and_replayed(dev):
+    """The one launch with the norm where its output is its input, on two streams at once, and from a HIP graph whose
+    input changes between replays: the separate launches' bits, and a workspace that is zero again."""
+    blocks = [_norm_block(dev, T, seed) for T, seed in ((32, 31), (117, 32))]
+    here = torch.cuda.current_stream().cuda_stream
+    want = []
+    for run, x, work, _ in blocks:
+        want.append(torch.empty_like(x))
+        run(x, want[-1], here, one=False)
+        y = x.clone()
+        run(y, y, here)  # in place
+        assert torch.equal(y, want[-1])
+    streams = [torch.cuda.Stream() for _ in blocks]
+    outs = [torch.zeros_like(x) for _, x, _, _ in blocks]
+    torch.cuda.synchronize()
+    for _ in range(20):
+        for (run, x, _, _), out, st in zip(blocks, outs, streams):
+            run(x, out, st.cuda_stream)
+    torch.cuda.synchronize()
+    for (_, _, work, _), out, ref in zip(blocks, outs, want):
+        assert torch.equal(out, ref) and int(work.abs().sum()) == 0
+
+    run, x, work, _ = blocks[0]
+    still, out = x.clone(), torch.empty_like(x)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        run(still, out, torch.cuda.current_stream().cuda_stream)
+    for scale in (1.0, 0.5, 3.0):
+        still.copy_(x * scale)
+        ref = torch.empty_like(x)
+        run(still, ref, here, one=False)
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, ref) and int(work.abs().sum()) == 0
