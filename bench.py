@@ -831,7 +831,8 @@ def ceiling_measurements(dev, x, weights, m0):
     `value`): (1) back-to-back bf16 MFMA instructions with operands held in registers, on zeros and on values
     drawn like the benchmark's activations and weights -- the sustained MFMA rate depends on the operand values
     (switching activity moves the clock the chip holds), so the nominal 2.5 PFLOP/s is not reachable on random
-    data; (2) the vendor GEMM (torch.matmul -> hipBLASLt) on the VL expert's two GEMM shapes with the benchmark's
+    data; in the GEMM kernels' form (16x16x32, one operand changing from each instruction to the next) and, on the
+    random values, in the two they do not use; (2) the vendor GEMM (torch.matmul -> hipBLASLt) on the VL expert's two GEMM shapes with the benchmark's
     own tensors, without the SwiGLU epilogue or the second expert."""
     import ctypes
     import torch
@@ -841,20 +842,23 @@ def ceiling_measurements(dev, x, weights, m0):
     probe = ctypes.CDLL(os.path.join(ROOT, "wall-x_amd", "wallx_mi355", "libwallx_probe.so"))
     probe.wxprobe_mfma_operand_bytes.restype = ctypes.c_size_t
     probe.wxprobe_mfma_rate.restype = ctypes.c_int
-    probe.wxprobe_mfma_rate.argtypes = [ctypes.c_void_p, ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p]
+    probe.wxprobe_mfma_rate.argtypes = [ctypes.c_void_p, ctypes.c_int, ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p]
     n = probe.wxprobe_mfma_operand_bytes() // 2
     sink = torch.zeros(1, dtype=torch.float32, device=dev)
     flops = ctypes.c_double(0.0)
     stream = torch.cuda.current_stream().cuda_stream
     g = torch.Generator(device=dev).manual_seed(1)
-    data = torch.randn(n, device=dev, generator=g)
-    data[n // 2:] *= 0.02  # half the fragments look like activations N(0, 1), half like weights N(0, 0.02)
-    for name, ops in (("zeros", torch.zeros(n, dtype=torch.bfloat16, device=dev)), ("normal", data.to(torch.bfloat16))):
+    data = torch.randn(4, 2, n // 8, device=dev, generator=g)
+    data[:, 1] *= 0.02  # each wavefront's A fragments look like activations N(0, 1), its B fragments like weights N(0, 0.02)
+    zeros, normal = torch.zeros(n, dtype=torch.bfloat16, device=dev), data.to(torch.bfloat16).contiguous()
+    for name, ops, form in (("zeros_operands", zeros, 2), ("normal_operands", normal, 2),
+                            ("normal_operands_both_change", normal, 1), ("normal_operands_32x32x16", normal, 0)):
         def run():
-            if probe.wxprobe_mfma_rate(ops.data_ptr(), 4000, sink.data_ptr(), ctypes.byref(flops), stream) != 0:
+            iters = 4000 if form == 0 else 8000  # (half the operations per instruction)
+            if probe.wxprobe_mfma_rate(ops.data_ptr(), form, iters, sink.data_ptr(), ctypes.byref(flops), stream) != 0:
                 raise RuntimeError("wxprobe_mfma_rate failed")
         t, _ = event_ms(run, 5, warm=2)
-        out[f"mfma_only_{name}_operands_tflops"] = round(flops.value / t / 1e9, 1)
+        out[f"mfma_only_{name}_tflops"] = round(flops.value / t / 1e9, 1)
     (g0, u0, d0) = weights[0]
     H, I0 = g0.shape[1], g0.shape[0]
     xv = x[:m0]

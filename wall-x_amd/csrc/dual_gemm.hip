@@ -88,9 +88,12 @@ struct TileShape {
 // of the four wavefronts on gate/up and behind them elsewhere.)
 using BigTile = TileShape<256, 256, 2, 4, 4>;
 // The small tile, for problems with too few large tiles to fill the chip: two workgroups per CU, each eight
-// wavefronts as 4 x 2 (wave tile 32 x 64), four of them loading, like the large tile.  (Four wavefronts of 64 x 64
-// measure 6 % slower on a denoise step; timestamps inside that kernel put 254 ns on a K step whose 8 MFMAs per
-// wavefront need 110, and 169 ns with the loads taken out.)
+// wavefronts as 4 x 2 (wave tile 32 x 64), four of them loading, like the large tile.  (Measured with 32x32x16 products:
+// four wavefronts of 64 x 64 are 6 % slower on a denoise step; timestamps inside that kernel put 254 ns on a K step whose
+// MFMAs need 110, and 169 ns with the loads taken out.)  16x16x32 products are faster here once every CU has two tiles or
+// one and a busy neighbour, and slower where most CUs are idle and the clock is high anyway: gate/up alone at 2048 rows
+// (hidden 2048, expert 1024) 20.4 -> 19.3 us, at 512 rows 13.4 -> 14.7; a denoise layer in one launch, permute inside, 2048
+// rows 35.3 -> 33.5, 512 rows 28.0 -> 28.1.
 using SmallTile = TileShape<128, 128, 4, 2, 4>;
 // the same eight wavefronts as 4 x 2: wave tile 64 x 128, for the epilogue that needs a wavefront to hold whole
 // 128-column heads (the rotation partner of a channel is 64 columns away)
@@ -373,8 +376,10 @@ __device__ __forceinline__ float swiglu_bf16(float gate, float up) {
 // memory latencies in place of K / 32 barriers.  Each row block reads the weights again (through L2: the tiles of a
 // column are on one XCD where the column tiles are a multiple of eight), which is why many rows keep the large tiles.
 // Measured (hidden 2048, experts 11008 / 1024, per layer): 32 rows 17 us where the 128 x 128 tiles take 35, 217 rows 22 where
-// they take 34.  The line lies where the tiles of a round of their own run out (256 rows at these widths): beyond it a second
-// round of small tiles re-reads the weights as often as the larger tiles' K loop takes.
+// they take 34.  The line lies where the tiles of a round of their own run out (256 rows at these widths): in a second round
+// the weights are read as often again and the next tile's chain of latencies begins.  36 layers with the norm, two rounds of
+// small tiles / 128 x 128 tiles: 260 rows 1471 / 1459 us, 320 rows 1510 / 1463, 512 rows 1520 / 1460; 256 rows, one round,
+// 1040.
 constexpr int kFewCols = 64;       // rows of B per tile
 constexpr int kFewMaxFm = 2;       // row blocks of 16 per tile: 1 or 2
 constexpr int kFewWavesPerSimd = 4;  // two workgroups per CU, which the fused launch counts on (128 registers)
@@ -1157,8 +1162,9 @@ __device__ __forceinline__ void dual_gemm_body(const Params& p, const int wg, co
   // first half of the products, its second half only for the second.  So the cut operand has one register set (each
   // half is refilled while the other half's products run) and the other one has two, by the step's parity.
   // Why 16x16x32 and not 32x32x16 (the same operations per cycle): on normally distributed operands the chip holds a
-  // clock that depends on what the instructions switch, and back-to-back MFMAs reach 2.04 PFLOP/s in this shape
-  // against 1.81 in the other; 2.09 when each differs from the one before in one operand only (the serpentine below).
+  // clock that depends on what the instructions switch, and back-to-back MFMAs reach 1.96 PFLOP/s in this shape
+  // against 1.77 in the other; 2.06 when each differs from the one before in one operand only (the serpentine below);
+  // probe.hip measures all three.
   // 28160 + 1024 rows, before and after on one chip: gate/up 1.892 -> 1.757 ms (1.35 -> 1.45 PFLOP/s), down 0.950 ->
   // 0.887 ms; the row-major op at 28160 x 11008 x 2048: forward 0.967 -> 0.900 ms, dX 0.967 -> 0.917, dW (half the
   // tokens) 0.540 -> 0.511.  On all-zero operands, where the clock is the same for both shapes, neither is faster.
