@@ -44,10 +44,11 @@ def parse():
     ap.add_argument("--cpu-seqs", type=int, default=32, help="sequences of the batch the CPU baseline runs (32 = all)")
     ap.add_argument("--kernel-loop", default=None,
                     choices=["gate_up", "down", "down_unpermute", "permute", "permute_plain", "unpermute", "partition", "copy",
-                             "layer_one_launch", "mrope", "mrope_packed", "mrope_copy", "config2_index"],
+                             "layer_one_launch", "layer_with_norm", "mrope", "mrope_packed", "mrope_copy", "config2_index"],
                     help="profiling aid: run only this kernel --steps times (no JSON line); 'layer_one_launch' is "
                          "permute, gate/up and down as the one launch a denoise step gets (three launches at config "
-                         "3, where it does not apply); 'copy' is a plain "
+                         "3, where it does not apply), 'layer_with_norm' the block with its RMSNorm and the residual (one "
+                         "launch for few rows, a norm launch in front otherwise); 'copy' is a plain "
                          "device-to-device copy of the [T, H] activations, the known-size yardstick for HBM counters; "
                          "'mrope' / 'mrope_packed' are the M-RoPE apply at config 2 from the two tables / from the "
                          "packed table, 'mrope_copy' a device copy of q and k of the same shape, 'config2_index' the "
@@ -56,9 +57,10 @@ def parse():
                     help="with --kernel-loop: the benchmark's normally distributed activations and weights, or all-zero "
                          "ones (same launches and cycle counts, far less switching activity: the pair shows which clock "
                          "the chip holds under each)")
-    ap.add_argument("--kernel-shape", default="config3", choices=["config3", "denoise"],
+    ap.add_argument("--kernel-shape", default="config3", choices=["config3", "denoise", "denoise_1"],
                     help="with --kernel-loop: the batch the kernel runs on -- config 3 (29184 tokens, 28160 VL + 1024 "
-                         "action) or config 4's denoise step (2048 action tokens, VL group empty)")
+                         "action), config 4's denoise step (2048 action tokens, VL group empty) or one robot's (32 action "
+                         "tokens)")
     return ap.parse_args()
 
 
@@ -105,8 +107,8 @@ def main():
 
     # ---- synthetic inputs, resident in HBM ----------------------------------------------------------
     x_cpu, types_cpu, w_cpu = wl.config3()
-    if args.kernel_loop and args.kernel_shape == "denoise":
-        T = 2048
+    if args.kernel_loop and args.kernel_shape != "config3":
+        T = 2048 if args.kernel_shape == "denoise" else 32
         x_cpu = wl.randn((1, T, H), 1.0, torch.bfloat16, torch.Generator().manual_seed(4))
         types_cpu = torch.ones(1, T, dtype=torch.bool)
     x = x_cpu.view(T, H).to(dev)
@@ -172,6 +174,14 @@ def main():
                   pg0.data_ptr(), pu0.data_ptr(), pd0.data_ptr(), pg1.data_ptr(), pu1.data_ptr(), pd1.data_ptr(),
                   hmid.data_ptr(), T, H, I0, I1, _lib.i64x2((m0, m1)), inverse.data_ptr(), counters.data_ptr(), stream)
 
+    norm = torch.ones(H, dtype=torch.bfloat16, device=dev)
+
+    def layer_with_norm():
+        _lib.call("wx_moe_block_forward", x.data_ptr(), y.data_ptr(), row_id_map.data_ptr(), inverse.data_ptr(),
+                  offsets.data_ptr(), pg0.data_ptr(), pu0.data_ptr(), pd0.data_ptr(), pg1.data_ptr(), pu1.data_ptr(),
+                  pd1.data_ptr(), x_tiled.data_ptr(), hmid.data_ptr(), T, H, I0, I1, _lib.i64x2((m0, m1)), norm.data_ptr(),
+                  1e-6, 1, counters.data_ptr(), stream)
+
     def step():  # partition -> permute -> gate/up + SwiGLU -> down with the unpermute in its stores
         partition()
         permute()
@@ -184,7 +194,7 @@ def main():
                 t.zero_()
         permute(); gate_up(); down()
         fn = {"gate_up": gate_up, "down": down, "down_unpermute": down_unpermute, "permute": permute,
-              "permute_plain": permute_plain, "layer_one_launch": layer_one_launch,
+              "permute_plain": permute_plain, "layer_one_launch": layer_one_launch, "layer_with_norm": layer_with_norm,
               "unpermute": unpermute, "partition": partition,
               "copy": lambda: x_sorted.copy_(x)}[args.kernel_loop]
         for _ in range(args.steps):
