@@ -867,7 +867,7 @@ def ceiling_measurements(dev, x, weights, m0):
             iters = 4000 if form == 0 else 8000  # (half the operations per instruction)
             if probe.wxprobe_mfma_rate(ops.data_ptr(), form, iters, sink.data_ptr(), ctypes.byref(flops), stream) != 0:
                 raise RuntimeError("wxprobe_mfma_rate failed")
-        t, _ = event_ms(run, 5, warm=2)
+        t, _ = event_ms(run, 10, warm=40)  # (~0.1 s for the clock to settle at what these values allow)
         out[f"mfma_only_{name}_tflops"] = round(flops.value / t / 1e9, 1)
     (g0, u0, d0) = weights[0]
     H, I0 = g0.shape[1], g0.shape[0]
