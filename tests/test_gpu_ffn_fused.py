@@ -273,7 +273,8 @@ def test_few_rows(dev, T, m0, H, I0, I1):
 
 
 @pytest.mark.parametrize("T,m0,H,I0,I1", [(32, 0, 2048, 1536, 1024), (217, 0, 2048, 1536, 1024), (19, 0, 768, 512, 1024),
-                                          (40, 23, 512, 448, 96), (1, 0, 256, 64, 32)])
+                                          (40, 23, 512, 448, 96), (1, 0, 256, 64, 32),
+                                          (9, 4, 1024, 64, 32), (9, 4, 1280, 64, 32), (9, 4, 1536, 64, 32), (9, 4, 1792, 64, 32)])
 def test_few_rows_with_the_norm_inside(dev, T, m0, H, I0, I1):
     """The RMSNorm inside the few-rows launch gives what the norm's own launch gives, bit for bit; row counts on the host
     that are not the device's change neither the launch's result nor its workspace.  (217 rows have tiles of 32 rows and a norm
