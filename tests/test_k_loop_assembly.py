@@ -24,8 +24,8 @@ def compile_to_assembly(source, out):
 
 
 def k_loops(text):
-    """(kernel, instructions) of every innermost loop with MFMAs, from the block of its first MFMA on: what lies before it
-    runs where a tile ends, not in every pass."""
+    """(kernel, instructions) of every innermost loop with MFMAs, from the block of its first MFMA to its last MFMA or
+    barrier: what lies before and behind runs where a tile ends, not in every pass."""
     for kernel, body in re.findall(r"^(_ZN\S+):[^\n]*\n(.*?)^\.Lfunc_end", text, re.M | re.S):
         lines = [line.split(";")[0].strip() for line in body.split("\n")]
         labels = {line[:-1]: i for i, line in enumerate(lines) if line.startswith(".LBB") and line.endswith(":")}
@@ -39,7 +39,8 @@ def k_loops(text):
                 continue
             first = next(i for i in range(a, b) if "v_mfma" in lines[i])
             start = max(i for i in range(a, first) if lines[i].startswith(".LBB"))
-            yield kernel, [line for line in lines[start:b + 1] if line and not line.startswith(".")]
+            stop = max(i for i in range(a, b) if "v_mfma" in lines[i] or lines[i].startswith("s_barrier"))
+            yield kernel, [line for line in lines[start:stop + 1] if line and not line.startswith(".")]
 
 
 def stray_waits(loop):

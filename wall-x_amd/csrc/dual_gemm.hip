@@ -90,10 +90,7 @@ using BigTile = TileShape<256, 256, 2, 4, 4>;
 // The small tile, for problems with too few large tiles to fill the chip: two workgroups per CU, each eight
 // wavefronts as 4 x 2 (wave tile 32 x 64), four of them loading, like the large tile.  (Measured with 32x32x16 products:
 // four wavefronts of 64 x 64 are 6 % slower on a denoise step; timestamps inside that kernel put 254 ns on a K step whose
-// MFMAs need 110, and 169 ns with the loads taken out.)  16x16x32 products are faster here once every CU has two tiles or
-// one and a busy neighbour, and slower where most CUs are idle and the clock is high anyway: gate/up alone at 2048 rows
-// (hidden 2048, expert 1024) 20.4 -> 19.3 us, at 512 rows 13.4 -> 14.7; a denoise layer in one launch, permute inside, 2048
-// rows 35.3 -> 33.5, 512 rows 28.0 -> 28.1.
+// MFMAs need 110, and 169 ns with the loads taken out.)
 using SmallTile = TileShape<128, 128, 4, 2, 4>;
 // the same eight wavefronts as 4 x 2: wave tile 64 x 128, for the epilogue that needs a wavefront to hold whole
 // 128-column heads (the rotation partner of a channel is 64 columns away)
@@ -1171,10 +1168,12 @@ __device__ __forceinline__ void dual_gemm_body(const Params& p, const int wg, co
   // The operands go in as (B, A), so a lane's four accumulator registers are four consecutive COLUMNS of one row of C:
   // the epilogue packs them into 8 bytes without exchanging anything between lanes.
   constexpr bool kCutA = FM >= FN;
+  // The FFN's small tile has the registers for all of two K steps' fragments and does not cut its products: k_step_whole.
+  constexpr bool kWhole = TILED_IN && std::is_same_v<TS, SmallTile>;
   constexpr int kFirstReads = (kCutA ? FM / 2 : FM) * (KA ? 2 : 1) + (kCutA ? FN : FN / 2) * (KB ? 2 : 1);
   constexpr int kSecondReads = kCutA ? FM / 2 * (KA ? 2 : 1) : FN / 2 * (KB ? 2 : 1);
   f32x4 acc[FM][FN];
-  bf16x8 fa[kCutA ? 1 : 2][FM], fb[kCutA ? 2 : 1][FN];
+  bf16x8 fa[kCutA && !kWhole ? 1 : 2][FM], fb[kCutA || kWhole ? 2 : 1][FN];
 
   // K-major slot: K values [8 lq, +8) for the lane's column of 16-column block `blk` (counted from the wave's first
   // block): two transposing reads of four rows each.
@@ -1313,6 +1312,51 @@ __device__ __forceinline__ void dual_gemm_body(const Params& p, const int wg, co
     read_first(slot_a((S + 1) % kStages), slot_b((S + 1) % kStages), (S + 1) & 1, ld_ks);
     mma(1, S & 1);
     schedule_after(std::integral_constant<int, (LD && kOdd) ? kPairLoadsA : 0>{});
+  };
+  // The same step with whole fragment sets: on entry set S & 1 holds all of slot S, every wavefront has read it, and slot
+  // S + 1 is complete.  Slot S is refilled and slot S + 1 read into the other set while the products run, and one wait and
+  // barrier end the step.  A step cut in two waits for the LDS twice, one after the other (the reads behind its first
+  // products are held up by the wait for those products' operands), which shows where few CUs are busy and the memory is
+  // quick: gate/up by itself at 512 rows (hidden 2048, expert 1024) 14.6 -> 13.8 us, down 10.1 -> 9.9, at 2048 rows 17.4 -> 17.0
+  // and 12.2 -> 11.9; 36 layers, the block alone, 640 rows 1198 -> 1183 us.  The reads go out among the first half of the
+  // products and the loads, at which a loading wavefront stalls, behind them, one at a time (all of them among the first
+  // products: 14.4; among the last: 15.1; the reads among the first quarter 15.3, three quarters 14.6).
+  auto read_whole = [&](const unsigned char* sa, const unsigned char* sb, int par, int step) {
+    fb[par][0] = read_b(sb, 0, step);
+#pragma unroll
+    for (int i = 0; i < FM; ++i) fa[par][i] = read_a(sa, i, step);
+#pragma unroll
+    for (int j = 1; j < FN; ++j) fb[par][j] = read_b(sb, j, step);
+  };
+  auto k_step_whole = [&](auto with_loads, auto step_c, Loader& L, int ld_ks) {
+    constexpr bool LD = decltype(with_loads)::value;
+    constexpr int S = decltype(step_c)::value, kMfma = FM * FN, kReads = FM + FN;
+    if constexpr (LD) {
+      issue_a(L, ld_ks + S, slot_a(S), pend);
+      issue_b(pend, slot_b(S), ld_ks);
+    }
+    read_whole(slot_a((S + 1) % kStages), slot_b((S + 1) % kStages), (S + 1) & 1, ld_ks);
+#pragma unroll
+    for (int j = 0; j < FN; ++j)
+#pragma unroll
+      for (int ii = 0; ii < FM; ++ii) {
+        const int i = (j & 1) ? FM - 1 - ii : ii;
+        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[S & 1][j], fa[S & 1][i], acc[i][j], 0, 0, 0);
+      }
+    constexpr unsigned kLoadBefore = 0x74;  // one load each before products 2, 4, 5 and 6 (of 0 .. 7)
+    static_assert(!kWhole || (kMfma == 8 && kLoadsPerStep == 4), "the loads' places");
+#pragma unroll
+    for (int m = 0; m < kMfma; ++m) {
+      const int reads = m < kMfma / 2 ? (m + 1) * kReads / (kMfma / 2) - m * kReads / (kMfma / 2) : 0;
+#pragma unroll
+      for (int q = 0; q < reads; ++q) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+      if (LD && (kLoadBefore >> m & 1)) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    // my reads of slot S + 1 have returned; slot S + 2 is complete (the loads of this step and the one before may be in flight)
+    __builtin_amdgcn_s_waitcnt(waitcnt_imm(LD ? (kStages - 2) * kLoadsPerStep : 63, 0));
+    barrier_no_fence();
   };
   // ... and with A alone in pairs (NN).  B keeps the slot-by-slot schedule of k_step_as (the refill of slot S - 1 at
   // the start of step S, its descriptor prepared after the barrier of step S - 1), A the pairs' (after the barrier of
@@ -1584,12 +1628,12 @@ __device__ __forceinline__ void dual_gemm_body(const Params& p, const int wg, co
     setup_store(tc, S);
     // Consumer of a fused launch: every tile starts from an empty ring.  The weights of the first ring slots are
     // fetched at once, the intermediate only after the row block's producers have finished; then the ring is as the
-    // plain prologue leaves it (the last slot's B half goes out in the first K step), with every load landed.
+    // plain prologue leaves it, with every load landed.
     auto consumer_prologue = [&]() {
-      static_assert(ROLE != 2 || TILED_IN, "the fused launch runs the tiled forms");
+      static_assert(ROLE != 2 || kWhole, "the fused launch runs the FFN's small tile");
       if constexpr (LD) {
 #pragma unroll
-        for (int s = 0; s + 1 < kStages; ++s) issue_b_ahead(L, s, slot_b(s));
+        for (int s = 0; s < kStages; ++s) issue_b_ahead(L, s, slot_b(s));
       }
       if constexpr (!LD && ASYM) {
         if (warm_pending) {
@@ -1630,13 +1674,23 @@ __device__ __forceinline__ void dual_gemm_body(const Params& p, const int wg, co
 #pragma unroll
       for (int s = 0; s < kStages; ++s) {
         issue_a(L, s, slot_a(s), pend);
-        if (s + 1 < kStages) issue_b(pend, slot_b(s));  // the last slot's B half goes out in the first K step
+        if (kWhole || s + 1 < kStages) issue_b(pend, slot_b(s));  // (else the last slot's B half goes out in the first K step)
       }
-      // slot 0 must be complete before its first fragments are read: the younger loads may remain in flight
-      __builtin_amdgcn_s_waitcnt(waitcnt_imm((kStages - 2) * kLoadsPerStep + kLoadsA, 15));
+      // slot 0 (and 1, where the first K step reads it) must be complete: the younger loads may remain in flight
+      __builtin_amdgcn_s_waitcnt(waitcnt_imm((kStages - 2) * kLoadsPerStep + (kWhole ? 0 : kLoadsA), 15));
     }
-    __syncthreads();
-    read_first(slot_a(0), slot_b(0), 0, 0);
+    auto read_slot_0 = [&]() {
+      if constexpr (kWhole) {
+        barrier_no_fence();  // (the loads of slots 2 and 3 stay in flight)
+        read_whole(slot_a(0), slot_b(0), 0, 0);
+        __builtin_amdgcn_s_waitcnt(waitcnt_imm(63, 0));
+        barrier_no_fence();  // slot 0 has been read: the first K step refills it
+      } else {
+        __syncthreads();
+        read_first(slot_a(0), slot_b(0), 0, 0);
+      }
+    };
+    read_slot_0();
 
     while (have) {
 #pragma unroll
@@ -1673,6 +1727,11 @@ __device__ __forceinline__ void dual_gemm_body(const Params& p, const int wg, co
           k_step_pair(with_loads, std::integral_constant<int, 1>{}, L, ld_ks);
           k_step_pair(with_loads, std::integral_constant<int, 2>{}, L, ld_ks);
           k_step_pair(with_loads, std::integral_constant<int, 3>{}, L, ld_ks);
+        } else if constexpr (kWhole) {
+          k_step_whole(with_loads, std::integral_constant<int, 0>{}, L, ld_ks);
+          k_step_whole(with_loads, std::integral_constant<int, 1>{}, L, ld_ks);
+          k_step_whole(with_loads, std::integral_constant<int, 2>{}, L, ld_ks);
+          k_step_whole(with_loads, std::integral_constant<int, 3>{}, L, ld_ks);
         } else {
           k_step_as(with_loads, std::integral_constant<int, 0>{}, L, ld_ks);
           k_step_as(with_loads, std::integral_constant<int, 1>{}, L, ld_ks);
@@ -1689,8 +1748,7 @@ __device__ __forceinline__ void dual_gemm_body(const Params& p, const int wg, co
           if constexpr (LD) setup_loader(tc, L);
           setup_store(tc, S);
           consumer_prologue();
-          __syncthreads();
-          read_first(slot_a(0), slot_b(0), 0, 0);
+          read_slot_0();
         }
       }
     }
