@@ -415,8 +415,8 @@ int wx_unpermute_rows_rmsnorm_bwd(const void* grad_sorted, const void* x, const 
  * buffers of wx_tiled_bytes(wx_padded_sorted_rows(num_rows), hidden) bytes and wx_padded_sorted_rows(num_rows) *
  * max(inter0, inter1) bf16; norm_weight: bf16 [hidden] or NULL (no norm); add_residual != 0 returns x + block(x).
  * ffn_workspace: NULL, or the workspace of wx_dual_swiglu_ffn_fused (same rules), which then runs the two GEMMs
- * and, when there is no norm, the permute as well; with a norm and the row counts on the host, few rows (a denoise step
- * of one robot or a few) run all of it, the norm included, as one launch. */
+ * and, when there is no norm, the permute as well; few rows (a denoise step of one robot or a few) run all of
+ * it, the norm included, as one launch. */
 int wx_moe_block_forward(const void* x, void* out, const int32_t* row_id_map, const int32_t* sorted_row_id,
                          const int32_t* expert_offsets, const void* gate0, const void* up0, const void* down0,
                          const void* gate1, const void* up1, const void* down1, void* x_tiled, void* hmid,

@@ -300,6 +300,55 @@ def test_few_rows_with_the_norm_inside(dev, T, m0, H, I0, I1):
     torch.cuda.synchronize()
 
 
+# The tile shapes of the one launch at their edges (its rows are taken for the narrow expert's where the host does not know
+# better), several tiles per workgroup on a wide expert and on a mix, a contraction longer than one round of loads, and hidden
+# sizes whose last column tile is short.
+@pytest.mark.parametrize("T,m0,H,I0,I1", [
+    (33, 0, 2048, 11008, 1024), (64, 0, 2048, 11008, 1024), (65, 1, 2048, 11008, 1024), (128, 64, 2048, 11008, 1024),
+    (129, 128, 2048, 11008, 1024), (224, 0, 2048, 1536, 1024), (225, 0, 2048, 1536, 1024), (256, 200, 2048, 4096, 1024),
+    (31, 31, 2048, 11008, 1024), (70, 70, 4096, 96, 64), (40, 9, 288, 320, 32), (200, 100, 1056, 640, 96),
+])
+def test_few_rows_tiles_whatever_rows_the_host_expects(dev, T, m0, H, I0, I1):
+    """One launch equals two, bit for bit, with the row counts known, unknown, and not the device's; with the norm inside it
+    equals the norm's own launch and those."""
+    ws_, packed, types, x, res, off, inv, xt = _case(dev, T, m0, H, I0, I1, T + I0)
+    p = [t.data_ptr() for t in packed]
+    stream = torch.cuda.current_stream().cuda_stream
+    pad = native.padded_sorted_rows(T)
+    work = _workspace(dev)
+    hm = [torch.zeros(pad * max(I0, I1), dtype=torch.bfloat16, device=dev) for _ in range(2)]
+    out = [torch.full((T, H), 7.0, dtype=torch.bfloat16, device=dev) for _ in range(2)]
+    _two_launches(p, xt, hm[0], out[0], res, off, inv, T, H, I0, I1, None, stream)
+    for counts in ((m0, T - m0), None, (0, T), (T, 0), (T // 2, T - T // 2)):
+        for rows_in in (x, None):
+            out[1].fill_(9.0)
+            hm[1].zero_()
+            _one_launch(p, xt, hm[1], out[1], res, off, inv, T, H, I0, I1, None if counts is None else _lib.i64x2(counts), work,
+                        stream, x_rows=rows_in)
+            torch.cuda.synchronize()
+            assert torch.equal(out[0], out[1]) and torch.equal(hm[0], hm[1]), f"counts {counts}"
+            assert int(work.abs().sum()) == 0, f"counts {counts}"
+    wc = [tuple(w.cpu() for w in ws_[:3]), tuple(w.cpu() for w in ws_[3:])]
+    ref = oracle.sparse_moe_block_ref(x.cpu()[None], types.cpu()[None], wc)[0].float()
+    ref = (res.cpu().float() + ref).to(torch.bfloat16).float()
+    err = (out[0].cpu().float() - ref).abs()
+    # (the bound of the other tests of this FFN, widened with the root of the contraction where it is longer than theirs)
+    assert not (err > 2e-2 * max(1.0, I0 / 2048) ** 0.5 + 1e-2 * ref.abs()).any(), float(err.max())
+    if H % 256 == 0 and H <= 2048:
+        rmap = native.partition(types, 2, 0, None, want_sorted=True)[0]
+        experts = native.PackedExperts(packed, (H, I0, I1))
+        norm = (torch.randn(H, generator=torch.Generator().manual_seed(3)) * 0.1 + 1).to(torch.bfloat16).to(dev)
+        got = []
+        for one, counts in ((False, (m0, T - m0)), (True, (m0, T - m0)), (True, None), (True, (0, T)), (True, (T, 0))):
+            old = native.set_one_launch_ffn(one)
+            try:
+                got.append(native.packed_block_forward(experts, x, rmap, inv, off, None if counts is None else _lib.i64x2(counts),
+                                                       (norm, 1e-6), True))
+            finally:
+                native.set_one_launch_ffn(old)
+        assert all(torch.equal(got[0], g) for g in got[1:])
+
+
 @pytest.mark.parametrize("T,m0,H,I0,I1", [(33, 0, 512, 448, 256), (40, 23, 512, 448, 96), (200, 90, 256, 384, 128)])
 def test_few_rows_keep_the_projections(dev, T, m0, H, I0, I1):
     """With the gate and up projections kept for a backward pass the intermediate is the same, and it is their SwiGLU."""

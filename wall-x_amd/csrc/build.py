@@ -55,8 +55,8 @@ def _newer(target: str, deps) -> bool:
 # The GEMM kernels use every register a wave can have; a small source change can push values of the K loop into scratch
 # memory, which costs a factor of three and shows in no test of results.  Their compile prints the resource-usage remarks
 # and this limit on "ScratchSize [bytes/lane]" of any kernel of the file turns a spill into a loud warning.
-# (Values that are only live outside the K loop do spill: 64 bytes in the few-rows gate/up kernel, 24 in the one with the
-# norm, 8 in the large tile with a K-major A; tests/test_k_loop_assembly.py shows that none is inside a loop.)
+# (Values that are only live outside the K loop do spill: 56 bytes in the few-rows kernel with the norm and 64-row B tiles, 8 in
+# the large tile with a K-major A; tests/test_k_loop_assembly.py shows that none is inside a loop.)
 RESOURCE_CHECKED = {"dual_gemm.hip": 96}
 
 

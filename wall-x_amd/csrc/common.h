@@ -107,8 +107,8 @@ __device__ __forceinline__ int64_t load_index(const void* p, int itype, int64_t 
 // Number of compute units of the current device (cached per thread); 256 on MI355X.
 int device_cu_count();
 
-// The block forward [RMSNorm -> permute -> FFN -> unpermute (+ residual)] as one launch, for few rows whose counts the
-// host knows (dual_gemm.hip).  1 = not such a call: nothing was launched, and nothing was refused.  The weights are gate,
+// The block forward [RMSNorm -> permute -> FFN -> unpermute (+ residual)] as one launch, for few rows
+// (dual_gemm.hip).  1 = not such a call: nothing was launched, and nothing was refused.  The weights are gate,
 // up and down of one expert each.
 int launch_norm_ffn_few_rows(const void* x, const void* x_tiled, void* out, const void* residual, const int32_t* sorted_row_id,
                              const int32_t* expert_offsets, const void* const* weights0, const void* const* weights1, void* hmid,

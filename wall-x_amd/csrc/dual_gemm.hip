@@ -133,8 +133,6 @@ struct Params {
   // number of 256 x 256 tiles is on its side of `gate_tiles`.  0 = always run, 1 = run if at most gate_tiles,
   // 2 = run if more.
   int gate, gate_tiles;
-  // CUs that the few-rows form may fill (see few_rows_fm); 0 = this launch does not take that form.
-  int few_rows_cus;
   // Tail split (see tail_split_point): 0 = off; 1 = this launch does the whole rounds of 256 x 256 tiles and leaves
   // the ragged last round to a second launch; 2 = this is that second launch, with 128 x 128 tiles.
   // split_cus = workgroups of the first launch (one per CU).
@@ -269,6 +267,13 @@ __device__ __forceinline__ void barrier_no_fence() {
   asm volatile("" ::: "memory");
 }
 
+// ... and behind this wavefront's own LDS writes.
+__device__ __forceinline__ void lds_barrier() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_waitcnt(waitcnt_imm(63, 0));
+  barrier_no_fence();
+}
+
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {
   const bf16x2 v = {static_cast<__bf16>(lo), static_cast<__bf16>(hi)};  // one packed convert
@@ -312,6 +317,7 @@ struct FusedSync {
   // (sorted position -> token)
   const __bf16* x;
   const int32_t* gather;
+  int guess[2];  // few-rows form: the rows per expert that the host sized the grid for
   // few-rows form with the norm folded in: the token rows pass through an RMSNorm on their way to the MFMAs
   const __bf16* norm_weight;
   float norm_eps;
@@ -346,6 +352,50 @@ __device__ __forceinline__ void wait_for_count(const FusedSync& fs, int tid, int
   }
   barrier_no_fence();  // (no wait for the counter's answer here)
 }
+// The same two for the few-rows form, whose launch is a chain of latencies.  A row block has up to 64 gate/up tiles and as
+// many down tiles here, and one counter for all of them was worth a queue: 64 increments and 64 pollers of one word took
+// 4.2 us from the last increment to the end of the wait (32 rows, hidden 2048, expert 1024), the words of a counter's 256
+// bytes, one per gate/up tile and stored, not added to, take 2.4.  A poll is one load of all 64 words by a wavefront.
+// (More than 64 tiles of a row block share the words, tile ct the word ct % 64, and add.)
+__device__ __forceinline__ void flag_done(const FusedSync& fs, int tid, int rb, int ct, int tiles) {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+  __builtin_amdgcn_s_waitcnt(waitcnt_imm(0, 0));
+  __syncthreads();
+  if (tid == 0) {
+    int* const word = fs.ready + rb * kFusedCounterStride + ct % kFusedCounterStride;
+    if (tiles <= kFusedCounterStride) __hip_atomic_store(word, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    else __hip_atomic_fetch_add(word, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+}
+// A first look at the words, ahead of the tile's other loads; `seen` of wait_for_flags.
+__device__ __forceinline__ int poll_flags(const FusedSync& fs, int tid, int rb) {
+  return tid < 64 ? __hip_atomic_load(fs.ready + rb * kFusedCounterStride + tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0;
+}
+__device__ __forceinline__ void wait_for_flags(const FusedSync& fs, int tid, int rb, int tiles, int seen, int& before) {
+  if (tid < 64) {
+    const int need = (tiles - tid + kFusedCounterStride - 1) / kFusedCounterStride;
+    if (__ballot(seen < need) != 0) {
+      const long long start = __builtin_amdgcn_s_memrealtime();
+      do {
+        if (static_cast<long long>(__builtin_amdgcn_s_memrealtime()) - start > kFusedWaitTicks) {
+          if (tid == 0) __hip_atomic_store(fs.error, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          break;
+        }
+        __builtin_amdgcn_s_sleep(1);
+        seen = poll_flags(fs, tid, rb);
+      } while (__ballot(seen < need) != 0);
+    }
+    if (tid == 0)
+      before = __hip_atomic_fetch_add(fs.passed + rb * kFusedCounterStride, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  barrier_no_fence();
+}
+__device__ __forceinline__ void clear_flags_if_last(const FusedSync& fs, int tid, int rb, int before, int waiters) {
+  if (tid >= 64) return;
+  if (__builtin_amdgcn_readfirstlane(before) != waiters - 1) return;
+  __hip_atomic_store(fs.ready + rb * kFusedCounterStride + tid, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (tid == 0) __hip_atomic_store(fs.passed + rb * kFusedCounterStride, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
 // ... and once the tile is done: the workgroup that was the last of its row block to get past the wait (everything
 // the wait was for is done, and every other waiter is past its wait as well) leaves the two counters at zero for
 // the next launch
@@ -367,277 +417,409 @@ __device__ __forceinline__ float swiglu_bf16(float gate, float up) {
 // ---- few rows ------------------------------------------------------------------------------------------------
 // A denoise step of one robot is 32 rows.  As 128 x 128 tiles its two GEMMs occupy 16 CUs each, and every K step of those
 // waits for the one before it (~250 ns, 96 of them).  This form makes the tiles small and cuts the contraction instead:
-// a workgroup computes 16 FM rows x 64 operand rows of B (32 gate + 32 up, or 64 output columns), its eight wavefronts
+// a workgroup computes 16 FM rows x 16 NB operand rows of B (half gate and half up, or output columns), its eight wavefronts
 // take an eighth of the K steps each, and the partial sums meet in LDS.  Fragments go from memory to registers (a block
-// of a K-tiled matrix is one fragment of a 16x16x32 MFMA), a ring of them in flight per wavefront, so a tile costs a few
-// memory latencies in place of K / 32 barriers.  Each row block reads the weights again (through L2: the tiles of a
-// column are on one XCD where the column tiles are a multiple of eight), which is why many rows keep the large tiles.
-// Measured (hidden 2048, experts 11008 / 1024, per layer): 32 rows 17 us where the 128 x 128 tiles take 35, 217 rows 22 where
-// they take 34.  The line lies where the tiles of a round of their own run out (256 rows at these widths): in a second round
-// the weights are read as often again and the next tile's chain of latencies begins.  36 layers with the norm, two rounds of
-// small tiles / 128 x 128 tiles: 260 rows 1471 / 1459 us, 320 rows 1510 / 1463, 512 rows 1520 / 1460; 256 rows, one round,
-// 1040.
-constexpr int kFewCols = 64;       // rows of B per tile
-constexpr int kFewMaxFm = 2;       // row blocks of 16 per tile: 1 or 2
-constexpr int kFewWavesPerSimd = 4;  // two workgroups per CU, which the fused launch counts on (128 registers)
-constexpr int kFewMaxRows = 1024;  // (a bound for the host; few_rows_fm decides)
+// of a K-tiled matrix is one fragment of a 16x16x32 MFMA), a wavefront's whole share of a contraction of 2048 at once, so a
+// tile costs a few memory latencies in place of K / 32 barriers.  Each row block reads the weights again (through L2: the
+// tiles of a column are on one XCD where the column tiles are a multiple of eight), which is why many rows keep the large
+// tiles.
+// A layer's launch is a chain of latencies (timestamps at 32 rows with the norm, weights from HBM, us after the first workgroup's
+// entry): arguments 0.6, row ids and first weights requested 1.6, rows requested 3.4, squares of the rows 6.0, products 7.1,
+// sums 8.0, stored 8.4, in memory 8.8, flags seen 12, intermediate multiplied 12.6, stored 13.  36 layers with distinct weights
+// from a graph, us per layer, as two kernels' worth of 128 registers with the norm's pass over the rows in front of the
+// products, a counter per row block and tiles of 16 or 32 rows x 64 / as it is: with the norm inside 32 rows 20.9 / 15.4, 64 rows
+// 21.0 / 16.5, 128 rows 22.5 / 19.4, 217 rows (the norm was a launch) 29.8 / 23.2; without a norm 18.8 / 13.6, 18.6 / 14.5,
+// 20.5 / 16.8, 24.2 / 18.8.
+constexpr int kFewThreads = 512;   // eight wavefronts
+constexpr int kFewMaxRows = 1024;  // (a bound for the host; few_rows decides)
 
-// Row blocks per tile of the few-rows form, or 0 where the problem keeps the 128 x 128 (256 x 256) tiles: the smaller
-// tile whose gate/up and down tiles each fit the CUs in one round.  Evaluated identically by the host (when it knows the
-// row counts) and on the device, by every launch form, so that they all add up in one order.
-__host__ __device__ inline int few_rows_fm(int64_t m0, int64_t m1, int64_t inter0, int64_t inter1, int64_t hidden, int cus) {
-  if (cus <= 0 || m0 + m1 > kFewMaxRows) return 0;
-  for (int fm = 1; fm <= kFewMaxFm; ++fm) {
-    const int64_t r0 = (m0 + 16 * fm - 1) / (16 * fm), r1 = (m1 + 16 * fm - 1) / (16 * fm);
-    if (r0 * (inter0 / 32) + r1 * (inter1 / 32) <= cus && (r0 + r1) * ((hidden + kFewCols - 1) / kFewCols) <= cus) return fm;
-  }
-  return 0;
+// Whether the few-rows form takes the problem: with every row on the narrower expert the tiles of 32 rows x 64 rows of B of
+// each GEMM are at most one per CU.  The split of the rows does not enter, so the host always knows, and every launch form
+// adds up in the same order.  The
+// line is where a round of the tiles ends (256 rows at hidden 2048, experts 11008 / 1024): 36 layers with the norm 950 us at 256
+// rows, as two rounds of tiles 1520 at 512 where the 128 x 128 tiles take 1460.  Rows on the wide expert are many tiles per
+// workgroup, and ahead of the 128 x 128 tiles up to that line too: 4 layers with the norm, every row on the expert of 11008,
+// 32 rows 513 / 292 us, 96 rows 517 / 353, 217 rows 560 / 478, 256 rows 560 / 547.
+inline bool few_rows(int64_t rows, int64_t inter0, int64_t inter1, int64_t hidden, int cus) {
+  const int64_t blocks = (rows + 31) / 32, inter = inter0 < inter1 ? inter0 : inter1;
+  return rows <= kFewMaxRows && blocks * (inter / 32) <= cus && blocks * ((hidden + 63) / 64) <= cus;
 }
 
-// One row's bf16 pair through the RMSNorm: w * bf16(x * inv), rounded, as the norm's own kernel has it.
-__device__ __forceinline__ uint32_t rms_scale(uint32_t x, uint32_t w, float inv) {
-  return pack_bf16x2(__uint_as_float(w << 16) * round_bf16(__uint_as_float(x << 16) * inv),
-                     __uint_as_float(w & 0xffff0000u) * round_bf16(__uint_as_float(x & 0xffff0000u) * inv));
+// One row's bf16 pair through the RMSNorm: w * bf16(x * inv), rounded, as the norm's own kernel has it (w_lo, w_hi: the pair of
+// weights).  A tile of 32 rows x 2048 spends 3 us of its CU's vector ALU on this and on the squares, so both roundings are one
+// packed convert each and the squares are fused multiply-adds (the square of a bf16 value is exact in fp32: the same sum).
+__device__ __forceinline__ uint32_t rms_scale(uint32_t x, float w_lo, float w_hi, float inv) {
+  const uint32_t n = pack_bf16x2(__uint_as_float(x << 16) * inv, __uint_as_float(x & 0xffff0000u) * inv);
+  return pack_bf16x2(w_lo * __uint_as_float(n << 16), w_hi * __uint_as_float(n & 0xffff0000u));
 }
 
 // MODE, ROLE, AROWS as in dual_gemm_body.  512 threads.
-// NORM (with AROWS; k a multiple of 256): the rows are normalised here.  Every tile sums the squares of its own rows while
-// its first weights are on their way from memory, which takes the norm's launch (6 us at 32 rows, all of it latency) out
-// of the layer.  The sums are formed in the order of rmsnorm_permute_tiled128_kernel, so the values are the same.
-template <int MODE, int FM, int ROLE, bool AROWS, bool NORM = false>
+// FM: row blocks of 16 per tile.  NB: blocks of 16 rows of B per tile (half gate, half up; or output columns).  R: K steps in
+// flight per wavefront, of which RL hold their B in LDS (the registers of a tile of 32 x 64 do not hold eight steps).
+// None of the four decides what is added to what, so every shape gives the same bits: wavefront w takes every other K step of
+// a quarter of the contraction (w / 2 the quarter, w % 2 the step's parity), in order, and the eight partial sums are added in
+// the order of the wavefronts.
+// NORM (with AROWS; k a multiple of 256, at most 32 * 8 R): the rows are normalised here.  A wavefront holds its share of the
+// rows, so it reads them once, for the squares and for the products.  The quarters and parities are those of the lanes of
+// rmsnorm_permute_tiled128_kernel, and the squares are added in its order: the same values.
+// NBP (ROLE 2): NB of the producers.
+template <int MODE, int FM, int NB, int R, int RV, int RL, int ROLE, bool AROWS, bool NORM = false, int NBP = NB>
 __device__ __forceinline__ void few_rows_body(const Params& p, const int wg, const int n_wg, const FusedSync& fs) {
 #if defined(__HIP_DEVICE_COMPILE__)
   static_assert(MODE == kGateUp || MODE == kDown, "the FFN's two GEMMs");
+  static_assert(!NORM || AROWS, "the norm reads token rows");
   constexpr bool SWIGLU = MODE == kGateUp;
   constexpr int kRows = 16 * FM;
-  // K steps in flight per wavefront: what 128 registers hold.  (Eight of them, a wavefront's whole share of 2048, at one
-  // workgroup per CU: 21.5 us in place of 20.4 for a layer of 32 rows.)
-  constexpr int kRing = FM == 1 ? 4 : 3;
+  static_assert(RV + RL == R || (RL == 0 && R % RV == 0), "steps of B in flight");
+  // where the finished blocks go: block q of the tile (row block q / NB, column block q % NB) is summed by wavefront q % 8
+  constexpr int kSums = SWIGLU ? 1 : (FM * NB + 7) / 8;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l16 = lane & 15, lq = lane >> 4;
-  // the partial sums of wavefront w, one KiB per 16 x 16 block: in the LDS of the 128 x 128 tile's ring
-  unsigned char* const part[8] = {lds_array<8192, 1024, 0>(), lds_array<8192, 1024, 1>(), lds_array<8192, 1024, 2>(),
-                                  lds_array<8192, 1024, 3>(), lds_array<8192, 1024, 4>(), lds_array<8192, 1024, 5>(),
-                                  lds_array<8192, 1024, 6>(), lds_array<8192, 1024, 7>()};
-  unsigned char* const stage = lds_array<SmallTile::kWaves * SmallTile::kStageBytes, 1024, 12>();
-  static_assert(SmallTile::kSlotBytesA == 8192 && SmallTile::kSlotBytesB == 8192 && FM * 4 * 1024 <= 8192, "ring slots hold the partial sums");
-  unsigned char* mine = part[0];
-#pragma unroll
-  for (int w = 1; w < 8; ++w) mine = wave == w ? part[w] : mine;
+  // one KiB per 16 x 16 block of partial sums (or per fragment of B) and wavefront: eight blocks in the first array, eight more
+  // in the second
+  constexpr int kBlocksLds = FM * NB > RL * NB ? FM * NB : RL * NB;
+  static_assert(kBlocksLds <= 16, "LDS of a wavefront");
+  constexpr bool kMore = kBlocksLds > 8;
+  unsigned char* const part = lds_array<65536, 1024, 0>();
+  unsigned char* const more = lds_array<kMore ? 65536 : 16, 1024, 1>();
+  unsigned char* const norm_lds = lds_array<NORM ? 4096 : 16, 16, 2>();              // the norm's weights
+  float* const ss_of = reinterpret_cast<float*>(lds_array<NORM ? kRows * 32 : 16, 16, 3>());  // [row][wavefront]
+  auto own_block = [&](int q) { return (q < 8 ? part + q * 1024 : more + (q - 8) * 1024) + wave * 8192; };
 
-  const int o0 = p.offsets[0], o1 = p.offsets[1], o2 = p.offsets[2];
-  const int m[2] = {o1 - o0, o2 - o1};
-  const int pad0 = static_cast<int>(round_up_256(m[0])), pad1 = static_cast<int>(round_up_256(m[1]));
-  constexpr int kTileN = SWIGLU ? kFewCols / 2 : kFewCols;  // output columns per tile
-  const int blocks[2] = {(m[0] + kRows - 1) / kRows, (m[1] + kRows - 1) / kRows};
+  constexpr int kTileN = SWIGLU ? 8 * NB : 16 * NB;  // output columns per tile
   const int cols[2] = {(p.g[0].n + kTileN - 1) / kTileN, (p.g[1].n + kTileN - 1) / kTileN};
-  const int total0 = blocks[0] * cols[0], total = total0 + blocks[1] * cols[1];
   const int frag = (l16 << 6) + ((lq ^ ((l16 >> 2) & 3)) << 4);  // this lane's 16 bytes of a K-tiled block
 
-  for (int t = wg; t < total; t += n_wg) {
-    const int e = t >= total0 ? 1 : 0;
+  // The row counts, and this workgroup's tiles: t, t + step, .. below end, in the order expert, row block, column tile.  At
+  // most one tile each where there are workgroups enough; else a workgroup stays with a row block, whose rows it then reads (and
+  // normalises) once, and the row blocks' workgroups of one column are on one XCD.
+  int m[2], blocks[2], total0, t, step, end;
+  auto place = [&](int m0, int m1) {
+    m[0] = m0;
+    m[1] = m1;
+    blocks[0] = (m0 + kRows - 1) / kRows;
+    blocks[1] = (m1 + kRows - 1) / kRows;
+    total0 = blocks[0] * cols[0];
+    t = wg;
+    step = n_wg;
+    end = total0 + blocks[1] * cols[1];
+    if (end > n_wg) {
+      for (int i = 2; i < 64; ++i) {
+        const int slots0 = (cols[0] + 8 * i - 1) / (8 * i) * 8, slots1 = (cols[1] + 8 * i - 1) / (8 * i) * 8;
+        if (blocks[0] * slots0 + blocks[1] * slots1 > n_wg) continue;
+        const int e = wg >= blocks[0] * slots0 ? 1 : 0, nct = e ? cols[1] : cols[0];
+        const int w = e ? wg - blocks[0] * slots0 : wg;
+        step = e ? slots1 : slots0;
+        const int rb = __builtin_amdgcn_readfirstlane(w / step);
+        const int first = (e ? total0 : 0) + rb * nct;
+        t = first + w - rb * step;
+        end = rb < (e ? blocks[1] : blocks[0]) ? first + nct : 0;
+        break;
+      }
+    }
+  };
+  struct Tile {
+    int e, rb, ct;
+  };
+  auto tile_of = [&](int at) {
+    Tile x;
+    x.e = at >= total0 ? 1 : 0;
+    const int te = x.e ? at - total0 : at, nct = x.e ? cols[1] : cols[0];
+    x.rb = __builtin_amdgcn_readfirstlane(te / nct);
+    x.ct = te - x.rb * nct;
+    return x;
+  };
+  // Where a tile's B comes from.  A K step's descriptor begins at that step (scalar work) and ends with it, so the lanes'
+  // offsets are the same in every step; steps past a wavefront's share have an empty descriptor and read as zeros.  A wavefront's
+  // steps are k_first + 2 i, i < share.
+  struct Stream {
+    const char *b0, *b1;
+    uint32_t step, off;
+    int steps, share, k_first;
+  };
+  auto stream_of = [&](const Tile& x) {
+    const Group& G = x.e ? p.g[1] : p.g[0];
+    Stream b;
+    b.b0 = reinterpret_cast<const char*>(G.b0);
+    b.b1 = reinterpret_cast<const char*>(SWIGLU ? G.b1 : G.b0);
+    b.step = static_cast<uint32_t>(G.ldb) << 10;  // (blocks past the matrix's last row of B are past it)
+    b.off = (static_cast<uint32_t>(x.ct * kTileN / kBlkRows) << 10) + frag;
+    b.steps = G.k / 32;
+    b.share = (b.steps + 7) / 8;
+    b.k_first = 2 * b.share * (wave >> 1) + (wave & 1);
+    return b;
+  };
+  u32x4 fa[R][FM], fb[RV][NB];
+  auto b_rsrc = [&](const Stream& b, int i, bool up) {
+    const int ks = b.k_first + 2 * i;
+    return make_rsrc((up ? b.b1 : b.b0) + static_cast<int64_t>(ks) * b.step, i < b.share && ks < b.steps ? b.step : 0u);
+  };
+  auto b_block = [&](const Stream& b, int j) { return b.off + (SWIGLU ? j % (NB / 2) : j) * kBlkBytes; };
+  auto load_b = [&](const Stream& b, int slot, int i) {
+    const __amdgpu_buffer_rsrc_t r0 = b_rsrc(b, i, false), r1 = SWIGLU ? b_rsrc(b, i, true) : r0;
+#pragma unroll
+    for (int j = 0; j < NB; ++j) fb[slot][j] = __builtin_amdgcn_raw_buffer_load_b128(SWIGLU && j >= NB / 2 ? r1 : r0, b_block(b, j), 0, 0);
+  };
+  auto load_b_lds = [&](const Stream& b, int slot, int i) {
+    const __amdgpu_buffer_rsrc_t r0 = b_rsrc(b, i, false), r1 = SWIGLU ? b_rsrc(b, i, true) : r0;
+#pragma unroll
+    for (int j = 0; j < NB; ++j)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(SWIGLU && j >= NB / 2 ? r1 : r0, LDS_PTR(own_block(slot * NB + j)), 16, b_block(b, j), 0, 0, 0);
+  };
+  // The first loads of a tile.  Loads return in the order they are issued, so what the next address or the wait needs goes out
+  // first: the flags of the row block, the row ids; then weights, which come from HBM.
+  int flags = 0, row_id[AROWS ? FM : 1], out_row[kSums];
+  u32x2 norm_w = {0u, 0u};
+  const bool sums = wave < FM * (SWIGLU ? NB / 2 : NB);
+  constexpr int kBFirst = AROWS ? 2 : RV;
+  auto begin = [&](const Tile& x) {
+    const Group& G = x.e ? p.g[1] : p.g[0];
+    const int me = x.e ? m[1] : m[0], first_row = x.e ? m[0] : 0, row0 = x.rb * kRows;
+    if constexpr (ROLE == 2) flags = poll_flags(fs, tid, x.e * kFusedMaxRowBlocks + x.rb);
+    if constexpr (AROWS) {
+#pragma unroll
+      for (int f = 0; f < FM; ++f) {
+        const int r = row0 + 16 * f + l16;
+        row_id[f] = fs.gather[first_row + (r < me ? r : 0)];
+      }
+    }
+    if constexpr (!SWIGLU) {
+#pragma unroll
+      for (int u = 0; u < kSums; ++u) {
+        const int q = wave + 8 * u, r = row0 + (q / NB) * 16 + l16, c = x.ct * kTileN + (q % NB) * 16 + 4 * lq;
+        out_row[u] = -1;
+        if (sums && r < me && c < G.n) out_row[u] = p.scatter != nullptr ? p.scatter[first_row + r] : first_row + r;
+      }
+    }
+    if constexpr (NORM) norm_w = __builtin_amdgcn_raw_buffer_load_b64(make_rsrc(fs.norm_weight, static_cast<uint32_t>(G.k) * 2u), tid * 8, 0, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    const Stream b = stream_of(x);
+#pragma unroll
+    for (int i = 0; i < kBFirst; ++i) load_b(b, i, i);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+
+  // (as a vector load: scalar loads return in any order, and a wait for the launch's arguments would be one for these as well)
+  const u32x4 off = __builtin_amdgcn_raw_buffer_load_b128(make_rsrc(p.offsets, 12), 0, 0, 0);
+  __builtin_amdgcn_sched_barrier(0);
+  auto offset = [&](int q) { return static_cast<int>(__builtin_amdgcn_readfirstlane(off[q])); };
+  if constexpr (ROLE != 0) {
+    // The offsets are a memory latency away.  The row counts the host took for granted when it sized the grid are in the
+    // launch's arguments: the first tile begins with them, and begins again where they turn out not to be the device's.
+    place(fs.guess[0], fs.guess[1]);
+    if (t < end) begin(tile_of(t));
+    if (offset(0) != 0 || offset(1) != fs.guess[0] || offset(2) - offset(1) != fs.guess[1]) {
+      place(offset(1) - offset(0), offset(2) - offset(1));
+      if (t < end) begin(tile_of(t));
+    }
+  } else {
+    place(offset(1) - offset(0), offset(2) - offset(1));
+    if (t < end) begin(tile_of(t));
+  }
+  const int pad0 = static_cast<int>(round_up_256(m[0])), pad1 = static_cast<int>(round_up_256(m[1]));
+  int held = -1;  // the row block whose rows `fa` holds
+
+  for (; t < end; t += step) {
+    const Tile x = tile_of(t);
+    const int e = x.e, rb = x.rb, ct = x.ct;
     const Group G = e ? p.g[1] : p.g[0];
     const int nct = e ? cols[1] : cols[0], me = e ? m[1] : m[0], pad_e = e ? pad1 : pad0;
-    const int te = e ? t - total0 : t;
-    const int rb = __builtin_amdgcn_readfirstlane(te / nct), ct = te - rb * nct;
     const int row0 = rb * kRows, col0 = ct * kTileN;
     const int counter = e * kFusedMaxRowBlocks + rb;
-    const int steps = G.k / 32, share = (steps + 7) / 8;
-    const int k_first = wave * share, k_last = k_first + share < steps ? k_first + share : steps;
+    const Stream B = stream_of(x);
+    const bool fresh = !SWIGLU || held != counter;
+    held = B.share <= R ? counter : -1;
 
-    // A: K-tiled rows (the activations, or the intermediate of this expert), or the token rows themselves.  A K step's
-    // descriptor begins at that step (scalar work) and ends with it, so the lanes' offsets are the same in every step;
-    // steps past this wavefront's share have an empty descriptor and read as zeros.
+    // A: K-tiled rows (the activations, or the intermediate of this expert), or the token rows themselves
     const char* a_base;
     uint32_t a_off[FM], a_step, a_bytes;
+    auto load_a = [&](int slot, int i) {
+      const int ks = B.k_first + 2 * i;
+      const int64_t adv = static_cast<int64_t>(ks) * a_step;
+      const __amdgpu_buffer_rsrc_t r = make_rsrc(a_base + adv, i < B.share && ks < B.steps ? (AROWS ? a_bytes - static_cast<uint32_t>(adv) : a_bytes) : 0u);
+      // (the intermediate inside a fused launch: read past this XCD's L2, since a cache line of it may have two writers)
+#pragma unroll
+      for (int f = 0; f < FM; ++f) fa[slot][f] = __builtin_amdgcn_raw_buffer_load_b128(r, a_off[f], 0, ROLE == 2 ? 16 /* sc1 */ : 0);
+    };
+    if constexpr (!AROWS) {
+#pragma unroll
+      for (int i = R - RL; i < R; ++i) load_b_lds(B, i - RV, i);
+    }
+    __builtin_amdgcn_sched_barrier(0);
     if constexpr (AROWS) {
       a_base = reinterpret_cast<const char*>(fs.x);
       a_step = 64;
-      a_bytes = static_cast<uint32_t>(o2) * static_cast<uint32_t>(G.k) * 2u;
+      a_bytes = static_cast<uint32_t>(m[0] + m[1]) * static_cast<uint32_t>(G.k) * 2u;
 #pragma unroll
-      for (int i = 0; i < FM; ++i) {
-        const int r = row0 + 16 * i + l16;
-        a_off[i] = r < me ? static_cast<uint32_t>(fs.gather[(e ? o1 : o0) + r]) * static_cast<uint32_t>(G.k) * 2u + lq * 16u : 0x80000000u;
-      }
+      for (int f = 0; f < FM; ++f)
+        a_off[f] = row0 + 16 * f + l16 < me ? static_cast<uint32_t>(row_id[f]) * static_cast<uint32_t>(G.k) * 2u + lq * 16u : 0x80000000u;
     } else {
       const int a_blocks = SWIGLU ? G.lda : pad_e / kBlkRows;
       const int first = (SWIGLU && e ? pad0 : 0) / kBlkRows + row0 / kBlkRows;
       a_base = reinterpret_cast<const char*>(SWIGLU ? G.a : G.a + (e ? static_cast<int64_t>(pad0) * p.g[0].k : 0));
       a_step = a_bytes = static_cast<uint32_t>(a_blocks) << 10;
 #pragma unroll
-      for (int i = 0; i < FM; ++i) a_off[i] = (static_cast<uint32_t>(first + i) << 10) + frag;
-    }
-    const uint32_t b_step = static_cast<uint32_t>(G.ldb) << 10;  // (blocks past the matrix's last row of B are past it)
-    const uint32_t b_off = (static_cast<uint32_t>(col0 / kBlkRows) << 10) + frag;
-    u32x4 fa[kRing][FM], fb[kRing][4], fw[NORM ? kRing : 1];
-    auto load_a = [&](int slot, int ks) {
-      const int64_t adv = static_cast<int64_t>(ks) * a_step;
-      const __amdgpu_buffer_rsrc_t r = make_rsrc(a_base + adv, ks >= k_last ? 0u : (AROWS ? a_bytes - static_cast<uint32_t>(adv) : a_bytes));
-#pragma unroll
-      for (int i = 0; i < FM; ++i) fa[slot][i] = __builtin_amdgcn_raw_buffer_load_b128(r, a_off[i], 0, 0);
-      if constexpr (NORM)
-        fw[slot] = __builtin_amdgcn_raw_buffer_load_b128(make_rsrc(fs.norm_weight + ks * 32, ks < k_last ? 64u : 0u), lq * 16, 0, 0);
-    };
-    auto load_b = [&](int slot, int ks) {
-      const int64_t adv = static_cast<int64_t>(ks) * b_step;
-      const uint32_t bytes = ks < k_last ? b_step : 0u;
-      const __amdgpu_buffer_rsrc_t r0 = make_rsrc(reinterpret_cast<const char*>(G.b0) + adv, bytes);
-      const __amdgpu_buffer_rsrc_t r1 = SWIGLU ? make_rsrc(reinterpret_cast<const char*>(G.b1) + adv, bytes) : r0;
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-        fb[slot][j] = __builtin_amdgcn_raw_buffer_load_b128(SWIGLU && j >= 2 ? r1 : r0, b_off + (SWIGLU ? j & 1 : j) * kBlkBytes, 0, 0);
-    };
-    f32x4 acc[FM][4];
-#pragma unroll
-    for (int i = 0; i < FM; ++i)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-    // where the finished blocks go: block q of the tile (row block q / 4, column block q % 4) is summed by wavefront q
-    const bool sums = wave < FM * (SWIGLU ? 2 : 4);
-    int out_row = -1;
-    u32x2 res = {0u, 0u};
-#pragma unroll
-    for (int s = 0; s < kRing; ++s) load_b(s, k_first + s);
-    if constexpr (!SWIGLU) {
-      const int r = row0 + (wave >> 2) * 16 + l16, c = col0 + (wave & 3) * 16 + 4 * lq;
-      if (sums && r < me && c < G.n) {
-        const int sorted = (e ? o1 : o0) + r;
-        out_row = p.scatter != nullptr ? p.scatter[sorted] : sorted;
-        if (p.residual != nullptr) res = *reinterpret_cast<const u32x2*>(p.residual + static_cast<int64_t>(out_row) * G.ldc + c);
-      }
-    }
-    float inv[FM];
-    if constexpr (NORM) {
-      // wavefront: quarter wave % 4 of the row, eight rows wave / 4; lane: row lane / 8, 16 bytes of each 128
-      float* const ss_of = reinterpret_cast<float*>(stage + 8192);  // [row][quarter]
-      const int quarter = wave & 3, r8 = 8 * (wave >> 2) + (lane >> 3), per_quarter = G.k / 256;
-      const __amdgpu_buffer_rsrc_t rx = make_rsrc(a_base, a_bytes);
-      constexpr int kAtOnce = 4;
-#pragma unroll
-      for (int i = 0; i < FM; ++i) {
-        const int r = row0 + 16 * i + r8;
-        uint32_t off = 0x80000000u;
-        if (r < me)
-          off = static_cast<uint32_t>(fs.gather[(e ? o1 : o0) + r]) * static_cast<uint32_t>(G.k) * 2u +
-                static_cast<uint32_t>(quarter * per_quarter * 8 + (lane & 7)) * 16u;
-        float ss = 0.f;
-        for (int u = 0; u < per_quarter; u += kAtOnce) {
-          u32x4 v[kAtOnce];
-#pragma unroll
-          for (int q = 0; q < kAtOnce; ++q)
-            v[q] = __builtin_amdgcn_raw_buffer_load_b128(rx, u + q < per_quarter ? off + (u + q) * 128 : 0x80000000u, 0, 0);
-#pragma unroll
-          for (int q = 0; q < kAtOnce; ++q)
-#pragma unroll
-            for (int w = 0; w < 4; ++w) {
-              const float lo = __uint_as_float(v[q][w] << 16), hi = __uint_as_float(v[q][w] & 0xffff0000u);
-              ss += lo * lo;
-              ss += hi * hi;
-            }
-        }
-        ss += __shfl_xor(ss, 1);
-        ss += __shfl_xor(ss, 2);
-        ss += __shfl_xor(ss, 4);
-        if ((lane & 7) == 0) ss_of[(16 * i + r8) * 4 + quarter] = ss;
-      }
-      __syncthreads();
-#pragma unroll
-      for (int i = 0; i < FM; ++i) {
-        const f32x4 q = *reinterpret_cast<const f32x4*>(ss_of + (16 * i + l16) * 4);
-        inv[i] = __frsqrt_rn((q[0] + q[1] + q[2] + q[3]) / static_cast<float>(G.k) + fs.norm_eps);
-      }
+      for (int f = 0; f < FM; ++f) a_off[f] = (static_cast<uint32_t>(first + f) << 10) + frag;
     }
     int before = 0;
-    if constexpr (ROLE == 2) wait_for_count(fs, tid, counter, (e ? p.g[1].k : p.g[0].k) / 32, before);
+    if constexpr (ROLE == 2) wait_for_flags(fs, tid, counter, (e ? p.g[1].k : p.g[0].k) / (8 * NBP), flags, before);
+    if (fresh) {
 #pragma unroll
-    for (int s = 0; s < kRing; ++s) load_a(s, k_first + s);
-    for (int ks = 0; ks < share; ks += kRing) {
+      for (int i = 0; i < R; ++i) load_a(i, i);
+    }
+    u32x2 res[kSums];
+    if constexpr (!SWIGLU) {
 #pragma unroll
-      for (int s = 0; s < kRing; ++s) {
-        if constexpr (NORM) {
-#pragma unroll
-          for (int i = 0; i < FM; ++i)
-#pragma unroll
-            for (int w = 0; w < 4; ++w) fa[s][i][w] = rms_scale(fa[s][i][w], fw[s][w], inv[i]);
-        }
-#pragma unroll
-        for (int i = 0; i < FM; ++i)
-#pragma unroll
-          for (int j = 0; j < 4; ++j)
-            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, fb[s][j]), __builtin_bit_cast(bf16x8, fa[s][i]), acc[i][j], 0, 0, 0);
-        load_b(s, k_first + ks + s + kRing);
-        load_a(s, k_first + ks + s + kRing);
+      for (int u = 0; u < kSums; ++u) {
+        res[u] = u32x2{0u, 0u};
+        if (p.residual != nullptr && out_row[u] >= 0)
+          res[u] = *reinterpret_cast<const u32x2*>(p.residual + static_cast<int64_t>(out_row[u]) * G.ldc + col0 + ((wave + 8 * u) % NB) * 16 + 4 * lq);
       }
     }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = kBFirst; i < RV; ++i) load_b(B, i, i);
+    if constexpr (AROWS) {
+#pragma unroll
+      for (int i = R - RL; i < R; ++i) load_b_lds(B, i - RV, i);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    float inv[FM];
+    if constexpr (NORM) {
+      if (fresh) {
+#pragma unroll
+        for (int f = 0; f < FM; ++f) {
+          float ss = 0.f;
+#pragma unroll
+          for (int i = 0; i < R; ++i)
+#pragma unroll
+            for (int w = 0; w < 4; ++w) {
+              const float lo = __uint_as_float(fa[i][f][w] << 16), hi = __uint_as_float(fa[i][f][w] & 0xffff0000u);
+              ss = __builtin_fmaf(lo, lo, ss);
+              ss = __builtin_fmaf(hi, hi, ss);
+            }
+          ss += __shfl_xor(ss, 16);
+          ss += __shfl_xor(ss, 32);
+          if (lane < 16) ss_of[(16 * f + l16) * 8 + wave] = ss;
+        }
+        *reinterpret_cast<u32x2*>(norm_lds + tid * 8) = norm_w;  // (zeros past the row's end)
+        lds_barrier();  // (the weights' loads stay in flight)
+#pragma unroll
+        for (int f = 0; f < FM; ++f) {
+          const f32x4 a = *reinterpret_cast<const f32x4*>(ss_of + (16 * f + l16) * 8), b = *reinterpret_cast<const f32x4*>(ss_of + (16 * f + l16) * 8 + 4);
+          inv[f] = __frsqrt_rn(((a[0] + a[1]) + (a[2] + a[3]) + (b[0] + b[1]) + (b[2] + b[3])) / static_cast<float>(G.k) + fs.norm_eps);
+        }
+      }
+    }
+    f32x4 acc[FM][NB];
+#pragma unroll
+    for (int f = 0; f < FM; ++f)
+#pragma unroll
+      for (int j = 0; j < NB; ++j) acc[f][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int base = 0; base < B.share; base += R) {  // (once, for a contraction of at most 256 R)
+#pragma unroll
+      for (int i = 0; i < R; ++i) {
+        if constexpr (NORM) {
+          if (fresh) {
+            const u32x4 w4 = *reinterpret_cast<const u32x4*>(norm_lds + (B.k_first + 2 * i) * 64 + lq * 16);
+#pragma unroll
+            for (int w = 0; w < 4; ++w) {
+              const float w_lo = __uint_as_float(w4[w] << 16), w_hi = __uint_as_float(w4[w] & 0xffff0000u);
+#pragma unroll
+              for (int f = 0; f < FM; ++f) fa[i][f][w] = rms_scale(fa[i][f][w], w_lo, w_hi, inv[f]);
+            }
+          }
+        }
+        if (RL > 0 && i == RV) {
+          asm volatile("" ::: "memory");
+          __builtin_amdgcn_s_waitcnt(waitcnt_imm(0, 15));
+          asm volatile("" ::: "memory");
+        }
+#pragma unroll
+        for (int j = 0; j < NB; ++j) {
+          const bf16x8 b = i < R - RL ? __builtin_bit_cast(bf16x8, fb[i % RV][j]) : *reinterpret_cast<const bf16x8*>(own_block((i - RV) * NB + j) + lane * 16);
+#pragma unroll
+          for (int f = 0; f < FM; ++f)
+            acc[f][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b, __builtin_bit_cast(bf16x8, fa[i][f]), acc[f][j], 0, 0, 0);
+        }
+        if (RV < R && RL == 0 && i + RV < R) load_b(B, i % RV, base + i + RV);
+        if (!NORM && base + R < B.share) {
+          if (i >= R - RL - RV && i < R - RL) load_b(B, i % RV, base + R + i % RV);
+          load_a(i, base + i + R);
+        }
+      }
+      if (RL > 0 && !NORM && base + R < B.share) {
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the fragments in LDS have been read
+#pragma unroll
+        for (int i = R - RL; i < R; ++i) load_b_lds(B, i - RV, base + i + R);
+      }
+    }
+    // (the last tile's sums need what `begin` changes)
+    int out_now[kSums];
+#pragma unroll
+    for (int u = 0; u < kSums; ++u) out_now[u] = out_row[u];
+    if (t + step < end) begin(tile_of(t + step));  // the next tile's first loads, while this one's sums meet
     // partial sums: lane l of a block holds row l % 16, columns 4 (l / 16) .. + 3
+    if constexpr (RL > 0) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
 #pragma unroll
-    for (int i = 0; i < FM; ++i)
+    for (int f = 0; f < FM; ++f)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) *reinterpret_cast<f32x4*>(mine + (i * 4 + j) * 1024 + lane * 16) = acc[i][j];
+      for (int j = 0; j < NB; ++j) *reinterpret_cast<f32x4*>(own_block(f * NB + j) + lane * 16) = acc[f][j];
     __syncthreads();
     auto sum_of = [&](int block) {
-      f32x4 v = *reinterpret_cast<const f32x4*>(part[0] + block * 1024 + lane * 16);
+      const unsigned char* const at = (!kMore || block < 8 ? part + block * 1024 : more + (block - 8) * 1024) + lane * 16;
+      f32x4 v = *reinterpret_cast<const f32x4*>(at);
 #pragma unroll
-      for (int w = 1; w < 8; ++w) v += *reinterpret_cast<const f32x4*>(part[w] + block * 1024 + lane * 16);
+      for (int w = 1; w < 8; ++w) v += *reinterpret_cast<const f32x4*>(at + w * 8192);
       return v;
     };
     if constexpr (SWIGLU) {
-      if (sums) {  // wavefront 2 i + j: row block i, columns 16 j .. of the tile's 32
-        const int i = wave >> 1, j = wave & 1;
-        const f32x4 g = sum_of(i * 4 + j), u = sum_of(i * 4 + j + 2);
+      if (sums) {  // wavefront (NB / 2) i + j: row block i, columns 16 j .. of the tile
+        const int i = wave / (NB / 2), j = wave % (NB / 2);
+        const f32x4 g = sum_of(i * NB + j), u = sum_of(i * NB + j + NB / 2);
         float h[4];
 #pragma unroll
         for (int r = 0; r < 4; ++r) h[r] = swiglu_bf16(g[r], u[r]);
-        const int chunk = 2 * j + (lq >> 1);
+        // four columns of a row of the K-tiled intermediate, written through where another XCD waits for them
+        const int c16 = (col0 >> 4) + j, chunk = 2 * (c16 & 1) + (lq >> 1);
         const int in_block = l16 * 64 + ((chunk ^ ((l16 >> 2) & 3)) << 4) + (lq & 1) * 8;
-        *reinterpret_cast<u32x2*>(stage + i * kBlkBytes + in_block) = u32x2{pack_bf16x2(h[0], h[1]), pack_bf16x2(h[2], h[3])};
-        if constexpr (ROLE == 0) {  // the projections themselves, for a backward pass
-          if (p.keep_gate != nullptr) {
-            const int64_t off = (e ? static_cast<int64_t>(pad0) * p.g[0].n * 2 : 0) +
-                                ((static_cast<int64_t>(ct) * (pad_e / kBlkRows) + row0 / kBlkRows + i) << 10) + in_block;
-            *reinterpret_cast<u32x2*>(reinterpret_cast<unsigned char*>(p.keep_gate) + off) = u32x2{pack_bf16x2(g[0], g[1]), pack_bf16x2(g[2], g[3])};
-            *reinterpret_cast<u32x2*>(reinterpret_cast<unsigned char*>(p.keep_up) + off) = u32x2{pack_bf16x2(u[0], u[1]), pack_bf16x2(u[2], u[3])};
+        const int64_t block = (e ? static_cast<int64_t>(pad0) * p.g[0].n * 2 : 0) +
+                              ((static_cast<int64_t>(c16 >> 1) * (pad_e / kBlkRows) + row0 / kBlkRows + i) << 10);
+        const u32x2 v = {pack_bf16x2(h[0], h[1]), pack_bf16x2(h[2], h[3])};
+        unsigned char* const dst = reinterpret_cast<unsigned char*>(p.g[0].c) + block;
+        // (a last tile of half a gate and half an up block more than the matrix has: nothing to store)
+        if (col0 + 16 * j < G.n) {
+          if constexpr (ROLE == 1) __builtin_amdgcn_raw_buffer_store_b64(v, make_rsrc(dst, kBlkBytes), in_block, 0, 16 /* sc1 */);
+          else *reinterpret_cast<u32x2*>(dst + in_block) = v;
+          if constexpr (ROLE == 0) {  // the projections themselves, for a backward pass
+            if (p.keep_gate != nullptr) {
+              *reinterpret_cast<u32x2*>(reinterpret_cast<unsigned char*>(p.keep_gate) + block + in_block) = u32x2{pack_bf16x2(g[0], g[1]), pack_bf16x2(g[2], g[3])};
+              *reinterpret_cast<u32x2*>(reinterpret_cast<unsigned char*>(p.keep_up) + block + in_block) = u32x2{pack_bf16x2(u[0], u[1]), pack_bf16x2(u[2], u[3])};
+            }
           }
         }
       }
-      __syncthreads();
-      if (wave < FM) {  // whole blocks of the K-tiled intermediate, written through where another XCD waits for them
-        const u32x4 v = *reinterpret_cast<const u32x4*>(stage + wave * kBlkBytes + lane * 16);
-        unsigned char* dst = reinterpret_cast<unsigned char*>(p.g[0].c + (e ? static_cast<int64_t>(pad0) * p.g[0].n : 0)) +
-                             ((static_cast<int64_t>(ct) * (pad_e / kBlkRows) + row0 / kBlkRows + wave) << 10);
-        if constexpr (ROLE == 1) __builtin_amdgcn_raw_buffer_store_b128(v, make_rsrc(dst, kBlkBytes), lane * 16, 0, 16 /* sc1 */);
-        else *reinterpret_cast<u32x4*>(dst + lane * 16) = v;
-      }
-      if constexpr (ROLE == 1) count_done(fs, tid, counter);
+      if constexpr (ROLE == 1) flag_done(fs, tid, counter, ct, nct);
     } else {
-      if (sums && out_row >= 0) {
-        const f32x4 y = sum_of(wave);
+#pragma unroll
+      for (int u = 0; u < kSums; ++u) {
+        if (out_now[u] < 0) continue;
+        const int q = wave + 8 * u;
+        const f32x4 y = sum_of(q);
         u32x2 v = {pack_bf16x2(y[0], y[1]), pack_bf16x2(y[2], y[3])};
         if (p.residual != nullptr) {
 #pragma unroll
-          for (int q = 0; q < 2; ++q)
-            v[q] = pack_bf16x2(__uint_as_float(v[q] << 16) + __uint_as_float(res[q] << 16),
-                               __uint_as_float(v[q] & 0xffff0000u) + __uint_as_float(res[q] & 0xffff0000u));
+          for (int w = 0; w < 2; ++w)
+            v[w] = pack_bf16x2(__uint_as_float(v[w] << 16) + __uint_as_float(res[u][w] << 16),
+                               __uint_as_float(v[w] & 0xffff0000u) + __uint_as_float(res[u][w] & 0xffff0000u));
         }
-        *reinterpret_cast<u32x2*>(p.g[0].c + static_cast<int64_t>(out_row) * G.ldc + col0 + (wave & 3) * 16 + 4 * lq) = v;
+        *reinterpret_cast<u32x2*>(p.g[0].c + static_cast<int64_t>(out_now[u]) * G.ldc + col0 + (q % NB) * 16 + 4 * lq) = v;
       }
-      if constexpr (ROLE == 2) clear_if_last(fs, tid, counter, before, nct);
+      if constexpr (ROLE == 2) clear_flags_if_last(fs, tid, counter, before, nct);
     }
     __syncthreads();  // the partial sums' LDS is written by the next tile
   }
 #endif
-}
-// The form for the row counts in p.offsets; false: the caller runs the tiles.
-template <int MODE, int ROLE, bool AROWS = false>
-__device__ __forceinline__ bool few_rows(const Params& p, const int wg, const int n_wg, const FusedSync& fs) {
-  const int inter0 = MODE == kGateUp ? p.g[0].n : p.g[0].k, inter1 = MODE == kGateUp ? p.g[1].n : p.g[1].k;
-  const int hidden = MODE == kGateUp ? p.g[0].k : p.g[0].n;
-  const int fm = few_rows_fm(p.offsets[1] - p.offsets[0], p.offsets[2] - p.offsets[1], inter0, inter1, hidden, p.few_rows_cus);
-  if (fm == 0) return false;
-  if (fm == 1) few_rows_body<MODE, 1, ROLE, AROWS>(p, wg, n_wg, fs);
-  else few_rows_body<MODE, 2, ROLE, AROWS>(p, wg, n_wg, fs);
-  return true;
 }
 
 // KA / KB (generic mode only): the operand is stored with K as its slow dimension -- A as [k, m], B as [k, n] --
@@ -1767,11 +1949,12 @@ __global__ __launch_bounds__(TS::kThreads, TS::kWgPerCu) void dual_gemm_kernel(P
   dual_gemm_body<MODE, TS, KA, KB, 0>(p, blockIdx.x, gridDim.x, FusedSync{});
 }
 
-// The same launch where the row counts may call for the few-rows form (MODE: gate/up or down).
-template <int MODE>
-__global__ __launch_bounds__(SmallTile::kThreads, kFewWavesPerSimd) void dual_gemm_few_rows_kernel(Params p) {
-  if (!few_rows<MODE, 0>(p, blockIdx.x, gridDim.x, FusedSync{}))
-    dual_gemm_body<MODE, SmallTile, false, false, 0>(p, blockIdx.x, gridDim.x, FusedSync{});
+// The few-rows form of the same launch (MODE: gate/up or down).
+template <int MODE, int FM, int NB>
+__global__ __launch_bounds__(kFewThreads, 2) void dual_gemm_few_rows_kernel(Params p) {
+  constexpr int R = MODE == kGateUp ? 8 : 4;
+  constexpr int RL = MODE == kGateUp && NB == 4 ? 4 : 0;
+  few_rows_body<MODE, FM, NB, R, R - RL, RL, 0, false>(p, blockIdx.x, gridDim.x, FusedSync{});
 }
 
 // The fused FFN launch (see FusedSync): workgroups [0, producers) run the gate/up form on `pg`, the rest the down
@@ -1780,32 +1963,32 @@ __global__ __launch_bounds__(SmallTile::kThreads, kFewWavesPerSimd) void dual_ge
 // it waits for belongs to workgroups with lower indices, which never wait: whatever part of the grid is resident,
 // the launch makes progress.)
 // AROWS: the producers read the token rows (fs.x through fs.gather) in place of the K-tiled activations.
-// FEW: the row counts may call for the few-rows form (a kernel of its own, so that the other's registers are its own).
-template <bool AROWS, bool FEW>
-__global__ __launch_bounds__(SmallTile::kThreads, FEW ? kFewWavesPerSimd : SmallTile::kWgPerCu) void ffn_fused_kernel(Params pg, Params pd,
-                                                                                             FusedSync fs,
-                                                                                             int producers) {
+template <bool AROWS>
+__global__ __launch_bounds__(SmallTile::kThreads, SmallTile::kWgPerCu) void ffn_fused_kernel(Params pg, Params pd, FusedSync fs, int producers) {
   const int wg = blockIdx.x, consumers = static_cast<int>(gridDim.x) - producers;
-  if (wg < producers) {
-    if constexpr (FEW)
-      if (few_rows<kGateUp, 1, AROWS>(pg, wg, producers, fs)) return;
-    dual_gemm_body<kGateUp, SmallTile, false, false, 1, AROWS>(pg, wg, producers, fs);
-  } else {
-    if constexpr (FEW)
-      if (few_rows<kDown, 2>(pd, wg - producers, consumers, fs)) return;
-    dual_gemm_body<kDown, SmallTile, false, false, 2>(pd, wg - producers, consumers, fs);
-  }
+  if (wg < producers) dual_gemm_body<kGateUp, SmallTile, false, false, 1, AROWS>(pg, wg, producers, fs);
+  else dual_gemm_body<kDown, SmallTile, false, false, 2>(pd, wg - producers, consumers, fs);
 }
 
-// The one launch in the few-rows form alone, with the RMSNorm in front of the FFN folded in: the host knows the row
-// counts.  (Tiles of 16 rows, whatever the device's counts are: the tile list is right for any split.)  At 32 rows a layer
-// takes 20.7 us where the norm's launch and the FFN's take 24; with tiles of 32 rows (217 rows) the norm's registers spill
-// and it takes 30 in place of 29, so those keep the two launches.
-__global__ __launch_bounds__(SmallTile::kThreads, kFewWavesPerSimd) void ffn_few_rows_norm_kernel(Params pg, Params pd, FusedSync fs,
-                                                                                                  int producers) {
+// The one launch in the few-rows form.  NB / NBC: the blocks of a gate/up and of a down tile.  WG: workgroups per CU that the
+// registers are divided among.  ffn_few_rows_norm_kernel: with the RMSNorm in front of the FFN inside.
+template <int FM, int NB, int NBC, int WG, bool AROWS, bool NORM>
+__device__ __forceinline__ void ffn_few_rows(const Params& pg, const Params& pd, const FusedSync& fs, int producers) {
   const int wg = blockIdx.x, consumers = static_cast<int>(gridDim.x) - producers;
-  if (wg < producers) few_rows_body<kGateUp, 1, 1, true, true>(pg, wg, producers, fs);
-  else few_rows_body<kDown, 1, 2, false>(pd, wg - producers, consumers, fs);
+  if (wg < producers) {
+    if constexpr (WG == 2) few_rows_body<kGateUp, FM, NB, NORM || NB == 2 ? 8 : 4, NB == 2 ? 8 : 4, 0, 1, AROWS, NORM>(pg, wg, producers, fs);
+    else few_rows_body<kGateUp, FM, NB, 8, NB == 4 ? 4 : 8, NB == 4 ? 4 : 0, 1, AROWS, NORM>(pg, wg, producers, fs);
+  } else {
+    few_rows_body<kDown, FM, NBC, 4, NBC == 8 ? 2 : 4, NBC == 8 ? 2 : 0, 2, false, false, NB>(pd, wg - producers, consumers, fs);
+  }
+}
+template <int FM, int NB, int NBC, int WG, bool AROWS>
+__global__ __launch_bounds__(kFewThreads, 2 * WG) void ffn_few_rows_kernel(Params pg, Params pd, FusedSync fs, int producers) {
+  ffn_few_rows<FM, NB, NBC, WG, AROWS, false>(pg, pd, fs, producers);
+}
+template <int FM, int NB, int NBC, int WG>
+__global__ __launch_bounds__(kFewThreads, 2 * WG) void ffn_few_rows_norm_kernel(Params pg, Params pd, FusedSync fs, int producers) {
+  ffn_few_rows<FM, NB, NBC, WG, true, true>(pg, pd, fs, producers);
 }
 
 // ---- plain FMA tiles: any transpose combination, any k --------------------------------------------------------
@@ -1901,22 +2084,21 @@ int check_dims(const char* who, int64_t m, int64_t n, int64_t k, bool k_in_rows 
 // second launch with 128 x 128 tiles takes the ragged last round when that pays (the row-major op, whose sizes the
 // host knows, decides it on the host); when the host cannot tell, both launches are made and the device decides (the
 // second returns at once if there is nothing to split).
-// few: whether the few-rows form (few_rows_fm) takes the problem; kFewMaybe = the device finds out.
-enum Few { kFewNever, kFewMaybe, kFewAlways };
+// few: the few-rows form takes the problem; its number of rows, or 0.
 template <int MODE, bool KA = false, bool KB = false>
 int launch_mfma(Params p, int64_t tiles_lo, int64_t tiles_hi, hipStream_t s, const char* who,
-                const int64_t* tiles_by_expert = nullptr, Few few = kFewNever) {
+                const int64_t* tiles_by_expert = nullptr, int64_t few = 0) {
   const int cus = device_cu_count();
   const int threshold = cus / 2;
-  p.few_rows_cus = few == kFewNever ? 0 : cus;
   if constexpr (MODE == kGateUp || MODE == kDown) {
-    if (few == kFewAlways) {
+    if (few > 0) {
       p.gate = p.split = 0;
-      hipLaunchKernelGGL((dual_gemm_few_rows_kernel<MODE>), dim3(cus), dim3(SmallTile::kThreads), 0, s, p);
+      if (few <= 64) hipLaunchKernelGGL((dual_gemm_few_rows_kernel<MODE, 1, 2>), dim3(cus), dim3(kFewThreads), 0, s, p);
+      else hipLaunchKernelGGL((dual_gemm_few_rows_kernel<MODE, 2, 4>), dim3(cus), dim3(kFewThreads), 0, s, p);
       return check_launch(who);
     }
   }
-  bool small = tiles_lo <= threshold || few == kFewMaybe, big = tiles_hi > threshold;
+  bool small = tiles_lo <= threshold, big = tiles_hi > threshold;
   if (tiles_by_expert != nullptr) {  // the host knows the split: the count that decides is shape_deciding_tiles'
     small = shape_deciding_tiles(tiles_by_expert[0], tiles_by_expert[1], p.g[0].k, p.g[1].k) <= threshold;
     big = !small;
@@ -1929,16 +2111,9 @@ int launch_mfma(Params p, int64_t tiles_lo, int64_t tiles_hi, hipStream_t s, con
   p.split_cus = cus;
   if (small) {
     p.gate = big ? 1 : 0;
-    if constexpr (MODE == kGateUp || MODE == kDown) {
-      if (few == kFewMaybe)
-        hipLaunchKernelGGL((dual_gemm_few_rows_kernel<MODE>), dim3(cus * SmallTile::kWgPerCu), dim3(SmallTile::kThreads), 0, s, p);
-    }
-    if (few != kFewMaybe) hipLaunchKernelGGL((dual_gemm_kernel<MODE, SmallTile, KA, KB>), dim3(cus * SmallTile::kWgPerCu),
-                       dim3(SmallTile::kThreads), 0, s, p);
+    hipLaunchKernelGGL((dual_gemm_kernel<MODE, SmallTile, KA, KB>), dim3(cus * SmallTile::kWgPerCu), dim3(SmallTile::kThreads), 0, s, p);
   }
   if (big) {
-    // (a problem of the few-rows form has at most cus / 4 + 4 large tiles, a quarter of its own and one row block's
-    // remainder each: this launch leaves it alone)
     p.gate = small ? 2 : 0;
     using Big = BigTileFor<MODE>;
     static_assert(Big::kWgPerCu == 1, "the split counts one large tile per CU and round");
@@ -2218,19 +2393,14 @@ Params gate_up_params(const FfnArgs& a) {
   return p;
 }
 
-// Whether the few-rows form takes this FFN.  Not with matrices beyond 31-bit byte offsets.  (Where the projections are kept
-// for a backward pass it does, as everywhere: a block's forward is the same with and without gradients.)
-Few few_rows_of(const FfnArgs& a) {
-  const int cus = device_cu_count();
+// The number of rows if the few-rows form takes this FFN, else 0.  Not with matrices beyond 31-bit byte offsets.  (Where the
+// projections are kept for a backward pass it does, as everywhere: a block's forward is the same with and without gradients.)
+int64_t few_rows_of(const FfnArgs& a) {
   const int64_t max_inter = a.inter[0] > a.inter[1] ? a.inter[0] : a.inter[1];
-  if (a.rows > kFewMaxRows || (max_inter + 16) * (a.hidden + 32) * 2 >= (1ll << 31) ||
+  if ((max_inter + 16) * (a.hidden + 32) * 2 >= (1ll << 31) ||
       padded_sorted_rows(a.rows) * (a.hidden > max_inter ? a.hidden : max_inter) * 2 >= (1ll << 31))
-    return kFewNever;
-  if (a.host_rows != nullptr)
-    return few_rows_fm(a.host_rows[0], a.host_rows[1], a.inter[0], a.inter[1], a.hidden, cus) ? kFewAlways : kFewNever;
-  // the split lies with the device: possible if it is with every row on the narrower expert
-  const int64_t i0 = a.inter[0], i1 = a.inter[1];
-  return few_rows_fm(i0 <= i1 ? a.rows : 0, i0 <= i1 ? 0 : a.rows, i0, i1, a.hidden, cus) ? kFewMaybe : kFewNever;
+    return 0;
+  return few_rows(a.rows, a.inter[0], a.inter[1], a.hidden, device_cu_count()) ? a.rows : 0;
 }
 
 int launch_gate_up(const FfnArgs& a, hipStream_t s) {
@@ -2307,6 +2477,20 @@ bool weights_of_last_launch(const void* ws, const FfnArgs& a) {
   return false;
 }
 
+// Tiles of the one launch in the few-rows form: row blocks of 16, blocks of 16 weight rows of a gate/up tile (half gate, half
+// up) and of a down tile, workgroups per CU.
+constexpr int kFewShapes = 4;
+constexpr int kFewShape[kFewShapes][4] = {{1, 2, 2, 2}, {1, 4, 4, 2}, {2, 4, 4, 1}, {2, 4, 8, 1}};
+using FfnKernel = void (*)(Params, Params, FusedSync, int);
+template <int Q>
+FfnKernel few_rows_kernel(bool x_rows, bool norm) {
+  constexpr int fm = kFewShape[Q][0], nb = kFewShape[Q][1], nbc = kFewShape[Q][2], wg = kFewShape[Q][3];
+  if (norm) return ffn_few_rows_norm_kernel<fm, nb, nbc, wg>;
+  if constexpr (wg == 1)
+    if (!x_rows) return ffn_few_rows_kernel<fm, nb, nbc, wg, false>;
+  return ffn_few_rows_kernel<fm, nb, nbc, wg, true>;
+}
+
 constexpr size_t kFusedWorkspaceInts = 2 * static_cast<size_t>(kFusedCounters) + 1;  // two counter arrays, then the error flag
 int launch_ffn_fused(const FfnArgs& a, int* ws, hipStream_t s) {
   if (ws == nullptr || a.keep_gate != nullptr) return 1;
@@ -2327,14 +2511,37 @@ int launch_ffn_fused(const FfnArgs& a, int* ws, hipStream_t s) {
     }
   }
   const bool rows_known = a.host_rows != nullptr;
-  const Few few = few_rows_of(a);
-  const int few_fm = few == kFewAlways ? few_rows_fm(a.host_rows[0], a.host_rows[1], a.inter[0], a.inter[1], a.hidden, cus) : 0;
-  if (a.norm_weight != nullptr && few_fm != 1) return 1;
-  if (few == kFewAlways) {  // tiles of the few-rows form (at most one per CU)
-    const int rows = 16 * few_fm;
-    const int64_t r0 = ceil_div(a.host_rows[0], rows), r1 = ceil_div(a.host_rows[1], rows);
-    gate_tiles = r0 * (a.inter[0] / 32) + r1 * (a.inter[1] / 32);
-    down_tiles = (r0 + r1) * ceil_div(a.hidden, kFewCols);
+  const bool few = few_rows_of(a) > 0;
+  if (a.norm_weight != nullptr && !few) return 1;
+  int shape = kFewShapes - 1, guess[2] = {0, 0};
+  int64_t places = cus;
+  if (few) {
+    // Where the split of the rows is not known on the host it is taken to be all rows on the narrower expert.  The launch is
+    // right for any split (a workgroup takes as many tiles as there are).
+    const int narrow = a.inter[1] <= a.inter[0] ? 1 : 0;
+    const int64_t rows[2] = {rows_known ? a.host_rows[0] : (narrow ? 0 : a.rows), rows_known ? a.host_rows[1] : (narrow ? a.rows : 0)};
+    guess[0] = static_cast<int>(rows[0]);
+    guess[1] = static_cast<int>(rows[1]);
+    // the smallest tile with at most one gate/up tile per CU whose down tiles have a place beside them, or (as the registers of
+    // the larger tiles leave no such place) behind them
+    for (int q = a.x_rows != nullptr ? 0 : kFewShapes - 2; q < kFewShapes; ++q) {  // (K-tiled rows: the larger tiles only)
+      const int fm = kFewShape[q][0], nb = kFewShape[q][1], nbc = kFewShape[q][2];
+      const int64_t r0 = ceil_div(rows[0], 16 * fm), r1 = ceil_div(rows[1], 16 * fm);
+      gate_tiles = r0 * ceil_div(a.inter[0], 8 * nb) + r1 * ceil_div(a.inter[1], 8 * nb);
+      down_tiles = (r0 + r1) * ceil_div(a.hidden, 16 * nbc);
+      places = static_cast<int64_t>(cus) * kFewShape[q][3];
+      shape = q;
+      if (gate_tiles <= cus && down_tiles <= (places == cus ? cus - kXcds : cus)) break;
+    }
+    // (Fewer down tiles in the grid than an XCD has places: with two launches in flight together the gate/up tiles of either
+    // then find a place however many workgroups wait.)
+    if (!rows_known) {  // (for rows that are on the wide expert after all)
+      const int64_t spare = places - ceil_div(down_tiles, kXcds) * kXcds;
+      gate_tiles = gate_tiles < spare ? spare : cus;
+    }
+    gate_tiles = gate_tiles < cus ? gate_tiles : cus;
+    const int64_t most = places == cus ? cus - kXcds : cus;
+    down_tiles = down_tiles < most ? down_tiles : most;
   } else if (!rows_known) {
     // The split of the rows is only known on the device.  The launch is right for any split (workgroups take as
     // many tiles as there are), so what the host has to settle is whether it is the faster form whatever the split.
@@ -2351,7 +2558,6 @@ int launch_ffn_fused(const FfnArgs& a, int* ws, hipStream_t s) {
   Params pg = gate_up_params(a), pd = down_params(a);
   pg.gate = pd.gate = 0;
   pg.split = pd.split = 0;
-  pg.few_rows_cus = pd.few_rows_cus = few == kFewNever ? 0 : cus;
   FusedSync fs{};
   fs.ready = ws;
   fs.passed = ws + kFusedCounters;
@@ -2371,14 +2577,20 @@ int launch_ffn_fused(const FfnArgs& a, int* ws, hipStream_t s) {
   fs.gather = a.out_row_id;
   const int producers = static_cast<int>((gate_tiles + kXcds - 1) / kXcds * kXcds);
   const int consumers = static_cast<int>((down_tiles + kXcds - 1) / kXcds * kXcds);
-  if (a.norm_weight != nullptr) {
+  if (few) {
+    fs.guess[0] = guess[0];
+    fs.guess[1] = guess[1];
     fs.norm_weight = static_cast<const __bf16*>(a.norm_weight);
     fs.norm_eps = a.norm_eps;
-    hipLaunchKernelGGL(ffn_few_rows_norm_kernel, dim3(producers + consumers), dim3(SmallTile::kThreads), 0, s, pg, pd, fs, producers);
-    return check_launch("ffn_few_rows_norm_kernel");
+    const bool x_rows = a.x_rows != nullptr, norm = a.norm_weight != nullptr;
+    const FfnKernel kernel = shape == 0   ? few_rows_kernel<0>(x_rows, norm)
+                             : shape == 1 ? few_rows_kernel<1>(x_rows, norm)
+                             : shape == 2 ? few_rows_kernel<2>(x_rows, norm)
+                                          : few_rows_kernel<3>(x_rows, norm);
+    hipLaunchKernelGGL(kernel, dim3(producers + consumers), dim3(kFewThreads), 0, s, pg, pd, fs, producers);
+    return check_launch("ffn_few_rows_kernel");
   }
-  const auto kernel = a.x_rows != nullptr ? (few != kFewNever ? ffn_fused_kernel<true, true> : ffn_fused_kernel<true, false>)
-                                          : (few != kFewNever ? ffn_fused_kernel<false, true> : ffn_fused_kernel<false, false>);
+  const FfnKernel kernel = a.x_rows != nullptr ? ffn_fused_kernel<true> : ffn_fused_kernel<false>;
   hipLaunchKernelGGL(kernel, dim3(producers + consumers), dim3(SmallTile::kThreads), 0, s, pg, pd, fs, producers);
   return check_launch("ffn_fused_kernel");
 }
@@ -2391,7 +2603,7 @@ int launch_norm_ffn_few_rows(const void* x, const void* x_tiled, void* out, cons
                              int64_t num_rows, int64_t hidden, int64_t inter0, int64_t inter1, const int64_t* host_rows,
                              const void* norm_weight, float eps, void* workspace, hipStream_t stream) {
   // (hidden: what the norm's kernel takes in its whole-line form)
-  if (!x || !x_tiled || !out || !sorted_row_id || !host_rows || !norm_weight || !workspace || !(eps >= 0.f) || num_rows <= 0 ||
+  if (!x || !x_tiled || !out || !sorted_row_id || !norm_weight || !workspace || !(eps >= 0.f) || num_rows <= 0 ||
       num_rows > kFewMaxRows || hidden <= 0 || hidden % 256 != 0 || hidden > 2048)
     return 1;
   if ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(x_tiled) | reinterpret_cast<uintptr_t>(norm_weight) |
