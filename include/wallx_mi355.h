@@ -113,6 +113,11 @@ int wx_unpermute_rows(const void* y, void* out, const int32_t* row_id_map, const
 int wx_unpermute_rows_bwd(const void* grad_out, const void* y_fwd, void* act_grad, float* prob_grad,
                           const int32_t* row_id_map, const float* probs, int64_t num_tokens,
                           int num_topk, int64_t num_cols, int dtype, wx_stream_t stream);
+/* The same with the num_rows rows of act_grad that no token maps to set to zero. */
+int wx_unpermute_rows_bwd_clear(const void* grad_out, const void* y_fwd, void* act_grad, int64_t num_rows,
+                                float* prob_grad, const int32_t* row_id_map, const float* probs,
+                                int64_t num_tokens, int num_topk, int64_t num_cols, int dtype,
+                                wx_stream_t stream);
 
 /* ------------------------------------------------------------------------------------------------
  * Dual asymmetric grouped GEMM: out_e = op(in_e) @ op(w_e), e in {0, 1}, in ONE launch; bf16 in/out,

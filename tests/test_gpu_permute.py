@@ -194,3 +194,49 @@ def test_permute_autograd_and_unpermute_backward(dev):
     rag, rpg, _ = oracle.unpermute_bwd_ref(gb, yb, ref_map, probs)
     assert torch.equal(ag.cpu(), rag)
     assert torch.allclose(pg.cpu(), rpg, rtol=1e-5, atol=1e-4)
+
+
+@pytest.mark.parametrize("T,K,R,H,dtype", [
+    (1, 1, 1, 8, torch.bfloat16), (65, 1, 400, 72, torch.float16), (700, 1, 500, 2048, torch.bfloat16),
+    (130, 3, 129, 520, torch.float32), (513, 2, 70001, 32, torch.bfloat16), (9, 1, 4194433, 8, torch.bfloat16),
+])
+def test_unpermute_backward_clears_the_rows_without_a_token(dev, T, K, R, H, dtype):
+    """A map that leaves rows out (and drops some of the tokens), into memory that held something else before: the rows it
+    names are the gradients, all others zeros.  129 and 400 rows end inside a workgroup's share of 128 or fewer; 4194433 is
+    one share of 65537 each, more than a workgroup's bitmap holds at a time."""
+    g = torch.Generator().manual_seed(T + R)
+    rmap = torch.full((T * K,), -1, dtype=torch.int32)
+    live = min(T * K, R) * 3 // 4
+    at = torch.randperm(T * K, generator=g)[:live]
+    rows = torch.cat((torch.tensor([R - 1, 0]), 1 + torch.randperm(max(R - 2, 0), generator=g)))[:live]
+    rmap[at] = rows.to(torch.int32)
+    dy = torch.randn(T, H, generator=g).to(dtype)
+    y = torch.randn(min(R, 70001), H, generator=g).to(dtype)
+    probs = torch.rand(T, K, generator=g)
+    y_dev = torch.zeros(R, H, dtype=dtype, device=dev)
+    y_dev[:y.size(0)] = y.to(dev)
+    torch.full((R, H), 7.0, dtype=dtype, device=dev)  # (freed: the result's memory)
+    got, dp = native.unpermute_bwd(dy.to(dev), y_dev, rmap.to(dev), probs.to(dev))
+    want = torch.zeros(R, H, dtype=dtype)
+    tok = torch.arange(T).repeat(K)[at]
+    if K == 1:
+        want[rows] = dy[tok]
+        assert torch.equal(native.unpermute_rows_bwd(dy.to(dev), y_dev, rmap.to(dev)).cpu(), want)
+        assert not dp.any()
+    else:
+        p = probs.t().reshape(-1)[at]  # entry k * T + t of the map
+        want[rows] = (dy[tok].float() * p.to(dtype).float()[:, None]).to(dtype)
+        dropped = (rmap < 0).view(K, T).t()
+        assert not dp.cpu()[dropped].any() and dp.cpu()[~dropped].all()
+    assert torch.equal(got.cpu(), want)
+
+
+@pytest.mark.parametrize("T,E", [(4097, 2), (6145, 200), (14593, 2)])
+def test_partition_of_ragged_segments(dev, T, E):
+    """The keys of 512 per wavefront are asked for together; the last wavefronts' are cut short or not there at all."""
+    g = torch.Generator().manual_seed(T)
+    ids = torch.randint(0, E, (T,), generator=g, dtype=torch.int32)
+    rmap, off, srt, _ = native.partition(ids.to(dev), E, 0, None, want_sorted=True)
+    _, ref_map, ref_sorted = oracle.permute_ref(torch.zeros(T, 8), ids)
+    assert torch.equal(rmap.cpu(), ref_map) and torch.equal(srt.cpu(), ref_sorted)
+    assert torch.equal(off.cpu(), oracle.expert_offsets_ref(ids, E))

@@ -33,6 +33,20 @@ __device__ __forceinline__ int load_key(const void* ids, int itype, int64_t i, i
   return static_cast<int>(v);
 }
 
+// The keys of kAhead groups of 64 from `base` on (a lane past `end` holds 0).  They are asked for together: a wavefront that
+// loads one group at a time waits out a memory latency per group (14593 int32 keys, us: count 7.6 -> 5.6; scatter, which
+// waits for its sums over the histograms first, 9.1 either way).
+constexpr int kAhead = 8;
+__device__ __forceinline__ void load_keys(const void* ids, int itype, int64_t base, int64_t end, int num_experts, int (&key)[kAhead],
+                                          bool& bad) {
+  const int64_t first = base + lane_id();
+#pragma unroll
+  for (int u = 0; u < kAhead; ++u) {
+    const int64_t i = first + u * kWave;
+    key[u] = i < end ? load_key(ids, itype, i, num_experts, bad) : 0;
+  }
+}
+
 // Calls f(key, mask) once per distinct key among the active lanes; mask = lanes holding that key.
 template <typename F>
 __device__ __forceinline__ void for_each_key_group(int key, bool active, F f) {
@@ -56,13 +70,15 @@ __global__ __launch_bounds__(kBlock) void partition_count(const void* __restrict
   const int64_t begin = seg * seg_len;
   const int64_t end = begin + seg_len < n ? begin + seg_len : n;
   bool bad = false;
-  for (int64_t base = begin; base < end; base += kWave) {
-    const int64_t i = base + lane;
-    const bool active = i < end;
-    const int key = active ? load_key(ids, itype, i, num_experts, bad) : 0;
-    for_each_key_group(key, active, [&](int k, uint64_t mask) {
-      if (lane == 0) s_hist[w][k] += __popcll(mask);
-    });
+  for (int64_t base = begin; base < end; base += kAhead * kWave) {
+    int key[kAhead];
+    load_keys(ids, itype, base, end, num_experts, key, bad);
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) {
+      for_each_key_group(key[u], base + u * kWave + lane < end, [&](int k, uint64_t mask) {
+        if (lane == 0) s_hist[w][k] += __popcll(mask);
+      });
+    }
   }
   if (begin < n) {
     for (int i = lane; i < kBins; i += kWave) hist[seg * kBins + i] = s_hist[w][i];
@@ -128,22 +144,26 @@ __global__ __launch_bounds__(kBlock) void partition_scatter(
   const int64_t end = begin + seg_len < n ? begin + seg_len : n;
   const uint64_t below = (1ull << lane) - 1ull;
   bool bad = false;
-  for (int64_t base = begin; base < end; base += kWave) {
-    const int64_t i = base + lane;
-    const bool active = i < end;
-    const int key = active ? load_key(ids, itype, i, num_experts, bad) : 0;
-    int32_t pos = 0;
-    for_each_key_group(key, active, [&](int k, uint64_t mask) {
-      const int32_t start = s_run[w][k];  // same address for the whole wave: LDS broadcast
-      if (active && key == k) pos = start + __popcll(mask & below);
-      __builtin_amdgcn_wave_barrier();
-      if (lane == 0) s_run[w][k] = start + __popcll(mask);
-      __builtin_amdgcn_wave_barrier();
-    });
-    if (active) {
-      const int64_t t = i / num_topk, k = i - t * num_topk;
-      row_id_map[k * num_tokens + t] = pos < num_out ? pos : -1;
-      if (sorted_row_id != nullptr) sorted_row_id[pos] = static_cast<int32_t>(i);
+  for (int64_t base = begin; base < end; base += kAhead * kWave) {
+    int key[kAhead];
+    load_keys(ids, itype, base, end, num_experts, key, bad);
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) {
+      const int64_t i = base + u * kWave + lane;
+      const bool active = i < end;
+      int32_t pos = 0;
+      for_each_key_group(key[u], active, [&](int k, uint64_t mask) {
+        const int32_t start = s_run[w][k];  // same address for the whole wave: LDS broadcast
+        if (active && key[u] == k) pos = start + __popcll(mask & below);
+        __builtin_amdgcn_wave_barrier();
+        if (lane == 0) s_run[w][k] = start + __popcll(mask);
+        __builtin_amdgcn_wave_barrier();
+      });
+      if (active) {
+        const int64_t t = num_topk == 1 ? i : i / num_topk, k = i - t * num_topk;
+        row_id_map[k * num_tokens + t] = pos < num_out ? pos : -1;
+        if (sorted_row_id != nullptr) sorted_row_id[pos] = static_cast<int32_t>(i);
+      }
     }
   }
 }
@@ -171,13 +191,15 @@ __global__ __launch_bounds__(kSmallWaves* kWave) void partition_small_kernel(
   const int64_t end = begin + chunk < n ? begin + chunk : n;
   bool bad = false;
   __builtin_amdgcn_wave_barrier();
-  for (int64_t base = begin; base < end; base += kWave) {
-    const int64_t i = base + lane;
-    const bool active = i < end;
-    const int key = active ? load_key(ids, itype, i, num_experts, bad) : 0;
-    for_each_key_group(key, active, [&](int k, uint64_t mask) {
-      if (lane == 0) s_run[w][k] += __popcll(mask);
-    });
+  for (int64_t base = begin; base < end; base += kAhead * kWave) {
+    int key[kAhead];
+    load_keys(ids, itype, base, end, num_experts, key, bad);
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) {
+      for_each_key_group(key[u], base + u * kWave + lane < end, [&](int k, uint64_t mask) {
+        if (lane == 0) s_run[w][k] += __popcll(mask);
+      });
+    }
   }
   if (status != nullptr && __ballot(bad) != 0 && lane == 0) *status = 1;
   __syncthreads();
@@ -209,22 +231,26 @@ __global__ __launch_bounds__(kSmallWaves* kWave) void partition_small_kernel(
   }
   __syncthreads();
   const uint64_t below = (1ull << lane) - 1ull;
-  for (int64_t base = begin; base < end; base += kWave) {
-    const int64_t i = base + lane;
-    const bool active = i < end;
-    const int key = active ? load_key(ids, itype, i, num_experts, bad) : 0;
-    int32_t pos = 0;
-    for_each_key_group(key, active, [&](int k, uint64_t mask) {
-      const int32_t start = s_run[w][k];  // same address for the whole wave: LDS broadcast
-      if (active && key == k) pos = start + __popcll(mask & below);
-      __builtin_amdgcn_wave_barrier();
-      if (lane == 0) s_run[w][k] = start + __popcll(mask);
-      __builtin_amdgcn_wave_barrier();
-    });
-    if (active) {
-      const int64_t t = i / num_topk, k = i - t * num_topk;
-      row_id_map[k * num_tokens + t] = pos < num_out ? pos : -1;
-      if (sorted_row_id != nullptr) sorted_row_id[pos] = static_cast<int32_t>(i);
+  for (int64_t base = begin; base < end; base += kAhead * kWave) {
+    int key[kAhead];
+    load_keys(ids, itype, base, end, num_experts, key, bad);
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) {
+      const int64_t i = base + u * kWave + lane;
+      const bool active = i < end;
+      int32_t pos = 0;
+      for_each_key_group(key[u], active, [&](int k, uint64_t mask) {
+        const int32_t start = s_run[w][k];  // same address for the whole wave: LDS broadcast
+        if (active && key[u] == k) pos = start + __popcll(mask & below);
+        __builtin_amdgcn_wave_barrier();
+        if (lane == 0) s_run[w][k] = start + __popcll(mask);
+        __builtin_amdgcn_wave_barrier();
+      });
+      if (active) {
+        const int64_t t = num_topk == 1 ? i : i / num_topk, k = i - t * num_topk;
+        row_id_map[k * num_tokens + t] = pos < num_out ? pos : -1;
+        if (sorted_row_id != nullptr) sorted_row_id[pos] = static_cast<int32_t>(i);
+      }
     }
   }
 }
@@ -460,41 +486,98 @@ __global__ __launch_bounds__(kMoverWaves* kWave) void combine_rows_kernel(
   }
 }
 
-// Backward of the weighted combine; one wavefront per token.
+// Backward of the weighted combine; one wavefront per token.  The rows of act_grad that no token maps to are zeros: the
+// first `clearers` workgroups find them in their share of the num_rows rows by reading the whole map into a bitmap in LDS, and
+// clear them, beside the workgroups that move rows.  (Clearing all of act_grad in a launch of its own ahead of this one
+// writes every row twice: 14593 rows of 4 KiB 10.4 us + 25.5 -> 28.8.)  No share when clearers is 0.
+typedef int32_t i32x4_word __attribute__((ext_vector_type(4), aligned(4)));  // four entries at any entry's address
+constexpr int kClearRows = 65536;  // rows of act_grad one workgroup looks after at a time: 8 KiB of bits
 template <int DT>
 __global__ __launch_bounds__(kMoverWaves* kWave) void combine_rows_bwd_kernel(
     const u32x4* __restrict__ grad_out, const u32x4* __restrict__ y_fwd, u32x4* __restrict__ act_grad,
     float* __restrict__ prob_grad, const int32_t* __restrict__ row_id_map, const float* __restrict__ probs,
-    int64_t num_tokens, int num_topk, int64_t vec_per_row) {
+    int64_t num_tokens, int num_topk, int64_t vec_per_row, int64_t num_rows, int clearers) {
   constexpr int E = elems_per_16<DT>();
   const int lane = lane_id();
-  const int64_t wave = static_cast<int64_t>(blockIdx.x) * kMoverWaves + threadIdx.x / kWave;
-  const int64_t n_waves = static_cast<int64_t>(gridDim.x) * kMoverWaves;
+  if (static_cast<int>(blockIdx.x) < clearers) {
+    __shared__ uint32_t s_mapped[kClearRows / 32];
+    const int64_t share = (num_rows + clearers - 1) / clearers;
+    const int64_t last = share * (blockIdx.x + 1) < num_rows ? share * (blockIdx.x + 1) : num_rows;
+    const int64_t n = num_tokens * num_topk;
+    for (int64_t r0 = share * blockIdx.x; r0 < last; r0 += kClearRows) {
+      const int rows = static_cast<int>(last - r0 < kClearRows ? last - r0 : kClearRows);
+      for (int i = threadIdx.x; i < (rows + 31) / 32; i += kMoverWaves * kWave) s_mapped[i] = 0;
+      __syncthreads();
+      // (32 entries per thread and trip, all asked for together: beside the movers a load is back after 2 - 3 us)
+      constexpr int kLoads = 8, kTrip = kLoads * 4 * kMoverWaves * kWave;
+      auto mark = [&](int32_t entry) {
+        const int64_t r = entry - r0;
+        if (r >= 0 && r < rows) atomicOr(&s_mapped[r >> 5], 1u << (r & 31));
+      };
+      int64_t i = 4 * threadIdx.x;
+      for (; i + (kTrip - 4 * kMoverWaves * kWave) + 4 <= n; i += kTrip) {
+        i32x4_word e[kLoads];
+#pragma unroll
+        for (int u = 0; u < kLoads; ++u) e[u] = *reinterpret_cast<const i32x4_word*>(row_id_map + i + u * 4 * kMoverWaves * kWave);
+#pragma unroll
+        for (int u = 0; u < kLoads; ++u)
+#pragma unroll
+          for (int c = 0; c < 4; ++c) mark(e[u][c]);
+      }
+      i32x4_word e[kLoads];
+#pragma unroll
+      for (int u = 0; u < kLoads; ++u)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+          const int64_t at = i + u * 4 * kMoverWaves * kWave + c;
+          e[u][c] = at < n ? row_id_map[at] : -1;
+        }
+#pragma unroll
+      for (int u = 0; u < kLoads; ++u)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) mark(e[u][c]);
+      __syncthreads();
+      for (int i = threadIdx.x / kWave; i < rows; i += kMoverWaves)
+        if (!(s_mapped[i >> 5] >> (i & 31) & 1))
+          for (int64_t v = lane; v < vec_per_row; v += kWave) st16(act_grad + (r0 + i) * vec_per_row + v, u32x4{0, 0, 0, 0});
+      __syncthreads();
+    }
+    return;
+  }
+  const int64_t wave = static_cast<int64_t>(blockIdx.x - clearers) * kMoverWaves + threadIdx.x / kWave;
+  const int64_t n_waves = static_cast<int64_t>(gridDim.x - clearers) * kMoverWaves;
   const bool weighted = num_topk > 1 && probs != nullptr;
   for (int64_t t = wave; t < num_tokens; t += n_waves) {
+    const u32x4* src = grad_out + t * vec_per_row;
     for (int k = 0; k < num_topk; ++k) {
       const int32_t r = row_id_map[k * num_tokens + t];
+      u32x4* dst = act_grad + static_cast<int64_t>(r) * vec_per_row;
+      if (!weighted) {
+        if (r < 0) continue;
+        int64_t v = lane;
+        for (; v + 3 * kWave < vec_per_row; v += 4 * kWave) {
+          const u32x4 a = ld16(src + v), b = ld16(src + v + kWave), c = ld16(src + v + 2 * kWave), d = ld16(src + v + 3 * kWave);
+          st16(dst + v, a); st16(dst + v + kWave, b); st16(dst + v + 2 * kWave, c); st16(dst + v + 3 * kWave, d);
+        }
+        for (; v < vec_per_row; v += kWave) st16(dst + v, ld16(src + v));
+        continue;
+      }
       float dot = 0.f;
       if (r >= 0) {
-        const float p = weighted ? Elem<DT>::round(probs[t * num_topk + k]) : 1.f;
+        const float p = Elem<DT>::round(probs[t * num_topk + k]);
         for (int64_t v = lane; v < vec_per_row; v += kWave) {
-          const u32x4 g16 = ld16(grad_out + t * vec_per_row + v);
-          if (!weighted) {
-            st16(act_grad + static_cast<int64_t>(r) * vec_per_row + v, g16);
-            continue;
-          }
           float g[E], yv[E], o[E];
-          unpack16<DT>(g16, g);
+          unpack16<DT>(ld16(src + v), g);
           unpack16<DT>(ld16(y_fwd + static_cast<int64_t>(r) * vec_per_row + v), yv);
 #pragma unroll
           for (int e = 0; e < E; ++e) {
             o[e] = Elem<DT>::round(g[e] * p);
             dot += Elem<DT>::round(g[e] * yv[e]);
           }
-          st16(act_grad + static_cast<int64_t>(r) * vec_per_row + v, pack16<DT>(o));
+          st16(dst + v, pack16<DT>(o));
         }
       }
-      if (weighted && prob_grad != nullptr) {
+      if (prob_grad != nullptr) {
 #pragma unroll
         for (int d = kWave / 2; d > 0; d >>= 1) dot += __shfl_xor(dot, d);
         if (lane == 0) prob_grad[t * num_topk + k] = dot;
@@ -752,30 +835,52 @@ extern "C" int wx_unpermute_rows(const void* y, void* out, const int32_t* row_id
   return check_launch("wx_unpermute_rows");
 }
 
-extern "C" int wx_unpermute_rows_bwd(const void* grad_out, const void* y_fwd, void* act_grad, float* prob_grad,
-                                     const int32_t* row_id_map, const float* probs, int64_t num_tokens,
-                                     int num_topk, int64_t num_cols, int dtype, wx_stream_t stream) {
-  if (int rc = check_rows("wx_unpermute_rows_bwd", grad_out, act_grad, row_id_map, num_tokens, num_topk, num_cols,
-                          dtype))
-    return rc;
+namespace {
+
+// num_rows: rows of act_grad, those without a token to be cleared; 0 = act_grad is the caller's to clear.
+int unpermute_rows_bwd(const char* who, const void* grad_out, const void* y_fwd, void* act_grad, int64_t num_rows, float* prob_grad,
+                       const int32_t* row_id_map, const float* probs, int64_t num_tokens, int num_topk, int64_t num_cols, int dtype,
+                       hipStream_t s) {
+  if (int rc = check_rows(who, grad_out, act_grad, row_id_map, num_tokens, num_topk, num_cols, dtype)) return rc;
+  if (num_rows < 0 || num_rows > INT32_MAX) return fail(WX_ERR_INVALID_ARGUMENT, "%s: bad sizes", who);
+  if (num_rows > 0 && act_grad == nullptr) return fail(WX_ERR_INVALID_ARGUMENT, "%s: null pointer", who);
   if (num_topk > 1 && (probs == nullptr || y_fwd == nullptr || prob_grad == nullptr))
-    return fail(WX_ERR_INVALID_ARGUMENT, "wx_unpermute_rows_bwd: probs, y_fwd and prob_grad are required for topK > 1");
-  if (num_tokens == 0) return WX_OK;
+    return fail(WX_ERR_INVALID_ARGUMENT, "%s: probs, y_fwd and prob_grad are required for topK > 1", who);
+  if (num_tokens == 0 && num_rows == 0) return WX_OK;
   const int64_t vec = num_cols * elem_bytes(dtype) / 16;
-  const dim3 grid(mover_grid(num_tokens)), block(kMoverWaves * kWave);
-  hipStream_t s = as_stream(stream);
+  // (a workgroup's share of the rows: what it reads is the whole map, so few of them, but enough to clear many rows quickly)
+  const int64_t shares = (num_rows + 127) / 128;
+  const int clearers = static_cast<int>(shares < 64 ? shares : 64);
+  const int movers = mover_grid(num_tokens), places = device_cu_count() * 8 - clearers;  // (all of them have a place at once)
+  const dim3 grid(static_cast<unsigned>((movers < places ? movers : places) + clearers)), block(kMoverWaves * kWave);
   const u32x4* g = static_cast<const u32x4*>(grad_out);
   const u32x4* yf = static_cast<const u32x4*>(y_fwd);
   u32x4* ag = static_cast<u32x4*>(act_grad);
   if (dtype == WX_F32) {
     hipLaunchKernelGGL(combine_rows_bwd_kernel<WX_F32>, grid, block, 0, s, g, yf, ag, prob_grad, row_id_map, probs,
-                       num_tokens, num_topk, vec);
+                       num_tokens, num_topk, vec, num_rows, clearers);
   } else if (dtype == WX_F16) {
     hipLaunchKernelGGL(combine_rows_bwd_kernel<WX_F16>, grid, block, 0, s, g, yf, ag, prob_grad, row_id_map, probs,
-                       num_tokens, num_topk, vec);
+                       num_tokens, num_topk, vec, num_rows, clearers);
   } else {
     hipLaunchKernelGGL(combine_rows_bwd_kernel<WX_BF16>, grid, block, 0, s, g, yf, ag, prob_grad, row_id_map, probs,
-                       num_tokens, num_topk, vec);
+                       num_tokens, num_topk, vec, num_rows, clearers);
   }
-  return check_launch("wx_unpermute_rows_bwd");
+  return check_launch(who);
+}
+
+}  // namespace
+
+extern "C" int wx_unpermute_rows_bwd(const void* grad_out, const void* y_fwd, void* act_grad, float* prob_grad,
+                                     const int32_t* row_id_map, const float* probs, int64_t num_tokens,
+                                     int num_topk, int64_t num_cols, int dtype, wx_stream_t stream) {
+  return unpermute_rows_bwd("wx_unpermute_rows_bwd", grad_out, y_fwd, act_grad, 0, prob_grad, row_id_map, probs, num_tokens,
+                            num_topk, num_cols, dtype, as_stream(stream));
+}
+
+extern "C" int wx_unpermute_rows_bwd_clear(const void* grad_out, const void* y_fwd, void* act_grad, int64_t num_rows,
+                                           float* prob_grad, const int32_t* row_id_map, const float* probs, int64_t num_tokens,
+                                           int num_topk, int64_t num_cols, int dtype, wx_stream_t stream) {
+  return unpermute_rows_bwd("wx_unpermute_rows_bwd_clear", grad_out, y_fwd, act_grad, num_rows, prob_grad, row_id_map, probs,
+                            num_tokens, num_topk, num_cols, dtype, as_stream(stream));
 }

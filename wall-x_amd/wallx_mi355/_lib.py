@@ -33,6 +33,7 @@ PROTOTYPES = {
     "wx_permute_rows": (_i32, [_vp, _vp, _vp, _i64, _i32, _i64, _i32, _vp]),
     "wx_unpermute_rows": (_i32, [_vp, _vp, _vp, _vp, _i64, _i32, _i64, _i32, _vp]),
     "wx_unpermute_rows_bwd": (_i32, [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i32, _i64, _i32, _vp]),
+    "wx_unpermute_rows_bwd_clear": (_i32, [_vp, _vp, _vp, _i64, _vp, _vp, _vp, _i64, _i32, _i64, _i32, _vp]),
     "wx_dual_gemm": (_i32, [_vp] * 6 + [_i64] * 6 + [_i32, _i32, _vp]),
     "wx_dual_gemm_add": (_i32, [_vp] * 8 + [_i64] * 6 + [_i32, _i32, _vp]),
     "wx_tiled_bytes": (_sz, [_i64, _i64]),

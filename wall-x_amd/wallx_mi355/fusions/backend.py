@@ -50,6 +50,11 @@ def unpermute_bwd(input_bwd, input_fwd, row_id_map, prob):
     return native.unpermute_bwd(input_bwd, input_fwd, row_id_map, prob)
 
 
+def unpermute_rows_bwd(input_bwd, input_fwd, row_id_map):
+    """No counterpart in backend.py: unpermute_bwd's first result for one expert per token and no weights."""
+    return native.unpermute_rows_bwd(input_bwd, input_fwd, row_id_map)
+
+
 def rope(q, k, cos, sin, q_out, k_out, mrope_section_doubled, layout: str = "csrc") -> None:
     """backend.py:233-262.  layout: "csrc" = the channel map of the reference's kernel, "hf" = its PyTorch path."""
     return native.rope(q, k, cos, sin, q_out, k_out, mrope_section_doubled, layout)

@@ -105,6 +105,8 @@ class PermuteMoE_topK(torch.autograd.Function):
             cls.workspace_fw = []
         permuted_act, row_id_map, cls.workspace_fw = backend.permute(
             input_act, indices, num_out_tokens, cls.workspace_fw, cls.max_expanded_token_num)
+        ctx.set_materialize_grads(False)  # no zeros for row_id_map's gradient, which nothing reads
+        ctx.permuted_like = (permuted_act.shape, permuted_act.dtype, permuted_act.device)
         ctx.row_id_map = row_id_map
         ctx.num_tokens = indices.size(0)
         ctx.num_topK = num_topK
@@ -113,6 +115,9 @@ class PermuteMoE_topK(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, permuted_act_grad, _):
+        if permuted_act_grad is None:
+            shape, dtype, device = ctx.permuted_like
+            permuted_act_grad = torch.zeros(shape, dtype=dtype, device=device)
         if not permuted_act_grad.numel():
             return permuted_act_grad, None, None, None
         grad = backend.unpermute(permuted_act_grad.contiguous(), ctx.row_id_map, torch.tensor([]),
@@ -171,8 +176,11 @@ class UnpermuteMoE_topK(torch.autograd.Function):
         input_act, row_id_map, probs = ctx.saved_tensors
         act_grad = prob_grad = None
         if ctx.needs_input_grad[0]:
-            act_grad, prob_grad = backend.unpermute_bwd(unpermuted_act_grad.contiguous(), input_act, row_id_map,
-                                                        probs)
+            if probs is None:
+                act_grad = backend.unpermute_rows_bwd(unpermuted_act_grad.contiguous(), input_act, row_id_map)
+            else:
+                act_grad, prob_grad = backend.unpermute_bwd(unpermuted_act_grad.contiguous(), input_act, row_id_map,
+                                                            probs)
         if not ctx.needs_input_grad[2]:
             prob_grad = None
         return act_grad, None, prob_grad

@@ -265,17 +265,28 @@ def unpermute_bwd(input_bwd: torch.Tensor, input_fwd: torch.Tensor, row_id_map: 
     """
     _need_cuda("input_bwd", input_bwd)
     T, K = prob.shape
+    prob = prob.to(device=input_bwd.device, dtype=torch.float32).contiguous()
+    # (K > 1: the kernel writes every entry)
+    prob_grad = (torch.empty if K > 1 else torch.zeros)((T, K), dtype=torch.float32, device=input_bwd.device)
+    return _unpermute_rows_bwd(input_bwd, input_fwd, row_id_map, prob, prob_grad, T, K), prob_grad
+
+
+def unpermute_rows_bwd(input_bwd: torch.Tensor, input_fwd: torch.Tensor, row_id_map: torch.Tensor) -> torch.Tensor:
+    """act_grad of `unpermute_bwd` for one expert per token and no weights: neither weights nor their gradient exist."""
+    _need_cuda("input_bwd", input_bwd)
+    return _unpermute_rows_bwd(input_bwd, input_fwd, row_id_map, None, None, input_bwd.size(0), 1)
+
+
+def _unpermute_rows_bwd(input_bwd, input_fwd, row_id_map, prob, prob_grad, T, K):
     input_bwd = input_bwd.contiguous()
     input_fwd = input_fwd.contiguous()
     row_id_map = row_id_map.to(device=input_bwd.device, dtype=torch.int32).contiguous()
-    prob = prob.to(device=input_bwd.device, dtype=torch.float32).contiguous()
-    act_grad = torch.zeros((input_fwd.size(0), input_bwd.size(1)), dtype=input_bwd.dtype, device=input_bwd.device)
-    prob_grad = torch.zeros((T, K), dtype=torch.float32, device=input_bwd.device)
+    act_grad = torch.empty((input_fwd.size(0), input_bwd.size(1)), dtype=input_bwd.dtype, device=input_bwd.device)
     with _DeviceGuard(input_bwd):
-        _lib.call("wx_unpermute_rows_bwd", _ptr(input_bwd), _ptr(input_fwd), _ptr(act_grad), _ptr(prob_grad),
-                  _ptr(row_id_map), _ptr(prob), T, K, input_bwd.size(1), _dtype_code(input_bwd),
+        _lib.call("wx_unpermute_rows_bwd_clear", _ptr(input_bwd), _ptr(input_fwd), _ptr(act_grad), act_grad.size(0),
+                  _ptr(prob_grad), _ptr(row_id_map), _ptr(prob), T, K, input_bwd.size(1), _dtype_code(input_bwd),
                   _stream(input_bwd))
-    return act_grad, prob_grad
+    return act_grad
 
 
 # ----------------------------------------------------------------------------- M-RoPE
