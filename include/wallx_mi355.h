@@ -362,6 +362,11 @@ int wx_rot_pos_emb(const float* inv_freq, int n_freq, const void* grid_thw, int 
                    int64_t n_grid, int spatial_merge_size, int64_t total_patches, float* table,
                    int64_t* pos_ids, wx_stream_t stream);
 
+/* Host code: totals[0] = sum t*h*w, totals[1] = sum t*(h/m)*(w/m), totals[2] = sum t*ceil(h/m/ws)*ceil(w/m/ws) of a
+ * grid_thw [n_grid, 3] (int32 or int64) in HOST memory: the sizes of the results of wx_rot_pos_emb and wx_window_index. */
+int wx_grid_totals(const void* grid_thw_host, int grid_type, int64_t n_grid, int64_t spatial_merge_size,
+                   int64_t vit_merger_window_size, int64_t* totals);
+
 /* Vision-tower window permutation.  Replaces get_window_index_cuda (csrc/window_index.cu:208-286)
  * and follows get_window_index (vl.py:502-547) with one cumulative entry per non-empty window.
  * grid_thw [n_grid, 3] int32 or int64 on the device.  window_index int32 [total_tokens], total_tokens =

@@ -160,3 +160,28 @@ def test_wallx_csrc_shim_exposes_the_nine_native_names():
     for name in ("asym_dual_gmm", "permute", "unpermute", "unpermute_bwd", "rope", "rope_bwd", "rope_index",
                  "rot_pos_emb", "get_window_index"):
         assert callable(getattr(wallx_csrc, name))
+
+
+@pytest.mark.parametrize("dtype", [torch.int32, torch.int64])
+@pytest.mark.parametrize("merge,window", [(1, 1), (2, 4), (3, 5)])
+def test_grid_totals_are_those_of_the_rows(dtype, merge, window):
+    """Host code: sides that are no multiples of the merge size or the window, empty and negative ones (rounded down), and
+    rows that are not packed; a total beyond 64 bits is refused."""
+    import ctypes
+
+    from wallx_mi355 import _lib, native
+    grids = torch.tensor([[1, 32, 32], [2, 17, 31], [0, 8, 8], [3, 1, 70], [1, 7, 0], [2, -5, 9]], dtype=dtype)
+    for src in (grids, grids.t().contiguous().t(), grids[:0]):
+        rows = src.tolist()
+        cells = [(t, h // merge, w // merge) for t, h, w in rows]
+        want = (sum(t * h * w for t, h, w in rows), sum(t * h * w for t, h, w in cells),
+                sum(t * -(-h // window) * -(-w // window) for t, h, w in cells))
+        assert native._grid_totals(src, None, merge, window) == want
+        assert native._grid_totals(src.double(), None, merge, window) == want  # (read row by row)
+    huge = torch.tensor([[4, 2 ** 31, 2 ** 31]])
+    with pytest.raises(RuntimeError, match="patches"):
+        native._grid_totals(huge, None)
+    lib = _lib.load()
+    assert lib.wx_grid_totals(None, 7, 0, 1, 1, (ctypes.c_int64 * 3)()) == -1
+    assert lib.wx_grid_totals(None, _lib.WX_I64, 1, 1, 1, (ctypes.c_int64 * 3)()) == -1
+    assert lib.wx_grid_totals(None, _lib.WX_I64, 0, 0, 1, (ctypes.c_int64 * 3)()) == -1

@@ -155,6 +155,31 @@ int check_grid(const char* who, const void* grid_thw, int grid_type, int64_t n_g
 
 using namespace wx;
 
+// Host code: what the sizes of the two results below come to (divisions round down, as Python's do).
+extern "C" int wx_grid_totals(const void* grid_thw_host, int grid_type, int64_t n_grid, int64_t merge, int64_t window, int64_t* totals) {
+  const char* who = "wx_grid_totals";
+  if (grid_type != WX_I32 && grid_type != WX_I64) return fail(WX_ERR_INVALID_ARGUMENT, "%s: grid_thw must be int32 or int64", who);
+  if (n_grid < 0 || merge <= 0 || window <= 0) return fail(WX_ERR_INVALID_ARGUMENT, "%s: bad sizes", who);
+  if (totals == nullptr || (n_grid > 0 && grid_thw_host == nullptr)) return fail(WX_ERR_INVALID_ARGUMENT, "%s: null pointer", who);
+  auto at = [&](int64_t i) {
+    return grid_type == WX_I64 ? static_cast<const int64_t*>(grid_thw_host)[i] : static_cast<int64_t>(static_cast<const int32_t*>(grid_thw_host)[i]);
+  };
+  auto floor_div = [](int64_t a, int64_t b) { return a / b - (a % b != 0 && a < 0 ? 1 : 0); };
+  int64_t sum[3] = {0, 0, 0};
+  for (int64_t g = 0; g < n_grid; ++g) {
+    const int64_t t = at(3 * g), h = at(3 * g + 1), w = at(3 * g + 2);
+    const int64_t gh = floor_div(h, merge), gw = floor_div(w, merge);
+    const int64_t sides[3][2] = {{h, w}, {gh, gw}, {-floor_div(-gh, window), -floor_div(-gw, window)}};
+    for (int i = 0; i < 3; ++i) {
+      int64_t n;
+      if (__builtin_mul_overflow(t, sides[i][0], &n) || __builtin_mul_overflow(n, sides[i][1], &n) || __builtin_add_overflow(sum[i], n, &sum[i]))
+        return fail(WX_ERR_UNSUPPORTED, "%s: more than 2^63 - 1 patches", who);
+    }
+  }
+  for (int i = 0; i < 3; ++i) totals[i] = sum[i];
+  return WX_OK;
+}
+
 extern "C" int wx_rot_pos_emb(const float* inv_freq, int n_freq, const void* grid_thw, int grid_type, int64_t n_grid,
                               int spatial_merge_size, int64_t total_patches, float* table, int64_t* pos_ids,
                               wx_stream_t stream) {

@@ -61,6 +61,7 @@ PROTOTYPES = {
     "wx_rope_index_workspace_bytes": (_sz, [_i64, _i64]),
     "wx_rope_index": (_i32, [_vp, _vp, _vp, _i64, _vp, _i64, _vp, _i64, _i64, _i32, _i64, _i64, _i64, _f32,
                              _vp, _vp, _vp, _vp, _sz, _vp]),
+    "wx_grid_totals": (_i32, [_vp, _i32, _i64, _i64, _i64, _c.POINTER(_i64)]),
     "wx_rot_pos_emb": (_i32, [_vp, _i32, _vp, _i32, _i64, _i32, _i64, _vp, _vp, _vp]),
     "wx_window_index": (_i32, [_vp, _i32, _i64, _i32, _i32, _i32, _i64, _i64, _vp, _vp, _vp]),
     "wx_rmsnorm_permute_rows_tiled": (_i32, [_vp, _vp, _f32, _vp, _vp, _vp, _i64, _i64, _vp]),
@@ -109,7 +110,9 @@ def check(rc: int, exc=RuntimeError):
 
 
 def call(name: str, *args, exc=RuntimeError):
-    check(getattr(load(), name)(*args), exc)
+    rc = getattr(_lib or load(), name)(*args)
+    if rc != 0:
+        check(rc, exc)
 
 
 def i64x2(vals):

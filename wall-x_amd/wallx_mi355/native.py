@@ -50,7 +50,8 @@ def is_checked() -> bool:
 
 
 def _stream(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+    # what torch.cuda.current_stream(t.device).cuda_stream is, without the Stream object around it (2 us of a call)
+    return torch._C._cuda_getCurrentRawStream(t.get_device())
 
 
 def capture_id(stream: int) -> int:
@@ -85,13 +86,15 @@ def _dtype_code(t: torch.Tensor) -> int:
 class _DeviceGuard:
     """Makes the tensor's device current for the launch when it is not already."""
 
+    __slots__ = ("idx", "prev")
+
     def __init__(self, t: torch.Tensor):
-        self.idx = t.device.index
+        self.idx = t.get_device()
         self.prev = None
 
     def __enter__(self):
-        cur = torch.cuda.current_device()
-        if self.idx is not None and self.idx != cur:
+        cur = torch._C._cuda_getDevice()  # (torch.cuda.current_device() of a process that holds a CUDA tensor)
+        if self.idx >= 0 and self.idx != cur:
             self.prev = cur
             torch.cuda.set_device(self.idx)
 
@@ -479,7 +482,8 @@ def rope_index(input_ids, image_grid_thw, video_grid_thw, second_per_grid_ts, at
     spg = None if second_per_grid_ts is None else second_per_grid_ts.to(device=dev, dtype=torch.float32).contiguous()
     pos = torch.empty((3, B, S), dtype=torch.int64, device=dev)
     deltas = torch.empty((B, 1), dtype=torch.int64, device=dev)
-    status = torch.zeros(1, dtype=torch.int32, device=dev)
+    # (only where somebody looks at it: clearing it is a launch)
+    status = torch.zeros(1, dtype=torch.int32, device=dev) if _checked or return_status else None
     ws_bytes = _lib.load().wx_rope_index_workspace_bytes(B, S)
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
     with _DeviceGuard(ids):
@@ -487,7 +491,7 @@ def rope_index(input_ids, image_grid_thw, video_grid_thw, second_per_grid_ts, at
                   0 if ig is None else ig.size(0), None if vg is None else vg.data_ptr(),
                   0 if vg is None else vg.size(0), _ptr(spg), B, S, int(spatial_merge_size), int(image_token_id),
                   int(video_token_id), int(vision_start_token_id), float(tokens_per_second), _ptr(pos),
-                  _ptr(deltas), status.data_ptr(), ws.data_ptr(), ws_bytes, _stream(ids))
+                  _ptr(deltas), _ptr(status), ws.data_ptr(), ws_bytes, _stream(ids))
     if _checked and int(status.item()):
         # the Python path raises on such rows (list.index / grid indexing, act.py:1013-1045)
         raise ValueError("rope_index: a row's vision tokens, <vision_start> markers and grids do not add up "
@@ -497,13 +501,20 @@ def rope_index(input_ids, image_grid_thw, video_grid_thw, second_per_grid_ts, at
     return pos, deltas
 
 
-def _host_grid(grid_thw: torch.Tensor, grid_thw_host):
-    """grid_thw as a host list of (t, h, w); copies device -> host (one sync) unless a host copy is given."""
-    if grid_thw_host is not None:
-        src = grid_thw_host
-    else:
-        src = grid_thw
-    return [tuple(int(v) for v in row) for row in src.cpu().tolist()]
+def _grid_totals(grid_thw: torch.Tensor, grid_thw_host, merge: int = 1, window: int = 1):
+    """(sum t h w, sum t (h // merge) (w // merge), the windows of `window` x `window` merged cells) over the rows (t, h, w) of
+    grid_thw; copies device -> host (one sync) unless a host copy is given."""
+    src = grid_thw if grid_thw_host is None else grid_thw_host
+    src = src.cpu()
+    if src.dim() == 2 and src.size(1) == 3 and src.dtype in (torch.int32, torch.int64) and merge > 0 and window > 0:
+        src = src.contiguous()
+        out = (ctypes.c_int64 * 3)()
+        _lib.call("wx_grid_totals", src.data_ptr(), _ITYPES[src.dtype], src.size(0), merge, window, out)
+        return tuple(out)
+    rows = [tuple(int(v) for v in row) for row in src.tolist()]
+    cells = [(t, h // merge, w // merge) for t, h, w in rows]
+    return (sum(t * h * w for t, h, w in rows), sum(t * h * w for t, h, w in cells),
+            sum(t * (-(-h // window)) * (-(-w // window)) for t, h, w in cells))
 
 
 def rot_pos_emb(inv_freq: torch.Tensor, grid_thw: torch.Tensor, spatial_merge_size: int,
@@ -521,8 +532,7 @@ def rot_pos_emb(inv_freq: torch.Tensor, grid_thw: torch.Tensor, spatial_merge_si
         raise RuntimeError("grid_thw must be int32 or int64")
     grid = grid_thw.contiguous()
     inv = inv_freq.contiguous()
-    rows = _host_grid(grid, grid_thw_host)
-    total = sum(t * h * w for t, h, w in rows)
+    total = _grid_totals(grid, grid_thw_host)[0]
     F = inv.numel()
     table = torch.empty((total, 2 * F), dtype=torch.float32, device=inv.device)
     ids = torch.empty((total, 2), dtype=torch.int64, device=inv.device) if return_ids else None
@@ -545,10 +555,8 @@ def get_window_index(grid_thw: torch.Tensor, spatial_merge_size: int, vit_merger
     dev = grid.device
     if grid.size(0) == 0:  # csrc/window_index.cu:220-225
         return torch.empty(0, dtype=torch.int32, device=dev), torch.zeros(1, dtype=torch.int32, device=dev)
-    rows = _host_grid(grid, grid_thw_host)
     m, ws = int(spatial_merge_size), int(vit_merger_window_size)
-    n_tok = sum(t * (h // m) * (w // m) for t, h, w in rows)
-    n_win = sum(t * (-(-(h // m) // ws)) * (-(-(w // m) // ws)) for t, h, w in rows)
+    _, n_tok, n_win = _grid_totals(grid, grid_thw_host, m, ws)
     if n_tok == 0 or n_win == 0:  # csrc/window_index.cu:253-258
         return torch.empty(0, dtype=torch.int32, device=dev), torch.zeros(1, dtype=torch.int32, device=dev)
     window_index = torch.empty(n_tok, dtype=torch.int32, device=dev)
