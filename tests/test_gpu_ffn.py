@@ -868,3 +868,23 @@ def test_moe_block_under_bf16_autocast_takes_fp32_input(dev):
     assert torch.equal(y, yb)
     yb.float().sum().backward()
     assert torch.equal(x32.grad, xb.grad.float())
+
+
+@pytest.mark.parametrize("rows,inter", [((32768, 40), (64, 32)), ((32769, 40), (64, 32)), ((300, 0), (96, 32)), ((0, 300), (96, 32)),
+                                        ((70, 33000), (32, 64)), ((1, 1), (32, 32))])
+def test_input_grads_in_shared_launches(dev, rows, inter):
+    """dX = dG Wg + dU Wu on both sides of the line between a launch per product and a launch per expert (on 256 CUs 32768
+    rows of 256 columns are its last), with either expert empty or the wider: the bits of the two products and their bf16 sum."""
+    H = 256
+    g = torch.Generator(device=dev).manual_seed(rows[0] + rows[1])
+    n = lambda *s: torch.empty(s, dtype=torch.bfloat16, device=dev).normal_(0, 1, generator=g)
+    dg, du = ([n(m, i) for m, i in zip(rows, inter)] for _ in range(2))
+    wg, wu = ([n(i, H) for i in inter] for _ in range(2))
+    got = moe._input_grads(dg, du, wg, wu, H)
+    want = torch.empty(sum(rows), H, dtype=torch.bfloat16, device=dev)
+    o0, o1 = want[:rows[0]], want[rows[0]:]
+    native.asym_dual_gmm(dg[0], dg[1], wg[0], wg[1], o0, o1, False, False)
+    native.asym_dual_gmm(du[0], du[1], wu[0], wu[1], o0, o1, False, False, add_expert0=o0, add_expert1=o1)
+    assert torch.equal(got, want)
+    ref = torch.cat([a.float() @ b.float() + c.float() @ d.float() for a, b, c, d in zip(dg, wg, du, wu)])
+    assert float((got.float() - ref).norm()) <= 2 ** -7 * float(ref.norm())  # three bf16 roundings

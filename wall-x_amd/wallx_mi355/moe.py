@@ -196,6 +196,32 @@ def _weight_grads(a0, a1, b0, b1, n0, n1, want):
     return _dual(a0, a1, b0, b1, n0, n1, True, False, want=want)
 
 
+def _input_grads(dg, du, wg, wu, H):
+    """dX_e = dG_e Wg_e + dU_e Wu_e over the rows of both experts, [rows_0 + rows_1, H]: the two products rounded to bf16 and
+    their sum rounded once, what the two eager ops and their add give.
+
+    As a rule a launch per product, both experts in each, the second accumulating onto the first in its epilogue.  Where
+    the wide expert's product has few 256 x 256 tiles such a launch leaves CUs idle: two products of at most as many tiles as
+    CUs between them go into one launch as its two problems, the narrow expert's into another, and an add follows.
+    Experts of 11008 and 1024 at hidden 2048, rows of each, a launch per product -> paired with the add, us: 100 + 12
+    158 -> 91, 880 + 32 165 -> 105, 1760 + 64 182 -> 174, 2640 + 96 291 -> 217, 3520 + 128 326 -> 247, 4050 + 65 345 -> 267.
+    Beyond, two rounds of large tiles take what two launches of one round do.  The same bits either way."""
+    m0, m1 = dg[0].size(0), dg[1].size(0)
+    dev = dg[0].device
+    out = torch.empty(m0 + m1, H, dtype=torch.bfloat16, device=dev)
+    o0, o1 = out[:m0], out[m0:]
+    wide = 0 if wg[0].size(0) >= wg[1].size(0) else 1
+    if 2 * -(-dg[wide].size(0) // 256) * -(-H // 256) > _cus(dev):
+        native.asym_dual_gmm(dg[0], dg[1], wg[0], wg[1], o0, o1, False, False)
+        native.asym_dual_gmm(du[0], du[1], wu[0], wu[1], o0, o1, False, False, add_expert0=o0, add_expert1=o1)
+        return out
+    second = torch.empty_like(out)
+    for e, rows in enumerate((slice(0, m0), slice(m0, m0 + m1))):
+        if dg[e].size(0):
+            native.asym_dual_gmm(dg[e], du[e], wg[e], wu[e], out[rows], second[rows], False, False)
+    return out.add_(second)
+
+
 class _MoeBlockFunction(torch.autograd.Function):
     """[RMSNorm ->] permute -> both experts' SwiGLU FFN -> unpermute [+ residual] with a backward (act.py:105-162,
     and the decoder layer's lines around it, act.py:256-265, under autograd).
@@ -314,12 +340,7 @@ class _MoeBlockFunction(torch.autograd.Function):
             grads[2], grads[5] = _weight_grads(dy0, dy1, hm0, hm1, I0, I1, (need[7], need[10]))
         dx = dnorm = None
         if need_x or need_norm:
-            # dX = dG Wg + dU Wu: the second product accumulates onto the first in its epilogue (bf16 + bf16, rounded
-            # once -- what the two eager ops and their add give)
-            dxs = torch.empty(T, H, dtype=torch.bfloat16, device=x.device)
-            d0_, d1_ = dxs[:m0], dxs[m0:m0 + m1]
-            native.asym_dual_gmm(dg0, dg1, g0, g1, d0_, d1_, False, False)
-            native.asym_dual_gmm(du0, du1, u0, u1, d0_, d1_, False, False, add_expert0=d0_, add_expert1=d1_)
+            dxs = _input_grads((dg0, dg1), (du0, du1), (g0, g1), (u0, u1), H)
             if ctx.has_norm:
                 dx, dnorm = native.unpermute_rmsnorm_bwd(dxs, x.detach(), norm_weight.detach(), ctx.eps, row_id_map,
                                                          add=dy if ctx.residual else None)
