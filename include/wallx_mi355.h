@@ -233,6 +233,17 @@ int wx_dual_down_proj_residual(const void* hmid, void* out, const void* residual
                                int64_t num_rows, int64_t hidden, int64_t inter0, int64_t inter1,
                                const int64_t* host_rows_per_expert, const int32_t* out_row_id,
                                wx_stream_t stream);
+/* wx_dual_down_proj (residual NULL) or wx_dual_down_proj_residual with scratch for a launch that cuts its contraction into
+ * parts where its tiles would leave CUs idle (513 to about 1100 rows at hidden 2048 and an expert of 11008): the fp32 sums of
+ * the parts are added in order, so the result may differ from the form without in the last bit of a bf16, and is the same on
+ * every call.  split_scratch: NULL (the form without), or wx_ffn_split_scratch_bytes() bytes of device memory, 16-byte
+ * aligned, zeroed ONCE by the caller before the first use; each launch leaves it ready for the next one on its stream.  One per
+ * stream. */
+size_t wx_ffn_split_scratch_bytes(void);
+int wx_dual_down_proj_split(const void* hmid, void* out, const void* residual, const int32_t* expert_offsets,
+                            const void* down0, const void* down1, int64_t num_rows, int64_t hidden,
+                            int64_t inter0, int64_t inter1, const int64_t* host_rows_per_expert,
+                            const int32_t* out_row_id, void* split_scratch, wx_stream_t stream);
 /* wx_dual_swiglu_gate_up for a forward pass whose backward will follow: besides hmid it stores the two projections
  * themselves (rounded to bf16, before the SwiGLU) into gate_keep / up_keep, K-tiled buffers of hmid's size and
  * geometry, so that the backward does not run the two projections again.  The reference keeps these activations
@@ -433,6 +444,13 @@ int wx_moe_block_forward(const void* x, void* out, const int32_t* row_id_map, co
                          int64_t num_rows, int64_t hidden, int64_t inter0, int64_t inter1,
                          const int64_t* host_rows_per_expert, const void* norm_weight, float eps,
                          int add_residual, void* ffn_workspace, wx_stream_t stream);
+/* The same with the scratch of wx_dual_down_proj_split (or NULL) for its down launch. */
+int wx_moe_block_forward_split(const void* x, void* out, const int32_t* row_id_map, const int32_t* sorted_row_id,
+                               const int32_t* expert_offsets, const void* gate0, const void* up0, const void* down0,
+                               const void* gate1, const void* up1, const void* down1, void* x_tiled, void* hmid,
+                               int64_t num_rows, int64_t hidden, int64_t inter0, int64_t inter1,
+                               const int64_t* host_rows_per_expert, const void* norm_weight, float eps,
+                               int add_residual, void* ffn_workspace, void* split_scratch, wx_stream_t stream);
 
 /* Elementwise backward of h = silu(g) * u inside an expert FFN (act.py:79-82; the reference leaves it to autograd):
  * from gate, up (the two projections, kept by the forward or recomputed) and dh (gradient w.r.t. h) in one pass:

@@ -888,3 +888,51 @@ def test_input_grads_in_shared_launches(dev, rows, inter):
     assert torch.equal(got, want)
     ref = torch.cat([a.float() @ b.float() + c.float() @ d.float() for a, b, c, d in zip(dg, wg, du, wu)])
     assert float((got.float() - ref).norm()) <= 2 ** -7 * float(ref.norm())  # three bf16 roundings
+
+
+@pytest.mark.parametrize("rows,inter,hidden", [
+    ((513, 0), (11008, 1024), 256), ((880, 32), (11008, 1024), 2048), ((1024, 1), (11008, 1024), 2048), ((1025, 0), (11008, 1024), 2048),
+    ((300, 400), (8224, 96), 2048), ((40, 700), (64, 4128), 1056), ((520, 500), (4096, 4096), 512), ((512, 0), (11008, 1024), 256),
+])
+@pytest.mark.parametrize("known", [True, False])
+def test_down_projection_with_its_contraction_in_parts(dev, rows, inter, hidden, known):
+    """wx_dual_down_proj_split on both sides of each of its lines (513 rows, a quarter and half as many tiles as CUs, 2048 of K
+    per part, one expert or both cut, a last part that is short) against the form without parts: no further from 64-bit results,
+    the same bits on every call -- also where the library knows the row counts only on the device -- and the scratch's
+    counters left at zero.  With and without the residual at the tokens' places."""
+    T = sum(rows)
+    g = torch.Generator(device=dev).manual_seed(T + hidden)
+    n = lambda *s: torch.empty(s, dtype=torch.bfloat16, device=dev).normal_(0, 1, generator=g)
+    h, d = [n(m, i) for m, i in zip(rows, inter)], [n(hidden, i) for i in inter]
+    pads = [(m + 255) // 256 * 256 for m in rows]
+    hmid = torch.zeros(native.padded_sorted_rows(T) * max(inter), dtype=torch.bfloat16, device=dev)
+    first = 0
+    for m, i, pad, v in zip(rows, inter, pads, h):
+        if m:
+            tiled = native.pack_weight(torch.cat((v, v.new_zeros(pad - m, i))), cache=False).view(-1)
+            hmid[first:first + pad * i] = tiled[:pad * i]
+        first += pad * i
+    packed = [native.pack_weight(w, cache=False) for w in d]
+    off = torch.tensor([0, rows[0], T], dtype=torch.int32, device=dev)
+    stream = torch.cuda.current_stream().cuda_stream
+    host = _lib.i64x2(rows) if known else None
+    scratch = torch.empty(_lib.load().wx_ffn_split_scratch_bytes() // 4, dtype=torch.int32, device=dev)
+    scratch[:256] = 0
+
+    def run(split, residual=None, order=None):
+        out = torch.full((T, hidden), 9.0, dtype=torch.bfloat16, device=dev)
+        _lib.call("wx_dual_down_proj_split", hmid.data_ptr(), out.data_ptr(), None if residual is None else residual.data_ptr(),
+                  off.data_ptr(), packed[0].data_ptr(), packed[1].data_ptr(), T, hidden, *inter, host,
+                  None if order is None else order.data_ptr(), scratch.data_ptr() if split else None, stream)
+        return out
+    want = torch.cat([a.double() @ b.double().t() for a, b in zip(h, d)])
+    plain, got = run(False), run(True)
+    error = lambda v: float((v.double() - want).norm() / want.norm())
+    assert error(got) <= 1.01 * error(plain) < 2 ** -8
+    for _ in range(3):
+        assert torch.equal(run(True), got)
+    assert not scratch[:256].any()
+    order = torch.randperm(T, device=dev, generator=g).to(torch.int32)
+    res = n(T, hidden)
+    both = run(True, res, order)
+    assert torch.equal(both[order.long()], (res[order.long()].float() + got.float()).to(torch.bfloat16))

@@ -115,4 +115,10 @@ int launch_norm_ffn_few_rows(const void* x, const void* x_tiled, void* out, cons
                              int64_t num_rows, int64_t hidden, int64_t inter0, int64_t inter1, const int64_t* host_rows,
                              const void* norm_weight, float eps, void* workspace, hipStream_t stream);
 
+// wx_dual_swiglu_ffn_fused with the down launch's scratch for a split contraction (dual_gemm.hip); NULL = without.
+int ffn_fused(const void* x_rows, void* x_tiled, void* out, const void* residual, const int32_t* expert_offsets, const void* gate0,
+              const void* up0, const void* down0, const void* gate1, const void* up1, const void* down1, void* hmid,
+              int64_t num_rows, int64_t hidden, int64_t inter0, int64_t inter1, const int64_t* host_rows_per_expert,
+              const int32_t* out_row_id, void* workspace, void* split_scratch, wx_stream_t stream);
+
 }  // namespace wx

@@ -175,6 +175,7 @@ constexpr int waitcnt_imm(int vm, int lgkm) { return (vm & 15) | ((vm >> 4) << 1
 
 struct TileCoord {
   int group, tm, tn;
+  int part;  // split contraction: which part of it (down_parts)
 };
 
 // Linear tile id -> coordinates.  Ids are first spread so that each XCD (workgroup id mod 8) walks its own
@@ -257,6 +258,30 @@ __host__ __device__ inline long long shape_deciding_tiles(long long tiles0, long
   return tiles0 + tiles1;
 }
 
+// The down launch's contraction in parts.  A 128 x 128 tile's K step takes 250 ns however many CUs work and however deep the
+// ring is, so 512 .. 1024 rows of an expert of 11008 -- 64 .. 128 tiles of 344 steps -- took 87 us with half of the CUs or more
+// idle.  The tiles of the expert that decides the launch's length (both experts', unless one's contraction is at most half as
+// long as the other's) are cut into two or four parts along K while all parts have a CU of their own and 2048 of K; the part
+// that finishes last adds them up: 500 rows 87 -> 41 us, 513 .. 880 rows 87 -> 52 .. 54, 1024 rows 87 -> 61.  From half as many tiles as CUs on, two parts on every CU take what one did (1760
+// rows: 90 us; parts of 250 tiles would be at 470 ns a step, two workgroups to a CU).
+// Evaluated identically on the host and on the device, so that the sums' order does not depend on which of them knows the row
+// counts: not where a host that knows them takes the one launch for both GEMMs, nor up to the 2 * cus rows of which it takes
+// the one launch without knowing them.
+__host__ __device__ inline void down_parts(int m0, int m1, int k0, int k1, int hidden, int cus, int parts[2]) {
+  parts[0] = parts[1] = 1;
+  const long long rb0 = (static_cast<long long>(m0) + 127) / 128, rb1 = (static_cast<long long>(m1) + 127) / 128;
+  const long long cols = (static_cast<long long>(hidden) + 127) / 128;
+  if (static_cast<long long>(m0) + m1 <= 2ll * cus) return;
+  if (rb0 * ((k0 + 63) / 64) + rb1 * ((k1 + 63) / 64) <= cus && (rb0 + rb1) * cols <= cus) return;
+  const bool cut0 = rb0 > 0 && (rb1 == 0 || 2ll * k0 > k1), cut1 = rb1 > 0 && (rb0 == 0 || 2ll * k1 > k0);
+  const long long count = ((cut0 ? rb0 : 0) + (cut1 ? rb1 : 0)) * cols;
+  const int k = cut0 && cut1 ? (k0 < k1 ? k0 : k1) : (cut0 ? k0 : k1);
+  int n = 1;
+  while (n < 4 && count * n * 2 <= cus && k / (2 * n) >= 2048) n *= 2;
+  if (cut0) parts[0] = n;
+  if (cut1) parts[1] = n;
+}
+
 // Workgroup barrier without the fences of __syncthreads().  Those fences make the compiler wait for EVERY
 // outstanding LDS-direct load (vmcnt(0)) at the barrier, which drains the prefetch ring on each K step; the waits
 // the data flow needs (own LDS reads returned, own loads of the next slot landed) are written out before each call.
@@ -321,6 +346,10 @@ struct FusedSync {
   // few-rows form with the norm folded in: the token rows pass through an RMSNorm on their way to the MFMAs
   const __bf16* norm_weight;
   float norm_eps;
+  // split contraction (down_parts): fp32 sums of the parts, split_slots of a tile's size, and a counter per slot, all zero
+  float* split_sums;
+  int* split_count;
+  int split_slots;
 };
 
 // Fused launch: what this workgroup wrote for row block `rb` is in memory (its stores are write-through and every
@@ -949,6 +978,14 @@ __device__ __forceinline__ void dual_gemm_body(const Params& p, const int wg, co
     const bool few = shape_deciding_tiles(big(g0.m, g0.n), big(g1.m, g1.n), g0.k, g1.k) <= p.gate_tiles;
     if (few != (p.gate == 1)) return;  // uniform: the other tile shape's launch does this problem
   }
+  // split contraction: part q of a column tile is a column tile of its own, all columns' part 0 first
+  int parts[2] = {1, 1};
+  const int cols_n[2] = {tiles_n[0], tiles_n[1]};
+  if constexpr (ROLE == 3) {
+    down_parts(g0.m, g1.m, g0.k, g1.k, g0.n, fs.split_slots, parts);
+    tiles_n[0] *= parts[0];
+    tiles_n[1] *= parts[1];
+  }
   int total = tiles_m[0] * tiles_n[0] + tiles_m[1] * tiles_n[1];  // the host bounds this below 2^31
   // tail split: the first launch (256 x 256 tiles) stops at `split_at`; the second (this shape: 128 x 128)
   // takes virtual tiles [split_at, all) of the 256 x 256 tiling, kSubM x kSubN pieces each
@@ -1047,11 +1084,18 @@ __device__ __forceinline__ void dual_gemm_body(const Params& p, const int wg, co
     int rows, cols_left, ldc, nk;
     int row0, col0;         // first row / column of the tile inside its group's output
     int row_block;          // fused launch: index of the tile's (expert, row block) counters
+    int part, parts, slot;  // split contraction: this part, how many, the slot of the tile's first part
   };
 
   // K steps of a tile rounded up to whole ring rounds (padding steps read zeros).  The host never launches this
   // kernel with k == 0 and a non-empty output: the tile loop below advances only from inside the K loop.
   auto padded_steps = [](int k) { return ((k + BK - 1) / BK + kStages - 1) / kStages * kStages; };
+  // split contraction: the K steps of a part (whole ring rounds; the last part has what is left)
+  auto part_steps = [&](int k, int n) { return ((k / BK + n - 1) / n + kStages - 1) / kStages * kStages; };
+  auto part_k = [&](int k, int n, int part) {
+    const int left = k - part * part_steps(k, n) * BK, most = part_steps(k, n) * BK;
+    return left < most ? left : most;
+  };
   auto setup_store = [&](const TileCoord& tc, Store& S) {
     const Group G = tc.group ? g1 : g0;
     const int row0 = tc.tm * BM, col0 = tc.tn * kTileN;
@@ -1080,12 +1124,24 @@ __device__ __forceinline__ void dual_gemm_body(const Params& p, const int wg, co
     S.row_block = tc.group * kFusedMaxRowBlocks + tc.tm;
     S.ldc = G.ldc;
     S.nk = padded_steps(G.k);
+    if constexpr (ROLE == 3) {
+      S.part = tc.part;
+      S.parts = tc.group ? parts[1] : parts[0];
+      S.slot = (tc.group && parts[0] > 1 ? tiles_m[0] * tiles_n[0] : 0) + (tc.tm * (tc.group ? cols_n[1] : cols_n[0]) + tc.tn) * S.parts;
+      S.nk = padded_steps(part_k(G.k, S.parts, tc.part));
+    }
   };
   auto setup_loader = [&](const TileCoord& tc, Loader& L) {
     const Group G = tc.group ? g1 : g0;
     const int row0 = tc.tm * BM, col0 = tc.tn * kTileN;
     L.K = G.k;
-    L.nk = padded_steps(G.k);
+    int64_t first = 0;  // the tile's first K step
+    if constexpr (ROLE == 3) {
+      const int n = tc.group ? parts[1] : parts[0];
+      L.K = part_k(G.k, n, tc.part);
+      first = static_cast<int64_t>(tc.part) * part_steps(G.k, n);
+    }
+    L.nk = padded_steps(L.K);
     constexpr int kHalfWaves = kLoadWaves / 2;  // SwiGLU: the first half of the loading waves load gate rows, the rest up rows
     const bool up_half = SWIGLU && wave >= kHalfWaves;
     const __bf16* b_src = up_half ? G.b1 : G.b0;
@@ -1093,7 +1149,7 @@ __device__ __forceinline__ void dual_gemm_body(const Params& p, const int wg, co
     if constexpr (TILED_IN) {
       // this wave's row blocks of the A tile and of the B tile at K step 0; a K step later they sit one column
       // block further, i.e. (row blocks of the matrix) KiB ahead
-      const int64_t b_blk = col0 / kBlkRows + b_wave * kLoadsB;
+      const int64_t b_blk = first * G.ldb + col0 / kBlkRows + b_wave * kLoadsB;
       L.b_base = b_src + (b_blk << 9);
       L.b_step = static_cast<int64_t>(G.ldb) << 10;
       const int64_t b_left = (static_cast<int64_t>(G.k / kBlkCols) * G.ldb - b_blk) << 10;
@@ -1122,7 +1178,7 @@ __device__ __forceinline__ void dual_gemm_body(const Params& p, const int wg, co
           L.voff_a[i] = v;
         }
       } else {
-        const int64_t a_blk = (G.a_row0 + row0) / kBlkRows + wave * kLoadsA;
+        const int64_t a_blk = first * G.lda + (G.a_row0 + row0) / kBlkRows + wave * kLoadsA;
         L.a_base = G.a + (a_blk << 9);
         L.a_step = static_cast<int64_t>(G.lda) << 10;
         const int64_t a_left = (static_cast<int64_t>(G.k / kBlkCols) * G.lda - a_blk) << 10;
@@ -1774,6 +1830,54 @@ __device__ __forceinline__ void dual_gemm_body(const Params& p, const int wg, co
     }
   };
 
+  // Split contraction: leaves this part's sums in its slot and says whether it was the tile's last to do so; the sums of all
+  // parts, in their order, are then in the accumulators.  The slots are written through to memory and counted once they are
+  // there (like the fused launch's intermediate); nobody waits for anybody.
+  auto last_part = [&](const Store& S) {
+    if constexpr (ROLE == 3) {
+      constexpr uint32_t kWaveBytes = FM * FN * 1024;
+      auto sums_of = [&](int part) {
+        return make_rsrc(reinterpret_cast<char*>(fs.split_sums) + (static_cast<int64_t>(S.slot + part) * kWaves + wave) * kWaveBytes, kWaveBytes);
+      };
+      const __amdgpu_buffer_rsrc_t mine = sums_of(S.part);
+#pragma unroll
+      for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int j = 0; j < FN; ++j)
+          __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, acc[i][j]), mine, (i * FN + j) * 1024 + lane * 16, 0, 16 /* sc1 */);
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+      __builtin_amdgcn_s_waitcnt(waitcnt_imm(0, 0));
+      __syncthreads();
+      volatile int* const s_before = reinterpret_cast<volatile int*>(s_out);  // (the staging area is free between tiles)
+      if (tid == 0) *s_before = __hip_atomic_fetch_add(fs.split_count + S.slot, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      __syncthreads();
+      const bool last = __builtin_amdgcn_readfirstlane(*s_before) == S.parts - 1;
+      __syncthreads();
+      if (!last) return false;
+      if (tid == 0) __hip_atomic_store(fs.split_count + S.slot, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      f32x4 sum[FM][FN];
+      for (int q = 0; q < S.parts; ++q) {
+        const __amdgpu_buffer_rsrc_t from = sums_of(q);
+        f32x4 v[FM][FN];
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+#pragma unroll
+          for (int j = 0; j < FN; ++j)
+            v[i][j] = q == S.part ? acc[i][j]
+                                  : __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(from, (i * FN + j) * 1024 + lane * 16, 0, 16 /* sc1 */));
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+#pragma unroll
+          for (int j = 0; j < FN; ++j) sum[i][j] = q == 0 ? v[i][j] : sum[i][j] + v[i][j];
+      }
+#pragma unroll
+      for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int j = 0; j < FN; ++j) acc[i][j] = sum[i][j];
+    }
+    return true;
+  };
+
   // ---- persistent loop -------------------------------------------------------------------------------
   // The load stream runs kStages K steps ahead of the MFMAs and crosses tile boundaries: the last kStages steps
   // of a tile refill the ring with the first kStages steps of the next tile, so the pipeline never drains and
@@ -1795,6 +1899,11 @@ __device__ __forceinline__ void dual_gemm_body(const Params& p, const int wg, co
       return have;
     }
     for (; next_t < padded && !have; next_t += n_wg) have = map_tile(next_t, total, tiles_m, tiles_n, tc);
+    if constexpr (ROLE == 3) {
+      const int cols = tc.group ? cols_n[1] : cols_n[0];
+      tc.part = have ? __builtin_amdgcn_readfirstlane(tc.tn / cols) : 0;
+      tc.tn -= tc.part * cols;
+    }
     return have;
   };
   TileCoord tc;
@@ -1921,7 +2030,11 @@ __device__ __forceinline__ void dual_gemm_body(const Params& p, const int wg, co
           k_step_as(with_loads, std::integral_constant<int, 3>{}, L, ld_ks);
         }
       }
-      epilogue(done);
+      if constexpr (ROLE == 3) {
+        if (done.parts == 1 || last_part(done)) epilogue(done);
+      } else {
+        epilogue(done);
+      }
       if constexpr (ROLE == 1) count_done(fs, tid, done.row_block);
       if constexpr (ROLE == 2) {
         clear_if_last(fs, tid, done.row_block, passed_before, fs.consumers);
@@ -1950,6 +2063,11 @@ __global__ __launch_bounds__(TS::kThreads, TS::kWgPerCu) void dual_gemm_kernel(P
 }
 
 // The few-rows form of the same launch (MODE: gate/up or down).
+// the down launch of small tiles with the contraction in parts
+__global__ __launch_bounds__(SmallTile::kThreads, SmallTile::kWgPerCu) void down_split_kernel(Params p, FusedSync fs) {
+  dual_gemm_body<kDown, SmallTile, false, false, 3>(p, blockIdx.x, gridDim.x, fs);
+}
+
 template <int MODE, int FM, int NB>
 __global__ __launch_bounds__(kFewThreads, 2) void dual_gemm_few_rows_kernel(Params p) {
   constexpr int R = MODE == kGateUp ? 8 : 4;
@@ -2085,9 +2203,10 @@ int check_dims(const char* who, int64_t m, int64_t n, int64_t k, bool k_in_rows 
 // host knows, decides it on the host); when the host cannot tell, both launches are made and the device decides (the
 // second returns at once if there is nothing to split).
 // few: the few-rows form takes the problem; its number of rows, or 0.
+// split: the down launch's contraction may be in parts (down_parts) in small tiles, with this scratch.
 template <int MODE, bool KA = false, bool KB = false>
 int launch_mfma(Params p, int64_t tiles_lo, int64_t tiles_hi, hipStream_t s, const char* who,
-                const int64_t* tiles_by_expert = nullptr, int64_t few = 0) {
+                const int64_t* tiles_by_expert = nullptr, int64_t few = 0, const FusedSync* split_sync = nullptr) {
   const int cus = device_cu_count();
   const int threshold = cus / 2;
   if constexpr (MODE == kGateUp || MODE == kDown) {
@@ -2111,7 +2230,10 @@ int launch_mfma(Params p, int64_t tiles_lo, int64_t tiles_hi, hipStream_t s, con
   p.split_cus = cus;
   if (small) {
     p.gate = big ? 1 : 0;
-    hipLaunchKernelGGL((dual_gemm_kernel<MODE, SmallTile, KA, KB>), dim3(cus * SmallTile::kWgPerCu), dim3(SmallTile::kThreads), 0, s, p);
+    if (MODE == kDown && split_sync != nullptr)
+      hipLaunchKernelGGL(down_split_kernel, dim3(cus * SmallTile::kWgPerCu), dim3(SmallTile::kThreads), 0, s, p, *split_sync);
+    else
+      hipLaunchKernelGGL((dual_gemm_kernel<MODE, SmallTile, KA, KB>), dim3(cus * SmallTile::kWgPerCu), dim3(SmallTile::kThreads), 0, s, p);
   }
   if (big) {
     p.gate = small ? 2 : 0;
@@ -2347,6 +2469,7 @@ struct FfnArgs {
   const void* norm_weight = nullptr;  // optional (with x_rows): the rows pass through an RMSNorm first; few rows only
   float norm_eps = 0.f;
   const void* x_rows = nullptr;    // optional: the activations in token order; `x` is then built by the fused launch
+  void* split_scratch = nullptr;   // optional: wx_ffn_split_scratch_bytes() for the down launch's parts
 };
 
 int check_ffn(const char* who, const FfnArgs& a, bool need_gate_up, bool need_down) {
@@ -2438,17 +2561,35 @@ Params down_params(const FfnArgs& a) {
   return p;
 }
 
+constexpr size_t kSplitSlotBytes = static_cast<size_t>(SmallTile::BM) * SmallTile::BN * sizeof(float);
+// counters, a word per slot, in front of the slots
+size_t split_count_bytes() { return (static_cast<size_t>(device_cu_count()) * sizeof(int) + 1023) / 1024 * 1024; }
+
 int launch_down(const FfnArgs& a, hipStream_t s) {
   const Params p = down_params(a);
   const int64_t col_tiles = ceil_div(a.hidden, BigTile::BN);
+  FusedSync sync{};
+  const FusedSync* split = nullptr;
+  if (a.split_scratch != nullptr && a.rows > 2ll * device_cu_count() && a.rows < (1ll << 30)) {
+    int parts[2] = {0, 0};
+    if (a.host_rows != nullptr)
+      down_parts(static_cast<int>(a.host_rows[0]), static_cast<int>(a.host_rows[1]), static_cast<int>(a.inter[0]),
+                 static_cast<int>(a.inter[1]), static_cast<int>(a.hidden), device_cu_count(), parts);
+    if (parts[0] != 1 || parts[1] != 1) {  // (row counts unknown: the launch decides by the same rule)
+      sync.split_count = static_cast<int*>(a.split_scratch);
+      sync.split_sums = reinterpret_cast<float*>(static_cast<char*>(a.split_scratch) + split_count_bytes());
+      sync.split_slots = device_cu_count();
+      split = &sync;
+    }
+  }
   if (a.host_rows != nullptr) {
     const int64_t by_expert[2] = {ceil_div(a.host_rows[0], BigTile::BM) * col_tiles, ceil_div(a.host_rows[1], BigTile::BM) * col_tiles};
     const int64_t tiles = by_expert[0] + by_expert[1];
-    return launch_mfma<kDown>(p, tiles, tiles, s, "dual_gemm_kernel<down>", by_expert, few_rows_of(a));
+    return launch_mfma<kDown>(p, tiles, tiles, s, "dual_gemm_kernel<down>", by_expert, few_rows_of(a), split);
   }
   const int64_t row_tiles = ceil_div(a.rows, BigTile::BM);
   return launch_mfma<kDown>(p, row_tiles * col_tiles, (row_tiles + 1) * col_tiles, s, "dual_gemm_kernel<down>", nullptr,
-                            few_rows_of(a));
+                            few_rows_of(a), split);
 }
 
 // Both launches as one (ffn_fused_kernel), for the shapes where each is a single round of small tiles with the row
@@ -2623,12 +2764,22 @@ int launch_norm_ffn_few_rows(const void* x, const void* x_tiled, void* out, cons
 
 extern "C" size_t wx_ffn_fused_workspace_bytes(void) { return kFusedWorkspaceInts * sizeof(int); }
 
+extern "C" size_t wx_ffn_split_scratch_bytes(void) { return split_count_bytes() + device_cu_count() * kSplitSlotBytes; }
+
 extern "C" int wx_dual_swiglu_ffn_fused(const void* x_rows, void* x_tiled, void* out, const void* residual,
                                         const int32_t* expert_offsets, const void* gate0, const void* up0,
                                         const void* down0, const void* gate1, const void* up1, const void* down1,
                                         void* hmid, int64_t num_rows, int64_t hidden, int64_t inter0, int64_t inter1,
                                         const int64_t* host_rows_per_expert, const int32_t* out_row_id,
                                         void* workspace, wx_stream_t stream) {
+  return wx::ffn_fused(x_rows, x_tiled, out, residual, expert_offsets, gate0, up0, down0, gate1, up1, down1, hmid, num_rows, hidden,
+                       inter0, inter1, host_rows_per_expert, out_row_id, workspace, nullptr, stream);
+}
+
+int wx::ffn_fused(const void* x_rows, void* x_tiled, void* out, const void* residual, const int32_t* expert_offsets, const void* gate0,
+                  const void* up0, const void* down0, const void* gate1, const void* up1, const void* down1, void* hmid,
+                  int64_t num_rows, int64_t hidden, int64_t inter0, int64_t inter1, const int64_t* host_rows_per_expert,
+                  const int32_t* out_row_id, void* workspace, void* split_scratch, wx_stream_t stream) {
   const char* who = "wx_dual_swiglu_ffn_fused";
   FfnArgs a{x_tiled, {gate0, gate1}, {up0, up1}, {down0, down1}, out, hmid, host_rows_per_expert, expert_offsets,
             num_rows, hidden, {inter0, inter1}, out_row_id};
@@ -2645,6 +2796,7 @@ extern "C" int wx_dual_swiglu_ffn_fused(const void* x_rows, void* x_tiled, void*
     a.x_rows = x_rows;
   }
   if (reinterpret_cast<uintptr_t>(workspace) & 3) return fail(WX_ERR_INVALID_ARGUMENT, "%s: workspace must be 4-byte aligned", who);
+  a.split_scratch = split_scratch;
   const int rc = launch_ffn_fused(a, static_cast<int*>(workspace), as_stream(stream));
   if (rc <= 0) return rc;
   if (x_rows != nullptr)
@@ -2706,6 +2858,24 @@ extern "C" int wx_dual_down_proj_residual(const void* hmid, void* out, const voi
     return fail(WX_ERR_INVALID_ARGUMENT, "%s: residual and out_row_id are required (the sum is formed in token order)", who);
   if (reinterpret_cast<uintptr_t>(residual) & 15) return fail(WX_ERR_INVALID_ARGUMENT, "%s: residual must be 16-byte aligned", who);
   a.residual = residual;
+  return launch_down(a, as_stream(stream));
+}
+
+extern "C" int wx_dual_down_proj_split(const void* hmid, void* out, const void* residual, const int32_t* expert_offsets,
+                                       const void* down0, const void* down1, int64_t num_rows, int64_t hidden,
+                                       int64_t inter0, int64_t inter1, const int64_t* host_rows_per_expert,
+                                       const int32_t* out_row_id, void* split_scratch, wx_stream_t stream) {
+  const char* who = "wx_dual_down_proj_split";
+  FfnArgs a{nullptr, {nullptr, nullptr}, {nullptr, nullptr}, {down0, down1}, out, const_cast<void*>(hmid),
+            host_rows_per_expert, expert_offsets, num_rows, hidden, {inter0, inter1}, out_row_id};
+  if (int rc = check_ffn(who, a, false, true)) return rc;
+  if (num_rows == 0) return WX_OK;
+  if (residual != nullptr && !out_row_id)
+    return fail(WX_ERR_INVALID_ARGUMENT, "%s: a residual needs out_row_id (the sum is formed in token order)", who);
+  if ((reinterpret_cast<uintptr_t>(residual) | reinterpret_cast<uintptr_t>(split_scratch)) & 15)
+    return fail(WX_ERR_INVALID_ARGUMENT, "%s: residual and split_scratch must be 16-byte aligned", who);
+  a.residual = residual;
+  a.split_scratch = split_scratch;
   return launch_down(a, as_stream(stream));
 }
 

@@ -594,21 +594,22 @@ extern "C" int wx_unpermute_rows_rmsnorm_bwd(const void* grad_sorted, const void
   return check_launch("column_sums_kernel");
 }
 
-extern "C" int wx_moe_block_forward(const void* x, void* out, const int32_t* row_id_map, const int32_t* sorted_row_id,
+extern "C" int wx_moe_block_forward_split(const void* x, void* out, const int32_t* row_id_map, const int32_t* sorted_row_id,
                                     const int32_t* expert_offsets, const void* gate0, const void* up0,
                                     const void* down0, const void* gate1, const void* up1, const void* down1,
                                     void* x_tiled, void* hmid, int64_t num_rows, int64_t hidden, int64_t inter0,
                                     int64_t inter1, const int64_t* host_rows_per_expert, const void* norm_weight,
-                                    float eps, int add_residual, void* ffn_workspace, wx_stream_t stream) {
+                                    float eps, int add_residual, void* ffn_workspace, void* split_scratch, wx_stream_t stream) {
   const char* who = "wx_moe_block_forward";
   if (num_rows < 0) return fail(WX_ERR_INVALID_ARGUMENT, "%s: negative row count", who);
   if (num_rows == 0) return WX_OK;
+  if (reinterpret_cast<uintptr_t>(split_scratch) & 15)
+    return fail(WX_ERR_INVALID_ARGUMENT, "%s: split_scratch must be 16-byte aligned", who);
   if (!sorted_row_id) return fail(WX_ERR_INVALID_ARGUMENT, "%s: sorted_row_id is required", who);
   if (ffn_workspace != nullptr && norm_weight == nullptr)
     // one launch for the permute and both GEMMs where the shape allows it, else the launches below
-    return wx_dual_swiglu_ffn_fused(x, x_tiled, out, add_residual ? x : nullptr, expert_offsets, gate0, up0, down0, gate1,
-                                    up1, down1, hmid, num_rows, hidden, inter0, inter1, host_rows_per_expert,
-                                    sorted_row_id, ffn_workspace, stream);
+    return ffn_fused(x, x_tiled, out, add_residual ? x : nullptr, expert_offsets, gate0, up0, down0, gate1, up1, down1, hmid,
+                     num_rows, hidden, inter0, inter1, host_rows_per_expert, sorted_row_id, ffn_workspace, split_scratch, stream);
   if (norm_weight != nullptr) {  // few rows: all of it in one launch
     const void* w0[3] = {gate0, up0, down0};
     const void* w1[3] = {gate1, up1, down1};
@@ -624,15 +625,23 @@ extern "C" int wx_moe_block_forward(const void* x, void* out, const int32_t* row
                                            stream))
     return rc;
   if (ffn_workspace != nullptr)  // one launch for both GEMMs where the shape allows it, else the two below
-    return wx_dual_swiglu_ffn_fused(nullptr, x_tiled, out, add_residual ? x : nullptr, expert_offsets, gate0, up0, down0,
-                                    gate1, up1, down1, hmid, num_rows, hidden, inter0, inter1, host_rows_per_expert,
-                                    sorted_row_id, ffn_workspace, stream);
+    return ffn_fused(nullptr, x_tiled, out, add_residual ? x : nullptr, expert_offsets, gate0, up0, down0, gate1, up1, down1,
+                     hmid, num_rows, hidden, inter0, inter1, host_rows_per_expert, sorted_row_id, ffn_workspace, split_scratch,
+                     stream);
   if (int rc = wx_dual_swiglu_gate_up(x_tiled, hmid, expert_offsets, gate0, up0, gate1, up1, num_rows, hidden, inter0,
                                       inter1, host_rows_per_expert, stream))
     return rc;
-  if (add_residual)
-    return wx_dual_down_proj_residual(hmid, out, x, expert_offsets, down0, down1, num_rows, hidden, inter0, inter1,
-                                      host_rows_per_expert, sorted_row_id, stream);
-  return wx_dual_down_proj(hmid, out, expert_offsets, down0, down1, num_rows, hidden, inter0, inter1,
-                           host_rows_per_expert, sorted_row_id, stream);
+  return wx_dual_down_proj_split(hmid, out, add_residual ? x : nullptr, expert_offsets, down0, down1, num_rows, hidden, inter0,
+                                 inter1, host_rows_per_expert, sorted_row_id, split_scratch, stream);
+}
+
+extern "C" int wx_moe_block_forward(const void* x, void* out, const int32_t* row_id_map, const int32_t* sorted_row_id,
+                                    const int32_t* expert_offsets, const void* gate0, const void* up0,
+                                    const void* down0, const void* gate1, const void* up1, const void* down1,
+                                    void* x_tiled, void* hmid, int64_t num_rows, int64_t hidden, int64_t inter0,
+                                    int64_t inter1, const int64_t* host_rows_per_expert, const void* norm_weight,
+                                    float eps, int add_residual, void* ffn_workspace, wx_stream_t stream) {
+  return wx_moe_block_forward_split(x, out, row_id_map, sorted_row_id, expert_offsets, gate0, up0, down0, gate1, up1, down1, x_tiled,
+                                    hmid, num_rows, hidden, inter0, inter1, host_rows_per_expert, norm_weight, eps,
+                                    add_residual, ffn_workspace, nullptr, stream);
 }

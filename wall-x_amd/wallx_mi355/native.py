@@ -770,18 +770,15 @@ def dual_swiglu_ffn_packed(x_tiled: torch.Tensor, num_rows: int, expert_offsets:
     if residual is not None:
         _check_residual(residual, num_rows, H, dev, out_row_id)
     with _DeviceGuard(x_tiled):
-        if residual is not None and num_rows:
+        if num_rows:
+            stream = _stream(x_tiled)
+            split = _split_scratch(dev, stream, num_rows)
             _lib.call("wx_dual_swiglu_gate_up", x_tiled.data_ptr(), hmid.data_ptr(), expert_offsets.data_ptr(),
                       _ptr(packed[0]), _ptr(packed[1]), _ptr(packed[3]), _ptr(packed[4]), int(num_rows), H, I0, I1,
-                      _lib.i64x2(host_rows), _stream(x_tiled))
-            _lib.call("wx_dual_down_proj_residual", hmid.data_ptr(), _ptr(out), residual.data_ptr(),
-                      expert_offsets.data_ptr(), _ptr(packed[2]), _ptr(packed[5]), int(num_rows), H, I0, I1,
-                      _lib.i64x2(host_rows), _ptr(out_row_id), _stream(x_tiled))
-        else:
-            _lib.call("wx_dual_swiglu_ffn", x_tiled.data_ptr(), _ptr(out), expert_offsets.data_ptr(), _ptr(packed[0]),
-                      _ptr(packed[1]), _ptr(packed[2]), _ptr(packed[3]), _ptr(packed[4]), _ptr(packed[5]),
-                      hmid.data_ptr(), int(num_rows), H, I0, I1, _lib.i64x2(host_rows), _ptr(out_row_id),
-                      _stream(x_tiled))
+                      _lib.i64x2(host_rows), stream)
+            _lib.call("wx_dual_down_proj_split", hmid.data_ptr(), _ptr(out), _ptr(residual), expert_offsets.data_ptr(),
+                      _ptr(packed[2]), _ptr(packed[5]), int(num_rows), H, I0, I1, _lib.i64x2(host_rows), _ptr(out_row_id),
+                      _ptr(split), stream)
     return out
 
 
@@ -863,9 +860,31 @@ def _ffn_buffers(device: torch.device, stream: int, x_elems: int, h_elems: int, 
     return hit[0], hit[1], cap, hit[3]
 
 
+_split_scratches = {}  # (device index, stream handle, capturing) -> (scratch, capture id)
+
+
+def _split_scratch(device: torch.device, stream: int, num_rows: int, cap: Optional[int] = None) -> Optional[torch.Tensor]:
+    """The scratch of wx_dual_down_proj_split (16 MiB): one per device and stream, or per capture, like _ffn_buffers' and for
+    its reasons.  None for calls of so few rows that the library never cuts their contraction."""
+    if num_rows <= 512:
+        return None
+    if cap is None:
+        cap = capture_id(stream)
+    key = (device.index, stream, cap != 0)
+    hit = _split_scratches.get(key)
+    if hit is None or hit[1] != cap:
+        if len(_split_scratches) >= 64:  # streams come and go
+            _split_scratches.clear()
+        hit = (torch.empty(_lib.load().wx_ffn_split_scratch_bytes() // 4, dtype=torch.int32, device=device), cap)
+        hit[0][:1024].zero_()  # the counters in front (one per CU); the sums need no clearing
+        _split_scratches[key] = hit
+    return hit[0]
+
+
 def release_ffn_buffers() -> None:
-    """Drops the buffers _ffn_buffers keeps (they come back, sized for the next call, when needed)."""
+    """Drops the buffers _ffn_buffers and _split_scratch keep (they come back, sized for the next call, when needed)."""
     _ffn_scratch.clear()
+    _split_scratches.clear()
 
 
 class PackedExperts:
@@ -945,12 +964,13 @@ def packed_block_forward(experts: PackedExperts, x: torch.Tensor, row_id_map: to
                 not weight.is_contiguous():
             raise RuntimeError("the norm weight must be a contiguous BFloat16 tensor of the hidden size")
         norm_ptr = weight.data_ptr()
+    split = _split_scratch(dev, stream, T, cap)
     with _DeviceGuard(x):  # one library call: [RMSNorm +] permute, gate/up, down with the unpermute [and the residual]
-        _lib.check(lib.wx_moe_block_forward(x.data_ptr(), out.data_ptr(), row_id_map.data_ptr(),
-                                            sorted_row_id.data_ptr(), expert_offsets.data_ptr(), *experts.ptrs,
-                                            x_tiled.data_ptr(), hmid.data_ptr(), T, H, I0, I1, host_rows_c, norm_ptr,
-                                            float(eps), int(bool(residual)),
-                                            counters.data_ptr() if _one_launch_ffn else None, stream))
+        _lib.check(lib.wx_moe_block_forward_split(x.data_ptr(), out.data_ptr(), row_id_map.data_ptr(),
+                                                  sorted_row_id.data_ptr(), expert_offsets.data_ptr(), *experts.ptrs,
+                                                  x_tiled.data_ptr(), hmid.data_ptr(), T, H, I0, I1, host_rows_c,
+                                                  norm_ptr, float(eps), int(bool(residual)),
+                                                  counters.data_ptr() if _one_launch_ffn else None, _ptr(split), stream))
     if _checked and _one_launch_ffn and cap == 0 and int(counters[-1].item()):
         counters.zero_()
         raise RuntimeError("packed_block_forward: a wait inside the one-launch FFN ran into its bound (the result is "
@@ -980,6 +1000,17 @@ def dual_swiglu_ffn_keep(x_tiled: torch.Tensor, num_rows: int, expert_offsets: t
     out = torch.empty((num_rows, H), dtype=torch.bfloat16, device=dev)
     if num_rows == 0:
         return out, gate_keep, up_keep, hmid
+    if residual is not None:
+        _check_residual(residual, num_rows, H, dev, out_row_id)
+    with _DeviceGuard(x_tiled):
+        _lib.call("wx_dual_swiglu_gate_up_keep", x_tiled.data_ptr(), hmid.data_ptr(), gate_keep.data_ptr(),
+                  up_keep.data_ptr(), expert_offsets.data_ptr(), _ptr(packed[0]), _ptr(packed[1]), _ptr(packed[3]),
+                  _ptr(packed[4]), int(num_rows), H, I0, I1, _lib.i64x2(host_rows), _stream(x_tiled))
+        split = _split_scratch(dev, _stream(x_tiled), num_rows)
+        _lib.call("wx_dual_down_proj_split", hmid.data_ptr(), _ptr(out), _ptr(residual), expert_offsets.data_ptr(),
+                  _ptr(packed[2]), _ptr(packed[5]), int(num_rows), H, I0, I1, _lib.i64x2(host_rows), _ptr(out_row_id),
+                  _ptr(split), _stream(x_tiled))
+    return out, gate_keep, up_keep, hmid
     if residual is not None:
         _check_residual(residual, num_rows, H, dev, out_row_id)
     with _DeviceGuard(x_tiled):
