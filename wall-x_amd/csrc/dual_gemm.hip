@@ -262,24 +262,33 @@ __host__ __device__ inline long long shape_deciding_tiles(long long tiles0, long
 // ring is, so 512 .. 1024 rows of an expert of 11008 -- 64 .. 128 tiles of 344 steps -- took 87 us with half of the CUs or more
 // idle.  The tiles of the expert that decides the launch's length (both experts', unless one's contraction is at most half as
 // long as the other's) are cut into two or four parts along K while all parts have a CU of their own and 2048 of K; the part
-// that finishes last adds them up: 500 rows 87 -> 41 us, 513 .. 880 rows 87 -> 52 .. 54, 1024 rows 87 -> 61.  From half as many tiles as CUs on, two parts on every CU take what one did (1760
+// that finishes last adds them up: 500 rows 87 -> 38 us, 513 .. 880 rows 87 -> 52 .. 55, 1024 rows 87 -> 56.  From half as many tiles as CUs on, two parts on every CU take what one did (1760
 // rows: 90 us; parts of 250 tiles would be at 470 ns a step, two workgroups to a CU).
+// Where 256 x 256 tiles would be a quarter to half as many as CUs, two parts of them (`true` is the answer: large tiles) beat
+// one part of four times as many small tiles, two workgroups to a CU: 2640 + 96 rows 140 -> 115 us, 3520 + 128 159 -> 132.  The
+// other expert's tiles count there: a workgroup that takes one as a second helping costs what the parts gained (4050 + 65 rows,
+// 128 tiles and 8, alone 162 -> 160, in four layers of a prefill 17 us a layer slower).
 // Evaluated identically on the host and on the device, so that the sums' order does not depend on which of them knows the row
 // counts: not where a host that knows them takes the one launch for both GEMMs, nor up to the 2 * cus rows of which it takes
-// the one launch without knowing them.
-__host__ __device__ inline void down_parts(int m0, int m1, int k0, int k1, int hidden, int cus, int parts[2]) {
+// the one launch without knowing them, nor beyond one round of large tiles (from where on a host that does not know them
+// launches no small ones).
+__host__ __device__ inline bool down_parts(int m0, int m1, int k0, int k1, int hidden, int cus, int parts[2]) {
   parts[0] = parts[1] = 1;
   const long long rb0 = (static_cast<long long>(m0) + 127) / 128, rb1 = (static_cast<long long>(m1) + 127) / 128;
   const long long cols = (static_cast<long long>(hidden) + 127) / 128;
-  if (static_cast<long long>(m0) + m1 <= 2ll * cus) return;
-  if (rb0 * ((k0 + 63) / 64) + rb1 * ((k1 + 63) / 64) <= cus && (rb0 + rb1) * cols <= cus) return;
+  const long long large_cols = (cols + 1) / 2, large0 = (rb0 + 1) / 2 * large_cols, large1 = (rb1 + 1) / 2 * large_cols;
+  if (static_cast<long long>(m0) + m1 <= 2ll * cus || large0 + large1 > cus) return false;
+  if (rb0 * ((k0 + 63) / 64) + rb1 * ((k1 + 63) / 64) <= cus && (rb0 + rb1) * cols <= cus) return false;
   const bool cut0 = rb0 > 0 && (rb1 == 0 || 2ll * k0 > k1), cut1 = rb1 > 0 && (rb0 == 0 || 2ll * k1 > k0);
-  const long long count = ((cut0 ? rb0 : 0) + (cut1 ? rb1 : 0)) * cols;
+  const long long count = ((cut0 ? rb0 : 0) + (cut1 ? rb1 : 0)) * cols, large = (cut0 ? large0 : 0) + (cut1 ? large1 : 0);
   const int k = cut0 && cut1 ? (k0 < k1 ? k0 : k1) : (cut0 ? k0 : k1);
   int n = 1;
   while (n < 4 && count * n * 2 <= cus && k / (2 * n) >= 2048) n *= 2;
+  const bool use_large = n == 1 && 4 * large > cus && large0 + large1 + large <= cus && k / 2 >= 2048;
+  if (use_large) n = 2;
   if (cut0) parts[0] = n;
   if (cut1) parts[1] = n;
+  return use_large;
 }
 
 // Workgroup barrier without the fences of __syncthreads().  Those fences make the compiler wait for EVERY
@@ -972,17 +981,18 @@ __device__ __forceinline__ void dual_gemm_body(const Params& p, const int wg, co
   tiles_m[1] = (g1.m + BM - 1) / BM;
   tiles_n[1] = (g1.n + kTileN - 1) / kTileN;
   if (g1.m <= 0 || g1.n <= 0) tiles_m[1] = tiles_n[1] = 0;
-  if (p.gate != 0) {
-    constexpr int kBigN = SWIGLU ? BigTile::BN / 2 : BigTile::BN;
-    auto big = [](int m, int n) { return (m <= 0 || n <= 0) ? 0 : ((m + BigTile::BM - 1) / BigTile::BM) * ((n + kBigN - 1) / kBigN); };
-    const bool few = shape_deciding_tiles(big(g0.m, g0.n), big(g1.m, g1.n), g0.k, g1.k) <= p.gate_tiles;
-    if (few != (p.gate == 1)) return;  // uniform: the other tile shape's launch does this problem
-  }
   // split contraction: part q of a column tile is a column tile of its own, all columns' part 0 first
   int parts[2] = {1, 1};
   const int cols_n[2] = {tiles_n[0], tiles_n[1]};
+  bool large_parts = false;
+  if constexpr (ROLE == 3) large_parts = down_parts(g0.m, g1.m, g0.k, g1.k, g0.n, fs.split_slots, parts);
+  if (p.gate != 0) {
+    constexpr int kBigN = SWIGLU ? BigTile::BN / 2 : BigTile::BN;
+    auto big = [](int m, int n) { return (m <= 0 || n <= 0) ? 0 : ((m + BigTile::BM - 1) / BigTile::BM) * ((n + kBigN - 1) / kBigN); };
+    const bool few = !large_parts && shape_deciding_tiles(big(g0.m, g0.n), big(g1.m, g1.n), g0.k, g1.k) <= p.gate_tiles;
+    if (few != (p.gate == 1)) return;  // uniform: the other tile shape's launch does this problem
+  }
   if constexpr (ROLE == 3) {
-    down_parts(g0.m, g1.m, g0.k, g1.k, g0.n, fs.split_slots, parts);
     tiles_n[0] *= parts[0];
     tiles_n[1] *= parts[1];
   }
@@ -1003,7 +1013,7 @@ __device__ __forceinline__ void dual_gemm_body(const Params& p, const int wg, co
     const int all = big_m[0] * big_n[0] + big_m[1] * big_n[1];
     split_at = tail_split_point(big_m[0] * big_n[0], big_m[1] * big_n[1], g0.k, g1.k, p.split_cus);
     if constexpr (kIsBig) {
-      total = split_at;  // a multiple of 8 when smaller than `all`
+      if (!large_parts) total = split_at;  // a multiple of 8 when smaller than `all`
     } else {
       if (split_at == all) return;  // no split: the first launch did everything
       pieces = kSubM * kSubN * (all - split_at);
@@ -1855,25 +1865,39 @@ __device__ __forceinline__ void dual_gemm_body(const Params& p, const int wg, co
       __syncthreads();
       if (!last) return false;
       if (tid == 0) __hip_atomic_store(fs.split_count + S.slot, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      f32x4 sum[FM][FN];
-      for (int q = 0; q < S.parts; ++q) {
-        const __amdgpu_buffer_rsrc_t from = sums_of(q);
-        f32x4 v[FM][FN];
+      if constexpr (FM * FN > 16) {  // (two parts; no registers for a second set of sums)
+        const __amdgpu_buffer_rsrc_t from = sums_of(1 - S.part);
 #pragma unroll
         for (int i = 0; i < FM; ++i)
 #pragma unroll
           for (int j = 0; j < FN; ++j)
-            v[i][j] = q == S.part ? acc[i][j]
-                                  : __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(from, (i * FN + j) * 1024 + lane * 16, 0, 16 /* sc1 */));
-#pragma unroll
-        for (int i = 0; i < FM; ++i)
-#pragma unroll
-          for (int j = 0; j < FN; ++j) sum[i][j] = q == 0 ? v[i][j] : sum[i][j] + v[i][j];
+            acc[i][j] += __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(from, (i * FN + j) * 1024 + lane * 16, 0, 16 /* sc1 */));
+        return true;
       }
+      // (a row of blocks at a time: the sums of all of them at once, and the parts on their way, would take the registers that
+      // a second workgroup on the CU needs)
+#pragma unroll 1
+      for (int i = 0; i < FM; ++i) {
+        f32x4 own[FN], sum[FN];
 #pragma unroll
-      for (int i = 0; i < FM; ++i)
+        for (int j = 0; j < FN; ++j) own[j] = acc[FM - 1][j];
+        for (int q = 0; q < S.parts; ++q) {
+          const __amdgpu_buffer_rsrc_t from = sums_of(q);
 #pragma unroll
-        for (int j = 0; j < FN; ++j) acc[i][j] = sum[i][j];
+          for (int j = 0; j < FN; ++j) {
+            const f32x4 v = q == S.part ? own[j]
+                : __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(from, ((FM - 1 - i) * FN + j) * 1024 + lane * 16, 0, 16 /* sc1 */));
+            sum[j] = q == 0 ? v : sum[j] + v;
+          }
+        }
+        // the rows of blocks move up by one, the finished one to the front: after FM turns each is in its place
+#pragma unroll
+        for (int r = FM - 1; r > 0; --r)
+#pragma unroll
+          for (int j = 0; j < FN; ++j) acc[r][j] = acc[r - 1][j];
+#pragma unroll
+        for (int j = 0; j < FN; ++j) acc[0][j] = sum[j];
+      }
     }
     return true;
   };
@@ -2063,9 +2087,11 @@ __global__ __launch_bounds__(TS::kThreads, TS::kWgPerCu) void dual_gemm_kernel(P
 }
 
 // The few-rows form of the same launch (MODE: gate/up or down).
-// the down launch of small tiles with the contraction in parts
-__global__ __launch_bounds__(SmallTile::kThreads, SmallTile::kWgPerCu) void down_split_kernel(Params p, FusedSync fs) {
-  dual_gemm_body<kDown, SmallTile, false, false, 3>(p, blockIdx.x, gridDim.x, fs);
+// the down launch with the contraction in parts.  (Bounded by the wavefronts per SIMD that TS is made for: with 147
+// registers, no second workgroup on a CU, 4050 rows on unknown counts, whose tiles stay whole, took 180 us in place of 161.)
+template <typename TS>
+__global__ __launch_bounds__(TS::kThreads, TS::kWgPerCu * TS::kWaves / 4) void down_split_kernel(Params p, FusedSync fs) {
+  dual_gemm_body<kDown, TS, false, false, 3>(p, blockIdx.x, gridDim.x, fs);
 }
 
 template <int MODE, int FM, int NB>
@@ -2203,7 +2229,7 @@ int check_dims(const char* who, int64_t m, int64_t n, int64_t k, bool k_in_rows 
 // host knows, decides it on the host); when the host cannot tell, both launches are made and the device decides (the
 // second returns at once if there is nothing to split).
 // few: the few-rows form takes the problem; its number of rows, or 0.
-// split: the down launch's contraction may be in parts (down_parts) in small tiles, with this scratch.
+// split_sync: the down launch's contraction may be in parts (down_parts), with this scratch.
 template <int MODE, bool KA = false, bool KB = false>
 int launch_mfma(Params p, int64_t tiles_lo, int64_t tiles_hi, hipStream_t s, const char* who,
                 const int64_t* tiles_by_expert = nullptr, int64_t few = 0, const FusedSync* split_sync = nullptr) {
@@ -2225,13 +2251,17 @@ int launch_mfma(Params p, int64_t tiles_lo, int64_t tiles_hi, hipStream_t s, con
     // at most one round of large tiles, and one expert's tiles may not count: the device has to choose
     small = true;
   }
+  if (MODE == kDown && split_sync != nullptr) {  // parts of large tiles, if the tiles that count can be enough for them
+    const bool one_counts = 2ll * p.g[0].k <= p.g[1].k || 2ll * p.g[1].k <= p.g[0].k;
+    if (4 * (one_counts ? tiles_lo : tiles_hi) > cus && tiles_lo <= cus) big = true;
+  }
   p.gate_tiles = threshold;
   p.split = 0;
   p.split_cus = cus;
   if (small) {
     p.gate = big ? 1 : 0;
     if (MODE == kDown && split_sync != nullptr)
-      hipLaunchKernelGGL(down_split_kernel, dim3(cus * SmallTile::kWgPerCu), dim3(SmallTile::kThreads), 0, s, p, *split_sync);
+      hipLaunchKernelGGL(down_split_kernel<SmallTile>, dim3(cus * SmallTile::kWgPerCu), dim3(SmallTile::kThreads), 0, s, p, *split_sync);
     else
       hipLaunchKernelGGL((dual_gemm_kernel<MODE, SmallTile, KA, KB>), dim3(cus * SmallTile::kWgPerCu), dim3(SmallTile::kThreads), 0, s, p);
   }
@@ -2246,7 +2276,10 @@ int launch_mfma(Params p, int64_t tiles_lo, int64_t tiles_hi, hipStream_t s, con
                                                   p.g[0].k, p.g[1].k, cus) != all;
     }
     p.split = split ? 1 : 0;
-    hipLaunchKernelGGL((dual_gemm_kernel<MODE, Big, KA, KB>), dim3(cus), dim3(Big::kThreads), 0, s, p);
+    if (MODE == kDown && split_sync != nullptr)
+      hipLaunchKernelGGL(down_split_kernel<BigTile>, dim3(cus), dim3(BigTile::kThreads), 0, s, p, *split_sync);
+    else
+      hipLaunchKernelGGL((dual_gemm_kernel<MODE, Big, KA, KB>), dim3(cus), dim3(Big::kThreads), 0, s, p);
     if (split) {
       p.split = 2;
       hipLaunchKernelGGL((dual_gemm_kernel<MODE, TailTile, KA, KB>), dim3(cus * TailTile::kWgPerCu),
@@ -2561,31 +2594,39 @@ Params down_params(const FfnArgs& a) {
   return p;
 }
 
-constexpr size_t kSplitSlotBytes = static_cast<size_t>(SmallTile::BM) * SmallTile::BN * sizeof(float);
+constexpr size_t kSplitSlotBytes = static_cast<size_t>(BigTile::BM) * BigTile::BN * sizeof(float);
 // counters, a word per slot, in front of the slots
 size_t split_count_bytes() { return (static_cast<size_t>(device_cu_count()) * sizeof(int) + 1023) / 1024 * 1024; }
 
 int launch_down(const FfnArgs& a, hipStream_t s) {
   const Params p = down_params(a);
   const int64_t col_tiles = ceil_div(a.hidden, BigTile::BN);
+  const int cus = device_cu_count();
+  const bool rows_known = a.host_rows != nullptr;
   FusedSync sync{};
   const FusedSync* split = nullptr;
-  if (a.split_scratch != nullptr && a.rows > 2ll * device_cu_count() && a.rows < (1ll << 30)) {
-    int parts[2] = {0, 0};
-    if (a.host_rows != nullptr)
-      down_parts(static_cast<int>(a.host_rows[0]), static_cast<int>(a.host_rows[1]), static_cast<int>(a.inter[0]),
-                 static_cast<int>(a.inter[1]), static_cast<int>(a.hidden), device_cu_count(), parts);
-    if (parts[0] != 1 || parts[1] != 1) {  // (row counts unknown: the launch decides by the same rule)
-      sync.split_count = static_cast<int*>(a.split_scratch);
-      sync.split_sums = reinterpret_cast<float*>(static_cast<char*>(a.split_scratch) + split_count_bytes());
-      sync.split_slots = device_cu_count();
-      split = &sync;
+  // (one round of large tiles at most: down_parts; contractions of 4096 at least)
+  if (a.split_scratch != nullptr && a.rows > 2ll * cus && ceil_div(a.rows, BigTile::BM) * col_tiles <= cus &&
+      (a.inter[0] >= 4096 || a.inter[1] >= 4096)) {
+    sync.split_count = static_cast<int*>(a.split_scratch);
+    sync.split_sums = reinterpret_cast<float*>(static_cast<char*>(a.split_scratch) + split_count_bytes());
+    sync.split_slots = cus;
+    int parts[2];
+    if (rows_known) {
+      const bool large = down_parts(static_cast<int>(a.host_rows[0]), static_cast<int>(a.host_rows[1]), static_cast<int>(a.inter[0]),
+                                    static_cast<int>(a.inter[1]), static_cast<int>(a.hidden), cus, parts);
+      if (large) hipLaunchKernelGGL(down_split_kernel<BigTile>, dim3(cus), dim3(BigTile::kThreads), 0, s, p, sync);
+      else if (parts[0] > 1 || parts[1] > 1)
+        hipLaunchKernelGGL(down_split_kernel<SmallTile>, dim3(cus * SmallTile::kWgPerCu), dim3(SmallTile::kThreads), 0, s, p, sync);
+      if (parts[0] > 1 || parts[1] > 1) return check_launch("down_split_kernel");
+    } else {
+      split = &sync;  // the launches decide by the same rule
     }
   }
   if (a.host_rows != nullptr) {
     const int64_t by_expert[2] = {ceil_div(a.host_rows[0], BigTile::BM) * col_tiles, ceil_div(a.host_rows[1], BigTile::BM) * col_tiles};
     const int64_t tiles = by_expert[0] + by_expert[1];
-    return launch_mfma<kDown>(p, tiles, tiles, s, "dual_gemm_kernel<down>", by_expert, few_rows_of(a), split);
+    return launch_mfma<kDown>(p, tiles, tiles, s, "dual_gemm_kernel<down>", by_expert, few_rows_of(a));
   }
   const int64_t row_tiles = ceil_div(a.rows, BigTile::BM);
   return launch_mfma<kDown>(p, row_tiles * col_tiles, (row_tiles + 1) * col_tiles, s, "dual_gemm_kernel<down>", nullptr,
