@@ -894,12 +894,12 @@ def test_input_grads_in_shared_launches(dev, rows, inter):
     ((513, 0), (11008, 1024), 256), ((880, 32), (11008, 1024), 2048), ((1024, 1), (11008, 1024), 2048), ((1025, 0), (11008, 1024), 2048),
     ((300, 400), (8224, 96), 2048), ((40, 700), (64, 4128), 1056), ((520, 500), (4096, 4096), 512), ((512, 0), (11008, 1024), 256),
     ((2048, 1), (11008, 1024), 2048), ((2049, 70), (11008, 1024), 2048), ((3840, 65), (11008, 1024), 2048), ((3841, 65), (11008, 1024), 2048),
-    ((4097, 0), (11008, 1024), 2048), ((60, 2100), (512, 4160), 2080), ((2300, 6000), (4096, 32), 2048), ((600, 8000), (11008, 64), 2048),
+    ((3600, 496), (11008, 1024), 2048), ((3600, 497), (11008, 1024), 2048), ((60, 2100), (512, 4160), 2080), ((2300, 6000), (4096, 32), 2048), ((600, 8000), (11008, 64), 2048),
 ])
 @pytest.mark.parametrize("known", [True, False])
 def test_down_projection_with_its_contraction_in_parts(dev, rows, inter, hidden, known):
     """wx_dual_down_proj_split on both sides of each of its lines (513 rows, a quarter and half as many small or large tiles as
-    CUs, one round of large tiles of both experts, 2048 of K per part, one expert or both cut, a last part that is short) against the form without parts: no further from 64-bit results,
+    CUs, rows for half a round of large tiles, 2048 of K per part, one expert or both cut, a last part that is short) against the form without parts: no further from 64-bit results,
     the same bits on every call -- also where the library knows the row counts only on the device -- and the scratch's
     counters left at zero.  With and without the residual at the tokens' places."""
     T = sum(rows)

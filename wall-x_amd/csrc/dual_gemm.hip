@@ -261,7 +261,7 @@ __host__ __device__ inline long long shape_deciding_tiles(long long tiles0, long
 // The down launch's contraction in parts.  A 128 x 128 tile's K step takes 250 ns however many CUs work and however deep the
 // ring is, so 512 .. 1024 rows of an expert of 11008 -- 64 .. 128 tiles of 344 steps -- took 87 us with half of the CUs or more
 // idle.  The tiles of the expert that decides the launch's length (both experts', unless one's contraction is at most half as
-// long as the other's) are cut into two or four parts along K while all parts have a CU of their own and 2048 of K; the part
+// long as the other's) are cut into two or four parts (1 << lg_parts) along K while all parts have a CU of their own and 2048 of K; the part
 // that finishes last adds them up: 500 rows 87 -> 38 us, 513 .. 880 rows 87 -> 52 .. 55, 1024 rows 87 -> 56.  From half as many tiles as CUs on, two parts on every CU take what one did (1760
 // rows: 90 us; parts of 250 tiles would be at 470 ns a step, two workgroups to a CU).
 // Where 256 x 256 tiles would be a quarter to half as many as CUs, two parts of them (`true` is the answer: large tiles) beat
@@ -270,24 +270,25 @@ __host__ __device__ inline long long shape_deciding_tiles(long long tiles0, long
 // 128 tiles and 8, alone 162 -> 160, in four layers of a prefill 17 us a layer slower).
 // Evaluated identically on the host and on the device, so that the sums' order does not depend on which of them knows the row
 // counts: not where a host that knows them takes the one launch for both GEMMs, nor up to the 2 * cus rows of which it takes
-// the one launch without knowing them, nor beyond one round of large tiles (from where on a host that does not know them
-// launches no small ones).
-__host__ __device__ inline bool down_parts(int m0, int m1, int k0, int k1, int hidden, int cus, int parts[2]) {
-  parts[0] = parts[1] = 1;
+// the one launch without knowing them, nor beyond as many rows as fill half of the CUs with large tiles (where a host that does
+// not know the counts would launch these kernels, for parts that hardly ever are: 4115 rows, of 5 x 823, 4 us a layer).
+__host__ __device__ inline bool down_parts(int m0, int m1, int k0, int k1, int hidden, int cus, int lg_parts[2]) {
+  lg_parts[0] = lg_parts[1] = 0;
   const long long rb0 = (static_cast<long long>(m0) + 127) / 128, rb1 = (static_cast<long long>(m1) + 127) / 128;
   const long long cols = (static_cast<long long>(hidden) + 127) / 128;
   const long long large_cols = (cols + 1) / 2, large0 = (rb0 + 1) / 2 * large_cols, large1 = (rb1 + 1) / 2 * large_cols;
-  if (static_cast<long long>(m0) + m1 <= 2ll * cus || large0 + large1 > cus) return false;
+  const long long rows = static_cast<long long>(m0) + m1;
+  if (rows <= 2ll * cus || 2 * ((rows + 255) / 256 * large_cols) > cus) return false;
   if (rb0 * ((k0 + 63) / 64) + rb1 * ((k1 + 63) / 64) <= cus && (rb0 + rb1) * cols <= cus) return false;
   const bool cut0 = rb0 > 0 && (rb1 == 0 || 2ll * k0 > k1), cut1 = rb1 > 0 && (rb0 == 0 || 2ll * k1 > k0);
   const long long count = ((cut0 ? rb0 : 0) + (cut1 ? rb1 : 0)) * cols, large = (cut0 ? large0 : 0) + (cut1 ? large1 : 0);
   const int k = cut0 && cut1 ? (k0 < k1 ? k0 : k1) : (cut0 ? k0 : k1);
-  int n = 1;
-  while (n < 4 && count * n * 2 <= cus && k / (2 * n) >= 2048) n *= 2;
-  const bool use_large = n == 1 && 4 * large > cus && large0 + large1 + large <= cus && k / 2 >= 2048;
-  if (use_large) n = 2;
-  if (cut0) parts[0] = n;
-  if (cut1) parts[1] = n;
+  int lg = 0;
+  while (lg < 2 && count << (lg + 1) <= cus && k >> (lg + 1) >= 2048) ++lg;
+  const bool use_large = lg == 0 && 4 * large > cus && large0 + large1 + large <= cus && k / 2 >= 2048;
+  if (use_large) lg = 1;
+  if (cut0) lg_parts[0] = lg;
+  if (cut1) lg_parts[1] = lg;
   return use_large;
 }
 
@@ -982,10 +983,15 @@ __device__ __forceinline__ void dual_gemm_body(const Params& p, const int wg, co
   tiles_n[1] = (g1.n + kTileN - 1) / kTileN;
   if (g1.m <= 0 || g1.n <= 0) tiles_m[1] = tiles_n[1] = 0;
   // split contraction: part q of a column tile is a column tile of its own, all columns' part 0 first
-  int parts[2] = {1, 1};
-  const int cols_n[2] = {tiles_n[0], tiles_n[1]};
+  int lg_parts = 0;  // of expert 0, and of expert 1 four bits up: one register across the K loop
   bool large_parts = false;
-  if constexpr (ROLE == 3) large_parts = down_parts(g0.m, g1.m, g0.k, g1.k, g0.n, fs.split_slots, parts);
+  if constexpr (ROLE == 3) {
+    int lg[2];
+    large_parts = down_parts(g0.m, g1.m, g0.k, g1.k, g0.n, fs.split_slots, lg);
+    lg_parts = lg[0] | lg[1] << 4;
+  }
+  auto lg_of = [&](int group) { return lg_parts >> (4 * group) & 3; };
+  auto cols_of = [&](int group) { return ((group ? g1.n : g0.n) + kTileN - 1) / kTileN; };
   if (p.gate != 0) {
     constexpr int kBigN = SWIGLU ? BigTile::BN / 2 : BigTile::BN;
     auto big = [](int m, int n) { return (m <= 0 || n <= 0) ? 0 : ((m + BigTile::BM - 1) / BigTile::BM) * ((n + kBigN - 1) / kBigN); };
@@ -993,8 +999,8 @@ __device__ __forceinline__ void dual_gemm_body(const Params& p, const int wg, co
     if (few != (p.gate == 1)) return;  // uniform: the other tile shape's launch does this problem
   }
   if constexpr (ROLE == 3) {
-    tiles_n[0] *= parts[0];
-    tiles_n[1] *= parts[1];
+    tiles_n[0] <<= lg_of(0);
+    tiles_n[1] <<= lg_of(1);
   }
   int total = tiles_m[0] * tiles_n[0] + tiles_m[1] * tiles_n[1];  // the host bounds this below 2^31
   // tail split: the first launch (256 x 256 tiles) stops at `split_at`; the second (this shape: 128 x 128)
@@ -1094,16 +1100,16 @@ __device__ __forceinline__ void dual_gemm_body(const Params& p, const int wg, co
     int rows, cols_left, ldc, nk;
     int row0, col0;         // first row / column of the tile inside its group's output
     int row_block;          // fused launch: index of the tile's (expert, row block) counters
-    int part, parts, slot;  // split contraction: this part, how many, the slot of the tile's first part
+    int split;              // split contraction: (logarithm of the number of parts, this part, the slot of the tile's first)
   };
 
   // K steps of a tile rounded up to whole ring rounds (padding steps read zeros).  The host never launches this
   // kernel with k == 0 and a non-empty output: the tile loop below advances only from inside the K loop.
   auto padded_steps = [](int k) { return ((k + BK - 1) / BK + kStages - 1) / kStages * kStages; };
   // split contraction: the K steps of a part (whole ring rounds; the last part has what is left)
-  auto part_steps = [&](int k, int n) { return ((k / BK + n - 1) / n + kStages - 1) / kStages * kStages; };
-  auto part_k = [&](int k, int n, int part) {
-    const int left = k - part * part_steps(k, n) * BK, most = part_steps(k, n) * BK;
+  auto part_steps = [&](int k, int lg) { return (((k / BK + (1 << lg) - 1) >> lg) + kStages - 1) / kStages * kStages; };
+  auto part_k = [&](int k, int lg, int part) {
+    const int left = k - part * part_steps(k, lg) * BK, most = part_steps(k, lg) * BK;
     return left < most ? left : most;
   };
   auto setup_store = [&](const TileCoord& tc, Store& S) {
@@ -1135,10 +1141,10 @@ __device__ __forceinline__ void dual_gemm_body(const Params& p, const int wg, co
     S.ldc = G.ldc;
     S.nk = padded_steps(G.k);
     if constexpr (ROLE == 3) {
-      S.part = tc.part;
-      S.parts = tc.group ? parts[1] : parts[0];
-      S.slot = (tc.group && parts[0] > 1 ? tiles_m[0] * tiles_n[0] : 0) + (tc.tm * (tc.group ? cols_n[1] : cols_n[0]) + tc.tn) * S.parts;
-      S.nk = padded_steps(part_k(G.k, S.parts, tc.part));
+      const int lg = lg_of(tc.group);
+      const int slot = lg == 0 ? 0 : (tc.group && lg_of(0) > 0 ? tiles_m[0] * tiles_n[0] : 0) + ((tc.tm * cols_of(tc.group) + tc.tn) << lg);
+      S.split = lg | tc.part << 4 | slot << 8;
+      S.nk = padded_steps(part_k(G.k, lg, tc.part));
     }
   };
   auto setup_loader = [&](const TileCoord& tc, Loader& L) {
@@ -1147,9 +1153,9 @@ __device__ __forceinline__ void dual_gemm_body(const Params& p, const int wg, co
     L.K = G.k;
     int64_t first = 0;  // the tile's first K step
     if constexpr (ROLE == 3) {
-      const int n = tc.group ? parts[1] : parts[0];
-      L.K = part_k(G.k, n, tc.part);
-      first = static_cast<int64_t>(tc.part) * part_steps(G.k, n);
+      const int lg = lg_of(tc.group);
+      L.K = part_k(G.k, lg, tc.part);
+      first = static_cast<int64_t>(tc.part) * part_steps(G.k, lg);
     }
     L.nk = padded_steps(L.K);
     constexpr int kHalfWaves = kLoadWaves / 2;  // SwiGLU: the first half of the loading waves load gate rows, the rest up rows
@@ -1846,10 +1852,11 @@ __device__ __forceinline__ void dual_gemm_body(const Params& p, const int wg, co
   auto last_part = [&](const Store& S) {
     if constexpr (ROLE == 3) {
       constexpr uint32_t kWaveBytes = FM * FN * 1024;
+      const int parts = 1 << (S.split & 15), this_part = S.split >> 4 & 15, slot = S.split >> 8;
       auto sums_of = [&](int part) {
-        return make_rsrc(reinterpret_cast<char*>(fs.split_sums) + (static_cast<int64_t>(S.slot + part) * kWaves + wave) * kWaveBytes, kWaveBytes);
+        return make_rsrc(reinterpret_cast<char*>(fs.split_sums) + (static_cast<int64_t>(slot + part) * kWaves + wave) * kWaveBytes, kWaveBytes);
       };
-      const __amdgpu_buffer_rsrc_t mine = sums_of(S.part);
+      const __amdgpu_buffer_rsrc_t mine = sums_of(this_part);
 #pragma unroll
       for (int i = 0; i < FM; ++i)
 #pragma unroll
@@ -1859,14 +1866,14 @@ __device__ __forceinline__ void dual_gemm_body(const Params& p, const int wg, co
       __builtin_amdgcn_s_waitcnt(waitcnt_imm(0, 0));
       __syncthreads();
       volatile int* const s_before = reinterpret_cast<volatile int*>(s_out);  // (the staging area is free between tiles)
-      if (tid == 0) *s_before = __hip_atomic_fetch_add(fs.split_count + S.slot, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (tid == 0) *s_before = __hip_atomic_fetch_add(fs.split_count + slot, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       __syncthreads();
-      const bool last = __builtin_amdgcn_readfirstlane(*s_before) == S.parts - 1;
+      const bool last = __builtin_amdgcn_readfirstlane(*s_before) == parts - 1;
       __syncthreads();
       if (!last) return false;
-      if (tid == 0) __hip_atomic_store(fs.split_count + S.slot, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (tid == 0) __hip_atomic_store(fs.split_count + slot, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       if constexpr (FM * FN > 16) {  // (two parts; no registers for a second set of sums)
-        const __amdgpu_buffer_rsrc_t from = sums_of(1 - S.part);
+        const __amdgpu_buffer_rsrc_t from = sums_of(1 - this_part);
 #pragma unroll
         for (int i = 0; i < FM; ++i)
 #pragma unroll
@@ -1881,11 +1888,11 @@ __device__ __forceinline__ void dual_gemm_body(const Params& p, const int wg, co
         f32x4 own[FN], sum[FN];
 #pragma unroll
         for (int j = 0; j < FN; ++j) own[j] = acc[FM - 1][j];
-        for (int q = 0; q < S.parts; ++q) {
+        for (int q = 0; q < parts; ++q) {
           const __amdgpu_buffer_rsrc_t from = sums_of(q);
 #pragma unroll
           for (int j = 0; j < FN; ++j) {
-            const f32x4 v = q == S.part ? own[j]
+            const f32x4 v = q == this_part ? own[j]
                 : __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(from, ((FM - 1 - i) * FN + j) * 1024 + lane * 16, 0, 16 /* sc1 */));
             sum[j] = q == 0 ? v : sum[j] + v;
           }
@@ -1924,9 +1931,12 @@ __device__ __forceinline__ void dual_gemm_body(const Params& p, const int wg, co
     }
     for (; next_t < padded && !have; next_t += n_wg) have = map_tile(next_t, total, tiles_m, tiles_n, tc);
     if constexpr (ROLE == 3) {
-      const int cols = tc.group ? cols_n[1] : cols_n[0];
-      tc.part = have ? __builtin_amdgcn_readfirstlane(tc.tn / cols) : 0;
-      tc.tn -= tc.part * cols;
+      tc.part = 0;
+      const int cols = cols_of(tc.group);
+      while (have && tc.tn >= cols) {  // (four parts at most)
+        tc.tn -= cols;
+        ++tc.part;
+      }
     }
     return have;
   };
@@ -2055,7 +2065,7 @@ __device__ __forceinline__ void dual_gemm_body(const Params& p, const int wg, co
         }
       }
       if constexpr (ROLE == 3) {
-        if (done.parts == 1 || last_part(done)) epilogue(done);
+        if ((done.split & 15) == 0 || last_part(done)) epilogue(done);
       } else {
         epilogue(done);
       }
@@ -2253,7 +2263,7 @@ int launch_mfma(Params p, int64_t tiles_lo, int64_t tiles_hi, hipStream_t s, con
   }
   if (MODE == kDown && split_sync != nullptr) {  // parts of large tiles, if the tiles that count can be enough for them
     const bool one_counts = 2ll * p.g[0].k <= p.g[1].k || 2ll * p.g[1].k <= p.g[0].k;
-    if (4 * (one_counts ? tiles_lo : tiles_hi) > cus && tiles_lo <= cus) big = true;
+    if (4 * (one_counts ? tiles_lo : tiles_hi) > cus) big = true;
   }
   p.gate_tiles = threshold;
   p.split = 0;
@@ -2605,20 +2615,20 @@ int launch_down(const FfnArgs& a, hipStream_t s) {
   const bool rows_known = a.host_rows != nullptr;
   FusedSync sync{};
   const FusedSync* split = nullptr;
-  // (one round of large tiles at most: down_parts; contractions of 4096 at least)
-  if (a.split_scratch != nullptr && a.rows > 2ll * cus && ceil_div(a.rows, BigTile::BM) * col_tiles <= cus &&
+  // (half a round of large tiles at most: down_parts; contractions of 4096 at least)
+  if (a.split_scratch != nullptr && a.rows > 2ll * cus && 2 * (ceil_div(a.rows, BigTile::BM) * col_tiles) <= cus &&
       (a.inter[0] >= 4096 || a.inter[1] >= 4096)) {
     sync.split_count = static_cast<int*>(a.split_scratch);
     sync.split_sums = reinterpret_cast<float*>(static_cast<char*>(a.split_scratch) + split_count_bytes());
     sync.split_slots = cus;
-    int parts[2];
+    int lg_parts[2];
     if (rows_known) {
       const bool large = down_parts(static_cast<int>(a.host_rows[0]), static_cast<int>(a.host_rows[1]), static_cast<int>(a.inter[0]),
-                                    static_cast<int>(a.inter[1]), static_cast<int>(a.hidden), cus, parts);
+                                    static_cast<int>(a.inter[1]), static_cast<int>(a.hidden), cus, lg_parts);
       if (large) hipLaunchKernelGGL(down_split_kernel<BigTile>, dim3(cus), dim3(BigTile::kThreads), 0, s, p, sync);
-      else if (parts[0] > 1 || parts[1] > 1)
+      else if (lg_parts[0] > 0 || lg_parts[1] > 0)
         hipLaunchKernelGGL(down_split_kernel<SmallTile>, dim3(cus * SmallTile::kWgPerCu), dim3(SmallTile::kThreads), 0, s, p, sync);
-      if (parts[0] > 1 || parts[1] > 1) return check_launch("down_split_kernel");
+      if (lg_parts[0] > 0 || lg_parts[1] > 0) return check_launch("down_split_kernel");
     } else {
       split = &sync;  // the launches decide by the same rule
     }

@@ -34,8 +34,9 @@ __device__ __forceinline__ int load_key(const void* ids, int itype, int64_t i, i
 }
 
 // The keys of kAhead groups of 64 from `base` on (a lane past `end` holds 0).  They are asked for together: a wavefront that
-// loads one group at a time waits out a memory latency per group (14593 int32 keys, us: count 7.6 -> 5.6; scatter, which
-// waits for its sums over the histograms first, 9.1 either way).
+// loads one group at a time waits out a memory latency per group: partition_count of 14593 int32 keys 7.6 -> 5.6 us.  (Not in
+// the two kernels that rank: partition_scatter, which waits for its sums over the histograms first, takes 9.1 us either way, and
+// a wavefront of partition_small_kernel has a few groups only and lost 4 us on 1424 keys.)
 constexpr int kAhead = 8;
 __device__ __forceinline__ void load_keys(const void* ids, int itype, int64_t base, int64_t end, int num_experts, int (&key)[kAhead],
                                           bool& bad) {
@@ -144,26 +145,22 @@ __global__ __launch_bounds__(kBlock) void partition_scatter(
   const int64_t end = begin + seg_len < n ? begin + seg_len : n;
   const uint64_t below = (1ull << lane) - 1ull;
   bool bad = false;
-  for (int64_t base = begin; base < end; base += kAhead * kWave) {
-    int key[kAhead];
-    load_keys(ids, itype, base, end, num_experts, key, bad);
-#pragma unroll
-    for (int u = 0; u < kAhead; ++u) {
-      const int64_t i = base + u * kWave + lane;
-      const bool active = i < end;
-      int32_t pos = 0;
-      for_each_key_group(key[u], active, [&](int k, uint64_t mask) {
-        const int32_t start = s_run[w][k];  // same address for the whole wave: LDS broadcast
-        if (active && key[u] == k) pos = start + __popcll(mask & below);
-        __builtin_amdgcn_wave_barrier();
-        if (lane == 0) s_run[w][k] = start + __popcll(mask);
-        __builtin_amdgcn_wave_barrier();
-      });
-      if (active) {
-        const int64_t t = num_topk == 1 ? i : i / num_topk, k = i - t * num_topk;
-        row_id_map[k * num_tokens + t] = pos < num_out ? pos : -1;
-        if (sorted_row_id != nullptr) sorted_row_id[pos] = static_cast<int32_t>(i);
-      }
+  for (int64_t base = begin; base < end; base += kWave) {
+    const int64_t i = base + lane;
+    const bool active = i < end;
+    const int key = active ? load_key(ids, itype, i, num_experts, bad) : 0;
+    int32_t pos = 0;
+    for_each_key_group(key, active, [&](int k, uint64_t mask) {
+      const int32_t start = s_run[w][k];  // same address for the whole wave: LDS broadcast
+      if (active && key == k) pos = start + __popcll(mask & below);
+      __builtin_amdgcn_wave_barrier();
+      if (lane == 0) s_run[w][k] = start + __popcll(mask);
+      __builtin_amdgcn_wave_barrier();
+    });
+    if (active) {
+      const int64_t t = i / num_topk, k = i - t * num_topk;
+      row_id_map[k * num_tokens + t] = pos < num_out ? pos : -1;
+      if (sorted_row_id != nullptr) sorted_row_id[pos] = static_cast<int32_t>(i);
     }
   }
 }
@@ -191,15 +188,13 @@ __global__ __launch_bounds__(kSmallWaves* kWave) void partition_small_kernel(
   const int64_t end = begin + chunk < n ? begin + chunk : n;
   bool bad = false;
   __builtin_amdgcn_wave_barrier();
-  for (int64_t base = begin; base < end; base += kAhead * kWave) {
-    int key[kAhead];
-    load_keys(ids, itype, base, end, num_experts, key, bad);
-#pragma unroll
-    for (int u = 0; u < kAhead; ++u) {
-      for_each_key_group(key[u], base + u * kWave + lane < end, [&](int k, uint64_t mask) {
-        if (lane == 0) s_run[w][k] += __popcll(mask);
-      });
-    }
+  for (int64_t base = begin; base < end; base += kWave) {
+    const int64_t i = base + lane;
+    const bool active = i < end;
+    const int key = active ? load_key(ids, itype, i, num_experts, bad) : 0;
+    for_each_key_group(key, active, [&](int k, uint64_t mask) {
+      if (lane == 0) s_run[w][k] += __popcll(mask);
+    });
   }
   if (status != nullptr && __ballot(bad) != 0 && lane == 0) *status = 1;
   __syncthreads();
@@ -231,26 +226,22 @@ __global__ __launch_bounds__(kSmallWaves* kWave) void partition_small_kernel(
   }
   __syncthreads();
   const uint64_t below = (1ull << lane) - 1ull;
-  for (int64_t base = begin; base < end; base += kAhead * kWave) {
-    int key[kAhead];
-    load_keys(ids, itype, base, end, num_experts, key, bad);
-#pragma unroll
-    for (int u = 0; u < kAhead; ++u) {
-      const int64_t i = base + u * kWave + lane;
-      const bool active = i < end;
-      int32_t pos = 0;
-      for_each_key_group(key[u], active, [&](int k, uint64_t mask) {
-        const int32_t start = s_run[w][k];  // same address for the whole wave: LDS broadcast
-        if (active && key[u] == k) pos = start + __popcll(mask & below);
-        __builtin_amdgcn_wave_barrier();
-        if (lane == 0) s_run[w][k] = start + __popcll(mask);
-        __builtin_amdgcn_wave_barrier();
-      });
-      if (active) {
-        const int64_t t = num_topk == 1 ? i : i / num_topk, k = i - t * num_topk;
-        row_id_map[k * num_tokens + t] = pos < num_out ? pos : -1;
-        if (sorted_row_id != nullptr) sorted_row_id[pos] = static_cast<int32_t>(i);
-      }
+  for (int64_t base = begin; base < end; base += kWave) {
+    const int64_t i = base + lane;
+    const bool active = i < end;
+    const int key = active ? load_key(ids, itype, i, num_experts, bad) : 0;
+    int32_t pos = 0;
+    for_each_key_group(key, active, [&](int k, uint64_t mask) {
+      const int32_t start = s_run[w][k];  // same address for the whole wave: LDS broadcast
+      if (active && key == k) pos = start + __popcll(mask & below);
+      __builtin_amdgcn_wave_barrier();
+      if (lane == 0) s_run[w][k] = start + __popcll(mask);
+      __builtin_amdgcn_wave_barrier();
+    });
+    if (active) {
+      const int64_t t = i / num_topk, k = i - t * num_topk;
+      row_id_map[k * num_tokens + t] = pos < num_out ? pos : -1;
+      if (sorted_row_id != nullptr) sorted_row_id[pos] = static_cast<int32_t>(i);
     }
   }
 }

@@ -866,7 +866,7 @@ _split_scratches = {}  # (device index, stream handle, capturing) -> (scratch, c
 def _split_scratch(device: torch.device, stream: int, num_rows: int, cap: Optional[int] = None) -> Optional[torch.Tensor]:
     """The scratch of wx_dual_down_proj_split (64 MiB): one per device and stream, or per capture, like _ffn_buffers' and for
     its reasons.  None for calls of so few rows, or so many, that the library never cuts their contraction."""
-    if not 512 < num_rows <= 65536:
+    if not 512 < num_rows <= 32768:
         return None
     if cap is None:
         cap = capture_id(stream)
