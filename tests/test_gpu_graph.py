@@ -237,3 +237,57 @@ def test_row_counts_reach_the_host_without_a_sync_and_captures_ignore_them(dev):
         want, _r = moe.moe_layer_forward(x, new_types, weights)
         torch.cuda.synchronize()
         assert int((got != want).sum()) == 0 and int((got_captured != want).sum()) == 0
+
+
+def test_down_projection_in_parts_from_graphs_and_on_two_streams(dev):
+    """Blocks whose down launches cut their contraction (930 rows, an expert of 4128): the scratch belongs to a stream or to a
+    capture, so replays between eager calls, and two streams at once, give the eager bits every time, with and without the row
+    counts from the host."""
+    from types import SimpleNamespace
+
+    g = torch.Generator(device=dev).manual_seed(3)
+    hidden, inters, n_vl, T = 512, (4128, 96), 900, 930
+    config = SimpleNamespace(experts=[dict(hidden_size=hidden, intermediate_size=i, hidden_act="silu") for i in inters])
+    blocks = []
+    for _ in range(3):
+        block = moe.SparseMoeBlock(config, 2).to(torch.bfloat16).to(dev)
+        with torch.no_grad():
+            for p in block.parameters():
+                p.normal_(0.0, 0.05, generator=g)
+        blocks.append(block.pack_for_inference())
+    types = torch.zeros(1, T, dtype=torch.int64, device=dev)
+    types[0, torch.randperm(T, device=dev, generator=g)[:T - n_vl]] = 1
+    x = torch.randn(1, T, hidden, device=dev, generator=g).to(torch.bfloat16)
+    ranges = (torch.tensor([0, n_vl]), torch.tensor([n_vl, T]))
+
+    def layers(h, known=True):
+        with torch.no_grad():
+            for b in blocks:
+                h = b(h, types, *(ranges if known else (None, None)), residual=True)
+        return h
+
+    want = layers(x)
+    assert torch.equal(layers(x, known=False), want)
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    got = []
+    for s in streams:
+        s.wait_stream(torch.cuda.current_stream())
+    for _ in range(5):
+        for s in streams:
+            with torch.cuda.stream(s):
+                got.append(layers(x))
+    torch.cuda.synchronize()
+    assert all(torch.equal(v, want) for v in got)
+    for known in (True, False):
+        with torch.cuda.stream(streams[0]):
+            layers(x, known)
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            out = layers(x, known)
+        for _ in range(4):
+            out.zero_()
+            graph.replay()
+            assert torch.equal(layers(x), want)
+            torch.cuda.synchronize()
+            assert torch.equal(out, want)
