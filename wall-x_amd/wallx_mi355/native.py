@@ -835,7 +835,8 @@ def set_one_launch_ffn(flag: bool) -> bool:
 _ffn_scratch = {}  # (device index, stream handle, capturing) -> (tiled activations, intermediate, capture id, counters)
 
 
-def _ffn_buffers(device: torch.device, stream: int, x_elems: int, h_elems: int, cap: Optional[int] = None):
+def _ffn_buffers(device: torch.device, stream: int, x_elems: int, h_elems: int, cap: Optional[int] = None,
+                 num_rows: int = 0):
     """The tiled-activation and intermediate buffers of the block forward, one pair per device and stream: the
     layers of a model run one after the other on a stream, so they can all work in the same two buffers (a pair per
     block would hold 0.45 GB per layer at 29 184 tokens).  Calls that overlap on one stream's pair from two threads
@@ -852,8 +853,19 @@ def _ffn_buffers(device: torch.device, stream: int, x_elems: int, h_elems: int, 
     if hit is None or hit[0].numel() < x_elems or hit[1].numel() < h_elems:
         if hit is not None:
             x_elems, h_elems = max(x_elems, hit[0].numel()), max(h_elems, hit[1].numel())
-        counters = hit[3] if hit is not None and hit[2] == cap else \
-            torch.zeros(_lib.load().wx_ffn_fused_workspace_bytes() // 4 + 1, dtype=torch.int32, device=device)
+        if hit is not None:
+            counters = hit[3]
+        else:
+            n = _lib.load().wx_ffn_fused_workspace_bytes() // 4 + 1
+            if _may_split(num_rows) and (key not in _split_scratches or _split_scratches[key][1] != cap):
+                # with the scratch of _split_scratch behind them: one launch clears both (a graph replays it every time)
+                at = (n + 63) // 64 * 64
+                both = torch.empty(at + _lib.load().wx_ffn_split_scratch_bytes() // 4, dtype=torch.int32, device=device)
+                both[:at + 1024].zero_()
+                counters = both[:n]
+                _keep_split_scratch(key, both[at:], cap)
+            else:
+                counters = torch.zeros(n, dtype=torch.int32, device=device)
         hit = (torch.empty(x_elems, dtype=torch.bfloat16, device=device),
                torch.empty(h_elems, dtype=torch.bfloat16, device=device), cap, counters)
         _ffn_scratch[key] = hit
@@ -863,22 +875,32 @@ def _ffn_buffers(device: torch.device, stream: int, x_elems: int, h_elems: int, 
 _split_scratches = {}  # (device index, stream handle, capturing) -> (scratch, capture id)
 
 
+def _may_split(num_rows: int) -> bool:
+    """False for calls of so few rows, or so many, that the library never cuts their down launch's contraction."""
+    return 512 < num_rows <= 32768
+
+
+def _keep_split_scratch(key, scratch: torch.Tensor, cap: int) -> None:
+    if len(_split_scratches) >= 64:  # streams come and go
+        _split_scratches.clear()
+    _split_scratches[key] = (scratch, cap)
+
+
 def _split_scratch(device: torch.device, stream: int, num_rows: int, cap: Optional[int] = None) -> Optional[torch.Tensor]:
     """The scratch of wx_dual_down_proj_split (64 MiB): one per device and stream, or per capture, like _ffn_buffers' and for
-    its reasons.  None for calls of so few rows, or so many, that the library never cuts their contraction."""
-    if not 512 < num_rows <= 32768:
+    its reasons.  None where _may_split is False."""
+    if not _may_split(num_rows):
         return None
     if cap is None:
         cap = capture_id(stream)
     key = (device.index, stream, cap != 0)
     hit = _split_scratches.get(key)
-    if hit is None or hit[1] != cap:
-        if len(_split_scratches) >= 64:  # streams come and go
-            _split_scratches.clear()
-        hit = (torch.empty(_lib.load().wx_ffn_split_scratch_bytes() // 4, dtype=torch.int32, device=device), cap)
-        hit[0][:1024].zero_()  # the counters in front (one per CU); the sums need no clearing
-        _split_scratches[key] = hit
-    return hit[0]
+    if hit is not None and hit[1] == cap:
+        return hit[0]
+    scratch = torch.empty(_lib.load().wx_ffn_split_scratch_bytes() // 4, dtype=torch.int32, device=device)
+    scratch[:1024].zero_()  # the counters in front (one per CU); the sums need no clearing
+    _keep_split_scratch(key, scratch, cap)
+    return scratch
 
 
 def release_ffn_buffers() -> None:
@@ -953,7 +975,7 @@ def packed_block_forward(experts: PackedExperts, x: torch.Tensor, row_id_map: to
     if stream is None:
         stream = torch.cuda.current_stream(dev).cuda_stream
     x_elems, h_elems = experts.sizes(T)
-    x_tiled, hmid, cap, counters = _ffn_buffers(dev, stream, x_elems, h_elems, capture)
+    x_tiled, hmid, cap, counters = _ffn_buffers(dev, stream, x_elems, h_elems, capture, T)
     if host_rows_c is None and rows_when_ready is not None and cap == 0:
         host_rows_c = rows_when_ready()
     H, I0, I1 = experts.hidden, experts.inter0, experts.inter1
