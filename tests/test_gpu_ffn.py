@@ -938,3 +938,29 @@ def test_down_projection_with_its_contraction_in_parts(dev, rows, inter, hidden,
     res = n(T, hidden)
     both = run(True, res, order)
     assert torch.equal(both[order.long()], (res[order.long()].float() + got.float()).to(torch.bfloat16))
+
+
+@pytest.mark.parametrize("rows,inter,hidden", [((800, 0), (4096, 96), 256), ((600, 0), (11008, 256), 512), ((3, 1021), (64, 4096), 256),
+                                               ((513, 0), (4128, 4096), 64)])
+def test_narrow_matrices_sum_in_one_order_whatever_the_launch_form(dev, monkeypatch, rows, inter, hidden):
+    """Sizes that the few-rows form and the rule of the contraction in parts would both take (up to 1024 rows, a small hidden
+    size and one narrow expert; the last has no narrow one and is the parts'): the same bits as one launch and as two, with the
+    row counts known and unknown, and with the projections kept for a backward pass."""
+    T = sum(rows)
+    g = torch.Generator(device=dev).manual_seed(T + hidden)
+    n = lambda *s: torch.empty(s, dtype=torch.bfloat16, device=dev).normal_(0, 0.05, generator=g)
+    weights = [(n(i, hidden), n(i, hidden), n(hidden, i)) for i in inter]
+    experts = native.PackedExperts([native.pack_weight(w, cache=False) for e in weights for w in e], (hidden, *inter))
+    types = torch.arange(T, device=dev)[torch.randperm(T, device=dev, generator=g)] >= rows[0]
+    x = n(T, hidden) * 20
+    rmap, off, inv, _ = native.partition(types, 2, 0, None, want_sorted=True)
+    got = {}
+    for known in (True, False):
+        for one in (True, False):
+            monkeypatch.setattr(native, "_one_launch_ffn", one)
+            got[f"known {known}, one launch {one}"] = native.packed_block_forward(experts, x, rmap, inv, off, _lib.i64x2(rows) if known else None)
+        x_tiled = native.permute_rows_tiled(x, rmap, off, None, inv)
+        got[f"known {known}, kept"] = native.dual_swiglu_ffn_keep(x_tiled, T, off, weights, host_rows=_lib.i64x2(rows) if known else None,
+                                                                  out_row_id=inv)[0]
+    first = got["known True, one launch True"]
+    assert [form for form, y in got.items() if not torch.equal(y, first)] == []

@@ -2613,10 +2613,12 @@ int launch_down(const FfnArgs& a, hipStream_t s) {
   const int64_t col_tiles = ceil_div(a.hidden, BigTile::BN);
   const int cus = device_cu_count();
   const bool rows_known = a.host_rows != nullptr;
+  const int64_t few = few_rows_of(a);
   FusedSync sync{};
   const FusedSync* split = nullptr;
-  // (half a round of large tiles at most: down_parts; contractions of 4096 at least)
-  if (a.split_scratch != nullptr && a.rows > 2ll * cus && 2 * (ceil_div(a.rows, BigTile::BM) * col_tiles) <= cus &&
+  // (half a round of large tiles at most: down_parts; contractions of 4096 at least.  Not where the few-rows form takes the
+  // problem: narrow matrices of up to 1024 rows, which run as one launch, as two, and with the projections kept)
+  if (a.split_scratch != nullptr && few == 0 && a.rows > 2ll * cus && 2 * (ceil_div(a.rows, BigTile::BM) * col_tiles) <= cus &&
       (a.inter[0] >= 4096 || a.inter[1] >= 4096)) {
     sync.split_count = static_cast<int*>(a.split_scratch);
     sync.split_sums = reinterpret_cast<float*>(static_cast<char*>(a.split_scratch) + split_count_bytes());
@@ -2636,11 +2638,11 @@ int launch_down(const FfnArgs& a, hipStream_t s) {
   if (a.host_rows != nullptr) {
     const int64_t by_expert[2] = {ceil_div(a.host_rows[0], BigTile::BM) * col_tiles, ceil_div(a.host_rows[1], BigTile::BM) * col_tiles};
     const int64_t tiles = by_expert[0] + by_expert[1];
-    return launch_mfma<kDown>(p, tiles, tiles, s, "dual_gemm_kernel<down>", by_expert, few_rows_of(a));
+    return launch_mfma<kDown>(p, tiles, tiles, s, "dual_gemm_kernel<down>", by_expert, few);
   }
   const int64_t row_tiles = ceil_div(a.rows, BigTile::BM);
   return launch_mfma<kDown>(p, row_tiles * col_tiles, (row_tiles + 1) * col_tiles, s, "dual_gemm_kernel<down>", nullptr,
-                            few_rows_of(a), split);
+                            few, split);
 }
 
 // Both launches as one (ffn_fused_kernel), for the shapes where each is a single round of small tiles with the row
