@@ -871,10 +871,10 @@ def test_moe_block_under_bf16_autocast_takes_fp32_input(dev):
 
 
 @pytest.mark.parametrize("rows,inter", [((32768, 40), (64, 32)), ((32769, 40), (64, 32)), ((300, 0), (96, 32)), ((0, 300), (96, 32)),
-                                        ((70, 33000), (32, 64)), ((1, 1), (32, 32))])
+                                        ((70, 33000), (32, 64)), ((1, 1), (32, 32)), ((70, 33000), (64, 32)), ((33000, 70), (32, 64))])
 def test_input_grads_in_shared_launches(dev, rows, inter):
     """dX = dG Wg + dU Wu on both sides of the line between a launch per product and a launch per expert (on 256 CUs 32768
-    rows of 256 columns are its last), with either expert empty or the wider: the bits of the two products and their bf16 sum."""
+    rows of 256 columns are its last), with either expert empty or the wider, and with one expert on each side of it: the bits of the two products and their bf16 sum."""
     H = 256
     g = torch.Generator(device=dev).manual_seed(rows[0] + rows[1])
     n = lambda *s: torch.empty(s, dtype=torch.bfloat16, device=dev).normal_(0, 1, generator=g)

@@ -58,3 +58,41 @@ def test_expert_lists_other_than_two_silu_experts_select_the_generic_path():
     # the reference's parameter names (act.py:74-76, 101-103), whatever the path
     assert sorted(three.state_dict()) == sorted(f"experts.{e}.{p}_proj.weight" for e in range(3)
                                                 for p in ("gate", "up", "down"))
+
+
+@pytest.mark.parametrize("rows,inter,launches", [
+    # (rows of the launch's two problems, whether it accumulates), in order; 256 columns: 2 * ceil(rows / 256) <= 8 CUs is few
+    ((100, 20), (64, 16), [(100, 100, False), (20, 20, False)]),
+    ((1024, 1024), (64, 16), [(1024, 1024, False), (1024, 1024, False)]),
+    ((1025, 20), (64, 16), [(1025, 20, False), (1025, 20, True)]),  # many rows on the wide expert
+    ((100, 1025), (64, 16), [(100, 100, False), (0, 1025, False), (0, 1025, True)]),  # ... and on the narrow one
+    ((1025, 100), (16, 64), [(1025, 0, False), (1025, 0, True), (100, 100, False)]),
+    ((0, 1024), (64, 16), [(1024, 1024, False)]),
+    ((0, 1025), (64, 16), [(0, 1025, False), (0, 1025, True)]),  # no row on the wide expert
+    ((1025, 0), (16, 64), [(1025, 0, False), (1025, 0, True)]),
+    ((0, 0), (64, 16), [(0, 0, False), (0, 0, True)]),
+    ((100, 20), (32, 32), [(100, 20, False), (100, 20, True)]),  # neither is the wide one
+    ((100, 20), (31, 16), [(100, 20, False), (100, 20, True)]),
+    ((20, 0), (32, 32), [(20, 20, False)]),
+])
+def test_input_grads_share_launches_by_each_experts_own_tiles(monkeypatch, rows, inter, launches):
+    """Which launches dX = dG Wg + dU Wu takes, and that no split of the rows leaves a product, a row or the sum out."""
+    made = []
+
+    def dual(in0, in1, w0, w1, out0, out1, trans_a, trans_b, add_expert0=None, add_expert1=None):
+        made.append((in0.size(0), in1.size(0), add_expert0 is not None or add_expert1 is not None))
+        for a, w, out, add in ((in0, w0, out0, add_expert0), (in1, w1, out1, add_expert1)):
+            y = (a.float() @ w.float()).to(torch.bfloat16)
+            out.copy_(y if add is None else y + add)
+
+    monkeypatch.setattr(moe.native, "asym_dual_gmm", dual)
+    monkeypatch.setattr(moe, "_cus", lambda device: 8)
+    g = torch.Generator().manual_seed(sum(rows))
+    n = lambda *s: torch.randn(s, generator=g).to(torch.bfloat16)
+    dg, du = ([n(m, i) for m, i in zip(rows, inter)] for _ in range(2))
+    wg, wu = ([n(i, 256) for i in inter] for _ in range(2))
+    got = moe._input_grads(dg, du, wg, wu, 256)
+    assert made == launches
+    want = torch.cat([(a.float() @ b.float()).to(torch.bfloat16) + (c.float() @ d.float()).to(torch.bfloat16)
+                      for a, b, c, d in zip(dg, wg, du, wu)])
+    assert torch.equal(got, want)

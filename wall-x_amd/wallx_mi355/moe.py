@@ -201,25 +201,39 @@ def _input_grads(dg, du, wg, wu, H):
     their sum rounded once, what the two eager ops and their add give.
 
     As a rule a launch per product, both experts in each, the second accumulating onto the first in its epilogue.  Where
-    the wide expert's product has few 256 x 256 tiles such a launch leaves CUs idle: two products of at most as many tiles as
-    CUs between them go into one launch as its two problems, the narrow expert's into another, and an add follows.
-    Experts of 11008 and 1024 at hidden 2048, rows of each, a launch per product -> paired with the add, us: 100 + 12
-    158 -> 91, 880 + 32 165 -> 105, 1760 + 64 182 -> 174, 2640 + 96 291 -> 217, 3520 + 128 326 -> 247, 4050 + 65 345 -> 267.
-    Beyond, two rounds of large tiles take what two launches of one round do.  The same bits either way."""
-    m0, m1 = dg[0].size(0), dg[1].size(0)
+    the expert that decides how long a launch takes (the only one with rows, or the one at least twice as wide) has few
+    256 x 256 tiles, such a launch leaves CUs idle: both products of an expert with at most as many tiles as CUs between them
+    go into one launch as its two problems, and an add follows.  An expert with more tiles than that (many rows on the narrow
+    one) keeps the two accumulating launches, on its own.
+    Experts of 11008 and 1024 at hidden 2048, rows of each, a launch per product -> by expert, us: 100 + 12 158 -> 91,
+    880 + 32 167 -> 106, 1760 + 64 182 -> 174, 2640 + 96 291 -> 217, 3520 + 128 325 -> 249, 4050 + 65 355 -> 272,
+    100 + 8192 211 -> 152, 100 + 20000 315 -> 277, 880 + 16000 341 -> 252, 0 + 1000 25 -> 18.  What the rule leaves alone, as
+    a launch per product / in shared launches: 0 + 8192 71 / 75, 0 + 29184 232 / 256, two experts of 4096 with 1000 rows each
+    82 / 89, with 4096 each 202 / 212.  The same bits either way."""
+    m = m0, m1 = dg[0].size(0), dg[1].size(0)
     dev = dg[0].device
     out = torch.empty(m0 + m1, H, dtype=torch.bfloat16, device=dev)
-    o0, o1 = out[:m0], out[m0:]
-    wide = 0 if wg[0].size(0) >= wg[1].size(0) else 1
-    if 2 * -(-dg[wide].size(0) // 256) * -(-H // 256) > _cus(dev):
-        native.asym_dual_gmm(dg[0], dg[1], wg[0], wg[1], o0, o1, False, False)
-        native.asym_dual_gmm(du[0], du[1], wu[0], wu[1], o0, o1, False, False, add_expert0=o0, add_expert1=o1)
+    outs = out[:m0], out[m0:]
+    w0, w1 = wg[0].size(0), wg[1].size(0)
+    cus, cols = _cus(dev), -(-H // 256)
+    few = 0 < 2 * -(-m0 // 256) * cols <= cus, 0 < 2 * -(-m1 // 256) * cols <= cus
+    if not (few[0] and (m1 == 0 or w0 >= 2 * w1) or few[1] and (m0 == 0 or w1 >= 2 * w0)):
+        native.asym_dual_gmm(dg[0], dg[1], wg[0], wg[1], outs[0], outs[1], False, False)
+        native.asym_dual_gmm(du[0], du[1], wu[0], wu[1], outs[0], outs[1], False, False, add_expert0=outs[0], add_expert1=outs[1])
         return out
-    second = torch.empty_like(out)
-    for e, rows in enumerate((slice(0, m0), slice(m0, m0 + m1))):
-        if dg[e].size(0):
-            native.asym_dual_gmm(dg[e], du[e], wg[e], wu[e], out[rows], second[rows], False, False)
-    return out.add_(second)
+    shared = out[0 if few[0] else m0:m0 + m1 if few[1] else m0]  # the rows whose products share a launch
+    second = torch.empty_like(shared)
+    for e in (0, 1):
+        if few[e]:
+            native.asym_dual_gmm(dg[e], du[e], wg[e], wu[e], outs[e], second[m0 if e and few[0] else 0:][:m[e]], False, False)
+        elif m[e]:
+            for d, w, add in ((dg, wg, None), (du, wu, outs[e])):
+                own = d[e], w[e], outs[e], add
+                none = d[1 - e][:0], w[1 - e], outs[1 - e][:0], None  # the other expert without rows
+                (a0, b0, o0, add0), (a1, b1, o1, add1) = (none, own) if e else (own, none)
+                native.asym_dual_gmm(a0, a1, b0, b1, o0, o1, False, False, add_expert0=add0, add_expert1=add1)
+    shared.add_(second)
+    return out
 
 
 class _MoeBlockFunction(torch.autograd.Function):
