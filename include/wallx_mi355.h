@@ -240,6 +240,8 @@ int wx_dual_down_proj_residual(const void* hmid, void* out, const void* residual
  * aligned, zeroed ONCE by the caller before the first use; each launch leaves it ready for the next one on its stream.  One per
  * stream. */
 size_t wx_ffn_split_scratch_bytes(void);
+/* 1 if wx_dual_down_proj_split of these sizes uses its scratch for some split of the rows, 0 if it never does. */
+int wx_ffn_may_split(int64_t num_rows, int64_t hidden, int64_t inter0, int64_t inter1);
 int wx_dual_down_proj_split(const void* hmid, void* out, const void* residual, const int32_t* expert_offsets,
                             const void* down0, const void* down1, int64_t num_rows, int64_t hidden,
                             int64_t inter0, int64_t inter1, const int64_t* host_rows_per_expert,

@@ -185,3 +185,15 @@ def test_grid_totals_are_those_of_the_rows(dtype, merge, window):
     assert lib.wx_grid_totals(None, 7, 0, 1, 1, (ctypes.c_int64 * 3)()) == -1
     assert lib.wx_grid_totals(None, _lib.WX_I64, 1, 1, 1, (ctypes.c_int64 * 3)()) == -1
     assert lib.wx_grid_totals(None, _lib.WX_I64, 0, 0, 1, (ctypes.c_int64 * 3)()) == -1
+
+
+@pytest.mark.parametrize("sizes,want", [
+    ((512, 2048, 11008, 1024), 0), ((513, 2048, 11008, 1024), 1), ((4096, 2048, 11008, 1024), 1), ((4097, 2048, 11008, 1024), 0),
+    ((29184, 2048, 11008, 1024), 0), ((930, 2048, 4095, 1024), 0), ((930, 2048, 1024, 4096), 1), ((32768, 256, 11008, 64), 1),
+    ((32769, 256, 11008, 64), 0), ((800, 256, 4096, 96), 0), ((800, 256, 4096, 1024), 1), ((0, 2048, 11008, 1024), 0),
+])
+def test_sizes_that_use_the_split_scratch(sizes, want):
+    """On 256 CUs (what the library takes for granted without a GPU): more than 512 rows, at most 128 tiles of 256 x 256, a
+    contraction of 4096, and not what the few-rows form takes."""
+    from wallx_mi355 import _lib, native
+    assert _lib.load().wx_ffn_may_split(*sizes) == want and native._may_split(*sizes) is bool(want)

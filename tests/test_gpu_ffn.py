@@ -964,3 +964,23 @@ def test_narrow_matrices_sum_in_one_order_whatever_the_launch_form(dev, monkeypa
                                                                   out_row_id=inv)[0]
     first = got["known True, one launch True"]
     assert [form for form, y in got.items() if not torch.equal(y, first)] == []
+
+
+@pytest.mark.parametrize("rows,hidden,inter,held", [((4000, 97), 2048, (4096, 64), 0), ((900, 30), 512, (4064, 608), 0),
+                                                    ((900, 30), 512, (4096, 608), 1), ((800, 0), 256, (4096, 96), 0)])
+def test_split_scratch_is_held_for_the_sizes_that_use_it(dev, rows, hidden, inter, held):
+    """Neither an inference forward nor a training one leaves 64 MiB behind for a down launch that is never cut."""
+    T = sum(rows)
+    g = torch.Generator(device=dev).manual_seed(T)
+    n = lambda *s: torch.empty(s, dtype=torch.bfloat16, device=dev).normal_(0, 0.05, generator=g)
+    weights = [(n(i, hidden), n(i, hidden), n(hidden, i)) for i in inter]
+    experts = native.PackedExperts([native.pack_weight(w, cache=False) for e in weights for w in e], (hidden, *inter))
+    x, types = n(T, hidden), torch.arange(T, device=dev) >= rows[0]
+    rmap, off, inv, _ = native.partition(types, 2, 0, None, want_sorted=True)
+    native.release_ffn_buffers()
+    for known in (None, _lib.i64x2(rows)):
+        native.packed_block_forward(experts, x, rmap, inv, off, known)
+        assert len(native._split_scratches) == held
+    native.release_ffn_buffers()
+    native.dual_swiglu_ffn_keep(native.permute_rows_tiled(x, rmap, off, None, inv), T, off, weights, out_row_id=inv)
+    assert len(native._split_scratches) == held

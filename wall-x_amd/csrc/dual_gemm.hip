@@ -2608,18 +2608,23 @@ constexpr size_t kSplitSlotBytes = static_cast<size_t>(BigTile::BM) * BigTile::B
 // counters, a word per slot, in front of the slots
 size_t split_count_bytes() { return (static_cast<size_t>(device_cu_count()) * sizeof(int) + 1023) / 1024 * 1024; }
 
+// Whether the down launch's contraction is cut for some split of the rows (down_parts: more than 2 * cus rows, half a round of
+// large tiles at most, contractions of 4096 at least).  Not where the few-rows form takes the problem: narrow matrices of up
+// to 1024 rows, which run as one launch, as two, and with the projections kept.
+bool may_split(const FfnArgs& a) {
+  const int cus = device_cu_count();
+  return a.rows > 2ll * cus && 2 * (ceil_div(a.rows, BigTile::BM) * ceil_div(a.hidden, BigTile::BN)) <= cus &&
+         (a.inter[0] >= 4096 || a.inter[1] >= 4096) && few_rows_of(a) == 0;
+}
+
 int launch_down(const FfnArgs& a, hipStream_t s) {
   const Params p = down_params(a);
   const int64_t col_tiles = ceil_div(a.hidden, BigTile::BN);
   const int cus = device_cu_count();
   const bool rows_known = a.host_rows != nullptr;
-  const int64_t few = few_rows_of(a);
   FusedSync sync{};
   const FusedSync* split = nullptr;
-  // (half a round of large tiles at most: down_parts; contractions of 4096 at least.  Not where the few-rows form takes the
-  // problem: narrow matrices of up to 1024 rows, which run as one launch, as two, and with the projections kept)
-  if (a.split_scratch != nullptr && few == 0 && a.rows > 2ll * cus && 2 * (ceil_div(a.rows, BigTile::BM) * col_tiles) <= cus &&
-      (a.inter[0] >= 4096 || a.inter[1] >= 4096)) {
+  if (a.split_scratch != nullptr && may_split(a)) {
     sync.split_count = static_cast<int*>(a.split_scratch);
     sync.split_sums = reinterpret_cast<float*>(static_cast<char*>(a.split_scratch) + split_count_bytes());
     sync.split_slots = cus;
@@ -2638,11 +2643,11 @@ int launch_down(const FfnArgs& a, hipStream_t s) {
   if (a.host_rows != nullptr) {
     const int64_t by_expert[2] = {ceil_div(a.host_rows[0], BigTile::BM) * col_tiles, ceil_div(a.host_rows[1], BigTile::BM) * col_tiles};
     const int64_t tiles = by_expert[0] + by_expert[1];
-    return launch_mfma<kDown>(p, tiles, tiles, s, "dual_gemm_kernel<down>", by_expert, few);
+    return launch_mfma<kDown>(p, tiles, tiles, s, "dual_gemm_kernel<down>", by_expert, few_rows_of(a));
   }
   const int64_t row_tiles = ceil_div(a.rows, BigTile::BM);
   return launch_mfma<kDown>(p, row_tiles * col_tiles, (row_tiles + 1) * col_tiles, s, "dual_gemm_kernel<down>", nullptr,
-                            few, split);
+                            few_rows_of(a), split);
 }
 
 // Both launches as one (ffn_fused_kernel), for the shapes where each is a single round of small tiles with the row
@@ -2816,6 +2821,15 @@ int launch_norm_ffn_few_rows(const void* x, const void* x_tiled, void* out, cons
 }  // namespace wx
 
 extern "C" size_t wx_ffn_fused_workspace_bytes(void) { return kFusedWorkspaceInts * sizeof(int); }
+
+extern "C" int wx_ffn_may_split(int64_t num_rows, int64_t hidden, int64_t inter0, int64_t inter1) {
+  FfnArgs a{};
+  a.rows = num_rows;
+  a.hidden = hidden;
+  a.inter[0] = inter0;
+  a.inter[1] = inter1;
+  return may_split(a) ? 1 : 0;
+}
 
 extern "C" size_t wx_ffn_split_scratch_bytes(void) { return split_count_bytes() + device_cu_count() * kSplitSlotBytes; }
 

@@ -71,6 +71,7 @@ PROTOTYPES = {
     "wx_rmsnorm_bwd_workspace_bytes": (_sz, [_i64]),
     "wx_unpermute_rows_rmsnorm_bwd": (_i32, [_vp, _vp, _vp, _f32, _vp, _vp, _vp, _vp, _i64, _i64, _vp, _sz, _vp]),
     "wx_ffn_split_scratch_bytes": (_sz, []),
+    "wx_ffn_may_split": (_i32, [_i64] * 4),
     "wx_dual_down_proj_split": (_i32, [_vp] * 6 + [_i64] * 4 + [_vp] * 4),
     "wx_moe_block_forward_split": (_i32, [_vp] * 13 + [_i64] * 4 + [_vp, _vp, _f32, _i32, _vp, _vp, _vp]),
     "wx_moe_block_forward": (_i32, [_vp] * 13 + [_i64] * 4 + [_vp, _vp, _f32, _i32, _vp, _vp]),

@@ -6,6 +6,7 @@ Nothing here falls back to PyTorch math: without the library, or with CPU tensor
 """
 
 import ctypes
+import functools
 import os
 import warnings
 from typing import List, Optional, Tuple
@@ -772,7 +773,7 @@ def dual_swiglu_ffn_packed(x_tiled: torch.Tensor, num_rows: int, expert_offsets:
     with _DeviceGuard(x_tiled):
         if num_rows:
             stream = _stream(x_tiled)
-            split = _split_scratch(dev, stream, num_rows)
+            split = _split_scratch(dev, stream, (int(num_rows), H, I0, I1))
             _lib.call("wx_dual_swiglu_gate_up", x_tiled.data_ptr(), hmid.data_ptr(), expert_offsets.data_ptr(),
                       _ptr(packed[0]), _ptr(packed[1]), _ptr(packed[3]), _ptr(packed[4]), int(num_rows), H, I0, I1,
                       _lib.i64x2(host_rows), stream)
@@ -836,14 +837,15 @@ _ffn_scratch = {}  # (device index, stream handle, capturing) -> (tiled activati
 
 
 def _ffn_buffers(device: torch.device, stream: int, x_elems: int, h_elems: int, cap: Optional[int] = None,
-                 num_rows: int = 0):
+                 sizes=None):
     """The tiled-activation and intermediate buffers of the block forward, one pair per device and stream: the
     layers of a model run one after the other on a stream, so they can all work in the same two buffers (a pair per
     block would hold 0.45 GB per layer at 29 184 tokens).  Calls that overlap on one stream's pair from two threads
     race, like any two launches writing one buffer.  Under HIP graph capture the pair belongs to that capture (its
     memory comes from the graph's pool and its replays write it): eager calls never share it, and a later capture on
     the same stream replaces it.  With them comes the zeroed counter workspace of the one-launch FFN
-    (wx_dual_swiglu_ffn_fused), which every launch leaves zero again."""
+    (wx_dual_swiglu_ffn_fused), which every launch leaves zero again.  sizes: those of _split_scratch, for callers that ask
+    for it next."""
     if cap is None:
         cap = capture_id(stream)
     key = (device.index, stream, cap != 0)
@@ -857,7 +859,7 @@ def _ffn_buffers(device: torch.device, stream: int, x_elems: int, h_elems: int, 
             counters = hit[3]
         else:
             n = _lib.load().wx_ffn_fused_workspace_bytes() // 4 + 1
-            if _may_split(num_rows) and (key not in _split_scratches or _split_scratches[key][1] != cap):
+            if sizes is not None and _may_split(*sizes) and (key not in _split_scratches or _split_scratches[key][1] != cap):
                 # with the scratch of _split_scratch behind them: one launch clears both (a graph replays it every time)
                 at = (n + 63) // 64 * 64
                 both = torch.empty(at + _lib.load().wx_ffn_split_scratch_bytes() // 4, dtype=torch.int32, device=device)
@@ -875,9 +877,10 @@ def _ffn_buffers(device: torch.device, stream: int, x_elems: int, h_elems: int, 
 _split_scratches = {}  # (device index, stream handle, capturing) -> (scratch, capture id)
 
 
-def _may_split(num_rows: int) -> bool:
-    """False for calls of so few rows, or so many, that the library never cuts their down launch's contraction."""
-    return 512 < num_rows <= 32768
+@functools.lru_cache(maxsize=256)
+def _may_split(num_rows: int, hidden: int, inter0: int, inter1: int) -> bool:
+    """False for sizes whose down launch's contraction the library never cuts, whatever the split of the rows."""
+    return _lib.load().wx_ffn_may_split(num_rows, hidden, inter0, inter1) != 0
 
 
 def _keep_split_scratch(key, scratch: torch.Tensor, cap: int) -> None:
@@ -886,10 +889,10 @@ def _keep_split_scratch(key, scratch: torch.Tensor, cap: int) -> None:
     _split_scratches[key] = (scratch, cap)
 
 
-def _split_scratch(device: torch.device, stream: int, num_rows: int, cap: Optional[int] = None) -> Optional[torch.Tensor]:
+def _split_scratch(device: torch.device, stream: int, sizes, cap: Optional[int] = None) -> Optional[torch.Tensor]:
     """The scratch of wx_dual_down_proj_split (64 MiB): one per device and stream, or per capture, like _ffn_buffers' and for
-    its reasons.  None where _may_split is False."""
-    if not _may_split(num_rows):
+    its reasons.  None where _may_split(*sizes) is False: sizes = (rows, hidden, inter0, inter1)."""
+    if not _may_split(*sizes):
         return None
     if cap is None:
         cap = capture_id(stream)
@@ -974,11 +977,11 @@ def packed_block_forward(experts: PackedExperts, x: torch.Tensor, row_id_map: to
     lib = _lib.load()
     if stream is None:
         stream = torch.cuda.current_stream(dev).cuda_stream
+    H, I0, I1 = experts.hidden, experts.inter0, experts.inter1
     x_elems, h_elems = experts.sizes(T)
-    x_tiled, hmid, cap, counters = _ffn_buffers(dev, stream, x_elems, h_elems, capture, T)
+    x_tiled, hmid, cap, counters = _ffn_buffers(dev, stream, x_elems, h_elems, capture, (T, H, I0, I1))
     if host_rows_c is None and rows_when_ready is not None and cap == 0:
         host_rows_c = rows_when_ready()
-    H, I0, I1 = experts.hidden, experts.inter0, experts.inter1
     norm_ptr, eps = None, 0.0
     if pre_norm is not None:
         weight, eps = pre_norm
@@ -986,7 +989,7 @@ def packed_block_forward(experts: PackedExperts, x: torch.Tensor, row_id_map: to
                 not weight.is_contiguous():
             raise RuntimeError("the norm weight must be a contiguous BFloat16 tensor of the hidden size")
         norm_ptr = weight.data_ptr()
-    split = _split_scratch(dev, stream, T, cap)
+    split = _split_scratch(dev, stream, (T, H, I0, I1), cap)
     with _DeviceGuard(x):  # one library call: [RMSNorm +] permute, gate/up, down with the unpermute [and the residual]
         _lib.check(lib.wx_moe_block_forward_split(x.data_ptr(), out.data_ptr(), row_id_map.data_ptr(),
                                                   sorted_row_id.data_ptr(), expert_offsets.data_ptr(), *experts.ptrs,
@@ -1028,7 +1031,7 @@ def dual_swiglu_ffn_keep(x_tiled: torch.Tensor, num_rows: int, expert_offsets: t
         _lib.call("wx_dual_swiglu_gate_up_keep", x_tiled.data_ptr(), hmid.data_ptr(), gate_keep.data_ptr(),
                   up_keep.data_ptr(), expert_offsets.data_ptr(), _ptr(packed[0]), _ptr(packed[1]), _ptr(packed[3]),
                   _ptr(packed[4]), int(num_rows), H, I0, I1, _lib.i64x2(host_rows), _stream(x_tiled))
-        split = _split_scratch(dev, _stream(x_tiled), num_rows)
+        split = _split_scratch(dev, _stream(x_tiled), (int(num_rows), H, I0, I1))
         _lib.call("wx_dual_down_proj_split", hmid.data_ptr(), _ptr(out), _ptr(residual), expert_offsets.data_ptr(),
                   _ptr(packed[2]), _ptr(packed[5]), int(num_rows), H, I0, I1, _lib.i64x2(host_rows), _ptr(out_row_id),
                   _ptr(split), _stream(x_tiled))
