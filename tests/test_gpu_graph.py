@@ -240,13 +240,13 @@ def test_row_counts_reach_the_host_without_a_sync_and_captures_ignore_them(dev):
 
 
 def test_down_projection_in_parts_from_graphs_and_on_two_streams(dev):
-    """Blocks whose down launches cut their contraction (930 rows, an expert of 4128): the scratch belongs to a stream or to a
-    capture, so replays between eager calls, and two streams at once, give the eager bits every time, with and without the row
-    counts from the host."""
+    """Blocks whose down launches cut their contraction (930 rows, an expert of 4128 and one too wide for the few-rows form): the
+    scratch belongs to a stream or to a capture, so replays between eager calls, and two streams at once, give the eager bits
+    every time, with and without the row counts from the host."""
     from types import SimpleNamespace
 
     g = torch.Generator(device=dev).manual_seed(3)
-    hidden, inters, n_vl, T = 512, (4128, 96), 900, 930
+    hidden, inters, n_vl, T = 512, (4128, 608), 900, 930
     config = SimpleNamespace(experts=[dict(hidden_size=hidden, intermediate_size=i, hidden_act="silu") for i in inters])
     blocks = []
     for _ in range(3):
@@ -266,7 +266,10 @@ def test_down_projection_in_parts_from_graphs_and_on_two_streams(dev):
                 h = b(h, types, *(ranges if known else (None, None)), residual=True)
         return h
 
+    native.release_ffn_buffers()
     want = layers(x)
+    (scratch, _cap), = native._split_scratches.values()
+    assert scratch[1024:].any() and not scratch[:256].any()  # sums have been left there, and their counters are zero again
     assert torch.equal(layers(x, known=False), want)
     streams = [torch.cuda.Stream() for _ in range(2)]
     got = []
