@@ -1036,21 +1036,6 @@ def dual_swiglu_ffn_keep(x_tiled: torch.Tensor, num_rows: int, expert_offsets: t
                   _ptr(packed[2]), _ptr(packed[5]), int(num_rows), H, I0, I1, _lib.i64x2(host_rows), _ptr(out_row_id),
                   _ptr(split), _stream(x_tiled))
     return out, gate_keep, up_keep, hmid
-    if residual is not None:
-        _check_residual(residual, num_rows, H, dev, out_row_id)
-    with _DeviceGuard(x_tiled):
-        _lib.call("wx_dual_swiglu_gate_up_keep", x_tiled.data_ptr(), hmid.data_ptr(), gate_keep.data_ptr(),
-                  up_keep.data_ptr(), expert_offsets.data_ptr(), _ptr(packed[0]), _ptr(packed[1]), _ptr(packed[3]),
-                  _ptr(packed[4]), int(num_rows), H, I0, I1, _lib.i64x2(host_rows), _stream(x_tiled))
-        if residual is not None:
-            _lib.call("wx_dual_down_proj_residual", hmid.data_ptr(), _ptr(out), residual.data_ptr(),
-                      expert_offsets.data_ptr(), _ptr(packed[2]), _ptr(packed[5]), int(num_rows), H, I0, I1,
-                      _lib.i64x2(host_rows), _ptr(out_row_id), _stream(x_tiled))
-        else:
-            _lib.call("wx_dual_down_proj", hmid.data_ptr(), _ptr(out), expert_offsets.data_ptr(), _ptr(packed[2]),
-                      _ptr(packed[5]), int(num_rows), H, I0, I1, _lib.i64x2(host_rows), _ptr(out_row_id),
-                      _stream(x_tiled))
-    return out, gate_keep, up_keep, hmid
 
 
 def swiglu_bwd_tiled(gate_keep: torch.Tensor, up_keep: torch.Tensor, elem_offset: int, tiled_rows: int,
