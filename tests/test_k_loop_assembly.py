@@ -67,7 +67,7 @@ def loops(tmp_path_factory):
 
 def test_the_k_loops_are_found(loops):
     names = {k for k, _ in loops}
-    for part in ("dual_gemm_kernel", "dual_gemm_few_rows_kernel", "ffn_fused_kernel", "ffn_few_rows_norm_kernel"):
+    for part in ("dual_gemm_kernel", "down_split_kernel", "dual_gemm_few_rows_kernel", "ffn_fused_kernel", "ffn_few_rows_norm_kernel"):
         assert any(part in n for n in names), part
     assert sum(any("lds" in x for x in body) for _, body in loops) >= 18  # loops that fill a ring
 
@@ -82,7 +82,7 @@ def test_no_k_loop_spills(loops):
     assert not bad, bad
 
 
-@pytest.mark.parametrize("kernel", ["dual_gemm_kernel", "dual_gemm_few_rows_kernel", "ffn_few_rows_norm_kernel", "ffn_fused_kernel"])
+@pytest.mark.parametrize("kernel", ["dual_gemm_kernel", "down_split_kernel", "dual_gemm_few_rows_kernel", "ffn_few_rows_norm_kernel", "ffn_fused_kernel"])
 def test_the_build_warns_of_a_spill_in_any_gemm_kernel(kernel, capsys):
     remark = "f.hip:1:1: remark: Function Name: _ZN2wx{}E [-Rpass]\nf.hip:1:1: remark:     ScratchSize [bytes/lane]: {} [-Rpass]\n"
     csrc_build._check_resources("dual_gemm.hip", remark.format(kernel, 96))

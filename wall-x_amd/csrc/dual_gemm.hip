@@ -175,7 +175,7 @@ constexpr int waitcnt_imm(int vm, int lgkm) { return (vm & 15) | ((vm >> 4) << 1
 
 struct TileCoord {
   int group, tm, tn;
-  int part;  // split contraction: which part of it (down_parts)
+  int part;  // split contraction: which part of it (PartsRule)
 };
 
 // Linear tile id -> coordinates.  Ids are first spread so that each XCD (workgroup id mod 8) walks its own
@@ -259,38 +259,59 @@ __host__ __device__ inline long long shape_deciding_tiles(long long tiles0, long
 }
 
 // The down launch's contraction in parts.  A 128 x 128 tile's K step takes 250 ns however many CUs work and however deep the
-// ring is, so 512 .. 1024 rows of an expert of 11008 -- 64 .. 128 tiles of 344 steps -- took 87 us with half of the CUs or more
+// ring is, so 513 .. 1024 rows of an expert of 11008 -- 80 .. 128 tiles of 344 steps -- took 87 us with half of the CUs or more
 // idle.  The tiles of the expert that decides the launch's length (both experts', unless one's contraction is at most half as
-// long as the other's) are cut into two or four parts (1 << lg_parts) along K while all parts have a CU of their own and 2048 of K; the part
-// that finishes last adds them up: 500 rows 87 -> 38 us, 513 .. 880 rows 87 -> 52 .. 55, 1024 rows 87 -> 56.  From half as many tiles as CUs on, two parts on every CU take what one did (1760
-// rows: 90 us; parts of 250 tiles would be at 470 ns a step, two workgroups to a CU).
-// Where 256 x 256 tiles would be a quarter to half as many as CUs, two parts of them (`true` is the answer: large tiles) beat
-// one part of four times as many small tiles, two workgroups to a CU: 2640 + 96 rows 140 -> 115 us, 3520 + 128 159 -> 132.  The
-// other expert's tiles count there: a workgroup that takes one as a second helping costs what the parts gained (4050 + 65 rows,
-// 128 tiles and 8, alone 162 -> 160, in four layers of a prefill 17 us a layer slower).
-// Evaluated identically on the host and on the device, so that the sums' order does not depend on which of them knows the row
-// counts: not where a host that knows them takes the one launch for both GEMMs, nor up to the 2 * cus rows of which it takes
-// the one launch without knowing them, nor beyond as many rows as fill half of the CUs with large tiles (where a host that does
-// not know the counts would launch these kernels, for parts that hardly ever are: 4115 rows, of 5 x 823, 4 us a layer).
-__host__ __device__ inline bool down_parts(int m0, int m1, int k0, int k1, int hidden, int cus, int lg_parts[2]) {
-  lg_parts[0] = lg_parts[1] = 0;
-  const long long rb0 = (static_cast<long long>(m0) + 127) / 128, rb1 = (static_cast<long long>(m1) + 127) / 128;
-  const long long cols = (static_cast<long long>(hidden) + 127) / 128;
-  const long long large_cols = (cols + 1) / 2, large0 = (rb0 + 1) / 2 * large_cols, large1 = (rb1 + 1) / 2 * large_cols;
-  const long long rows = static_cast<long long>(m0) + m1;
-  if (rows <= 2ll * cus || 2 * ((rows + 255) / 256 * large_cols) > cus) return false;
-  if (rb0 * ((k0 + 63) / 64) + rb1 * ((k1 + 63) / 64) <= cus && (rb0 + rb1) * cols <= cus) return false;
-  const bool cut0 = rb0 > 0 && (rb1 == 0 || 2ll * k0 > k1), cut1 = rb1 > 0 && (rb0 == 0 || 2ll * k1 > k0);
-  const long long count = ((cut0 ? rb0 : 0) + (cut1 ? rb1 : 0)) * cols, large = (cut0 ? large0 : 0) + (cut1 ? large1 : 0);
-  const int k = cut0 && cut1 ? (k0 < k1 ? k0 : k1) : (cut0 ? k0 : k1);
-  int lg = 0;
-  while (lg < 2 && count << (lg + 1) <= cus && k >> (lg + 1) >= 2048) ++lg;
-  const bool use_large = lg == 0 && 4 * large > cus && large0 + large1 + large <= cus && k / 2 >= 2048;
-  if (use_large) lg = 1;
-  if (cut0) lg_parts[0] = lg;
-  if (cut1) lg_parts[1] = lg;
-  return use_large;
-}
+// long as the other's) are cut into two or four parts (1 << lg) along K while all parts have a CU of their own and 2048 of K;
+// the part that finishes last adds them up: at hidden 2048 (two parts) 513 .. 880 rows 87 -> 52 .. 55 us, 1024 rows 87 -> 56,
+// 100 rows of the expert of 11008 beside 900 of one of 1024 (four) 92 -> 35.  From half as many tiles as CUs on, two parts on
+// every CU take what one did (1760 rows: 90 us; parts of 250 tiles would be at 470 ns a step, two workgroups to a CU).
+// Where 256 x 256 tiles would be a quarter to half as many as CUs, two parts of them beat one part of four times as many small
+// tiles, two workgroups to a CU: 2640 + 96 rows 140 -> 115 us, 3520 + 128 159 -> 132.  The other expert's tiles count there: a
+// workgroup that takes one as a second helping costs what the parts gained (4050 + 65 rows, 128 tiles and 8, alone 162 -> 160,
+// in four layers of a prefill 17 us a layer slower).
+// Asked with the same numbers on the host and on the device, so that the sums' order does not depend on which of them knows the
+// row counts, of sizes that may_split lets through (more rows than the one launch for both GEMMs takes without knowing the
+// counts, and no more than fill half of the CUs with large tiles: where a host that does not know the counts would make these
+// launches for parts that hardly ever are, 4115 rows, of 5 x 823, 4 us a layer); not where the one launch takes the rows
+// with their counts known.  Every workgroup of a launch on unknown counts asks first, so what depends on the sizes alone is
+// worked out on the host, and the rest is 32-bit.
+struct DownParts {
+  int lg;      // 1 << lg parts
+  bool large;  // of 256 x 256 tiles
+  bool cut[2]; // expert e's tiles are cut
+};
+struct PartsRule {
+  int cus, cols;      // CUs; column tiles of 128
+  int steps[2];       // column tiles of the gate/up launch, expert e
+  int beside[2];      // expert e is cut beside rows of the other one
+  int lg_most[2];     // parts that expert e's contraction has room for
+  __host__ __device__ inline DownParts parts(int m0, int m1) const {
+    DownParts d{};
+    const int rb0 = (m0 + 127) >> 7, rb1 = (m1 + 127) >> 7;
+    if (rb0 * steps[0] + rb1 * steps[1] <= cus && (rb0 + rb1) * cols <= cus) return d;
+    d.cut[0] = rb0 > 0 && (rb1 == 0 || beside[0] != 0);
+    d.cut[1] = rb1 > 0 && (rb0 == 0 || beside[1] != 0);
+    const int most0 = d.cut[0] ? lg_most[0] : 2, most1 = d.cut[1] ? lg_most[1] : 2, most = most0 < most1 ? most0 : most1;
+    const int count = ((d.cut[0] ? rb0 : 0) + (d.cut[1] ? rb1 : 0)) * cols;
+    d.lg = count * 4 <= cus ? 2 : (count * 2 <= cus ? 1 : 0);
+    if (d.lg > most) d.lg = most;
+    const int large_cols = (cols + 1) >> 1, large0 = ((rb0 + 1) >> 1) * large_cols, large1 = ((rb1 + 1) >> 1) * large_cols;
+    const int large = (d.cut[0] ? large0 : 0) + (d.cut[1] ? large1 : 0);
+    d.large = d.lg == 0 && most > 0 && 4 * large > cus && large0 + large1 + large <= cus;
+    if (d.large) d.lg = 1;
+    return d;
+  }
+};
+
+// fp32 sums of the parts, a tile's size each, at most as many as CUs, and a counter per slot, all zero
+struct DownSplit {
+  float* sums;
+  int* count;
+  PartsRule rule;
+};
+
+// Memory that no launch writes while it reads it: scalar loads, wherever they stand.
+using ScalarInts = const __attribute__((address_space(4))) int32_t*;
 
 // Workgroup barrier without the fences of __syncthreads().  Those fences make the compiler wait for EVERY
 // outstanding LDS-direct load (vmcnt(0)) at the barrier, which drains the prefetch ring on each K step; the waits
@@ -356,10 +377,7 @@ struct FusedSync {
   // few-rows form with the norm folded in: the token rows pass through an RMSNorm on their way to the MFMAs
   const __bf16* norm_weight;
   float norm_eps;
-  // split contraction (down_parts): fp32 sums of the parts, split_slots of a tile's size, and a counter per slot, all zero
-  float* split_sums;
-  int* split_count;
-  int split_slots;
+  DownSplit split;
 };
 
 // Fused launch: what this workgroup wrote for row block `rb` is in memory (its stores are write-through and every
@@ -867,10 +885,12 @@ __device__ __forceinline__ void few_rows_body(const Params& p, const int wg, con
 // The kernel's body is a function of its own so that one launch can run two of them side by side (the fused FFN
 // launch below: some workgroups run the gate/up form, the others the down form).  `wg` of `n_wg` is the workgroup's
 // place among those that share this body's tile list (blockIdx.x of gridDim.x in a plain launch).
-// ROLE: 0 = a plain launch; 1 / 2 = producer / consumer of a fused launch (see FusedSync).  AROWS (gate/up form of a fused launch): the A operand is read from the token rows themselves,
+// ROLE: 0 = a plain launch; 1 / 2 = producer / consumer of a fused launch (see FusedSync); 3 = the contraction in parts, as
+// `parts` says.  AROWS (gate/up form of a fused launch): the A operand is read from the token rows themselves,
 // fs.x through fs.gather, instead of from a K-tiled copy of them.
 template <int MODE, typename TS, bool KA, bool KB, int ROLE, bool AROWS = false>
-__device__ __forceinline__ void dual_gemm_body(const Params& p, const int wg, const int n_wg, const FusedSync& fs) {
+__device__ __forceinline__ void dual_gemm_body(const Params& p, const int wg, const int n_wg, const FusedSync& fs,
+                                               const DownParts parts = DownParts{}) {
 #if defined(__HIP_DEVICE_COMPILE__)  // the host pass only needs the launch stub; the body uses gfx950-only builtins
   constexpr int BM = TS::BM, BN = TS::BN, FM = TS::FM, FN = TS::FN;
   constexpr int kWavesN = TS::kWavesN, kWaves = TS::kWaves;
@@ -946,7 +966,8 @@ __device__ __forceinline__ void dual_gemm_body(const Params& p, const int wg, co
   int sorted_first[2] = {0, 0};  // tiled modes: sorted position of each expert's first row
   int sorted_total = 0;          // ... and the number of sorted rows
   if constexpr (TILED_IN) {
-    const int o0 = p.offsets[0], o1 = p.offsets[1], o2 = p.offsets[2];
+    const ScalarInts offsets = (ScalarInts)p.offsets;
+    const int o0 = offsets[0], o1 = offsets[1], o2 = offsets[2];
     g0.m = o1 - o0;
     g1.m = o2 - o1;
     const int pad0 = static_cast<int>(round_up_256(g0.m)), pad1 = static_cast<int>(round_up_256(g1.m));
@@ -983,19 +1004,14 @@ __device__ __forceinline__ void dual_gemm_body(const Params& p, const int wg, co
   tiles_n[1] = (g1.n + kTileN - 1) / kTileN;
   if (g1.m <= 0 || g1.n <= 0) tiles_m[1] = tiles_n[1] = 0;
   // split contraction: part q of a column tile is a column tile of its own, all columns' part 0 first
-  int lg_parts = 0;  // of expert 0, and of expert 1 four bits up: one register across the K loop
-  bool large_parts = false;
-  if constexpr (ROLE == 3) {
-    int lg[2];
-    large_parts = down_parts(g0.m, g1.m, g0.k, g1.k, g0.n, fs.split_slots, lg);
-    lg_parts = lg[0] | lg[1] << 4;
-  }
+  // (lg of expert 0, and of expert 1 four bits up: one register across the K loop)
+  const int lg_parts = ROLE == 3 ? (parts.cut[0] ? parts.lg : 0) | (parts.cut[1] ? parts.lg : 0) << 4 : 0;
   auto lg_of = [&](int group) { return lg_parts >> (4 * group) & 3; };
   auto cols_of = [&](int group) { return ((group ? g1.n : g0.n) + kTileN - 1) / kTileN; };
-  if (p.gate != 0) {
+  if (ROLE != 3 && p.gate != 0) {
     constexpr int kBigN = SWIGLU ? BigTile::BN / 2 : BigTile::BN;
     auto big = [](int m, int n) { return (m <= 0 || n <= 0) ? 0 : ((m + BigTile::BM - 1) / BigTile::BM) * ((n + kBigN - 1) / kBigN); };
-    const bool few = !large_parts && shape_deciding_tiles(big(g0.m, g0.n), big(g1.m, g1.n), g0.k, g1.k) <= p.gate_tiles;
+    const bool few = shape_deciding_tiles(big(g0.m, g0.n), big(g1.m, g1.n), g0.k, g1.k) <= p.gate_tiles;
     if (few != (p.gate == 1)) return;  // uniform: the other tile shape's launch does this problem
   }
   if constexpr (ROLE == 3) {
@@ -1008,7 +1024,7 @@ __device__ __forceinline__ void dual_gemm_body(const Params& p, const int wg, co
   constexpr bool kIsTail = std::is_same_v<TS, TailTileFor<MODE>>, kIsBig = std::is_same_v<TS, BigTileFor<MODE>>;
   constexpr int kSubM = BigTile::BM / BM, kSubN = BigTile::BN / BN;
   int big_m[2], big_n[2], split_at = 0, pieces = 0;
-  if ((kIsBig && p.split == 1) || (kIsTail && p.split == 2)) {
+  if (ROLE != 3 && ((kIsBig && p.split == 1) || (kIsTail && p.split == 2))) {
     constexpr int kBigN = SWIGLU ? BigTile::BN / 2 : BigTile::BN;
     big_m[0] = (g0.m + BigTile::BM - 1) / BigTile::BM;
     big_n[0] = (g0.n + kBigN - 1) / kBigN;
@@ -1019,7 +1035,7 @@ __device__ __forceinline__ void dual_gemm_body(const Params& p, const int wg, co
     const int all = big_m[0] * big_n[0] + big_m[1] * big_n[1];
     split_at = tail_split_point(big_m[0] * big_n[0], big_m[1] * big_n[1], g0.k, g1.k, p.split_cus);
     if constexpr (kIsBig) {
-      if (!large_parts) total = split_at;  // a multiple of 8 when smaller than `all`
+      total = split_at;  // a multiple of 8 when smaller than `all`
     } else {
       if (split_at == all) return;  // no split: the first launch did everything
       pieces = kSubM * kSubN * (all - split_at);
@@ -1854,7 +1870,7 @@ __device__ __forceinline__ void dual_gemm_body(const Params& p, const int wg, co
       constexpr uint32_t kWaveBytes = FM * FN * 1024;
       const int parts = 1 << (S.split & 15), this_part = S.split >> 4 & 15, slot = S.split >> 8;
       auto sums_of = [&](int part) {
-        return make_rsrc(reinterpret_cast<char*>(fs.split_sums) + (static_cast<int64_t>(slot + part) * kWaves + wave) * kWaveBytes, kWaveBytes);
+        return make_rsrc(reinterpret_cast<char*>(fs.split.sums) + (static_cast<int64_t>(slot + part) * kWaves + wave) * kWaveBytes, kWaveBytes);
       };
       const __amdgpu_buffer_rsrc_t mine = sums_of(this_part);
 #pragma unroll
@@ -1866,12 +1882,12 @@ __device__ __forceinline__ void dual_gemm_body(const Params& p, const int wg, co
       __builtin_amdgcn_s_waitcnt(waitcnt_imm(0, 0));
       __syncthreads();
       volatile int* const s_before = reinterpret_cast<volatile int*>(s_out);  // (the staging area is free between tiles)
-      if (tid == 0) *s_before = __hip_atomic_fetch_add(fs.split_count + slot, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (tid == 0) *s_before = __hip_atomic_fetch_add(fs.split.count + slot, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       __syncthreads();
       const bool last = __builtin_amdgcn_readfirstlane(*s_before) == parts - 1;
       __syncthreads();
       if (!last) return false;
-      if (tid == 0) __hip_atomic_store(fs.split_count + slot, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (tid == 0) __hip_atomic_store(fs.split.count + slot, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       if constexpr (FM * FN > 16) {  // (two parts; no registers for a second set of sums)
         const __amdgpu_buffer_rsrc_t from = sums_of(1 - this_part);
 #pragma unroll
@@ -2096,14 +2112,38 @@ __global__ __launch_bounds__(TS::kThreads, TS::kWgPerCu) void dual_gemm_kernel(P
   dual_gemm_body<MODE, TS, KA, KB, 0>(p, blockIdx.x, gridDim.x, FusedSync{});
 }
 
-// The few-rows form of the same launch (MODE: gate/up or down).
-// the down launch with the contraction in parts.  (Bounded by the wavefronts per SIMD that TS is made for: with 147
-// registers, no second workgroup on a CU, 4050 rows on unknown counts, whose tiles stay whole, took 180 us in place of 161.)
+// The down launch whose contraction may be in parts: the plain form or the parts', by the row counts.  Rows that are not cut
+// pay for the question alone, and their launch's arguments and offsets stay scalar loads that are asked for together: 960 rows
+// of the narrow expert on unknown counts 9.9 us, the plain kernel 9.7 (one body for both forms, asked in 64-bit numbers, 10.7;
+// two bodies that share their arguments 10.4).
+// (Bounded by the wavefronts per SIMD that TS is made for: with 147 registers, no second workgroup on a CU, 4050 rows on unknown
+// counts, whose tiles stay whole, took 180 us in place of 161.)
 template <typename TS>
-__global__ __launch_bounds__(TS::kThreads, TS::kWgPerCu * TS::kWaves / 4) void down_split_kernel(Params p, FusedSync fs) {
-  dual_gemm_body<kDown, TS, false, false, 3>(p, blockIdx.x, gridDim.x, fs);
+__global__ __launch_bounds__(TS::kThreads, TS::kWgPerCu * TS::kWaves / 4) void down_split_kernel(Params p, DownSplit split) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  // (every line of the launch's arguments, asked for at once, as the plain form does in front of its first wait)
+  const int n_wg = gridDim.x;
+  const ScalarInts offsets = (ScalarInts)p.offsets;
+  asm volatile("" ::"s"(p.g[0].a), "s"(p.g[1].a), "s"(p.gate), "s"(split.rule.cus), "s"(split.rule.lg_most[1]), "s"(n_wg), "s"(offsets));
+  const DownParts parts = split.rule.parts(offsets[1] - offsets[0], offsets[2] - offsets[1]);
+  // Each form reads its arguments for itself (they are the launch's first): values that both want, held across the question,
+  // are more than the scalar registers take.
+  using Arguments = const __attribute__((address_space(4))) Params*;
+  Arguments args = (Arguments)__builtin_amdgcn_kernarg_segment_ptr();
+  if (parts.lg == 0) {
+    asm volatile("" : "+s"(args));
+    dual_gemm_body<kDown, TS, false, false, 0>(*(const Params*)args, blockIdx.x, n_wg, FusedSync{});
+  } else {
+    if (parts.large != std::is_same_v<TS, BigTile>) return;  // uniform: the other tile shape's launch does this problem
+    asm volatile("" : "+s"(args));
+    FusedSync fs{};
+    fs.split = split;
+    dual_gemm_body<kDown, TS, false, false, 3>(*(const Params*)args, blockIdx.x, n_wg, fs, parts);
+  }
+#endif
 }
 
+// The few-rows form of the same launch (MODE: gate/up or down).
 template <int MODE, int FM, int NB>
 __global__ __launch_bounds__(kFewThreads, 2) void dual_gemm_few_rows_kernel(Params p) {
   constexpr int R = MODE == kGateUp ? 8 : 4;
@@ -2239,10 +2279,10 @@ int check_dims(const char* who, int64_t m, int64_t n, int64_t k, bool k_in_rows 
 // host knows, decides it on the host); when the host cannot tell, both launches are made and the device decides (the
 // second returns at once if there is nothing to split).
 // few: the few-rows form takes the problem; its number of rows, or 0.
-// split_sync: the down launch's contraction may be in parts (down_parts), with this scratch.
+// parts: the down launch's contraction may be in parts (PartsRule), with this scratch.
 template <int MODE, bool KA = false, bool KB = false>
 int launch_mfma(Params p, int64_t tiles_lo, int64_t tiles_hi, hipStream_t s, const char* who,
-                const int64_t* tiles_by_expert = nullptr, int64_t few = 0, const FusedSync* split_sync = nullptr) {
+                const int64_t* tiles_by_expert = nullptr, int64_t few = 0, const DownSplit* parts = nullptr) {
   const int cus = device_cu_count();
   const int threshold = cus / 2;
   if constexpr (MODE == kGateUp || MODE == kDown) {
@@ -2261,7 +2301,7 @@ int launch_mfma(Params p, int64_t tiles_lo, int64_t tiles_hi, hipStream_t s, con
     // at most one round of large tiles, and one expert's tiles may not count: the device has to choose
     small = true;
   }
-  if (MODE == kDown && split_sync != nullptr) {  // parts of large tiles, if the tiles that count can be enough for them
+  if (MODE == kDown && parts != nullptr) {  // parts of large tiles, if the tiles that count can be enough for them
     const bool one_counts = 2ll * p.g[0].k <= p.g[1].k || 2ll * p.g[1].k <= p.g[0].k;
     if (4 * (one_counts ? tiles_lo : tiles_hi) > cus) big = true;
   }
@@ -2270,8 +2310,8 @@ int launch_mfma(Params p, int64_t tiles_lo, int64_t tiles_hi, hipStream_t s, con
   p.split_cus = cus;
   if (small) {
     p.gate = big ? 1 : 0;
-    if (MODE == kDown && split_sync != nullptr)
-      hipLaunchKernelGGL(down_split_kernel<SmallTile>, dim3(cus * SmallTile::kWgPerCu), dim3(SmallTile::kThreads), 0, s, p, *split_sync);
+    if (MODE == kDown && parts != nullptr)
+      hipLaunchKernelGGL(down_split_kernel<SmallTile>, dim3(cus * SmallTile::kWgPerCu), dim3(SmallTile::kThreads), 0, s, p, *parts);
     else
       hipLaunchKernelGGL((dual_gemm_kernel<MODE, SmallTile, KA, KB>), dim3(cus * SmallTile::kWgPerCu), dim3(SmallTile::kThreads), 0, s, p);
   }
@@ -2286,8 +2326,8 @@ int launch_mfma(Params p, int64_t tiles_lo, int64_t tiles_hi, hipStream_t s, con
                                                   p.g[0].k, p.g[1].k, cus) != all;
     }
     p.split = split ? 1 : 0;
-    if (MODE == kDown && split_sync != nullptr)
-      hipLaunchKernelGGL(down_split_kernel<BigTile>, dim3(cus), dim3(BigTile::kThreads), 0, s, p, *split_sync);
+    if (MODE == kDown && parts != nullptr)
+      hipLaunchKernelGGL(down_split_kernel<BigTile>, dim3(cus), dim3(BigTile::kThreads), 0, s, p, *parts);
     else
       hipLaunchKernelGGL((dual_gemm_kernel<MODE, Big, KA, KB>), dim3(cus), dim3(Big::kThreads), 0, s, p);
     if (split) {
@@ -2608,8 +2648,8 @@ constexpr size_t kSplitSlotBytes = static_cast<size_t>(BigTile::BM) * BigTile::B
 // counters, a word per slot, in front of the slots
 size_t split_count_bytes() { return (static_cast<size_t>(device_cu_count()) * sizeof(int) + 1023) / 1024 * 1024; }
 
-// Whether the down launch's contraction is cut for some split of the rows (down_parts: more than 2 * cus rows, half a round of
-// large tiles at most, contractions of 4096 at least).  Not where the few-rows form takes the problem: narrow matrices of up
+// Whether the down launch's contraction is cut for some split of the rows (PartsRule): more than 2 * cus rows, half a round of
+// large tiles at most, contractions of 4096 at least.  Not where the few-rows form takes the problem: narrow matrices of up
 // to 1024 rows, which run as one launch, as two, and with the projections kept.
 bool may_split(const FfnArgs& a) {
   const int cus = device_cu_count();
@@ -2617,27 +2657,39 @@ bool may_split(const FfnArgs& a) {
          (a.inter[0] >= 4096 || a.inter[1] >= 4096) && few_rows_of(a) == 0;
 }
 
+// (of sizes that may_split lets through: at most 32768 rows)
+PartsRule parts_rule(const FfnArgs& a) {
+  PartsRule r{};
+  r.cus = device_cu_count();
+  r.cols = static_cast<int>(ceil_div(a.hidden, SmallTile::BN));
+  for (int e = 0; e < 2; ++e) {
+    const int64_t steps = ceil_div(a.inter[e], SmallTile::BN / 2);
+    r.steps[e] = static_cast<int>(steps <= r.cus ? steps : r.cus + 1);  // (more than one per CU is all that is asked)
+    r.beside[e] = 2 * a.inter[e] > a.inter[1 - e];
+    r.lg_most[e] = a.inter[e] >= 8192 ? 2 : (a.inter[e] >= 4096 ? 1 : 0);
+  }
+  return r;
+}
+
 int launch_down(const FfnArgs& a, hipStream_t s) {
   const Params p = down_params(a);
   const int64_t col_tiles = ceil_div(a.hidden, BigTile::BN);
   const int cus = device_cu_count();
   const bool rows_known = a.host_rows != nullptr;
-  FusedSync sync{};
-  const FusedSync* split = nullptr;
+  DownSplit parts_of{};
+  const DownSplit* split = nullptr;
   if (a.split_scratch != nullptr && may_split(a)) {
-    sync.split_count = static_cast<int*>(a.split_scratch);
-    sync.split_sums = reinterpret_cast<float*>(static_cast<char*>(a.split_scratch) + split_count_bytes());
-    sync.split_slots = cus;
-    int lg_parts[2];
+    parts_of.count = static_cast<int*>(a.split_scratch);
+    parts_of.sums = reinterpret_cast<float*>(static_cast<char*>(a.split_scratch) + split_count_bytes());
+    parts_of.rule = parts_rule(a);
     if (rows_known) {
-      const bool large = down_parts(static_cast<int>(a.host_rows[0]), static_cast<int>(a.host_rows[1]), static_cast<int>(a.inter[0]),
-                                    static_cast<int>(a.inter[1]), static_cast<int>(a.hidden), cus, lg_parts);
-      if (large) hipLaunchKernelGGL(down_split_kernel<BigTile>, dim3(cus), dim3(BigTile::kThreads), 0, s, p, sync);
-      else if (lg_parts[0] > 0 || lg_parts[1] > 0)
-        hipLaunchKernelGGL(down_split_kernel<SmallTile>, dim3(cus * SmallTile::kWgPerCu), dim3(SmallTile::kThreads), 0, s, p, sync);
-      if (lg_parts[0] > 0 || lg_parts[1] > 0) return check_launch("down_split_kernel");
+      const DownParts parts = parts_of.rule.parts(static_cast<int>(a.host_rows[0]), static_cast<int>(a.host_rows[1]));
+      if (parts.large) hipLaunchKernelGGL(down_split_kernel<BigTile>, dim3(cus), dim3(BigTile::kThreads), 0, s, p, parts_of);
+      else if (parts.lg > 0)
+        hipLaunchKernelGGL(down_split_kernel<SmallTile>, dim3(cus * SmallTile::kWgPerCu), dim3(SmallTile::kThreads), 0, s, p, parts_of);
+      if (parts.lg > 0) return check_launch("down_split_kernel");
     } else {
-      split = &sync;  // the launches decide by the same rule
+      split = &parts_of;  // the launches decide by the same rule
     }
   }
   if (a.host_rows != nullptr) {
