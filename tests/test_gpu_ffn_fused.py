@@ -391,10 +391,13 @@ def _norm_block(dev, T, seed):
     return run, x, work, (packed, norm, experts)
 
 
-def test_few_rows_with_the_norm_in_place_on_two_streams_and_replayed(dev):
+@pytest.mark.parametrize("rows", [(32, 117), (217, 256), (217, 32), (129, 224)])
+def test_few_rows_with_the_norm_in_place_on_two_streams_and_replayed(dev, rows):
     """The one launch with the norm where its output is its input, on two streams at once, and from a HIP graph whose
-    input changes between replays: the separate launches' bits, and a workspace that is zero again."""
-    blocks = [_norm_block(dev, T, seed) for T, seed in ((32, 31), (117, 32))]
+    input changes between replays: the separate launches' bits, and a workspace that is zero again.  Up to 128 rows two
+    workgroups share a CU and a launch's waiting ones take 32 of an XCD's 64 places at most; from 129 rows on a workgroup has
+    its CU to itself, and at most 31 of an XCD's 32 are taken by a launch that waits.  Both kinds, and one of each."""
+    blocks = [_norm_block(dev, T, seed) for T, seed in zip(rows, (31, 32))]
     here = torch.cuda.current_stream().cuda_stream
     want = []
     for run, x, work, _ in blocks:

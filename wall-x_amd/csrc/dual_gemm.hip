@@ -348,11 +348,18 @@ __device__ __forceinline__ unsigned char* lds_array() {
 // has reached the number of those tiles.  An XCD places its share of a launch's workgroups in index order and the
 // producers come first, so on every XCD the producers have their places before a consumer gets one, and producers
 // never wait: a launch alone on the chip always makes progress.  So do two of them in flight together on their own
-// workspaces (an XCD has 64 places for workgroups of this size, a launch at most 32 consumers per XCD, and a
-// launch's consumers hold no place on an XCD where its producers still wait for one: waiting workgroups cannot
-// fill an XCD).  The wait is bounded all the same (kFusedWaitTicks of the 100 MHz clock; then `*error` is set and
-// the tile goes ahead on whatever is there), which is what three or more concurrent launches would fall back on.  The last consumer past the wait of a row block clears the row block's counters, so a launch
-// leaves the workspace as it found it: all zero.
+// workspaces.  Where a launch's producers still wait for a place on an XCD, it has no consumer there, and the other launch's
+// consumers leave one:
+//   two workgroups per CU (128 x 128 tiles, few rows up to 128): an XCD has 64 places, a launch at most 32 consumers for it
+//     (one per CU in all);
+//   one workgroup per CU (the few-rows form's larger tiles, 129 .. 256 rows): 32 places, at most 31 consumers (the limit of
+//     kXcds less than a workgroup per CU in launch_ffn_fused), so a whole CU is left, for a workgroup of either kind;
+//   one launch of each kind: consumers of the first kind, one on each of 32 CUs, can keep workgroups of the second out, but
+//     their own producers find the CU that the second kind leaves, so they end, and the second launch goes on.
+// Three or more launches have no such guarantee (two others' consumers can take every place of an XCD), and the kind of one
+// per CU has the smaller margin: at 217 rows a launch has 28 consumers to an XCD.  The wait is bounded for them
+// (kFusedWaitTicks of the 100 MHz clock; then `*error` is set and the tile goes ahead on whatever is there).  The last consumer
+// past the wait of a row block clears the row block's counters, so a launch leaves the workspace as it found it: all zero.
 // The producers can read their A operand from the token rows themselves (AROWS below: `x` through `gather`), which
 // makes the permute into the K-tiled activation matrix part of the launch.
 constexpr int kFusedMaxRowBlocks = 256;   // 128-row blocks per expert
@@ -2784,8 +2791,7 @@ int launch_ffn_fused(const FfnArgs& a, int* ws, hipStream_t s) {
       shape = q;
       if (gate_tiles <= cus && down_tiles <= (places == cus ? cus - kXcds : cus)) break;
     }
-    // (Fewer down tiles in the grid than an XCD has places: with two launches in flight together the gate/up tiles of either
-    // then find a place however many workgroups wait.)
+    // (Fewer down tiles in the grid than an XCD has places: see FusedSync.)
     if (!rows_known) {  // (for rows that are on the wide expert after all)
       const int64_t spare = places - ceil_div(down_tiles, kXcds) * kXcds;
       gate_tiles = gate_tiles < spare ? spare : cus;
