@@ -384,7 +384,6 @@ struct FusedSync {
   // few-rows form with the norm folded in: the token rows pass through an RMSNorm on their way to the MFMAs
   const __bf16* norm_weight;
   float norm_eps;
-  DownSplit split;
 };
 
 // Fused launch: what this workgroup wrote for row block `rb` is in memory (its stores are write-through and every
@@ -893,11 +892,11 @@ __device__ __forceinline__ void few_rows_body(const Params& p, const int wg, con
 // launch below: some workgroups run the gate/up form, the others the down form).  `wg` of `n_wg` is the workgroup's
 // place among those that share this body's tile list (blockIdx.x of gridDim.x in a plain launch).
 // ROLE: 0 = a plain launch; 1 / 2 = producer / consumer of a fused launch (see FusedSync); 3 = the contraction in parts, as
-// `parts` says.  AROWS (gate/up form of a fused launch): the A operand is read from the token rows themselves,
+// `parts` says, with the scratch `split`.  AROWS (gate/up form of a fused launch): the A operand is read from the token rows themselves,
 // fs.x through fs.gather, instead of from a K-tiled copy of them.
 template <int MODE, typename TS, bool KA, bool KB, int ROLE, bool AROWS = false>
 __device__ __forceinline__ void dual_gemm_body(const Params& p, const int wg, const int n_wg, const FusedSync& fs,
-                                               const DownParts parts = DownParts{}) {
+                                               const DownParts parts = DownParts{}, const DownSplit& split = DownSplit{}) {
 #if defined(__HIP_DEVICE_COMPILE__)  // the host pass only needs the launch stub; the body uses gfx950-only builtins
   constexpr int BM = TS::BM, BN = TS::BN, FM = TS::FM, FN = TS::FN;
   constexpr int kWavesN = TS::kWavesN, kWaves = TS::kWaves;
@@ -973,7 +972,10 @@ __device__ __forceinline__ void dual_gemm_body(const Params& p, const int wg, co
   int sorted_first[2] = {0, 0};  // tiled modes: sorted position of each expert's first row
   int sorted_total = 0;          // ... and the number of sorted rows
   if constexpr (TILED_IN) {
-    const ScalarInts offsets = (ScalarInts)p.offsets;
+    // (Behind the asm statements of down_split_kernel they would be vector loads.  A fused launch's are scalar as they stand, and
+    // the other type moves its prologue about: 2048 rows 0.2 us a layer slower.)
+    using Offsets = std::conditional_t<ROLE == 1 || ROLE == 2, const int32_t*, ScalarInts>;
+    const Offsets offsets = (Offsets)p.offsets;
     const int o0 = offsets[0], o1 = offsets[1], o2 = offsets[2];
     g0.m = o1 - o0;
     g1.m = o2 - o1;
@@ -1877,7 +1879,7 @@ __device__ __forceinline__ void dual_gemm_body(const Params& p, const int wg, co
       constexpr uint32_t kWaveBytes = FM * FN * 1024;
       const int parts = 1 << (S.split & 15), this_part = S.split >> 4 & 15, slot = S.split >> 8;
       auto sums_of = [&](int part) {
-        return make_rsrc(reinterpret_cast<char*>(fs.split.sums) + (static_cast<int64_t>(slot + part) * kWaves + wave) * kWaveBytes, kWaveBytes);
+        return make_rsrc(reinterpret_cast<char*>(split.sums) + (static_cast<int64_t>(slot + part) * kWaves + wave) * kWaveBytes, kWaveBytes);
       };
       const __amdgpu_buffer_rsrc_t mine = sums_of(this_part);
 #pragma unroll
@@ -1889,12 +1891,12 @@ __device__ __forceinline__ void dual_gemm_body(const Params& p, const int wg, co
       __builtin_amdgcn_s_waitcnt(waitcnt_imm(0, 0));
       __syncthreads();
       volatile int* const s_before = reinterpret_cast<volatile int*>(s_out);  // (the staging area is free between tiles)
-      if (tid == 0) *s_before = __hip_atomic_fetch_add(fs.split.count + slot, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (tid == 0) *s_before = __hip_atomic_fetch_add(split.count + slot, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       __syncthreads();
       const bool last = __builtin_amdgcn_readfirstlane(*s_before) == parts - 1;
       __syncthreads();
       if (!last) return false;
-      if (tid == 0) __hip_atomic_store(fs.split.count + slot, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (tid == 0) __hip_atomic_store(split.count + slot, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       if constexpr (FM * FN > 16) {  // (two parts; no registers for a second set of sums)
         const __amdgpu_buffer_rsrc_t from = sums_of(1 - this_part);
 #pragma unroll
@@ -2143,9 +2145,7 @@ __global__ __launch_bounds__(TS::kThreads, TS::kWgPerCu * TS::kWaves / 4) void d
   } else {
     if (parts.large != std::is_same_v<TS, BigTile>) return;  // uniform: the other tile shape's launch does this problem
     asm volatile("" : "+s"(args));
-    FusedSync fs{};
-    fs.split = split;
-    dual_gemm_body<kDown, TS, false, false, 3>(*(const Params*)args, blockIdx.x, n_wg, fs, parts);
+    dual_gemm_body<kDown, TS, false, false, 3>(*(const Params*)args, blockIdx.x, n_wg, FusedSync{}, parts, split);
   }
 #endif
 }
