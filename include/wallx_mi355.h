@@ -234,11 +234,13 @@ int wx_dual_down_proj_residual(const void* hmid, void* out, const void* residual
                                const int64_t* host_rows_per_expert, const int32_t* out_row_id,
                                wx_stream_t stream);
 /* wx_dual_down_proj (residual NULL) or wx_dual_down_proj_residual with scratch for a launch that cuts its contraction into
- * parts where its tiles would leave CUs idle (513 .. 1024 and 2049 .. about 3900 rows at hidden 2048 and an expert of 11008): the fp32 sums of
- * the parts are added in order, so the result may differ from the form without in the last bit of a bf16, and is the same on
- * every call.  split_scratch: NULL (the form without), or wx_ffn_split_scratch_bytes() bytes of device memory, 16-byte
- * aligned, zeroed ONCE by the caller before the first use; each launch leaves it ready for the next one on its stream.  One per
- * stream. */
+ * parts where its tiles would leave CUs idle (513 .. about 1100 and 2049 .. about 3900 rows at hidden 2048 and an expert of
+ * 11008; wx_ffn_may_split has the bounds): the fp32 sums of the parts are added in order, so the result may differ from the
+ * form without in the last bit of a bf16, and is the same on every call.  Whether and where the contraction is cut depends
+ * on the rows of both experts: a token's last bit may change with the batch around it.  host_rows_per_expert that disagree
+ * with expert_offsets may leave the contraction whole.  split_scratch: NULL (the form without), or
+ * wx_ffn_split_scratch_bytes() bytes of device memory, 16-byte aligned, zeroed ONCE by the caller before the first use; each
+ * launch leaves it ready for the next one on its stream.  One per stream. */
 size_t wx_ffn_split_scratch_bytes(void);
 /* 1 if wx_dual_down_proj_split of these sizes uses its scratch for some split of the rows, 0 if it never does. */
 int wx_ffn_may_split(int64_t num_rows, int64_t hidden, int64_t inter0, int64_t inter1);

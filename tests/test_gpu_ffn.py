@@ -984,3 +984,35 @@ def test_split_scratch_is_held_for_the_sizes_that_use_it(dev, rows, hidden, inte
     native.release_ffn_buffers()
     native.dual_swiglu_ffn_keep(native.permute_rows_tiled(x, rmap, off, None, inv), T, off, weights, out_row_id=inv)
     assert len(native._split_scratches) == held
+
+
+@pytest.mark.parametrize("rows,told", [
+    # at hidden 2048, experts of 11008 and 1024: large tiles in two parts / small ones in two / small ones in four / none
+    ((2640, 96), (1000, 1736)), ((1000, 1736), (2640, 96)), ((100, 2636), (2640, 96)), ((2640, 96), (100, 2636)),
+    ((0, 2736), (2640, 96)), ((2640, 96), (0, 2736)), ((1000, 1736), (100, 2636)),
+])
+def test_parts_with_row_counts_that_are_not_the_devices(dev, rows, told):
+    """The host's row counts choose the launch, the device's decide what it does: counts that disagree may leave the contraction
+    whole, never an output or a counter.  No further from 64-bit results than the form without parts."""
+    T, hidden, inter = sum(rows), 2048, (11008, 1024)
+    g = torch.Generator(device=dev).manual_seed(T + rows[0])
+    n = lambda *s: torch.empty(s, dtype=torch.bfloat16, device=dev).normal_(0, 1, generator=g)
+    h, d = [n(m, i) for m, i in zip(rows, inter)], [n(hidden, i) for i in inter]
+    hmid = torch.zeros(native.padded_sorted_rows(T) * max(inter), dtype=torch.bfloat16, device=dev)
+    first = 0
+    for m, i, v in zip(rows, inter, h):
+        pad = (m + 255) // 256 * 256
+        if m:
+            hmid[first:first + pad * i] = native.pack_weight(torch.cat((v, v.new_zeros(pad - m, i))), cache=False).view(-1)[:pad * i]
+        first += pad * i
+    packed = [native.pack_weight(w, cache=False) for w in d]
+    off = torch.tensor([0, rows[0], T], dtype=torch.int32, device=dev)
+    scratch = torch.zeros(_lib.load().wx_ffn_split_scratch_bytes() // 4, dtype=torch.int32, device=dev)
+    out = [torch.full((T, hidden), 9.0, dtype=torch.bfloat16, device=dev) for _ in range(2)]
+    for y, split in zip(out, (None, scratch.data_ptr())):
+        _lib.call("wx_dual_down_proj_split", hmid.data_ptr(), y.data_ptr(), None, off.data_ptr(), packed[0].data_ptr(), packed[1].data_ptr(),
+                  T, hidden, *inter, _lib.i64x2(told), None, split, torch.cuda.current_stream().cuda_stream)
+    want = torch.cat([a.double() @ b.double().t() for a, b in zip(h, d)])
+    plain, got = (float((y.double() - want).norm() / want.norm()) for y in out)
+    assert got <= 1.01 * plain < 2 ** -8
+    assert not scratch[:256].any()

@@ -2139,11 +2139,12 @@ __global__ __launch_bounds__(TS::kThreads, TS::kWgPerCu * TS::kWaves / 4) void d
   // are more than the scalar registers take.
   using Arguments = const __attribute__((address_space(4))) Params*;
   Arguments args = (Arguments)__builtin_amdgcn_kernarg_segment_ptr();
-  if (parts.lg == 0) {
+  const bool other_shape = parts.lg > 0 && parts.large != std::is_same_v<TS, BigTile>;
+  if (other_shape && p.gate != 0) return;  // uniform: the other tile shape's launch does this problem
+  if (parts.lg == 0 || other_shape) {  // (the only launch, made for row counts that are not the device's: its tiles stay whole)
     asm volatile("" : "+s"(args));
     dual_gemm_body<kDown, TS, false, false, 0>(*(const Params*)args, blockIdx.x, n_wg, FusedSync{});
   } else {
-    if (parts.large != std::is_same_v<TS, BigTile>) return;  // uniform: the other tile shape's launch does this problem
     asm volatile("" : "+s"(args));
     dual_gemm_body<kDown, TS, false, false, 3>(*(const Params*)args, blockIdx.x, n_wg, FusedSync{}, parts, split);
   }
