@@ -190,10 +190,10 @@ def test_grid_totals_are_those_of_the_rows(dtype, merge, window):
 @pytest.mark.parametrize("sizes,want", [
     ((512, 2048, 11008, 1024), 0), ((513, 2048, 11008, 1024), 1), ((4096, 2048, 11008, 1024), 1), ((4097, 2048, 11008, 1024), 0),
     ((29184, 2048, 11008, 1024), 0), ((930, 2048, 4095, 1024), 0), ((930, 2048, 1024, 4096), 1), ((32768, 256, 11008, 64), 1),
-    ((32769, 256, 11008, 64), 0), ((800, 256, 4096, 96), 0), ((800, 256, 4096, 1024), 1), ((0, 2048, 11008, 1024), 0),
+    ((32769, 256, 11008, 64), 0), ((800, 256, 4096, 96), 1), ((256, 256, 4096, 96), 0), ((0, 2048, 11008, 1024), 0),
 ])
 def test_sizes_that_use_the_split_scratch(sizes, want):
-    """On 256 CUs (what the library takes for granted without a GPU): more than 512 rows, at most 128 tiles of 256 x 256, a
-    contraction of 4096, and not what the few-rows form takes."""
+    """On 256 CUs (what the library takes for granted without a GPU): more than 512 rows, at most 128 tiles of 256 x 256, and a
+    contraction of 4096."""
     from wallx_mi355 import _lib, native
     assert _lib.load().wx_ffn_may_split(*sizes) == want and native._may_split(*sizes) is bool(want)

@@ -941,11 +941,12 @@ def test_down_projection_with_its_contraction_in_parts(dev, rows, inter, hidden,
 
 
 @pytest.mark.parametrize("rows,inter,hidden", [((800, 0), (4096, 96), 256), ((600, 0), (11008, 256), 512), ((3, 1021), (64, 4096), 256),
-                                               ((513, 0), (4128, 4096), 64)])
+                                               ((513, 0), (4128, 4096), 64), ((512, 0), (4096, 96), 256), ((248, 8), (4096, 96), 256),
+                                               ((249, 8), (4096, 96), 256), ((0, 257), (64, 32), 256)])
 def test_narrow_matrices_sum_in_one_order_whatever_the_launch_form(dev, monkeypatch, rows, inter, hidden):
-    """Sizes that the few-rows form and the rule of the contraction in parts would both take (up to 1024 rows, a small hidden
-    size and one narrow expert; the last has no narrow one and is the parts'): the same bits as one launch and as two, with the
-    row counts known and unknown, and with the projections kept for a backward pass."""
+    """Small hidden sizes and a narrow expert, on both sides of the few-rows form's last row (256) and of the first whose
+    contraction may be in parts (513): the same bits as one launch and as two, with the row counts known and unknown, and with
+    the projections kept for a backward pass."""
     T = sum(rows)
     g = torch.Generator(device=dev).manual_seed(T + hidden)
     n = lambda *s: torch.empty(s, dtype=torch.bfloat16, device=dev).normal_(0, 0.05, generator=g)
@@ -967,7 +968,7 @@ def test_narrow_matrices_sum_in_one_order_whatever_the_launch_form(dev, monkeypa
 
 
 @pytest.mark.parametrize("rows,hidden,inter,held", [((4000, 97), 2048, (4096, 64), 0), ((900, 30), 512, (4064, 608), 0),
-                                                    ((900, 30), 512, (4096, 608), 1), ((800, 0), 256, (4096, 96), 0)])
+                                                    ((900, 30), 512, (4096, 608), 1), ((256, 0), 256, (4096, 96), 0)])
 def test_split_scratch_is_held_for_the_sizes_that_use_it(dev, rows, hidden, inter, held):
     """Neither an inference forward nor a training one leaves 64 MiB behind for a down launch that is never cut."""
     T = sum(rows)

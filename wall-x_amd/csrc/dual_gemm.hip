@@ -494,18 +494,19 @@ __device__ __forceinline__ float swiglu_bf16(float gate, float up) {
 // 21.0 / 16.5, 128 rows 22.5 / 19.4, 217 rows (the norm was a launch) 29.8 / 23.2; without a norm 18.8 / 13.6, 18.6 / 14.5,
 // 20.5 / 16.8, 24.2 / 18.8.
 constexpr int kFewThreads = 512;   // eight wavefronts
-constexpr int kFewMaxRows = 1024;  // (a bound for the host; few_rows decides)
 
-// Whether the few-rows form takes the problem: with every row on the narrower expert the tiles of 32 rows x 64 rows of B of
-// each GEMM are at most one per CU.  The split of the rows does not enter, so the host always knows, and every launch form
-// adds up in the same order.  The
-// line is where a round of the tiles ends (256 rows at hidden 2048, experts 11008 / 1024): 36 layers with the norm 950 us at 256
-// rows, as two rounds of tiles 1520 at 512 where the 128 x 128 tiles take 1460.  Rows on the wide expert are many tiles per
-// workgroup, and ahead of the 128 x 128 tiles up to that line too: 4 layers with the norm, every row on the expert of 11008,
-// 32 rows 513 / 292 us, 96 rows 517 / 353, 217 rows 560 / 478, 256 rows 560 / 547.
+// Whether the few-rows form takes the problem: at most a row per CU, and with every row on the narrower expert the tiles of 32
+// rows x 64 rows of B of each GEMM are at most one per CU.  The split of the rows does not enter, so the host always knows, and
+// every launch form adds up in the same order.  At hidden 2048, experts 11008 / 1024, both lines are 256 rows: 36 layers with the
+// norm 950 us at 256 rows, as two rounds of tiles 1520 at 512 where the 128 x 128 tiles take 1460.
+// Rows on the wide expert are many tiles per workgroup.  Layers with weights of their own (700 MB in turn), us a layer, 128 x 128
+// tiles / this form: 32 rows, all on the expert of 11008, 118 / 91, 64 of 128 120 / 100, 192 134 / 122, 256 134 / 136, 248 of 256
+// 135 / 159; none on it 28 / 22 at 256 rows.  Without the first line, at
+// narrower sizes: hidden 512, experts 2048 / 256, 504 of 512 rows on the wide one 24 / 47, none 13 / 9; hidden 256, 11008 / 64, 384
+// of 768 53 / 231; 1016 of 1024 68 / 262.
 inline bool few_rows(int64_t rows, int64_t inter0, int64_t inter1, int64_t hidden, int cus) {
   const int64_t blocks = (rows + 31) / 32, inter = inter0 < inter1 ? inter0 : inter1;
-  return rows <= kFewMaxRows && blocks * (inter / 32) <= cus && blocks * ((hidden + 63) / 64) <= cus;
+  return rows <= cus && blocks * (inter / 32) <= cus && blocks * ((hidden + 63) / 64) <= cus;
 }
 
 // One row's bf16 pair through the RMSNorm: w * bf16(x * inv), rounded, as the norm's own kernel has it (w_lo, w_hi: the pair of
@@ -2657,12 +2658,11 @@ constexpr size_t kSplitSlotBytes = static_cast<size_t>(BigTile::BM) * BigTile::B
 size_t split_count_bytes() { return (static_cast<size_t>(device_cu_count()) * sizeof(int) + 1023) / 1024 * 1024; }
 
 // Whether the down launch's contraction is cut for some split of the rows (PartsRule): more than 2 * cus rows, half a round of
-// large tiles at most, contractions of 4096 at least.  Not where the few-rows form takes the problem: narrow matrices of up
-// to 1024 rows, which run as one launch, as two, and with the projections kept.
+// large tiles at most, contractions of 4096 at least.  (The few-rows form ends before the first line.)
 bool may_split(const FfnArgs& a) {
   const int cus = device_cu_count();
   return a.rows > 2ll * cus && 2 * (ceil_div(a.rows, BigTile::BM) * ceil_div(a.hidden, BigTile::BN)) <= cus &&
-         (a.inter[0] >= 4096 || a.inter[1] >= 4096) && few_rows_of(a) == 0;
+         (a.inter[0] >= 4096 || a.inter[1] >= 4096);
 }
 
 // (of sizes that may_split lets through: at most 32768 rows)
@@ -2862,7 +2862,7 @@ int launch_norm_ffn_few_rows(const void* x, const void* x_tiled, void* out, cons
                              const void* norm_weight, float eps, void* workspace, hipStream_t stream) {
   // (hidden: what the norm's kernel takes in its whole-line form)
   if (!x || !x_tiled || !out || !sorted_row_id || !norm_weight || !workspace || !(eps >= 0.f) || num_rows <= 0 ||
-      num_rows > kFewMaxRows || hidden <= 0 || hidden % 256 != 0 || hidden > 2048)
+      hidden <= 0 || hidden % 256 != 0 || hidden > 2048)
     return 1;
   if ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(x_tiled) | reinterpret_cast<uintptr_t>(norm_weight) |
        reinterpret_cast<uintptr_t>(residual) | reinterpret_cast<uintptr_t>(out)) & 15)
