@@ -501,7 +501,7 @@ constexpr int kFewThreads = 512;   // eight wavefronts
 // norm 950 us at 256 rows, as two rounds of tiles 1520 at 512 where the 128 x 128 tiles take 1460.
 // Rows on the wide expert are many tiles per workgroup.  Layers with weights of their own (700 MB in turn), us a layer, 128 x 128
 // tiles / this form: 32 rows, all on the expert of 11008, 118 / 91, 64 of 128 120 / 100, 192 134 / 122, 256 134 / 136, 248 of 256
-// 135 / 159; none on it 28 / 22 at 256 rows.  Without the first line, at
+// 135 / 137; none on it 28 / 22 at 256 rows.  Without the first line, at
 // narrower sizes: hidden 512, experts 2048 / 256, 504 of 512 rows on the wide one 24 / 47, none 13 / 9; hidden 256, 11008 / 64, 384
 // of 768 53 / 231; 1016 of 1024 68 / 262.
 inline bool few_rows(int64_t rows, int64_t inter0, int64_t inter1, int64_t hidden, int cus) {
@@ -554,10 +554,13 @@ __device__ __forceinline__ void few_rows_body(const Params& p, const int wg, con
   const int cols[2] = {(p.g[0].n + kTileN - 1) / kTileN, (p.g[1].n + kTileN - 1) / kTileN};
   const int frag = (l16 << 6) + ((lq ^ ((l16 >> 2) & 3)) << 4);  // this lane's 16 bytes of a K-tiled block
 
-  // The row counts, and this workgroup's tiles: t, t + step, .. below end, in the order expert, row block, column tile.  At
-  // most one tile each where there are workgroups enough; else a workgroup stays with a row block, whose rows it then reads (and
-  // normalises) once, and the row blocks' workgroups of one column are on one XCD.
-  int m[2], blocks[2], total0, t, step, end;
+  // The row counts, and this workgroup's tiles: t, t + step, .. below end, in the order expert, row block, column tile, and then
+  // behind, behind + n_wg, .. below behind_end.  At most one tile each where there are workgroups enough; else a workgroup stays
+  // with a row block, whose rows it then reads (and normalises) once, and the row blocks' workgroups of one column are on one
+  // XCD, which takes them in eights: where that leaves many without a row block (nine blocks of 256 workgroups: 24 each, 15 tiles
+  // of 344; 248 rows of the expert of 11008 and 8 of the other 159 us a layer), the expert with less to do comes behind the other,
+  // a tile or a few for every workgroup (eight blocks of 32: 11 tiles and one; 137 us).
+  int m[2], blocks[2], total0, t, step, end, behind, behind_end;
   auto place = [&](int m0, int m1) {
     m[0] = m0;
     m[1] = m1;
@@ -567,18 +570,44 @@ __device__ __forceinline__ void few_rows_body(const Params& p, const int wg, con
     t = wg;
     step = n_wg;
     end = total0 + blocks[1] * cols[1];
+    behind = behind_end = 0;
     if (end > n_wg) {
-      for (int i = 2; i < 64; ++i) {
-        const int slots0 = (cols[0] + 8 * i - 1) / (8 * i) * 8, slots1 = (cols[1] + 8 * i - 1) / (8 * i) * 8;
-        if (blocks[0] * slots0 + blocks[1] * slots1 > n_wg) continue;
-        const int e = wg >= blocks[0] * slots0 ? 1 : 0, nct = e ? cols[1] : cols[0];
-        const int w = e ? wg - blocks[0] * slots0 : wg;
+      const int total1 = end - total0;
+      auto slots_of = [&](int e, int i) { return ((e ? cols[1] : cols[0]) + 8 * i - 1) / (8 * i) * 8; };
+      // tiles per workgroup: with both experts' row blocks side by side, and with those of `big` alone
+      const int big = static_cast<int64_t>(total1) * p.g[1].k > static_cast<int64_t>(total0) * p.g[0].k ? 1 : 0;
+      int both = (end + n_wg - 1) / n_wg, alone = 0;  // (fewer do not fit)
+      while (both < 64 && blocks[0] * slots_of(0, both) + blocks[1] * slots_of(1, both) > n_wg) ++both;
+      if (total0 > 0 && total1 > 0) {
+        const int k_big = big ? p.g[1].k : p.g[0].k, k_less = big ? p.g[0].k : p.g[1].k;
+        const int b = big ? blocks[1] : blocks[0], less = ((big ? total0 : total1) + n_wg - 1) / n_wg;
+        alone = ((big ? total1 : total0) + n_wg - 1) / n_wg;
+        while (alone < 64 && b * slots_of(big, alone) > n_wg) ++alone;
+        const int64_t most = k_big > k_less ? k_big : k_less;
+        if (alone >= 64 || (both < 64 && static_cast<int64_t>(alone) * k_big + static_cast<int64_t>(less) * k_less >= both * most)) alone = 0;
+      }
+      if (alone > 0 || both < 64) {
+        const int per = alone > 0 ? alone : both;
+        const int slots0 = slots_of(0, per), slots1 = slots_of(1, per);
+        const int used0 = alone > 0 && big ? 0 : blocks[0] * slots0, used1 = alone > 0 && !big ? 0 : blocks[1] * slots1;
+        const int e = wg >= used0 ? 1 : 0, nct = e ? cols[1] : cols[0];
+        const int w = e ? wg - used0 : wg;
         step = e ? slots1 : slots0;
         const int rb = __builtin_amdgcn_readfirstlane(w / step);
         const int first = (e ? total0 : 0) + rb * nct;
         t = first + w - rb * step;
-        end = rb < (e ? blocks[1] : blocks[0]) ? first + nct : 0;
-        break;
+        end = rb * step < (e ? used1 : used0) ? first + nct : 0;
+        if (alone > 0) {  // (workgroups without a row block first)
+          const int at = wg - (used0 + used1);
+          behind = (big ? 0 : total0) + (at < 0 ? at + n_wg : at);
+          behind_end = big ? total0 : total0 + total1;
+          if (t >= end) {
+            t = behind;
+            step = n_wg;
+            end = behind_end;
+            behind = behind_end;
+          }
+        }
       }
     }
   };
@@ -683,8 +712,14 @@ __device__ __forceinline__ void few_rows_body(const Params& p, const int wg, con
   const int pad0 = static_cast<int>(round_up_256(m[0])), pad1 = static_cast<int>(round_up_256(m[1]));
   int held = -1;  // the row block whose rows `fa` holds
 
-  for (; t < end; t += step) {
+  while (t < end) {
     const Tile x = tile_of(t);
+    int next = t + step;
+    if (next >= end && behind < behind_end) {
+      next = behind;
+      step = n_wg;
+      end = behind = behind_end;
+    }
     const int e = x.e, rb = x.rb, ct = x.ct;
     const Group G = e ? p.g[1] : p.g[0];
     const int nct = e ? cols[1] : cols[0], me = e ? m[1] : m[0], pad_e = e ? pad1 : pad0;
@@ -822,7 +857,7 @@ __device__ __forceinline__ void few_rows_body(const Params& p, const int wg, con
     int out_now[kSums];
 #pragma unroll
     for (int u = 0; u < kSums; ++u) out_now[u] = out_row[u];
-    if (t + step < end) begin(tile_of(t + step));  // the next tile's first loads, while this one's sums meet
+    if (next < end) begin(tile_of(next));  // the next tile's first loads, while this one's sums meet
     // partial sums: lane l of a block holds row l % 16, columns 4 (l / 16) .. + 3
     if constexpr (RL > 0) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
 #pragma unroll
@@ -882,6 +917,7 @@ __device__ __forceinline__ void few_rows_body(const Params& p, const int wg, con
       if constexpr (ROLE == 2) clear_flags_if_last(fs, tid, counter, before, nct);
     }
     __syncthreads();  // the partial sums' LDS is written by the next tile
+    t = next;
   }
 #endif
 }
@@ -2783,7 +2819,9 @@ int launch_ffn_fused(const FfnArgs& a, int* ws, hipStream_t s) {
     guess[1] = static_cast<int>(rows[1]);
     // the smallest tile with at most one gate/up tile per CU whose down tiles have a place beside them, or (as the registers of
     // the larger tiles leave no such place) behind them
-    for (int q = a.x_rows != nullptr ? 0 : kFewShapes - 2; q < kFewShapes; ++q) {  // (K-tiled rows: the larger tiles only)
+    // (K-tiled rows: the larger tiles only; and for half as many rows as CUs or more whose split is not known: at narrow sizes
+    // the smallest would do for all of them, and take 1.5 times as long where the rows are on the wide expert)
+    for (int q = a.x_rows != nullptr && (rows_known || a.rows <= cus / 2) ? 0 : kFewShapes - 2; q < kFewShapes; ++q) {
       const int fm = kFewShape[q][0], nb = kFewShape[q][1], nbc = kFewShape[q][2];
       const int64_t r0 = ceil_div(rows[0], 16 * fm), r1 = ceil_div(rows[1], 16 * fm);
       gate_tiles = r0 * ceil_div(a.inter[0], 8 * nb) + r1 * ceil_div(a.inter[1], 8 * nb);
@@ -2793,7 +2831,8 @@ int launch_ffn_fused(const FfnArgs& a, int* ws, hipStream_t s) {
       if (gate_tiles <= cus && down_tiles <= (places == cus ? cus - kXcds : cus)) break;
     }
     // (Fewer down tiles in the grid than an XCD has places: see FusedSync.)
-    if (!rows_known) {  // (for rows that are on the wide expert after all)
+    if (!rows_known) {  // (for rows that are on the wide expert after all, and a row block more where they are on both)
+      down_tiles += ceil_div(a.hidden, 16 * kFewShape[shape][2]);
       const int64_t spare = places - ceil_div(down_tiles, kXcds) * kXcds;
       gate_tiles = gate_tiles < spare ? spare : cus;
     }
