@@ -1017,3 +1017,24 @@ def test_parts_with_row_counts_that_are_not_the_devices(dev, rows, told):
     plain, got = (float((y.double() - want).norm() / want.norm()) for y in out)
     assert got <= 1.01 * plain < 2 ** -8
     assert not scratch[:256].any()
+
+
+@pytest.mark.parametrize("rows,inter,hidden,cut", [
+    ((513, 0), (4096, 4096), 2048, True), ((640, 0), (4064, 4096), 2048, False), ((1025, 0), (11008, 1024), 2048, False),
+    ((2200, 0), (4096, 4096), 2048, False), ((565, 1353), (4096, 4096), 2048, False), ((2200, 0), (8160, 1024), 2048, False),
+    ((2200, 0), (8192, 1024), 2048, True), ((565, 1353), (8192, 8192), 2048, True), ((565, 1353), (8192, 8160), 2048, False),
+])
+@pytest.mark.parametrize("known", [True, False])
+def test_sizes_whose_contraction_is_cut(dev, rows, inter, hidden, cut, known):
+    """A cut contraction leaves its parts' sums in the scratch.  Small tiles are cut into parts of 2048 and more, large ones (of the
+    rows that more than 256 small tiles hold) into parts of 4096 and more."""
+    T = sum(rows)
+    hmid = torch.ones(native.padded_sorted_rows(T) * max(inter), dtype=torch.bfloat16, device=dev)
+    packed = [native.pack_weight(torch.ones(hidden, i, dtype=torch.bfloat16, device=dev), cache=False) for i in inter]
+    off = torch.tensor([0, rows[0], T], dtype=torch.int32, device=dev)
+    scratch = torch.zeros(_lib.load().wx_ffn_split_scratch_bytes() // 4, dtype=torch.int32, device=dev)
+    out = torch.empty(T, hidden, dtype=torch.bfloat16, device=dev)
+    _lib.call("wx_dual_down_proj_split", hmid.data_ptr(), out.data_ptr(), None, off.data_ptr(), packed[0].data_ptr(), packed[1].data_ptr(),
+              T, hidden, *inter, _lib.i64x2(rows) if known else None, None, scratch.data_ptr(), torch.cuda.current_stream().cuda_stream)
+    assert bool(scratch.any()) is cut
+    assert (out[:rows[0]] == inter[0]).all() and (out[rows[0]:] == inter[1]).all()

@@ -265,8 +265,9 @@ __host__ __device__ inline long long shape_deciding_tiles(long long tiles0, long
 // the part that finishes last adds them up: at hidden 2048 (two parts) 513 .. 880 rows 87 -> 52 .. 55 us, 1024 rows 87 -> 56,
 // 100 rows of the expert of 11008 beside 900 of one of 1024 (four) 92 -> 35.  From half as many tiles as CUs on, two parts on
 // every CU take what one did (1760 rows: 90 us; parts of 250 tiles would be at 470 ns a step, two workgroups to a CU).
-// Where 256 x 256 tiles would be a quarter to half as many as CUs, two parts of them beat one part of four times as many small
-// tiles, two workgroups to a CU: 2640 + 96 rows 140 -> 115 us, 3520 + 128 159 -> 132.  The other expert's tiles count there: a
+// Where 256 x 256 tiles would be a quarter to half as many as CUs, two parts of 4096 and more of them beat one part of four
+// times as many small tiles, two workgroups to a CU: 2640 + 96 rows 140 -> 115 us, 3520 + 128 159 -> 132, an expert of 8192 and
+// 2410 rows 94 -> 88 (of 4096 they do not: 2200 rows 50 -> 55, 565 + 1353 of two 34 -> 58).  The other expert's tiles count there: a
 // workgroup that takes one as a second helping costs what the parts gained (4050 + 65 rows, 128 tiles and 8, alone 162 -> 160,
 // in four layers of a prefill 17 us a layer slower).
 // Asked with the same numbers on the host and on the device, so that the sums' order does not depend on which of them knows the
@@ -297,7 +298,7 @@ struct PartsRule {
     if (d.lg > most) d.lg = most;
     const int large_cols = (cols + 1) >> 1, large0 = ((rb0 + 1) >> 1) * large_cols, large1 = ((rb1 + 1) >> 1) * large_cols;
     const int large = (d.cut[0] ? large0 : 0) + (d.cut[1] ? large1 : 0);
-    d.large = d.lg == 0 && most > 0 && 4 * large > cus && large0 + large1 + large <= cus;
+    d.large = d.lg == 0 && most > 1 && 4 * large > cus && large0 + large1 + large <= cus;
     if (d.large) d.lg = 1;
     return d;
   }
@@ -2348,7 +2349,7 @@ int launch_mfma(Params p, int64_t tiles_lo, int64_t tiles_hi, hipStream_t s, con
   }
   if (MODE == kDown && parts != nullptr) {  // parts of large tiles, if the tiles that count can be enough for them
     const bool one_counts = 2ll * p.g[0].k <= p.g[1].k || 2ll * p.g[1].k <= p.g[0].k;
-    if (4 * (one_counts ? tiles_lo : tiles_hi) > cus) big = true;
+    if ((parts->rule.lg_most[0] > 1 || parts->rule.lg_most[1] > 1) && 4 * (one_counts ? tiles_lo : tiles_hi) > cus) big = true;
   }
   p.gate_tiles = threshold;
   p.split = 0;
