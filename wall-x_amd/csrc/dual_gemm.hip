@@ -577,12 +577,14 @@ __device__ __forceinline__ void few_rows_body(const Params& p, const int wg, con
       auto slots_of = [&](int e, int i) { return ((e ? cols[1] : cols[0]) + 8 * i - 1) / (8 * i) * 8; };
       // tiles per workgroup: with both experts' row blocks side by side, and with those of `big` alone
       const int big = static_cast<int64_t>(total1) * p.g[1].k > static_cast<int64_t>(total0) * p.g[0].k ? 1 : 0;
-      int both = (end + n_wg - 1) / n_wg, alone = 0;  // (fewer do not fit)
+      // (fewer do not fit; and none do where there are more row blocks than eights of workgroups: finding that out by trying, 64
+      // turns of divisions ahead of every workgroup's first load, was 11 us of a launch of 22)
+      int both = (blocks[0] + blocks[1]) * 8 <= n_wg ? (end + n_wg - 1) / n_wg : 64, alone = 0;
       while (both < 64 && blocks[0] * slots_of(0, both) + blocks[1] * slots_of(1, both) > n_wg) ++both;
       if (total0 > 0 && total1 > 0) {
         const int k_big = big ? p.g[1].k : p.g[0].k, k_less = big ? p.g[0].k : p.g[1].k;
         const int b = big ? blocks[1] : blocks[0], less = ((big ? total0 : total1) + n_wg - 1) / n_wg;
-        alone = ((big ? total1 : total0) + n_wg - 1) / n_wg;
+        alone = b * 8 <= n_wg ? ((big ? total1 : total0) + n_wg - 1) / n_wg : 64;
         while (alone < 64 && b * slots_of(big, alone) > n_wg) ++alone;
         const int64_t most = k_big > k_less ? k_big : k_less;
         if (alone >= 64 || (both < 64 && static_cast<int64_t>(alone) * k_big + static_cast<int64_t>(less) * k_less >= both * most)) alone = 0;
