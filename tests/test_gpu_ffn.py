@@ -942,11 +942,13 @@ def test_down_projection_with_its_contraction_in_parts(dev, rows, inter, hidden,
 
 @pytest.mark.parametrize("rows,inter,hidden", [((800, 0), (4096, 96), 256), ((600, 0), (11008, 256), 512), ((3, 1021), (64, 4096), 256),
                                                ((513, 0), (4128, 4096), 64), ((512, 0), (4096, 96), 256), ((248, 8), (4096, 96), 256),
-                                               ((249, 8), (4096, 96), 256), ((0, 257), (64, 32), 256)])
+                                               ((249, 8), (4096, 96), 256), ((0, 257), (64, 32), 256), ((504, 8), (64, 32), 256),
+                                               ((1016, 8), (64, 32), 256), ((1017, 8), (64, 32), 256), ((240, 240), (256, 256), 1024),
+                                               ((1, 480), (256, 256), 1024), ((496, 496), (256, 256), 512)])
 def test_narrow_matrices_sum_in_one_order_whatever_the_launch_form(dev, monkeypatch, rows, inter, hidden):
-    """Small hidden sizes and a narrow expert, on both sides of the few-rows form's last row (256) and of the first whose
-    contraction may be in parts (513): the same bits as one launch and as two, with the row counts known and unknown, and with
-    the projections kept for a backward pass."""
+    """Small hidden sizes and a narrow expert, on both sides of the few-rows form's last row (256 beside a wide expert, else 1024
+    or where rows on both experts are a tile to every CU) and of the first whose contraction may be in parts (513): the same bits
+    as one launch and as two, with the row counts known and unknown, and with the projections kept for a backward pass."""
     T = sum(rows)
     g = torch.Generator(device=dev).manual_seed(T + hidden)
     n = lambda *s: torch.empty(s, dtype=torch.bfloat16, device=dev).normal_(0, 0.05, generator=g)

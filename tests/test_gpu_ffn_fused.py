@@ -309,6 +309,8 @@ def test_few_rows_with_the_norm_inside(dev, T, m0, H, I0, I1):
     (31, 31, 2048, 11008, 1024), (70, 70, 4096, 96, 64), (40, 9, 288, 320, 32), (200, 100, 1056, 640, 96),
     # one expert's tiles behind the other's, in the gate/up part and in the down part, the first expert's and the second's
     (256, 248, 2048, 11008, 1024), (128, 120, 2048, 11008, 1024), (256, 8, 2048, 1024, 4096), (250, 3, 512, 96, 4064),
+    # more rows than CUs: a row block more than the grid has eights of workgroups for, and one tile to every CU
+    (512, 504, 256, 64, 32), (992, 496, 512, 256, 256), (1024, 1017, 256, 32, 64),
 ])
 def test_few_rows_tiles_whatever_rows_the_host_expects(dev, T, m0, H, I0, I1):
     """One launch equals two, bit for bit, with the row counts known, unknown, and not the device's; with the norm inside it

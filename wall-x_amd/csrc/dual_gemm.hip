@@ -351,9 +351,9 @@ __device__ __forceinline__ unsigned char* lds_array() {
 // never wait: a launch alone on the chip always makes progress.  So do two of them in flight together on their own
 // workspaces.  Where a launch's producers still wait for a place on an XCD, it has no consumer there, and the other launch's
 // consumers leave one:
-//   two workgroups per CU (128 x 128 tiles, few rows up to 128): an XCD has 64 places, a launch at most 32 consumers for it
-//     (one per CU in all);
-//   one workgroup per CU (the few-rows form's larger tiles, 129 .. 256 rows): 32 places, at most 31 consumers (the limit of
+//   two workgroups per CU (128 x 128 tiles, the few-rows form's smaller ones): an XCD has 64 places, a launch at most 32
+//     consumers for it (one per CU in all);
+//   one workgroup per CU (the few-rows form's larger tiles, at hidden 2048 129 .. 256 rows): 32 places, at most 31 consumers (the limit of
 //     kXcds less than a workgroup per CU in launch_ffn_fused), so a whole CU is left, for a workgroup of either kind;
 //   one launch of each kind: consumers of the first kind, one on each of 32 CUs, can keep workgroups of the second out, but
 //     their own producers find the CU that the second kind leaves, so they end, and the second launch goes on.
@@ -496,18 +496,23 @@ __device__ __forceinline__ float swiglu_bf16(float gate, float up) {
 // 20.5 / 16.8, 24.2 / 18.8.
 constexpr int kFewThreads = 512;   // eight wavefronts
 
-// Whether the few-rows form takes the problem: at most a row per CU, and with every row on the narrower expert the tiles of 32
-// rows x 64 rows of B of each GEMM are at most one per CU.  The split of the rows does not enter, so the host always knows, and
-// every launch form adds up in the same order.  At hidden 2048, experts 11008 / 1024, both lines are 256 rows: 36 layers with the
-// norm 950 us at 256 rows, as two rounds of tiles 1520 at 512 where the 128 x 128 tiles take 1460.
+// Whether the few-rows form takes the problem: at most a row per CU, where with every row on the narrower expert the tiles of 32
+// rows x 64 rows of B of each GEMM are at most one per CU; and up to kFewMaxRows where they are for any split of the rows.  The
+// split itself does not enter, so the host always knows, and every launch form adds up in the same order.  At hidden 2048, experts
+// 11008 / 1024, the line is 256 rows: 36 layers with the norm 950 us at 256 rows, as two rounds of tiles 1520 at 512 where the
+// 128 x 128 tiles take 1460.
 // Rows on the wide expert are many tiles per workgroup.  Layers with weights of their own (700 MB in turn), us a layer, 128 x 128
 // tiles / this form: 32 rows, all on the expert of 11008, 118 / 91, 64 of 128 120 / 100, 192 134 / 122, 256 134 / 136, 248 of 256
-// 135 / 137; none on it 28 / 22 at 256 rows.  Without the first line, at
-// narrower sizes: hidden 512, experts 2048 / 256, 504 of 512 rows on the wide one 24 / 47, none 13 / 9; hidden 256, 11008 / 64, 384
-// of 768 53 / 231; 1016 of 1024 68 / 262.
+// 135 / 137; none on it 28 / 22 at 256 rows.  Beyond a row per CU, at narrower sizes, they cost more than the form gains: hidden
+// 512, experts 2048 / 256, 504 of 512 rows on the wide one 24 / 47, none 13 / 9; hidden 256, 11008 / 64, 384 of 768 53 / 231.
+// Where both experts are narrow there is no such split: hidden 256, experts 64 / 32, 257 .. 992 rows 10.9 .. 11.5 / 7.9 .. 8.5
+// however they are split, 256 / 256 up to 512 rows 12 / 8.7; hidden 512, 256 / 256 14 / 9.5 at 384 rows, at 992 of which half are
+// on either 15.0 / 16.5, the one place where it is behind without a norm (with it from 768 rows of 256 / 256 on, 15.3 / 16.5).
+constexpr int kFewMaxRows = 1024;
 inline bool few_rows(int64_t rows, int64_t inter0, int64_t inter1, int64_t hidden, int cus) {
-  const int64_t blocks = (rows + 31) / 32, inter = inter0 < inter1 ? inter0 : inter1;
-  return rows <= cus && blocks * (inter / 32) <= cus && blocks * ((hidden + 63) / 64) <= cus;
+  auto one_per_cu = [&](int64_t blocks, int64_t inter) { return blocks * (inter / 32) <= cus && blocks * ((hidden + 63) / 64) <= cus; };
+  const int64_t blocks = (rows + 31) / 32, wide = inter0 > inter1 ? inter0 : inter1, narrow = inter0 + inter1 - wide;
+  return rows <= cus ? one_per_cu(blocks, narrow) : rows <= kFewMaxRows && one_per_cu(blocks + 1, wide);  // (+ 1: rows on both)
 }
 
 // One row's bf16 pair through the RMSNorm: w * bf16(x * inv), rounded, as the norm's own kernel has it (w_lo, w_hi: the pair of
@@ -2697,7 +2702,8 @@ constexpr size_t kSplitSlotBytes = static_cast<size_t>(BigTile::BM) * BigTile::B
 size_t split_count_bytes() { return (static_cast<size_t>(device_cu_count()) * sizeof(int) + 1023) / 1024 * 1024; }
 
 // Whether the down launch's contraction is cut for some split of the rows (PartsRule): more than 2 * cus rows, half a round of
-// large tiles at most, contractions of 4096 at least.  (The few-rows form ends before the first line.)
+// large tiles at most, contractions of 4096 at least.  (The few-rows form takes none of them: of so many rows only
+// where both experts are far narrower.)
 bool may_split(const FfnArgs& a) {
   const int cus = device_cu_count();
   return a.rows > 2ll * cus && 2 * (ceil_div(a.rows, BigTile::BM) * ceil_div(a.hidden, BigTile::BN)) <= cus &&
@@ -2822,10 +2828,17 @@ int launch_ffn_fused(const FfnArgs& a, int* ws, hipStream_t s) {
     guess[1] = static_cast<int>(rows[1]);
     // the smallest tile with at most one gate/up tile per CU whose down tiles have a place beside them, or (as the registers of
     // the larger tiles leave no such place) behind them
-    // (K-tiled rows: the larger tiles only; and for half as many rows as CUs or more whose split is not known: at narrow sizes
-    // the smallest would do for all of them, and take 1.5 times as long where the rows are on the wide expert)
-    for (int q = a.x_rows != nullptr && (rows_known || a.rows <= cus / 2) ? 0 : kFewShapes - 2; q < kFewShapes; ++q) {
+    // (K-tiled rows: the larger tiles only)
+    const int64_t wide = a.inter[0] > a.inter[1] ? a.inter[0] : a.inter[1];
+    for (int q = a.x_rows != nullptr ? 0 : kFewShapes - 2; q < kFewShapes; ++q) {
       const int fm = kFewShape[q][0], nb = kFewShape[q][1], nbc = kFewShape[q][2];
+      // Of more than half as many rows as CUs whose split is not known the smaller tiles have to fit with any split: at narrow
+      // sizes they would do for all rows on the narrow expert, and take 1.5 times as long where they are on the wide one
+      // (hidden 256, experts 11008 / 64, 224 rows 137 / 82 us; none on it 8 / 10).  Where they fit they are ahead whatever the
+      // split: experts of 64 and 32, 256 rows 8.3 .. 9.0 / 10.5 .. 11.3, with the norm 10.2 .. 11.0 / 14.7 .. 15.6.
+      if (q < kFewShapes - 2 && !rows_known && a.rows > cus / 2 &&
+          (ceil_div(a.rows, 16 * fm) + 1) * ceil_div(wide, 8 * nb) > cus)
+        continue;
       const int64_t r0 = ceil_div(rows[0], 16 * fm), r1 = ceil_div(rows[1], 16 * fm);
       gate_tiles = r0 * ceil_div(a.inter[0], 8 * nb) + r1 * ceil_div(a.inter[1], 8 * nb);
       down_tiles = (r0 + r1) * ceil_div(a.hidden, 16 * nbc);
