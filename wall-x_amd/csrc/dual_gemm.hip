@@ -533,7 +533,10 @@ __device__ __forceinline__ uint32_t rms_scale(uint32_t x, float w_lo, float w_hi
 // rows, so it reads them once, for the squares and for the products.  The quarters and parities are those of the lanes of
 // rmsnorm_permute_tiled128_kernel, and the squares are added in its order: the same values.
 // NBP (ROLE 2): NB of the producers.
-template <int MODE, int FM, int NB, int R, int RV, int RL, int ROLE, bool AROWS, bool NORM = false, int NBP = NB>
+// ROUNDS: there may be more tiles than workgroups by much.  (The search for their places, if it is not needed, costs the kernels
+// with the largest tiles the registers of 20 scalars: 225 .. 256 rows at hidden 2048 21.8 us a layer, with the norm 25.3; with the
+// search in the down part 22.4 and 26.1.)
+template <int MODE, int FM, int NB, int R, int RV, int RL, int ROLE, bool AROWS, bool NORM = false, int NBP = NB, bool ROUNDS = true>
 __device__ __forceinline__ void few_rows_body(const Params& p, const int wg, const int n_wg, const FusedSync& fs) {
 #if defined(__HIP_DEVICE_COMPILE__)
   static_assert(MODE == kGateUp || MODE == kDown, "the FFN's two GEMMs");
@@ -561,12 +564,19 @@ __device__ __forceinline__ void few_rows_body(const Params& p, const int wg, con
   const int frag = (l16 << 6) + ((lq ^ ((l16 >> 2) & 3)) << 4);  // this lane's 16 bytes of a K-tiled block
 
   // The row counts, and this workgroup's tiles: t, t + step, .. below end, in the order expert, row block, column tile, and then
-  // behind, behind + n_wg, .. below behind_end.  At most one tile each where there are workgroups enough; else a workgroup stays
-  // with a row block, whose rows it then reads (and normalises) once, and the row blocks' workgroups of one column are on one
-  // XCD, which takes them in eights: where that leaves many without a row block (nine blocks of 256 workgroups: 24 each, 15 tiles
-  // of 344; 248 rows of the expert of 11008 and 8 of the other 159 us a layer), the expert with less to do comes behind the other,
-  // a tile or a few for every workgroup (eight blocks of 32: 11 tiles and one; 137 us).
-  int m[2], blocks[2], total0, t, step, end, behind, behind_end;
+  // (if behind is not negative) behind, behind + n_wg, .. of the other expert.  At most one tile each where there are workgroups
+  // enough; else a workgroup stays with a row block, whose rows it then reads (and normalises) once, and the row blocks'
+  // workgroups of one column are on one XCD, which takes them in eights: where that leaves many without a row block (nine blocks
+  // of 256 workgroups: 24 each, 15 tiles of 344; 248 rows of the expert of 11008 and 8 of the other 159 us a layer), the expert
+  // with less to do comes behind the other, a tile or a few for every workgroup (eight blocks of 32: 11 tiles and one; 137 us).
+  int m[2], blocks[2], total0, t, step, end, behind;
+  auto go_behind = [&](int& next) {
+    if (!ROUNDS || behind < 0) return;
+    next = behind;
+    step = n_wg;
+    end = behind < total0 ? total0 : total0 + blocks[1] * cols[1];
+    behind = -1;
+  };
   auto place = [&](int m0, int m1) {
     m[0] = m0;
     m[1] = m1;
@@ -576,8 +586,8 @@ __device__ __forceinline__ void few_rows_body(const Params& p, const int wg, con
     t = wg;
     step = n_wg;
     end = total0 + blocks[1] * cols[1];
-    behind = behind_end = 0;
-    if (end > n_wg) {
+    behind = -1;
+    if (ROUNDS && __builtin_expect(end > n_wg, 0)) {
       const int total1 = end - total0;
       auto slots_of = [&](int e, int i) { return ((e ? cols[1] : cols[0]) + 8 * i - 1) / (8 * i) * 8; };
       // tiles per workgroup: with both experts' row blocks side by side, and with those of `big` alone
@@ -606,15 +616,9 @@ __device__ __forceinline__ void few_rows_body(const Params& p, const int wg, con
         t = first + w - rb * step;
         end = rb * step < (e ? used1 : used0) ? first + nct : 0;
         if (alone > 0) {  // (workgroups without a row block first)
-          const int at = wg - (used0 + used1);
-          behind = (big ? 0 : total0) + (at < 0 ? at + n_wg : at);
-          behind_end = big ? total0 : total0 + total1;
-          if (t >= end) {
-            t = behind;
-            step = n_wg;
-            end = behind_end;
-            behind = behind_end;
-          }
+          const int at = wg - (used0 + used1) < 0 ? wg - (used0 + used1) + n_wg : wg - (used0 + used1);
+          if (at < (big ? total0 : total1)) behind = (big ? 0 : total0) + at;
+          if (t >= end) go_behind(t);
         }
       }
     }
@@ -723,11 +727,7 @@ __device__ __forceinline__ void few_rows_body(const Params& p, const int wg, con
   while (t < end) {
     const Tile x = tile_of(t);
     int next = t + step;
-    if (next >= end && behind < behind_end) {
-      next = behind;
-      step = n_wg;
-      end = behind = behind_end;
-    }
+    if (next >= end) go_behind(next);
     const int e = x.e, rb = x.rb, ct = x.ct;
     const Group G = e ? p.g[1] : p.g[0];
     const int nct = e ? cols[1] : cols[0], me = e ? m[1] : m[0], pad_e = e ? pad1 : pad0;
@@ -2226,7 +2226,8 @@ __device__ __forceinline__ void ffn_few_rows(const Params& pg, const Params& pd,
     if constexpr (WG == 2) few_rows_body<kGateUp, FM, NB, NORM || NB == 2 ? 8 : 4, NB == 2 ? 8 : 4, 0, 1, AROWS, NORM>(pg, wg, producers, fs);
     else few_rows_body<kGateUp, FM, NB, 8, NB == 4 ? 4 : 8, NB == 4 ? 4 : 0, 1, AROWS, NORM>(pg, wg, producers, fs);
   } else {
-    few_rows_body<kDown, FM, NBC, 4, NBC == 8 ? 2 : 4, NBC == 8 ? 2 : 0, 2, false, false, NB>(pd, wg - producers, consumers, fs);
+    // (few_rows leaves at most 256 of the largest down tiles, and more than 192 from hidden 12320 on)
+    few_rows_body<kDown, FM, NBC, 4, NBC == 8 ? 2 : 4, NBC == 8 ? 2 : 0, 2, false, false, NB, NBC != 8>(pd, wg - producers, consumers, fs);
   }
 }
 template <int FM, int NB, int NBC, int WG, bool AROWS>
