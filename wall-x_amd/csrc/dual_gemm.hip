@@ -2828,18 +2828,9 @@ int launch_ffn_fused(const FfnArgs& a, int* ws, hipStream_t s) {
     guess[0] = static_cast<int>(rows[0]);
     guess[1] = static_cast<int>(rows[1]);
     // the smallest tile with at most one gate/up tile per CU whose down tiles have a place beside them, or (as the registers of
-    // the larger tiles leave no such place) behind them
-    // (K-tiled rows: the larger tiles only)
-    const int64_t wide = a.inter[0] > a.inter[1] ? a.inter[0] : a.inter[1];
+    // the larger tiles leave no such place) behind them; for K-tiled rows of the larger tiles only
     for (int q = a.x_rows != nullptr ? 0 : kFewShapes - 2; q < kFewShapes; ++q) {
       const int fm = kFewShape[q][0], nb = kFewShape[q][1], nbc = kFewShape[q][2];
-      // Of more than half as many rows as CUs whose split is not known the smaller tiles have to fit with any split: at narrow
-      // sizes they would do for all rows on the narrow expert, and take 1.5 times as long where they are on the wide one
-      // (hidden 256, experts 11008 / 64, 224 rows 137 / 82 us; none on it 8 / 10).  Where they fit they are ahead whatever the
-      // split: experts of 64 and 32, 256 rows 8.3 .. 9.0 / 10.5 .. 11.3, with the norm 10.2 .. 11.0 / 14.7 .. 15.6.
-      if (q < kFewShapes - 2 && !rows_known && a.rows > cus / 2 &&
-          (ceil_div(a.rows, 16 * fm) + 1) * ceil_div(wide, 8 * nb) > cus)
-        continue;
       const int64_t r0 = ceil_div(rows[0], 16 * fm), r1 = ceil_div(rows[1], 16 * fm);
       gate_tiles = r0 * ceil_div(a.inter[0], 8 * nb) + r1 * ceil_div(a.inter[1], 8 * nb);
       down_tiles = (r0 + r1) * ceil_div(a.hidden, 16 * nbc);
@@ -2847,15 +2838,16 @@ int launch_ffn_fused(const FfnArgs& a, int* ws, hipStream_t s) {
       shape = q;
       if (gate_tiles <= cus && down_tiles <= (places == cus ? cus - kXcds : cus)) break;
     }
+    // (a row block more where rows are on both experts)
+    if (!rows_known) down_tiles += ceil_div(a.hidden, 16 * kFewShape[shape][2]);
     // (Fewer down tiles in the grid than an XCD has places: see FusedSync.)
-    if (!rows_known) {  // (for rows that are on the wide expert after all, and a row block more where they are on both)
-      down_tiles += ceil_div(a.hidden, 16 * kFewShape[shape][2]);
+    const int64_t most = places == cus ? cus - kXcds : cus;
+    down_tiles = down_tiles < most ? down_tiles : most;
+    if (!rows_known) {  // (for rows that are on the wide expert after all)
       const int64_t spare = places - ceil_div(down_tiles, kXcds) * kXcds;
       gate_tiles = gate_tiles < spare ? spare : cus;
     }
     gate_tiles = gate_tiles < cus ? gate_tiles : cus;
-    const int64_t most = places == cus ? cus - kXcds : cus;
-    down_tiles = down_tiles < most ? down_tiles : most;
   } else if (!rows_known) {
     // The split of the rows is only known on the device.  The launch is right for any split (workgroups take as
     // many tiles as there are), so what the host has to settle is whether it is the faster form whatever the split.
