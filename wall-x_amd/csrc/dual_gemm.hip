@@ -499,7 +499,7 @@ constexpr int kFewThreads = 512;   // eight wavefronts
 // Whether the few-rows form takes the problem: at most a row per CU, where with every row on the narrower expert the tiles of 32
 // rows x 64 rows of B of each GEMM are at most one per CU; and up to kFewMaxRows where they are for any split of the rows.  The
 // split itself does not enter, so the host always knows, and every launch form adds up in the same order.  At hidden 2048, experts
-// 11008 / 1024, the line is 256 rows: 36 layers with the norm 950 us at 256 rows, as two rounds of tiles 1520 at 512 where the
+// 11008 / 1024, the line is 256 rows: 36 layers with the norm 910 us at 256 rows, as two rounds of tiles 1520 at 512 where the
 // 128 x 128 tiles take 1460.
 // Rows on the wide expert are many tiles per workgroup.  Layers with weights of their own (700 MB in turn), us a layer, 128 x 128
 // tiles / this form: 32 rows, all on the expert of 11008, 118 / 91, 64 of 128 120 / 100, 192 134 / 122, 256 134 / 136, 248 of 256
