@@ -269,6 +269,8 @@ def test_down_projection_in_parts_from_graphs_and_on_two_streams(dev):
     native.release_ffn_buffers()
     want = layers(x)
     (scratch, _cap), = native._split_scratches.values()
+    scratch[1024:].zero_()
+    assert torch.equal(layers(x), want)
     assert scratch[1024:].any() and not scratch[:256].any()  # sums have been left there, and their counters are zero again
     assert torch.equal(layers(x, known=False), want)
     streams = [torch.cuda.Stream() for _ in range(2)]
