@@ -1726,38 +1726,53 @@ __device__ __forceinline__ void dual_gemm_body(const Params& p, const int wg, co
     // a row is kPitch bytes = kLanesPerRow lanes; one store instruction writes kRowsPerStore rows
     const int rl = lane_e / kLanesPerRow, cc = lane_e % kLanesPerRow;
     const int col = wn * kOutCols + cc * 8;
+    // What the stores need from memory is asked for ahead of the first of them: the row ids of the whole tile, and the addend's
+    // chunks kAhead row blocks in front of their use.  (Asked for row block by row block, a tile of 256 rows waited for eight
+    // memory latencies one after the other, twice over with row ids and an addend: q / k / v and o projections of 14592 rows with
+    // the rotary table's loads a row block ahead as well 291.6 -> 283.9 us, a layer of 912 rows 157 -> 155, training on 29184 rows
+    // 9630 -> 9600.)  Three row blocks where the row ids take registers: with four the kernel with the parts spills 56 bytes.
+    // Rows past the tile's end read a row that is there.
+    constexpr int kMost = MODE == kDown ? 3 : 4, kAhead = FM < kMost ? FM : kMost;
+    auto row_of = [&](int i, int q) { return (wm * FM + i) * 16 + q * kRowsPerStore + rl; };
+    // (a wavefront's ids: a lane has those of rows lane, lane + 64, .. of its share, and hands them out)
+    constexpr int kIds = MODE == kDown ? (FM * 16 + 63) / 64 : 1;
+    int ids[kIds];
+    if constexpr (MODE == kDown) {
 #pragma unroll
-    for (int i = 0; i < FM; ++i) {
-      int out_row[kStores];
-      u32x4 resv[kStores];
+      for (int r = 0; r < kIds; ++r) {
+        const int row = wm * FM * 16 + 64 * r + lane_e;
+        ids[r] = row < S.rows ? row : 0;
+      }
+      if (S.row_id != nullptr) {
+#pragma unroll
+        for (int r = 0; r < kIds; ++r) ids[r] = S.row_id[ids[r]];
+      }
+      // The ids are waited for here, whether or not this lane stores a row.  (A row block with nothing to store skips
+      // the stores and with them the wait; the compiler then keeps the registers of the ids from being written again
+      // before the loads are back, with a wait of its own in the first K step of every ring round, which drains the
+      // ring: the one-launch layer of 260 .. 2048 rows took 28.3 us in place of 26.4 at 512 rows, hidden 2048, expert
+      // 1024.)
+#pragma unroll
+      for (int r = 0; r < kIds; ++r) asm volatile("" : "+v"(ids[r]));
+    }
+    auto out_row = [&](int i, int q) {
+      if constexpr (MODE == kDown) return __shfl(ids[(i * 16 + q * kRowsPerStore) / 64], (i * 16 + q * kRowsPerStore) % 64 + rl);
+      else return row_of(i, q) < S.rows ? row_of(i, q) : 0;
+    };
+    u32x4 resv[RES ? kAhead : 1][kStores];
+    auto load_res = [&](int i) {
 #pragma unroll
       for (int q = 0; q < kStores; ++q) {
-        const int row = (wm * FM + i) * 16 + q * kRowsPerStore + rl;
-        out_row[q] = row;
-        if constexpr (MODE == kDown) {
-          // scatter: the row ids of the round (and the residual's chunks) are fetched together, ahead of the
-          // staging writes and reads
-          if (S.row_id != nullptr && row < S.rows) out_row[q] = S.row_id[row];
-        }
+        resv[i % kAhead][q] = *reinterpret_cast<const u32x4*>(S.res + static_cast<int64_t>(out_row(i, q)) * S.ldc + (col < S.cols_left ? col : 0));
       }
-      if constexpr (MODE == kDown) {
-        // The ids are waited for here, whether or not this lane stores a row.  (A row block with nothing to store skips
-        // the stores and with them the wait; the compiler then keeps the registers of the ids from being written again
-        // before the loads are back, with a wait of its own in the first K step of every ring round, which drains the
-        // ring: the one-launch layer of 260 .. 2048 rows took 28.3 us in place of 26.4 at 512 rows, hidden 2048, expert
-        // 1024.)
+    };
+    if constexpr (RES) {
 #pragma unroll
-        for (int q = 0; q < kStores; ++q) asm volatile("" : "+v"(out_row[q]));
-      }
-      if constexpr (RES) {
+      for (int i = 0; i < kAhead; ++i) load_res(i);
+      __builtin_amdgcn_sched_barrier(0);
+    }
 #pragma unroll
-        for (int q = 0; q < kStores; ++q) {
-          const int row = (wm * FM + i) * 16 + q * kRowsPerStore + rl;
-          resv[q] = u32x4{0u, 0u, 0u, 0u};
-          if (row < S.rows && col < S.cols_left)
-            resv[q] = *reinterpret_cast<const u32x4*>(S.res + static_cast<int64_t>(out_row[q]) * S.ldc + col);
-        }
-      }
+    for (int i = 0; i < FM; ++i) {
 #pragma unroll
       for (int j = 0; j < FN; ++j)
         *reinterpret_cast<u32x2*>(stage + e16 * kPitch + (((2 * j + (eq >> 1)) ^ swz(e16)) << 4) + (eq & 1) * 8) =
@@ -1765,20 +1780,25 @@ __device__ __forceinline__ void dual_gemm_body(const Params& p, const int wg, co
       __builtin_amdgcn_s_waitcnt(waitcnt_imm(63, 0));
 #pragma unroll
       for (int q = 0; q < kStores; ++q) {
-        const int srow = q * kRowsPerStore + rl;
+        const int srow = q * kRowsPerStore + rl, to = out_row(i, q);
         u32x4 v = *reinterpret_cast<const u32x4*>(stage + srow * kPitch + ((cc ^ swz(srow)) << 4));
         const int row = (wm * FM + i) * 16 + srow;
         if constexpr (RES) {  // bf16(y) + bf16(residual), summed in fp32 and rounded once, like the eager add
+          asm volatile("" : "+v"(resv[i % kAhead][q]));  // (waited for whether or not this lane stores a row, like the ids)
 #pragma unroll
           for (int w = 0; w < 4; ++w) {
-            const float lo = __builtin_bit_cast(float, v[w] << 16) + __builtin_bit_cast(float, resv[q][w] << 16);
+            const float lo = __builtin_bit_cast(float, v[w] << 16) + __builtin_bit_cast(float, resv[i % kAhead][q][w] << 16);
             const float hi = __builtin_bit_cast(float, v[w] & 0xFFFF0000u) +
-                             __builtin_bit_cast(float, resv[q][w] & 0xFFFF0000u);
+                             __builtin_bit_cast(float, resv[i % kAhead][q][w] & 0xFFFF0000u);
             v[w] = pack_bf16x2(lo, hi);
           }
         }
         if (row < S.rows && col < S.cols_left)
-          *reinterpret_cast<u32x4*>(S.c_base + static_cast<int64_t>(out_row[q]) * S.ldc + col) = v;
+          *reinterpret_cast<u32x4*>(S.c_base + static_cast<int64_t>(to) * S.ldc + col) = v;
+      }
+      if constexpr (RES) {
+        if (i + kAhead < FM) load_res(i + kAhead);
+        __builtin_amdgcn_sched_barrier(0);
       }
       __builtin_amdgcn_s_waitcnt(waitcnt_imm(63, 0));
     }
@@ -1875,17 +1895,21 @@ __device__ __forceinline__ void dual_gemm_body(const Params& p, const int wg, co
         };
         const bool rotate = live && col_w < p.rope_cols;  // wave-uniform: q and k heads rotate, v heads do not
         constexpr int kWidth = MODE == kQkvRope ? 64 : 128;  // table entries per token: shared by d and d + 64, or one each
+        // cos | sin of this lane's channels, four per load (the table need only be word-aligned), a row block ahead of their use
+        // (the table with an entry per channel: ahead of their first use, there are no registers for two row blocks of it)
+        constexpr int kCs = kWidth == 64 ? 2 : 1;
+        u32x4 cs[kCs][kWidth / 16];
+        auto load_cs = [&](int i) {
+          const int row = (wm * FM + i) * 16 + e16;
+          const uint32_t* t = p.rope_table + static_cast<int64_t>(S.row0 + (row < S.rows ? row : 0)) * kWidth + 4 * eq;
+#pragma unroll
+          for (int j = 0; j < kWidth / 16; ++j) cs[i % kCs][j] = *reinterpret_cast<const u32x4_word*>(t + j * 16);
+        };
+        if (rotate && kCs > 1) load_cs(0);
 #pragma unroll
         for (int i = 0; i < FM; ++i) {
-          // cos | sin of this lane's channels, four per load (the table need only be word-aligned), all loads ahead of their
-          // first use
-          u32x4 cs[kWidth / 16];
-          if (rotate) {
-            const int row = (wm * FM + i) * 16 + e16;
-            const uint32_t* t = p.rope_table + static_cast<int64_t>(S.row0 + (row < S.rows ? row : 0)) * kWidth + 4 * eq;
-#pragma unroll
-            for (int j = 0; j < kWidth / 16; ++j) cs[j] = *reinterpret_cast<const u32x4_word*>(t + j * 16);
-          }
+          if (rotate && i + kCs - 1 < FM) load_cs(i + kCs - 1);
+          if constexpr (kCs > 1) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
           for (int j = 0; j < 4; ++j) {
 #pragma unroll
@@ -1893,7 +1917,7 @@ __device__ __forceinline__ void dual_gemm_body(const Params& p, const int wg, co
               const float lo = round_bf16(acc[i][j][r] + bias_of(j, r));
               const float hi = round_bf16(acc[i][j + 4][r] + bias_of(j + 4, r));
               if (rotate) {
-                const uint32_t t_lo = cs[j][r], t_hi = cs[MODE == kQkvRope ? j : j + 4][r];
+                const uint32_t t_lo = cs[i % kCs][j][r], t_hi = cs[i % kCs][MODE == kQkvRope ? j : j + 4][r];
                 const float c_lo = __uint_as_float(t_lo << 16), s_lo = __uint_as_float(t_lo & 0xffff0000u);
                 const float c_hi = __uint_as_float(t_hi << 16), s_hi = __uint_as_float(t_hi & 0xffff0000u);
                 acc[i][j][r] = round_bf16(lo * c_lo) - round_bf16(hi * s_lo);
