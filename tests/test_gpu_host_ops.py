@@ -1,0 +1,123 @@
+"""The native host side of the row and rotary ops (csrc/host_ops.cpp) against the general path in native.py: what it takes
+gives the same bits, and whatever has to be warned of, copied or refused it leaves alone."""
+import pytest
+import torch
+
+from wallx_mi355 import _lib, native, workloads as wl
+from wallx_mi355.fusions import ops
+
+SECTION = list(wl.MROPE_SECTION)
+
+
+def _rope_inputs(dev, form, dtype, layout, order, rows=2, row_len=5):
+    g = torch.Generator(device=dev).manual_seed(3)
+    D = 128
+    make = {"bshd": lambda n: torch.randn((rows, row_len, n, D), generator=g, device=dev).to(dtype).transpose(1, 2),
+            "bhsd": lambda n: torch.randn((rows, n, row_len, D), generator=g, device=dev).to(dtype),
+            "packed": lambda n: torch.randn((rows, row_len, n + 3, D), generator=g, device=dev).to(dtype)[:, :, 2:2 + n].transpose(1, 2),
+            "expanded": lambda n: torch.randn((1, n, 1, D), generator=g, device=dev).to(dtype).expand(rows, n, row_len, D)}[order]
+    q, k = make(4), make(2)
+    pos = torch.randint(0, 300, (3, rows, row_len), generator=g, device=dev)
+    freq = wl.text_inv_freq(D).to(dev)
+    if form == 1:
+        return q, k, pos, freq
+    if form == 2:
+        return q, k, native.mrope_table(pos, freq, SECTION, layout), None
+    angle = pos.float()[..., None] * torch.cat((freq, freq))
+    return q, k, angle.cos().to(dtype), angle.sin().to(dtype)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("order", ["bshd", "bhsd", "packed", "expanded"])
+@pytest.mark.parametrize("form,dtype", [(0, torch.bfloat16), (0, torch.float16), (0, torch.float32), (1, torch.bfloat16), (1, torch.float32),
+                                        (2, torch.bfloat16)])
+@pytest.mark.parametrize("layout", ["hf", "csrc"])
+def test_rope_as_the_general_path(dev, form, dtype, layout, order):
+    q, k, a, b = _rope_inputs(dev, form, dtype, layout, order)
+    doubled = [2 * v for v in SECTION]
+    for backward in (0, 1):
+        made = _lib.host().rope(form, q, k, a, b, SECTION, layout, backward)
+        want = torch.empty(q.shape, dtype=dtype, device=dev), torch.empty(k.shape, dtype=dtype, device=dev)
+        if form == 0:
+            (native.rope_bwd(q, k, None, None, a, b, *want, doubled, layout) if backward else native.rope(q, k, a, b, *want, doubled, layout))
+        elif form == 1:
+            native.rope_from_positions(q, k, a, b, *want, doubled, backward=bool(backward), layout=layout)
+        else:
+            native.rope_from_table(q, k, a, *want, doubled, backward=bool(backward), layout=layout)
+        for x, w in zip(made, want):
+            assert x.is_contiguous() and x.shape == w.shape and torch.equal(x, w)
+
+
+@pytest.mark.gpu
+def test_rope_leaves_alone_what_the_general_path_is_for(dev):
+    q, k, c, s = _rope_inputs(dev, 0, torch.bfloat16, "hf", "bshd")
+    rope = _lib.host().rope
+
+    class Sub(torch.Tensor):
+        pass
+
+    assert rope(0, q, k, c, s, SECTION, "hf", 0) is not None
+    for args in ((q.cpu(), k, c, s), (q, k.float(), c, s), (q, k, c.transpose(1, 2), s), (q, k[:1], c, s), (q[..., ::2], k, c, s),
+                 (q, k, c[:2], s), (q.as_subclass(Sub), k, c, s), (q, k, c, None), (q.double(), k.double(), c.double(), s.double())):
+        assert rope(0, *args, SECTION, "hf", 0) is None
+    for section, layout in (([16, 24], "hf"), ([16.0, 24, 24], "hf"), ("abc", "hf"), (SECTION, "other"), (SECTION, 0)):
+        assert rope(0, q, k, c, s, section, layout, 0) is None
+    with pytest.raises(RuntimeError, match="covers 120 channels"):
+        ops.multimodal_rope(q, k, c, s, [16, 24, 20])
+    with pytest.raises(RuntimeError, match="list of 3 integers"):
+        ops.multimodal_rope(q, k, c, s, [16, 24])
+    with pytest.warns(UserWarning, match="`cos` of multimodal_rope op is discontiguous"):
+        got = ops.multimodal_rope(q, k, c.transpose(1, 2).contiguous().transpose(1, 2), s, SECTION)
+    assert all(torch.equal(x, y) for x, y in zip(got, ops.multimodal_rope(q, k, c, s, SECTION)))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tokens,topk,num_out", [(1, 1, 0), (257, 1, 0), (257, 1, 100), (300, 3, 0), (4099, 2, 5000)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_permute_and_unpermute_as_the_general_path(dev, tokens, topk, num_out, dtype, monkeypatch):
+    g = torch.Generator(device=dev).manual_seed(tokens)
+    x = torch.randn((tokens, 72), generator=g, device=dev).to(dtype)
+    ids = torch.randint(0, 5, (tokens, topk), generator=g, device=dev, dtype=torch.int32)
+    host = _lib.host()
+    rmap, _, _, ws = native.partition(ids, native.MAX_EXPERTS, num_out)
+    want = native.permute_rows(x, rmap, topk, num_out or tokens * topk)
+    out, got = host.permute(x, ids, num_out, *ws, native.MAX_EXPERTS)
+    used = int((rmap >= 0).sum())
+    assert torch.equal(got, rmap) and torch.equal(out[:used], want[:used])
+    assert host.permute(x, ids, num_out, ws[0][:1], ws[1], native.MAX_EXPERTS) is None  # too little scratch
+    assert host.permute(x, ids.long(), num_out, *ws, native.MAX_EXPERTS) is None
+    assert host.permute(x.t(), ids, num_out, *ws, native.MAX_EXPERTS) is None
+    if not num_out:
+        probs = torch.rand((tokens, topk), generator=g, device=dev)
+        for p in (None, probs):
+            assert torch.equal(host.unpermute(out, rmap, p, tokens, topk), native.unpermute(out, rmap, torch.tensor([]) if p is None else p, tokens, topk))
+        assert host.unpermute(out, rmap[:-1], None, tokens, topk) is None  # a short map
+        assert host.unpermute(out, rmap.long(), None, tokens, topk) is None
+    if topk == 1:
+        grad = torch.randn((tokens, 72), generator=g, device=dev).to(dtype)
+        assert torch.equal(host.unpermute_bwd(grad, out, rmap), native.unpermute_rows_bwd(grad, out, rmap))
+        assert host.unpermute_bwd(grad, out[:, :40], rmap) is None
+
+
+@pytest.mark.gpu
+def test_permute_in_checked_mode_still_refuses_wild_ids(dev):
+    x = torch.randn((8, 64), device=dev)
+    ids = torch.full((8, 1), native.MAX_EXPERTS, dtype=torch.int32, device=dev)
+    _, _, ws = native.permute(x, ids, 0, [], 0)
+    native.set_checked(True)
+    try:
+        with pytest.raises(RuntimeError, match="outside"):
+            native.permute(x, ids, 0, ws, 0)
+    finally:
+        native.set_checked(False)
+
+
+def test_tensors_on_the_cpu_are_left_alone():
+    q, k, c = torch.zeros(1, 4, 2, 128), torch.zeros(1, 2, 2, 128), torch.zeros(3, 1, 2, 128)
+    x, ids = torch.zeros(4, 8), torch.zeros(4, 1, dtype=torch.int32)
+    host = _lib.host()
+    assert host.rope(0, q, k, c, c, SECTION, "hf", 0) is None
+    assert host.permute(x, ids, 0, x, ids, 256) is None
+    assert host.unpermute(x, ids.view(-1), None, 4, 1) is None and host.unpermute_bwd(x, x, ids.view(-1)) is None
+    with pytest.raises(TypeError):
+        host.bind(1)

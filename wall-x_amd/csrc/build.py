@@ -4,7 +4,8 @@
 
 Sources are compiled one by one (objects under csrc/build/) and linked into
 wall-x_amd/wallx_mi355/libwallx_mi355.so, next to the Python package that loads it.  The benchmark's MFMA rate
-probe (probe.hip) goes into a library of its own, libwallx_probe.so, beside it.
+probe (probe.hip) goes into a library of its own, libwallx_probe.so, beside it, and the host side of the row and rotary
+ops (host_ops.cpp) into the Python module _wallx_host.so.
 """
 
 import os
@@ -26,6 +27,10 @@ HEADERS = ["common.h", "grid_prefix.h", "k_major.h", "tiled_layout.h", os.path.j
 # benchmark-only MFMA rate probe: its own library, not part of the product library or its ABI
 PROBE_SOURCE = "probe.hip"
 PROBE_LIB = os.path.join(OUT_DIR, "libwallx_probe.so")
+
+# the ops' host side, a Python module against torch's headers (no GPU code, and no HIP runtime of its own)
+HOST_SOURCE = "host_ops.cpp"
+HOST_LIB = os.path.join(OUT_DIR, "_wallx_host.so")
 
 FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-fno-gpu-rdc",
@@ -97,6 +102,23 @@ def build_probe(force: bool = False, verbose: bool = True) -> str:
     return PROBE_LIB
 
 
+def build_host(force: bool = False, verbose: bool = True) -> str:
+    import sysconfig
+
+    path = os.path.join(HERE, HOST_SOURCE)
+    if force or not _newer(HOST_LIB, [path, os.path.join(INCLUDE, "wallx_mi355.h")]):
+        import torch
+
+        root = os.path.dirname(torch.__file__)
+        _run([_hipcc(), "-x", "c++", "-std=c++17", "-O2", "-fPIC", "-shared", "-no-hip-rt", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+              f"-I{root}/include", f"-I{root}/include/torch/csrc/api/include", f"-I{sysconfig.get_paths()['include']}",
+              f"-I{os.path.dirname(os.path.dirname(os.path.realpath(_hipcc())))}/include", f"-I{INCLUDE}", f"-L{root}/lib",
+              "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_python", path, "-o", HOST_LIB])
+        if verbose:
+            print(f"[wallx_mi355] built {HOST_LIB}", flush=True)
+    return HOST_LIB
+
+
 def build(force: bool = False, verbose: bool = True, probe: bool = True) -> str:
     hipcc = _hipcc()
     os.makedirs(OBJ_DIR, exist_ok=True)
@@ -118,6 +140,7 @@ def build(force: bool = False, verbose: bool = True, probe: bool = True) -> str:
         _run([hipcc, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", LIB] + objs)
         if verbose:
             print(f"[wallx_mi355] linked {LIB}", flush=True)
+    build_host(force, verbose)
     if probe:
         build_probe(force, verbose)
     return LIB

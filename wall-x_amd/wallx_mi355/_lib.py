@@ -5,11 +5,13 @@ missing, loading raises.
 """
 
 import ctypes
+import importlib.util
 import os
 import threading
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 # WALLX_MI355_LIB points at an alternative build of the same library (e.g. one compiled with other tuning flags)
+HOST_PATH = os.path.join(_HERE, "_wallx_host.so")
 LIB_PATH = os.environ.get("WALLX_MI355_LIB") or os.path.join(_HERE, "libwallx_mi355.so")
 
 WX_F32, WX_F16, WX_BF16 = 0, 1, 2
@@ -81,6 +83,7 @@ PROTOTYPES = {
 
 _lock = threading.Lock()
 _lib = None
+_host = None
 
 
 class WallxLibraryError(RuntimeError):
@@ -105,6 +108,25 @@ def load():
                 fn.argtypes = args
             _lib = lib
     return _lib
+
+
+def host():
+    """The module of csrc/host_ops.cpp (a call's checks, outputs and launches in native code), bound to the loaded library."""
+    global _host
+    if _host is None:
+        lib = load()
+        with _lock:
+            if _host is None:
+                if not os.path.exists(HOST_PATH):
+                    raise WallxLibraryError(f"{HOST_PATH} is missing: build it with `python wall-x_amd/csrc/build.py`.")
+                import torch  # noqa: F401  (its libraries, which the module is linked against)
+
+                spec = importlib.util.spec_from_file_location("_wallx_host", HOST_PATH)
+                mod = importlib.util.module_from_spec(spec)
+                spec.loader.exec_module(mod)
+                mod.bind(*(ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in mod.names()))
+                _host = mod
+    return _host
 
 
 def check(rc: int, exc=RuntimeError):

@@ -17,7 +17,11 @@ import warnings
 
 import torch
 
+from .. import _lib
 from . import backend
+
+# The forwards and backwards below hand plain calls to the native host module first (_lib.host(): checks, outputs and
+# launches in one call); it declines anything that has to be warned of, copied or refused, which then goes on here.
 
 
 # ----------------------------------------------------------------------------- asym_dual_gmm
@@ -120,8 +124,10 @@ class PermuteMoE_topK(torch.autograd.Function):
             permuted_act_grad = torch.zeros(shape, dtype=dtype, device=device)
         if not permuted_act_grad.numel():
             return permuted_act_grad, None, None, None
-        grad = backend.unpermute(permuted_act_grad.contiguous(), ctx.row_id_map, torch.tensor([]),
-                                 ctx.num_tokens, ctx.num_topK)
+        grad = _lib.host().unpermute(permuted_act_grad, ctx.row_id_map, None, ctx.num_tokens, ctx.num_topK)
+        if grad is None:
+            grad = backend.unpermute(permuted_act_grad.contiguous(), ctx.row_id_map, torch.tensor([]),
+                                     ctx.num_tokens, ctx.num_topK)
         return grad, None, None, None
 
 
@@ -164,8 +170,10 @@ class UnpermuteMoE_topK(torch.autograd.Function):
 
         num_tokens = probs.size(0) if probs is not None else input_act.size(0)
         num_topK = probs.size(1) if probs is not None else 1
-        out = backend.unpermute(input_act, row_id_map, probs if probs is not None else torch.tensor([]),
-                                num_tokens, num_topK)
+        out = _lib.host().unpermute(input_act, row_id_map, probs, num_tokens, num_topK)
+        if out is None:
+            out = backend.unpermute(input_act, row_id_map, probs if probs is not None else torch.tensor([]),
+                                    num_tokens, num_topK)
         ctx.save_for_backward(input_act, row_id_map, probs)
         return out
 
@@ -177,7 +185,9 @@ class UnpermuteMoE_topK(torch.autograd.Function):
         act_grad = prob_grad = None
         if ctx.needs_input_grad[0]:
             if probs is None:
-                act_grad = backend.unpermute_rows_bwd(unpermuted_act_grad.contiguous(), input_act, row_id_map)
+                act_grad = _lib.host().unpermute_bwd(unpermuted_act_grad, input_act, row_id_map)
+                if act_grad is None:
+                    act_grad = backend.unpermute_rows_bwd(unpermuted_act_grad.contiguous(), input_act, row_id_map)
             else:
                 act_grad, prob_grad = backend.unpermute_bwd(unpermuted_act_grad.contiguous(), input_act, row_id_map,
                                                             probs)
@@ -207,6 +217,12 @@ class MultimodalRoPE(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, q, k, cos, sin, mrope_section, layout="hf"):
+        ctx.layout = layout
+        made = _lib.host().rope(0, q, k, cos, sin, mrope_section, layout, 0)
+        if made is not None:
+            ctx.save_for_backward(q, k, cos, sin)
+            ctx.mrope_section = tuple(mrope_section)
+            return made
         for name, t in (("q", q), ("k", k), ("cos", cos), ("sin", sin)):
             if t.is_cpu:
                 raise RuntimeError(f"[Error] The input `{name}` of multimodal_rope op is on the device: CPU!")
@@ -229,8 +245,7 @@ class MultimodalRoPE(torch.autograd.Function):
         k_out = torch.empty(k.shape, dtype=k.dtype, device=k.device)
         backend.rope(q, k, cos, sin, q_out, k_out, doubled, layout)
         ctx.save_for_backward(q, k, cos, sin)
-        ctx.mrope_section_doubled = doubled
-        ctx.layout = layout
+        ctx.mrope_section = tuple(int(v) for v in mrope_section)
         return q_out, k_out
 
     @staticmethod
@@ -239,13 +254,16 @@ class MultimodalRoPE(torch.autograd.Function):
         want_q, want_k = ctx.needs_input_grad[0], ctx.needs_input_grad[1]
         if not (want_q or want_k):
             return None, None, None, None, None, None
+        made = _lib.host().rope(0, grad_q_out, grad_k_out, cos, sin, ctx.mrope_section, ctx.layout, 1)
+        if made is not None:
+            return (made[0] if want_q else None), (made[1] if want_k else None), None, None, None, None
         gq = torch.empty(q.shape, dtype=q.dtype, device=q.device)
         gk = torch.empty(k.shape, dtype=k.dtype, device=k.device)
         if grad_q_out.stride(-1) != 1:
             grad_q_out = grad_q_out.contiguous()
         if grad_k_out.stride(-1) != 1:
             grad_k_out = grad_k_out.contiguous()
-        backend.rope_bwd(grad_q_out, grad_k_out, q, k, cos, sin, gq, gk, ctx.mrope_section_doubled, ctx.layout)
+        backend.rope_bwd(grad_q_out, grad_k_out, q, k, cos, sin, gq, gk, [2 * v for v in ctx.mrope_section], ctx.layout)
         return (gq if want_q else None), (gk if want_k else None), None, None, None, None
 
 
@@ -263,6 +281,12 @@ class MultimodalRoPEFromPositions(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, q, k, position_ids, inv_freq, mrope_section, layout="hf"):
+        ctx.layout = layout
+        made = _lib.host().rope(1, q, k, position_ids, inv_freq, mrope_section, layout, 0)
+        if made is not None:
+            ctx.save_for_backward(position_ids, inv_freq)
+            ctx.mrope_section = tuple(mrope_section)
+            return made
         for name, t in (("q", q), ("k", k), ("position_ids", position_ids), ("inv_freq", inv_freq)):
             if t.is_cpu:
                 raise RuntimeError(f"[Error] The input `{name}` of multimodal_rope op is on the device: CPU!")
@@ -280,8 +304,7 @@ class MultimodalRoPEFromPositions(torch.autograd.Function):
         k_out = torch.empty(k.shape, dtype=k.dtype, device=k.device)
         backend.rope_from_positions(q, k, position_ids, inv_freq, q_out, k_out, doubled, layout=layout)
         ctx.save_for_backward(position_ids, inv_freq)
-        ctx.mrope_section_doubled = doubled
-        ctx.layout = layout
+        ctx.mrope_section = tuple(int(v) for v in mrope_section)
         return q_out, k_out
 
     @staticmethod
@@ -290,6 +313,9 @@ class MultimodalRoPEFromPositions(torch.autograd.Function):
         want_q, want_k = ctx.needs_input_grad[0], ctx.needs_input_grad[1]
         if not (want_q or want_k):
             return None, None, None, None, None, None
+        made = _lib.host().rope(1, grad_q_out, grad_k_out, position_ids, inv_freq, ctx.mrope_section, ctx.layout, 1)
+        if made is not None:
+            return (made[0] if want_q else None), (made[1] if want_k else None), None, None, None, None
         if grad_q_out.stride(-1) != 1:
             grad_q_out = grad_q_out.contiguous()
         if grad_k_out.stride(-1) != 1:
@@ -297,7 +323,7 @@ class MultimodalRoPEFromPositions(torch.autograd.Function):
         gq = torch.empty(grad_q_out.shape, dtype=grad_q_out.dtype, device=grad_q_out.device)
         gk = torch.empty(grad_k_out.shape, dtype=grad_k_out.dtype, device=grad_k_out.device)
         backend.rope_from_positions(grad_q_out, grad_k_out, position_ids, inv_freq, gq, gk,
-                                    ctx.mrope_section_doubled, backward=True, layout=ctx.layout)
+                                    [2 * v for v in ctx.mrope_section], backward=True, layout=ctx.layout)
         return (gq if want_q else None), (gk if want_k else None), None, None, None, None
 
 
@@ -323,6 +349,12 @@ class MultimodalRoPEFromTable(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, q, k, table, mrope_section, layout="hf"):
+        ctx.layout = layout
+        made = _lib.host().rope(2, q, k, table, None, mrope_section, layout, 0)
+        if made is not None:
+            ctx.save_for_backward(table)
+            ctx.mrope_section = tuple(mrope_section)
+            return made
         for name, t in (("q", q), ("k", k), ("table", table)):
             if t.is_cpu:
                 raise RuntimeError(f"[Error] The input `{name}` of multimodal_rope op is on the device: CPU!")
@@ -339,8 +371,7 @@ class MultimodalRoPEFromTable(torch.autograd.Function):
         k_out = torch.empty(k.shape, dtype=k.dtype, device=k.device)
         backend.rope_from_table(q, k, table, q_out, k_out, doubled, layout=layout)
         ctx.save_for_backward(table)
-        ctx.mrope_section_doubled = doubled
-        ctx.layout = layout
+        ctx.mrope_section = tuple(int(v) for v in mrope_section)
         return q_out, k_out
 
     @staticmethod
@@ -349,13 +380,16 @@ class MultimodalRoPEFromTable(torch.autograd.Function):
         want_q, want_k = ctx.needs_input_grad[0], ctx.needs_input_grad[1]
         if not (want_q or want_k):
             return None, None, None, None, None
+        made = _lib.host().rope(2, grad_q_out, grad_k_out, table, None, ctx.mrope_section, ctx.layout, 1)
+        if made is not None:
+            return (made[0] if want_q else None), (made[1] if want_k else None), None, None, None
         if grad_q_out.stride(-1) != 1:
             grad_q_out = grad_q_out.contiguous()
         if grad_k_out.stride(-1) != 1:
             grad_k_out = grad_k_out.contiguous()
         gq = torch.empty(grad_q_out.shape, dtype=grad_q_out.dtype, device=grad_q_out.device)
         gk = torch.empty(grad_k_out.shape, dtype=grad_k_out.dtype, device=grad_k_out.device)
-        backend.rope_from_table(grad_q_out, grad_k_out, table, gq, gk, ctx.mrope_section_doubled, backward=True,
+        backend.rope_from_table(grad_q_out, grad_k_out, table, gq, gk, [2 * v for v in ctx.mrope_section], backward=True,
                                 layout=ctx.layout)
         return (gq if want_q else None), (gk if want_k else None), None, None, None
 

@@ -222,6 +222,10 @@ MAX_EXPERTS = 256
 def permute(input: torch.Tensor, indices: torch.Tensor, num_out_tokens: int, workspace: List[torch.Tensor],
             max_expanded_token_num: int) -> Tuple[torch.Tensor, torch.Tensor, List[torch.Tensor]]:
     """csrc/permute.cu:450-630: (permuted [num_out, H], row_id_map int32 [T*K], workspace)."""
+    if workspace and not _checked:
+        made = _lib.host().permute(input, indices, num_out_tokens, workspace[0], workspace[1], MAX_EXPERTS)
+        if made is not None:
+            return made[0], made[1], workspace
     _need_cuda("input", input)
     _need_cuda("indices", indices)
     if input.dim() != 2 or indices.dim() != 2:
