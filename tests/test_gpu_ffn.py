@@ -237,6 +237,58 @@ def test_fused_ffn_small(dev, T, n_act, hidden, inters):
     _close(y, ref32, atol=2 * ATOL, rtol=2 * RTOL, what="moe layer vs fp32 math")
 
 
+@pytest.mark.parametrize("m0,m1,inters", [
+    (769, 0, (11008, 1024)), (896, 0, (11008, 1024)), (897, 0, (11008, 1024)),  # a strip of 1 and of 128 rows, and no strip
+    (880, 32, (11008, 1024)),     # both experts end in one; behind three whole row blocks and in place of the only one
+    (899, 300, (11008, 1024)),    # the short expert alone
+    (2400, 13, (11008, 1024)),    # three whole rounds in front
+    (40, 880, (1024, 11040)),     # the other way round, with a ragged last column
+])
+def test_last_rows_of_an_expert_as_a_strip_of_small_tiles(dev, m0, m1, inters):
+    """Row blocks of at most 128 rows behind more than one round of large gate/up tiles go to the launch of small tiles.
+    Whole output against the oracle, with the split known on the device only and handed over from the host (right and
+    wrong)."""
+    T, hidden = m0 + m1, 128
+    g = torch.Generator().manual_seed(T)
+    x = _bf((T, hidden), g)
+    types = torch.zeros(T, dtype=torch.bool)
+    types[torch.randperm(T, generator=g)[:m1]] = True
+    ws = _moe_weights(hidden, inters, g, 0.05)
+    ref = oracle.sparse_moe_block_ref(x[None], types[None], [w.as_tuple() for w in ws])[0]
+    wd = [w.to(dev).as_tuple() for w in ws]
+    y, routing = moe.moe_layer_forward(x.to(dev), types.to(dev), wd)
+    _close(y, ref, what="device-side split")
+    for hint in ((m0, m1), (m1, m0), (T, 0)):
+        yh, _ = moe.moe_layer_forward(x.to(dev), types.to(dev), wd, routing=routing, host_rows=hint)
+        if hint == (m0, m1):
+            assert torch.equal(yh, y)
+        else:  # (the down launch's contraction is then whole where it is in parts: another order of its sums)
+            _close(yh, ref, what=f"host row counts {hint}")
+
+
+@pytest.mark.parametrize("trans_a,trans_b", [(False, False), (False, True), (True, False), (True, True)])
+@pytest.mark.parametrize("m0,m1,n", [(872, 0, 20736), (776, 104, 20736), (896, 8, 22016), (904, 40, 20480), (2400, 0, 22016)])
+def test_dual_gemm_with_a_strip_of_small_tiles(dev, trans_a, trans_b, m0, m1, n):
+    """The same of the row-major op, in every layout, with and without an addend (and in place on it)."""
+    g = torch.Generator(device=dev).manual_seed(m0 + m1)
+    k = 72
+
+    def operand(rows, cols, transposed):
+        return torch.randn((cols, rows) if transposed else (rows, cols), device=dev, generator=g).to(torch.bfloat16)
+
+    a, w = [operand(m, k, trans_a) for m in (m0, m1)], [operand(k, c, trans_b) for c in (n, 520)]
+    add = [torch.randn((m, c), device=dev, generator=g).to(torch.bfloat16) for m, c in ((m0, n), (m1, 520))]
+    out = [torch.full_like(t, float("nan")) for t in add]
+    native.asym_dual_gmm(a[0], a[1], w[0], w[1], out[0], out[1], trans_a, trans_b)
+    for got, x, y in zip(out, a, w):
+        x, y = (x.t() if trans_a else x).float(), (y.t() if trans_b else y).float()
+        # one rounding to bf16 (2^-9 of the value) and fp32 sums of k products
+        assert bool(((got.float() - x @ y).abs() <= 2 ** -8 * (x @ y).abs() + 1e-5 * (x.abs() @ y.abs())).all())
+    summed = [o + t for o, t in zip(out, add)]
+    native.asym_dual_gmm(a[0], a[1], w[0], w[1], add[0], add[1], trans_a, trans_b, add_expert0=add[0], add_expert1=add[1])
+    assert torch.equal(add[0], summed[0]) and torch.equal(add[1], summed[1])
+
+
 @pytest.mark.parametrize("T,n_act,hidden,inters", [
     (8600, 300, 2048, (1056, 256)),   # gate/up: 301 large tiles, 45 left over, among them a ragged last column
     (8600, 8300, 2048, (256, 1056)),  # the action expert is the long one

@@ -44,7 +44,9 @@ def _reference(x, w, b, pos, nq, nkv, rows=None, layout="hf"):
 
 @pytest.mark.parametrize("layout", ["hf", "csrc"])
 @pytest.mark.parametrize("B,S,H,nq,nkv,with_bias", [(2, 300, 512, 4, 2, True), (1, 37, 256, 2, 1, False),
-                                                   (3, 256, 1024, 3, 1, True), (1, 1, 64, 1, 1, True)])
+                                                   (3, 256, 1024, 3, 1, True), (1, 1, 64, 1, 1, True),
+                                                   # more than a round of large tiles; the last 104 rows are a strip of small ones
+                                                   (2, 436, 64, 160, 1, True)])
 def test_qkv_rope_projection(dev, B, S, H, nq, nkv, with_bias, layout):
     g = torch.Generator().manual_seed(B * 1000 + S)
     x = torch.randn(B, S, H, generator=g).to(torch.bfloat16)

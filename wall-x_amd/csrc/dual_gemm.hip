@@ -98,7 +98,7 @@ using BigTileQ = TileShape<256, 256, 4, 2, 4>;
 // The large tile of a launch.
 template <int MODE>
 using BigTileFor = std::conditional_t<MODE == 3 || MODE == 4 /* kQkvRope, kQkvRopeFull */, BigTileQ, BigTile>;
-// the shape that runs the ragged last round of a launch (see tail_split_point): BigTile cut in four.  (Cut in two,
+// the shape that runs the ragged last round of a launch (see tail_plan): BigTile cut in four.  (Cut in two,
 // 256 x 128 with one workgroup per CU, measures the same.)
 using TailTile = SmallTile;
 // ... and for the projection that rotates heads: four wavefronts as 4 x 1, wave tile 32 x 128, so that a wavefront
@@ -133,7 +133,7 @@ struct Params {
   // number of 256 x 256 tiles is on its side of `gate_tiles`.  0 = always run, 1 = run if at most gate_tiles,
   // 2 = run if more.
   int gate, gate_tiles;
-  // Tail split (see tail_split_point): 0 = off; 1 = this launch does the whole rounds of 256 x 256 tiles and leaves
+  // Tail split (see tail_plan): 0 = off; 1 = this launch does the whole rounds of 256 x 256 tiles and leaves
   // the ragged last round to a second launch; 2 = this is that second launch, with 128 x 128 tiles.
   // split_cus = workgroups of the first launch (one per CU).
   int split, split_cus;
@@ -243,6 +243,44 @@ __host__ __device__ inline int tail_split_point(int tiles0, int tiles1, int k0, 
   const int tail1 = tail < tiles1 ? tail : tiles1, tail0 = tail - tail1;
   const int counted = (tiles1 > 0 && tiles0 > 0 && 2ll * k1 <= k0) ? tail0 : tail;
   return 2 * counted <= cus ? full : total;
+}
+
+// The two launches of a problem of more than one round of large tiles: the split above, or one that leaves an expert's last
+// rows to the second launch where they are 128 at most (`strips`).  As large tiles such a row block is half padding, and its
+// tiles take part in the whole rounds like any other: 880 rows of an expert of 11008 are 344 large gate/up tiles, one round
+// and 88 left over that take 37 us as small ones, where three whole row blocks and a strip are one round, two large tiles
+// and 172 small ones: us a layer 158 -> 146, 2310 to 2400 rows 318 to 323 -> 307 to 311, 1656 rows 240 -> 230.
+// The rounds are counted in kTailRound-ths of a round of large tiles: kTailOne for a launch of small tiles with one to a CU,
+// kTailTwo with two (contractions of 2048, us: 47 to 53, 20, 37).
+struct TailPlan {
+  int rows[2];  // row blocks of 256 of each expert that are large tiles
+  int first;    // large tiles of the first launch
+  bool split;   // whether there is a second one
+};
+constexpr int kTailRound = 10, kTailOne = 4, kTailTwo = 8;
+__host__ __device__ inline TailPlan tail_plan(int m0, int m1, int cols0, int cols1, int k0, int k1, int cus, bool strips) {
+  TailPlan p;
+  p.rows[0] = (m0 + 255) >> 8;
+  p.rows[1] = (m1 + 255) >> 8;
+  const int tiles0 = p.rows[0] * cols0, tiles1 = p.rows[1] * cols1, total = tiles0 + tiles1;
+  p.first = tail_split_point(tiles0, tiles1, k0, k1, cus);
+  p.split = p.first != total;
+  // (experts whose tiles differ in length: the rule above, which does not count the short ones)
+  if (!strips || cus <= 0 || total <= cus || (tiles0 > 0 && tiles1 > 0 && (2ll * k1 <= k0 || 2ll * k0 <= k1))) return p;
+  const int strip0 = ((m0 - 1) & 255) < 128 && tiles0 > 0 ? 1 : 0, strip1 = ((m1 - 1) & 255) < 128 && tiles1 > 0 ? 1 : 0;
+  const int pieces = 2 * (strip0 * cols0 + strip1 * cols1);
+  if (pieces == 0) return p;
+  const int large = total - pieces / 2, full = large / cus, left = large - full * cus, whole = total / cus;
+  auto small = [&](int n) { return n <= 0 ? 0 : (n <= cus ? kTailOne : (n <= 2 * cus ? kTailTwo : 4 * kTailRound)); };
+  const int as_is = whole * kTailRound + (p.split ? small(4 * (total - p.first)) : (total > whole * cus ? kTailRound : 0));
+  const int both = full > 0 ? full * kTailRound + small(4 * left + pieces) : as_is;  // strips and what the whole rounds leave
+  const int alone = (full + (left > 0 ? 1 : 0)) * kTailRound + small(pieces);       // strips alone
+  if (both >= as_is && alone >= as_is) return p;
+  p.rows[0] -= strip0;
+  p.rows[1] -= strip1;
+  p.first = both <= alone ? full * cus : large;
+  p.split = true;
+  return p;
 }
 
 // The tile count that decides between the two tile shapes.  The small shape pays when the large tiles would leave
@@ -1073,26 +1111,35 @@ __device__ __forceinline__ void dual_gemm_body(const Params& p, const int wg, co
     tiles_n[1] <<= lg_of(1);
   }
   int total = tiles_m[0] * tiles_n[0] + tiles_m[1] * tiles_n[1];  // the host bounds this below 2^31
-  // tail split: the first launch (256 x 256 tiles) stops at `split_at`; the second (this shape: 128 x 128)
-  // takes virtual tiles [split_at, all) of the 256 x 256 tiling, kSubM x kSubN pieces each
+  // tail split (tail_plan): the first launch (256 x 256 tiles) stops at `split_at`; the second (this shape: 128 x 128)
+  // takes virtual tiles [split_at, all) of the 256 x 256 tiling, kSubM x kSubN pieces each, and then the strips
   constexpr bool kIsTail = std::is_same_v<TS, TailTileFor<MODE>>, kIsBig = std::is_same_v<TS, BigTileFor<MODE>>;
   constexpr int kSubM = BigTile::BM / BM, kSubN = BigTile::BN / BN;
-  int big_m[2], big_n[2], split_at = 0, pieces = 0;
+  int big_m[2], big_n[2], split_at = 0, pieces = 0, strip_cols[2] = {0, 0};
   if (ROLE != 3 && ((kIsBig && p.split == 1) || (kIsTail && p.split == 2))) {
     constexpr int kBigN = SWIGLU ? BigTile::BN / 2 : BigTile::BN;
-    big_m[0] = (g0.m + BigTile::BM - 1) / BigTile::BM;
     big_n[0] = (g0.n + kBigN - 1) / kBigN;
-    if (g0.m <= 0 || g0.n <= 0) big_m[0] = big_n[0] = 0;
-    big_m[1] = (g1.m + BigTile::BM - 1) / BigTile::BM;
     big_n[1] = (g1.n + kBigN - 1) / kBigN;
-    if (g1.m <= 0 || g1.n <= 0) big_m[1] = big_n[1] = 0;
-    const int all = big_m[0] * big_n[0] + big_m[1] * big_n[1];
-    split_at = tail_split_point(big_m[0] * big_n[0], big_m[1] * big_n[1], g0.k, g1.k, p.split_cus);
+    const bool any0 = g0.m > 0 && g0.n > 0, any1 = g1.m > 0 && g1.n > 0;
+    const TailPlan plan = tail_plan(any0 ? g0.m : 0, any1 ? g1.m : 0, any0 ? big_n[0] : 0, any1 ? big_n[1] : 0, g0.k, g1.k, p.split_cus, MODE != kDown);
+    if (!any0) big_n[0] = 0;
+    if (!any1) big_n[1] = 0;
+    big_m[0] = plan.rows[0];
+    big_m[1] = plan.rows[1];
+    split_at = plan.first;
     if constexpr (kIsBig) {
-      total = split_at;  // a multiple of 8 when smaller than `all`
+      total = split_at;
+      if (MODE != kDown) {
+        tiles_m[0] = big_m[0];
+        tiles_m[1] = big_m[1];
+      }
     } else {
-      if (split_at == all) return;  // no split: the first launch did everything
-      pieces = kSubM * kSubN * (all - split_at);
+      if (!plan.split) return;  // the first launch did everything
+      pieces = kSubM * kSubN * (big_m[0] * big_n[0] + big_m[1] * big_n[1] - split_at);
+      if (MODE != kDown) {  // strips: the row of small tiles behind an expert's large ones
+        strip_cols[0] = kSubM * big_m[0] < tiles_m[0] ? tiles_n[0] : 0;
+        strip_cols[1] = kSubM * big_m[1] < tiles_m[1] ? tiles_n[1] : 0;
+      }
     }
   }
   const int padded = (total + kXcds - 1) / kXcds * kXcds;
@@ -2021,6 +2068,14 @@ __device__ __forceinline__ void dual_gemm_body(const Params& p, const int wg, co
         // pieces past a ragged last row / column of tiles are empty
         have = tc.tm < (tc.group ? tiles_m[1] : tiles_m[0]) && tc.tn < (tc.group ? tiles_n[1] : tiles_n[0]);
       }
+      if (MODE != kDown && !have && next_t < pieces + strip_cols[0] + strip_cols[1]) {
+        const int at = next_t - pieces;
+        tc.group = at >= strip_cols[0] ? 1 : 0;
+        tc.tm = kSubM * (tc.group ? big_m[1] : big_m[0]);
+        tc.tn = tc.group ? at - strip_cols[0] : at;
+        next_t += n_wg;
+        have = true;
+      }
       return have;
     }
     for (; next_t < padded && !have; next_t += n_wg) have = map_tile(next_t, total, tiles_m, tiles_n, tc);
@@ -2358,9 +2413,12 @@ int check_dims(const char* who, int64_t m, int64_t n, int64_t k, bool k_in_rows 
 // second returns at once if there is nothing to split).
 // few: the few-rows form takes the problem; its number of rows, or 0.
 // parts: the down launch's contraction may be in parts (PartsRule), with this scratch.
+int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
+
 template <int MODE, bool KA = false, bool KB = false>
 int launch_mfma(Params p, int64_t tiles_lo, int64_t tiles_hi, hipStream_t s, const char* who,
-                const int64_t* tiles_by_expert = nullptr, int64_t few = 0, const DownSplit* parts = nullptr) {
+                const int64_t* tiles_by_expert = nullptr, int64_t few = 0, const DownSplit* parts = nullptr,
+                const int64_t* rows = nullptr) {
   const int cus = device_cu_count();
   const int threshold = cus / 2;
   if constexpr (MODE == kGateUp || MODE == kDown) {
@@ -2400,8 +2458,14 @@ int launch_mfma(Params p, int64_t tiles_lo, int64_t tiles_hi, hipStream_t s, con
     bool split = (MODE != kGeneric || tiles_by_expert != nullptr) && tiles_hi > cus;
     if (split && tiles_by_expert != nullptr) {
       const int64_t all = tiles_by_expert[0] + tiles_by_expert[1];
-      split = all < INT32_MAX && tail_split_point(static_cast<int>(tiles_by_expert[0]), static_cast<int>(tiles_by_expert[1]),
-                                                  p.g[0].k, p.g[1].k, cus) != all;
+      if (all >= INT32_MAX) {
+        split = false;
+      } else if (rows != nullptr) {
+        auto cols = [&](int e) { return rows[e] > 0 ? static_cast<int>(tiles_by_expert[e] / ceil_div(rows[e], BigTile::BM)) : 0; };
+        split = tail_plan(static_cast<int>(rows[0]), static_cast<int>(rows[1]), cols(0), cols(1), p.g[0].k, p.g[1].k, cus, true).split;
+      } else {
+        split = tail_split_point(static_cast<int>(tiles_by_expert[0]), static_cast<int>(tiles_by_expert[1]), p.g[0].k, p.g[1].k, cus) != all;
+      }
     }
     p.split = split ? 1 : 0;
     if (MODE == kDown && parts != nullptr)
@@ -2416,8 +2480,6 @@ int launch_mfma(Params p, int64_t tiles_lo, int64_t tiles_hi, hipStream_t s, con
   }
   return check_launch(who);
 }
-
-int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
 }  // namespace
 }  // namespace wx
@@ -2517,10 +2579,11 @@ int dual_gemm_impl(const void* in0, const void* in1, const void* w0, const void*
     // (the host knows both problems' sizes: it settles the tile shape and the split of a ragged last round itself)
     const int64_t by_expert[2] = {ceil_div(mm0, BigTile::BM) * ceil_div(n0, BigTile::BN),
                                   ceil_div(mm1, BigTile::BM) * ceil_div(n1, BigTile::BN)};
-    if (!trans_a && trans_b) return launch_mfma<kGeneric, false, false>(p, tiles, tiles, s, who, by_expert);
-    if (!trans_a && !trans_b) return launch_mfma<kGeneric, false, true>(p, tiles, tiles, s, who, by_expert);
-    if (trans_a && trans_b) return launch_mfma<kGeneric, true, false>(p, tiles, tiles, s, who, by_expert);
-    return launch_mfma<kGeneric, true, true>(p, tiles, tiles, s, who, by_expert);
+    const int64_t by_rows[2] = {n0 > 0 ? mm0 : 0, n1 > 0 ? mm1 : 0};
+    if (!trans_a && trans_b) return launch_mfma<kGeneric, false, false>(p, tiles, tiles, s, who, by_expert, 0, nullptr, by_rows);
+    if (!trans_a && !trans_b) return launch_mfma<kGeneric, false, true>(p, tiles, tiles, s, who, by_expert, 0, nullptr, by_rows);
+    if (trans_a && trans_b) return launch_mfma<kGeneric, true, false>(p, tiles, tiles, s, who, by_expert, 0, nullptr, by_rows);
+    return launch_mfma<kGeneric, true, true>(p, tiles, tiles, s, who, by_expert, 0, nullptr, by_rows);
   }
   gemm_path_note(WX_GEMM_PATH_FMA);
   hipLaunchKernelGGL(dual_gemm_reference_layout_kernel, dim3(device_cu_count() * 4), dim3(256), 0, s, p, trans_a, trans_b);
@@ -2560,7 +2623,7 @@ extern "C" int wx_qkv_rope_proj(const void* x, const void* weight, const void* b
   p.rope_cols = (n_q_heads + n_kv_heads) * head_dim;
   p.rope_width = table_width;
   // Tiles whose wavefronts cover whole heads only (a 64-column wave tile would split a rotation pair): the large
-  // tile, and for a ragged last round (see tail_split_point) a second launch of 128 x 128 tiles with 32 x 128 wave tiles
+  // tile, and for a ragged last round (see tail_plan) a second launch of 128 x 128 tiles with 32 x 128 wave tiles
   using Tile = BigTileFor<kQkvRope>;
   using Tail = TailTileFor<kQkvRope>;
   const int cus = device_cu_count();
@@ -2569,7 +2632,7 @@ extern "C" int wx_qkv_rope_proj(const void* x, const void* weight, const void* b
   // The table, this launch and the o projection at n 2560, k 2048: 32 rows 66 -> 45 us, 1024 rows 70 -> 48, 2048 rows
   // 73 -> 63, 3072 rows 83 -> 76; one more row of large tiles is past the line.
   const bool small = tiles <= cus / 2;
-  const bool split = !small && tiles < INT32_MAX && tail_split_point(static_cast<int>(tiles), 0, g.k, 0, cus) != tiles;
+  const bool split = !small && tiles < INT32_MAX && tail_plan(g.m, 0, static_cast<int>(ceil_div(g.n, Tile::BN)), 0, g.k, 0, cus, true).split;
   p.split = split ? 1 : 0;
   p.split_cus = cus;
   hipStream_t s = as_stream(stream);
@@ -2693,7 +2756,7 @@ int launch_gate_up(const FfnArgs& a, hipStream_t s) {
   if (a.host_rows != nullptr) {  // the caller knows the split: one launch of the right tile shape
     const int64_t by_expert[2] = {ceil_div(a.host_rows[0], BigTile::BM) * t0, ceil_div(a.host_rows[1], BigTile::BM) * t1};
     const int64_t tiles = by_expert[0] + by_expert[1];
-    return launch_mfma<kGateUp>(p, tiles, tiles, s, "dual_gemm_kernel<gate_up>", by_expert, few_rows_of(a));
+    return launch_mfma<kGateUp>(p, tiles, tiles, s, "dual_gemm_kernel<gate_up>", by_expert, few_rows_of(a), nullptr, a.host_rows);
   }
   // the split of the rows between the experts is only known on the device: bound the tile count from the total
   const int64_t row_tiles = ceil_div(a.rows, BigTile::BM);
