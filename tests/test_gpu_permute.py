@@ -21,7 +21,7 @@ def _quiet(fn, *a, **k):
 @pytest.mark.parametrize("T,E,K,dtype", [
     (1, 2, 1, torch.bfloat16), (63, 2, 1, torch.float32), (64, 2, 1, torch.float16), (65, 2, 1, torch.bfloat16),
     (513, 3, 1, torch.bfloat16), (4096, 2, 1, torch.bfloat16), (1000, 4, 2, torch.float32),
-    (777, 8, 3, torch.bfloat16), (2049, 200, 1, torch.float16),
+    (777, 8, 3, torch.bfloat16), (2049, 200, 1, torch.float16), (4133, 9, 5, torch.bfloat16), (3000, 256, 2, torch.float16),
 ])
 def test_permute_unpermute_small(dev, T, E, K, dtype):
     g = torch.Generator().manual_seed(T + E + K)
@@ -199,6 +199,8 @@ def test_permute_autograd_and_unpermute_backward(dev):
 @pytest.mark.parametrize("T,K,R,H,dtype", [
     (1, 1, 1, 8, torch.bfloat16), (65, 1, 400, 72, torch.float16), (700, 1, 500, 2048, torch.bfloat16),
     (130, 3, 129, 520, torch.float32), (513, 2, 70001, 32, torch.bfloat16), (9, 1, 4194433, 8, torch.bfloat16),
+    # the copies' groups: two, four, and four and one; whole chunks of a row and a remainder; a map of fewer than four entries
+    (200, 2, 500, 2056, torch.bfloat16), (130, 4, 600, 2048, torch.float16), (77, 5, 400, 520, torch.bfloat16), (1, 3, 40, 2048, torch.float32),
 ])
 def test_unpermute_backward_clears_the_rows_without_a_token(dev, T, K, R, H, dtype):
     """A map that leaves rows out (and drops some of the tokens), into memory that held something else before: the rows it

@@ -8,6 +8,7 @@
 //   pass 2  partition_scatter  per-block prefix over hist (bins, then earlier segments), then ranks
 // The row movers are pure HBM streams: one wavefront per token row, 16-byte lanes, several rows in flight.
 #include <mutex>
+#include <type_traits>
 
 #include "common.h"
 #include "tiled_layout.h"
@@ -35,9 +36,10 @@ __device__ __forceinline__ int load_key(const void* ids, int itype, int64_t i, i
 
 // The keys of kAhead groups of 64 from `base` on (a lane past `end` holds 0).  They are asked for together: a wavefront that
 // loads one group at a time waits out a memory latency per group: partition_count of 14593 int32 keys 7.6 -> 5.6 us.  (Not in
-// the two kernels that rank: partition_scatter, which waits for its sums over the histograms first, takes 9.1 us either way, and
-// a wavefront of partition_small_kernel has a few groups only and lost 4 us on 1424 keys.)
+// partition_small_kernel: its wavefronts have a few groups only and lost 4 us on 1424 keys.)
 constexpr int kAhead = 8;
+constexpr int kHistAhead = 32;  // histograms
+static_assert(kHistAhead % kWavesPerBlock == 0, "a block's segments lie in one trip");
 __device__ __forceinline__ void load_keys(const void* ids, int itype, int64_t base, int64_t end, int num_experts, int (&key)[kAhead],
                                           bool& bad) {
   const int64_t first = base + lane_id();
@@ -48,17 +50,30 @@ __device__ __forceinline__ void load_keys(const void* ids, int itype, int64_t ba
   }
 }
 
-// Calls f(key, mask) once per distinct key among the active lanes; mask = lanes holding that key.
-template <typename F>
-__device__ __forceinline__ void for_each_key_group(int key, bool active, F f) {
-  uint64_t todo = __ballot(active);
+// The active lanes that hold this lane's key (none for a lane that is not active).
+__device__ __forceinline__ uint64_t lanes_of_key(int key, bool active) {
+  uint64_t todo = __ballot(active), mine = 0;
   while (todo) {
     const int leader = __ffsll(static_cast<long long>(todo)) - 1;
     const int k = __builtin_amdgcn_readlane(key, leader);
     const uint64_t mask = __ballot(active && key == k);
-    f(k, mask);
+    if (key == k) mine = mask;
     todo &= ~mask;
   }
+  return active ? mine : 0;
+}
+// Adds a group of 64 keys to the wavefront's counts `bins`, one read and one write of LDS for all its keys (with a read and a write per
+// key, one after the other, 24000 keys of eight experts took 9.7 us to count and 15.8 to rank, now 7.3 and 12), and returns this lane's place: its key's count before the group plus
+// the lanes of that key below it.
+__device__ __forceinline__ int32_t count_keys(int32_t* bins, int key, bool active) {
+  const uint64_t mine = lanes_of_key(key, active);
+  const int below = __popcll(mine & ((1ull << lane_id()) - 1ull));
+  int32_t start = 0;
+  if (active) start = bins[key];
+  __builtin_amdgcn_wave_barrier();
+  if (active && below == 0) bins[key] = start + __popcll(mine);
+  __builtin_amdgcn_wave_barrier();
+  return start + below;
 }
 
 __global__ __launch_bounds__(kBlock) void partition_count(const void* __restrict__ ids, int itype, int64_t n,
@@ -76,9 +91,7 @@ __global__ __launch_bounds__(kBlock) void partition_count(const void* __restrict
     load_keys(ids, itype, base, end, num_experts, key, bad);
 #pragma unroll
     for (int u = 0; u < kAhead; ++u) {
-      for_each_key_group(key[u], base + u * kWave + lane < end, [&](int k, uint64_t mask) {
-        if (lane == 0) s_hist[w][k] += __popcll(mask);
-      });
+      count_keys(s_hist[w], key[u], base + u * kWave + lane < end);
     }
   }
   if (begin < n) {
@@ -99,23 +112,24 @@ __global__ __launch_bounds__(kBlock) void partition_scatter(
   const int64_t first_seg = static_cast<int64_t>(blockIdx.x) * kWavesPerBlock;
 
   // bin `tid`: rows of this bin in all segments (total) and in segments before this block (before)
-  // (eight independent loads per trip: with one load per trip the loop costs a memory latency per segment)
-  int32_t total = 0, before = 0;
-  int64_t s = 0;
-  for (; s + 8 <= num_seg; s += 8) {
-    int32_t v[8];
+  // (kHistAhead independent loads per trip, a memory latency each trip, and ahead of them the keys, which are wanted next)
+  const int64_t seg = first_seg + w;
+  const int64_t begin = seg * seg_len;
+  const int64_t end = begin + seg_len < n ? begin + seg_len : n;
+  bool bad = false;
+  int key[kAhead];
+  load_keys(ids, itype, begin, end, num_experts, key, bad);
+  int32_t total = 0, before = 0, own[kWavesPerBlock] = {0};
+  for (int64_t s = 0; s < num_seg; s += kHistAhead) {
+    int32_t v[kHistAhead];
 #pragma unroll
-    for (int u = 0; u < 8; ++u) v[u] = hist[(s + u) * kBins + tid];
+    for (int u = 0; u < kHistAhead; ++u) v[u] = s + u < num_seg ? hist[(s + u) * kBins + tid] : 0;
 #pragma unroll
-    for (int u = 0; u < 8; ++u) {
+    for (int u = 0; u < kHistAhead; ++u) {
       total += v[u];
       if (s + u < first_seg) before += v[u];
+      if (s + u - u % kWavesPerBlock == first_seg) own[u % kWavesPerBlock] = v[u];  // (the segments of this block)
     }
-  }
-  for (; s < num_seg; ++s) {
-    const int32_t v = hist[s * kBins + tid];
-    total += v;
-    if (s < first_seg) before += v;
   }
   // exclusive prefix of `total` over the 256 bins: wave scan, then wave totals through LDS
   int32_t incl = total;
@@ -136,31 +150,22 @@ __global__ __launch_bounds__(kBlock) void partition_scatter(
 #pragma unroll
   for (int i = 0; i < kWavesPerBlock; ++i) {
     s_run[i][tid] = run;
-    if (first_seg + i < num_seg) run += hist[(first_seg + i) * kBins + tid];
+    run += own[i];
   }
   __syncthreads();
 
-  const int64_t seg = first_seg + w;
-  const int64_t begin = seg * seg_len;
-  const int64_t end = begin + seg_len < n ? begin + seg_len : n;
-  const uint64_t below = (1ull << lane) - 1ull;
-  bool bad = false;
-  for (int64_t base = begin; base < end; base += kWave) {
-    const int64_t i = base + lane;
-    const bool active = i < end;
-    const int key = active ? load_key(ids, itype, i, num_experts, bad) : 0;
-    int32_t pos = 0;
-    for_each_key_group(key, active, [&](int k, uint64_t mask) {
-      const int32_t start = s_run[w][k];  // same address for the whole wave: LDS broadcast
-      if (active && key == k) pos = start + __popcll(mask & below);
-      __builtin_amdgcn_wave_barrier();
-      if (lane == 0) s_run[w][k] = start + __popcll(mask);
-      __builtin_amdgcn_wave_barrier();
-    });
-    if (active) {
-      const int64_t t = i / num_topk, k = i - t * num_topk;
-      row_id_map[k * num_tokens + t] = pos < num_out ? pos : -1;
-      if (sorted_row_id != nullptr) sorted_row_id[pos] = static_cast<int32_t>(i);
+  for (int64_t base = begin; base < end; base += kAhead * kWave) {
+    if (base > begin) load_keys(ids, itype, base, end, num_experts, key, bad);
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) {
+      const int64_t i = base + u * kWave + lane;
+      const bool active = i < end;
+      const int32_t pos = count_keys(s_run[w], key[u], active);
+      if (active) {
+        const int64_t t = i / num_topk, k = i - t * num_topk;
+        row_id_map[k * num_tokens + t] = pos < num_out ? pos : -1;
+        if (sorted_row_id != nullptr) sorted_row_id[pos] = static_cast<int32_t>(i);
+      }
     }
   }
 }
@@ -192,9 +197,7 @@ __global__ __launch_bounds__(kSmallWaves* kWave) void partition_small_kernel(
     const int64_t i = base + lane;
     const bool active = i < end;
     const int key = active ? load_key(ids, itype, i, num_experts, bad) : 0;
-    for_each_key_group(key, active, [&](int k, uint64_t mask) {
-      if (lane == 0) s_run[w][k] += __popcll(mask);
-    });
+    count_keys(s_run[w], key, active);
   }
   if (status != nullptr && __ballot(bad) != 0 && lane == 0) *status = 1;
   __syncthreads();
@@ -225,19 +228,11 @@ __global__ __launch_bounds__(kSmallWaves* kWave) void partition_small_kernel(
     }
   }
   __syncthreads();
-  const uint64_t below = (1ull << lane) - 1ull;
   for (int64_t base = begin; base < end; base += kWave) {
     const int64_t i = base + lane;
     const bool active = i < end;
     const int key = active ? load_key(ids, itype, i, num_experts, bad) : 0;
-    int32_t pos = 0;
-    for_each_key_group(key, active, [&](int k, uint64_t mask) {
-      const int32_t start = s_run[w][k];  // same address for the whole wave: LDS broadcast
-      if (active && key == k) pos = start + __popcll(mask & below);
-      __builtin_amdgcn_wave_barrier();
-      if (lane == 0) s_run[w][k] = start + __popcll(mask);
-      __builtin_amdgcn_wave_barrier();
-    });
+    const int32_t pos = count_keys(s_run[w], key, active);
     if (active) {
       const int64_t t = i / num_topk, k = i - t * num_topk;
       row_id_map[k * num_tokens + t] = pos < num_out ? pos : -1;
@@ -248,9 +243,19 @@ __global__ __launch_bounds__(kSmallWaves* kWave) void partition_small_kernel(
 
 // ---- row movers ---------------------------------------------------------------------------------
 constexpr int kMoverWaves = 4;
+constexpr int kMoverPlaces = 8;  // wavefronts per SIMD that the grids count on
 
 __device__ __forceinline__ u32x4 ld16(const u32x4* p) { return __builtin_nontemporal_load(p); }
 __device__ __forceinline__ void st16(u32x4* p, const u32x4& v) { __builtin_nontemporal_store(v, p); }
+
+// f(v, N) for this lane's 16-byte chunks v, v + 64, .. (N of them) of a row: MOST at a time while there are so many, for their
+// loads to be in flight together.
+template <int MOST, typename F>
+__device__ __forceinline__ void chunks_of_a_row(int lane, int64_t vec_per_row, F f) {
+  int64_t v = lane;
+  for (; v + (MOST - 1) * kWave < vec_per_row; v += MOST * kWave) f(v, std::integral_constant<int, MOST>{});
+  for (; v < vec_per_row; v += kWave) f(v, std::integral_constant<int, 1>{});
+}
 
 // out[row_id_map[k*T + t]] = x[t] for every k; one wavefront per source row.
 __global__ __launch_bounds__(kMoverWaves* kWave) void permute_rows_kernel(
@@ -273,13 +278,19 @@ __global__ __launch_bounds__(kMoverWaves* kWave) void permute_rows_kernel(
       }
       for (; v < vec_per_row; v += kWave) st16(dst + v, ld16(src + v));
     } else {
-      for (int64_t v = lane; v < vec_per_row; v += kWave) {
-        const u32x4 a = ld16(src + v);
+      chunks_of_a_row<4>(lane, vec_per_row, [&](int64_t v, auto n) {
+        constexpr int N = decltype(n)::value;
+        u32x4 a[N];
+#pragma unroll
+        for (int u = 0; u < N; ++u) a[u] = ld16(src + v + u * kWave);
         for (int k = 0; k < num_topk; ++k) {
           const int32_t dst_row = row_id_map[k * num_tokens + t];
-          if (dst_row >= 0) st16(out + static_cast<int64_t>(dst_row) * vec_per_row + v, a);
+          if (dst_row < 0) continue;
+          u32x4* dst = out + static_cast<int64_t>(dst_row) * vec_per_row + v;
+#pragma unroll
+          for (int u = 0; u < N; ++u) st16(dst + u * kWave, a[u]);
         }
-      }
+      });
     }
   }
 }
@@ -444,7 +455,8 @@ __global__ __launch_bounds__(kMoverWaves* kWave) void gather_rows_kernel(
   }
 }
 
-// out[t] = sum_k prob[t,k] * y[row_id_map[k*T+t]] for topK > 1.  The reference kernel multiplies and
+// out[t] = sum_k prob[t,k] * y[row_id_map[k*T+t]] for topK > 1 (a row's chunks four at a time: 8000 tokens, two copies in bf16
+// 21.1 -> 17.5 us, three in fp32 49 -> 45; the scatter of their rows 23.2 -> 18.5, 52 -> 49).  The reference kernel multiplies and
 // accumulates in the storage type (csrc/permute.cu:69-154 with TCompute == T for 16-bit types), one
 // rounding per operation in k order; Elem<DT>::round reproduces that.
 template <int DT>
@@ -456,35 +468,49 @@ __global__ __launch_bounds__(kMoverWaves* kWave) void combine_rows_kernel(
   const int64_t wave = static_cast<int64_t>(blockIdx.x) * kMoverWaves + threadIdx.x / kWave;
   const int64_t n_waves = static_cast<int64_t>(gridDim.x) * kMoverWaves;
   for (int64_t t = wave; t < num_tokens; t += n_waves) {
-    for (int64_t v = lane; v < vec_per_row; v += kWave) {
-      float acc[E];
+    chunks_of_a_row<4>(lane, vec_per_row, [&](int64_t v, auto n) {
+      constexpr int N = decltype(n)::value;
+      float acc[N][E];
 #pragma unroll
-      for (int e = 0; e < E; ++e) acc[e] = 0.f;
+      for (int u = 0; u < N; ++u)
+#pragma unroll
+        for (int e = 0; e < E; ++e) acc[u][e] = 0.f;
       for (int k = 0; k < num_topk; ++k) {
         const int32_t r = row_id_map[k * num_tokens + t];
         if (r < 0) continue;  // a dropped copy adds nothing (for k == 0 the sum starts at zero)
-        float f[E];
-        unpack16<DT>(ld16(y + static_cast<int64_t>(r) * vec_per_row + v), f);
+        u32x4 raw[N];
+#pragma unroll
+        for (int u = 0; u < N; ++u) raw[u] = ld16(y + static_cast<int64_t>(r) * vec_per_row + v + u * kWave);
         const float p = probs != nullptr ? Elem<DT>::round(probs[t * num_topk + k]) : 1.f;
 #pragma unroll
-        for (int e = 0; e < E; ++e) {
-          const float term = probs != nullptr ? Elem<DT>::round(f[e] * p) : f[e];
-          acc[e] = k == 0 ? term : Elem<DT>::round(acc[e] + term);
+        for (int u = 0; u < N; ++u) {
+          float f[E];
+          unpack16<DT>(raw[u], f);
+#pragma unroll
+          for (int e = 0; e < E; ++e) {
+            const float term = probs != nullptr ? Elem<DT>::round(f[e] * p) : f[e];
+            acc[u][e] = k == 0 ? term : Elem<DT>::round(acc[u][e] + term);
+          }
         }
       }
-      st16(out + t * vec_per_row + v, pack16<DT>(acc));
-    }
+#pragma unroll
+      for (int u = 0; u < N; ++u) st16(out + t * vec_per_row + v + u * kWave, pack16<DT>(acc[u]));
+    });
   }
 }
 
-// Backward of the weighted combine; one wavefront per token.  The rows of act_grad that no token maps to are zeros: the
+// Backward of the weighted combine; one wavefront per token.  (With the copies one after the other and their gradient's row read
+// for each: 8000 tokens of 2048, us, two copies in bf16 39.0 -> 32.8, three in fp32 110 -> 90.)  The rows of act_grad that no token maps to are zeros: the
 // first `clearers` workgroups find them in their share of the num_rows rows by reading the whole map into a bitmap in LDS, and
 // clear them, beside the workgroups that move rows.  (Clearing all of act_grad in a launch of its own ahead of this one
-// writes every row twice: 14593 rows of 4 KiB 10.4 us + 25.5 -> 28.8.)  No share when clearers is 0.
+// writes every row twice: 14593 rows of 4 KiB 10.4 us + 25.5.)  The search must not take longer than the moving: with 64-bit
+// compares, a remainder of its own and a look at each row's bit those rows took 28 us and 29184 of them 51.6, now 22.7 and 42.
+// No share when clearers is 0.
 typedef int32_t i32x4_word __attribute__((ext_vector_type(4), aligned(4)));  // four entries at any entry's address
 constexpr int kClearRows = 65536;  // rows of act_grad one workgroup looks after at a time: 8 KiB of bits
-template <int DT>
-__global__ __launch_bounds__(kMoverWaves* kWave) void combine_rows_bwd_kernel(
+// COPIES: copies of a token handled together (its gradient's row is read once for all of them); 0 = rows without weights.
+template <int DT, int COPIES>
+__global__ __launch_bounds__(kMoverWaves* kWave, COPIES == 0 ? kMoverPlaces : 5) void combine_rows_bwd_kernel(
     const u32x4* __restrict__ grad_out, const u32x4* __restrict__ y_fwd, u32x4* __restrict__ act_grad,
     float* __restrict__ prob_grad, const int32_t* __restrict__ row_id_map, const float* __restrict__ probs,
     int64_t num_tokens, int num_topk, int64_t vec_per_row, int64_t num_rows, int clearers) {
@@ -499,79 +525,101 @@ __global__ __launch_bounds__(kMoverWaves* kWave) void combine_rows_bwd_kernel(
       const int rows = static_cast<int>(last - r0 < kClearRows ? last - r0 : kClearRows);
       for (int i = threadIdx.x; i < (rows + 31) / 32; i += kMoverWaves * kWave) s_mapped[i] = 0;
       __syncthreads();
-      // (32 entries per thread and trip, all asked for together: beside the movers a load is back after 2 - 3 us)
+      // (32 entries per thread and trip, all asked for together: beside the movers a load is back after 2 - 3 us.  Threads past the
+      // end mark the last entries once more.)
       constexpr int kLoads = 8, kTrip = kLoads * 4 * kMoverWaves * kWave;
       auto mark = [&](int32_t entry) {
-        const int64_t r = entry - r0;
-        if (r >= 0 && r < rows) atomicOr(&s_mapped[r >> 5], 1u << (r & 31));
+        const uint32_t r = static_cast<uint32_t>(entry) - static_cast<uint32_t>(r0);
+        if (r < static_cast<uint32_t>(rows)) atomicOr(&s_mapped[r >> 5], 1u << (r & 31));
       };
-      int64_t i = 4 * threadIdx.x;
-      for (; i + (kTrip - 4 * kMoverWaves * kWave) + 4 <= n; i += kTrip) {
-        i32x4_word e[kLoads];
+      if (n < 4) {
+        if (threadIdx.x < n) mark(row_id_map[threadIdx.x]);
+      } else {
+        const uint32_t last4 = static_cast<uint32_t>(n - 4);
+        for (uint32_t i = 4 * threadIdx.x; i < n; i += kTrip) {
+          i32x4_word e[kLoads];
 #pragma unroll
-        for (int u = 0; u < kLoads; ++u) e[u] = *reinterpret_cast<const i32x4_word*>(row_id_map + i + u * 4 * kMoverWaves * kWave);
+          for (int u = 0; u < kLoads; ++u) {
+            const uint32_t at = i + u * 4 * kMoverWaves * kWave;
+            e[u] = *reinterpret_cast<const i32x4_word*>(row_id_map + (at < last4 ? at : last4));
+          }
 #pragma unroll
-        for (int u = 0; u < kLoads; ++u)
+          for (int u = 0; u < kLoads; ++u)
 #pragma unroll
-          for (int c = 0; c < 4; ++c) mark(e[u][c]);
-      }
-      i32x4_word e[kLoads];
-#pragma unroll
-      for (int u = 0; u < kLoads; ++u)
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-          const int64_t at = i + u * 4 * kMoverWaves * kWave + c;
-          e[u][c] = at < n ? row_id_map[at] : -1;
+            for (int c = 0; c < 4; ++c) mark(e[u][c]);
         }
-#pragma unroll
-      for (int u = 0; u < kLoads; ++u)
-#pragma unroll
-        for (int c = 0; c < 4; ++c) mark(e[u][c]);
+      }
       __syncthreads();
-      for (int i = threadIdx.x / kWave; i < rows; i += kMoverWaves)
-        if (!(s_mapped[i >> 5] >> (i & 31) & 1))
-          for (int64_t v = lane; v < vec_per_row; v += kWave) st16(act_grad + (r0 + i) * vec_per_row + v, u32x4{0, 0, 0, 0});
+      // 32 rows at a time, hardly ever one of them to clear
+      for (int i = threadIdx.x / kWave; i < (rows + 31) / 32; i += kMoverWaves) {
+        uint32_t clear = ~s_mapped[i] & (rows - 32 * i < 32 ? (1u << (rows - 32 * i)) - 1u : ~0u);
+        clear = __builtin_amdgcn_readfirstlane(clear);
+        while (clear != 0) {
+          const int r = 32 * i + __ffs(static_cast<int>(clear)) - 1;
+          clear &= clear - 1;
+          for (int64_t v = lane; v < vec_per_row; v += kWave) st16(act_grad + (r0 + r) * vec_per_row + v, u32x4{0, 0, 0, 0});
+        }
+      }
       __syncthreads();
     }
     return;
   }
   const int64_t wave = static_cast<int64_t>(blockIdx.x - clearers) * kMoverWaves + threadIdx.x / kWave;
   const int64_t n_waves = static_cast<int64_t>(gridDim.x - clearers) * kMoverWaves;
-  const bool weighted = num_topk > 1 && probs != nullptr;
   for (int64_t t = wave; t < num_tokens; t += n_waves) {
     const u32x4* src = grad_out + t * vec_per_row;
-    for (int k = 0; k < num_topk; ++k) {
-      const int32_t r = row_id_map[k * num_tokens + t];
-      u32x4* dst = act_grad + static_cast<int64_t>(r) * vec_per_row;
-      if (!weighted) {
+    if constexpr (COPIES == 0) {
+      for (int k = 0; k < num_topk; ++k) {
+        const int32_t r = row_id_map[k * num_tokens + t];
         if (r < 0) continue;
+        u32x4* dst = act_grad + static_cast<int64_t>(r) * vec_per_row;
         int64_t v = lane;
         for (; v + 3 * kWave < vec_per_row; v += 4 * kWave) {
           const u32x4 a = ld16(src + v), b = ld16(src + v + kWave), c = ld16(src + v + 2 * kWave), d = ld16(src + v + 3 * kWave);
           st16(dst + v, a); st16(dst + v + kWave, b); st16(dst + v + 2 * kWave, c); st16(dst + v + 3 * kWave, d);
         }
         for (; v < vec_per_row; v += kWave) st16(dst + v, ld16(src + v));
-        continue;
       }
-      float dot = 0.f;
-      if (r >= 0) {
-        const float p = Elem<DT>::round(probs[t * num_topk + k]);
-        for (int64_t v = lane; v < vec_per_row; v += kWave) {
-          float g[E], yv[E], o[E];
-          unpack16<DT>(ld16(src + v), g);
-          unpack16<DT>(ld16(y_fwd + static_cast<int64_t>(r) * vec_per_row + v), yv);
+    } else {
+      constexpr int kCopies = COPIES;
+      for (int k0 = 0; k0 < num_topk; k0 += kCopies) {
+        int32_t r[kCopies];
+        float p[kCopies], dot[kCopies];
 #pragma unroll
-          for (int e = 0; e < E; ++e) {
-            o[e] = Elem<DT>::round(g[e] * p);
-            dot += Elem<DT>::round(g[e] * yv[e]);
-          }
-          st16(dst + v, pack16<DT>(o));
+        for (int c = 0; c < kCopies; ++c) {
+          const int k = k0 + c < num_topk ? k0 + c : num_topk - 1;
+          r[c] = k0 + c < num_topk ? row_id_map[k * num_tokens + t] : -1;
+          p[c] = Elem<DT>::round(probs[t * num_topk + k]);
+          dot[c] = 0.f;
         }
-      }
-      if (prob_grad != nullptr) {
+        for (int64_t v = lane; v < vec_per_row; v += kWave) {
+          const u32x4 graw = ld16(src + v);
+          u32x4 yraw[kCopies];
 #pragma unroll
-        for (int d = kWave / 2; d > 0; d >>= 1) dot += __shfl_xor(dot, d);
-        if (lane == 0) prob_grad[t * num_topk + k] = dot;
+          for (int c = 0; c < kCopies; ++c)
+            if (r[c] >= 0) yraw[c] = ld16(y_fwd + static_cast<int64_t>(r[c]) * vec_per_row + v);
+          float g[E];
+          unpack16<DT>(graw, g);
+#pragma unroll
+          for (int c = 0; c < kCopies; ++c) {
+            if (r[c] < 0) continue;
+            float yv[E], o[E];
+            unpack16<DT>(yraw[c], yv);
+#pragma unroll
+            for (int e = 0; e < E; ++e) {
+              o[e] = Elem<DT>::round(g[e] * p[c]);
+              dot[c] += Elem<DT>::round(g[e] * yv[e]);
+            }
+            st16(act_grad + static_cast<int64_t>(r[c]) * vec_per_row + v, pack16<DT>(o));
+          }
+        }
+#pragma unroll
+        for (int c = 0; c < kCopies; ++c) {
+          if (k0 + c >= num_topk) continue;
+#pragma unroll
+          for (int d = kWave / 2; d > 0; d >>= 1) dot[c] += __shfl_xor(dot[c], d);
+          if (lane == 0 && prob_grad != nullptr) prob_grad[t * num_topk + k0 + c] = dot[c];
+        }
       }
     }
   }
@@ -847,16 +895,18 @@ int unpermute_rows_bwd(const char* who, const void* grad_out, const void* y_fwd,
   const u32x4* g = static_cast<const u32x4*>(grad_out);
   const u32x4* yf = static_cast<const u32x4*>(y_fwd);
   u32x4* ag = static_cast<u32x4*>(act_grad);
-  if (dtype == WX_F32) {
-    hipLaunchKernelGGL(combine_rows_bwd_kernel<WX_F32>, grid, block, 0, s, g, yf, ag, prob_grad, row_id_map, probs,
-                       num_tokens, num_topk, vec, num_rows, clearers);
-  } else if (dtype == WX_F16) {
-    hipLaunchKernelGGL(combine_rows_bwd_kernel<WX_F16>, grid, block, 0, s, g, yf, ag, prob_grad, row_id_map, probs,
-                       num_tokens, num_topk, vec, num_rows, clearers);
-  } else {
-    hipLaunchKernelGGL(combine_rows_bwd_kernel<WX_BF16>, grid, block, 0, s, g, yf, ag, prob_grad, row_id_map, probs,
-                       num_tokens, num_topk, vec, num_rows, clearers);
-  }
+  auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, grid, block, 0, s, g, yf, ag, prob_grad, row_id_map, probs, num_tokens, num_topk, vec, num_rows, clearers);
+  };
+  auto launch_weighted = [&](auto copies) {
+    constexpr int C = decltype(copies)::value;
+    if (dtype == WX_F32) launch(combine_rows_bwd_kernel<WX_F32, C>);
+    else if (dtype == WX_F16) launch(combine_rows_bwd_kernel<WX_F16, C>);
+    else launch(combine_rows_bwd_kernel<WX_BF16, C>);
+  };
+  if (num_topk == 1) launch(combine_rows_bwd_kernel<WX_BF16, 0>);  // (rows as they are, whatever their type)
+  else if (num_topk == 2) launch_weighted(std::integral_constant<int, 2>{});
+  else launch_weighted(std::integral_constant<int, 4>{});
   return check_launch(who);
 }
 
