@@ -343,6 +343,16 @@ int wx_mrope_apply_packed(const void* q, const void* k, const uint32_t* table, v
                           const int64_t q_strides[3], const int64_t k_strides[3], const int64_t qo_strides[3],
                           const int64_t ko_strides[3], const int mrope_section[3], int layout, int dtype,
                           int backward, wx_stream_t stream);
+/* The gradient of wx_qkv_rope_proj's result before the rotation: grad_out [batch * seq, (n_q + 2 n_kv) * 128] = the q and k
+ * heads' gradients rotated back with the projection's own table (width table_width), the v heads' as they are; and, where
+ * grad_bias is not NULL, grad_bias = its column sums (fp32, rounded to bf16).  Each gradient is [batch, heads, seq, 128] bf16
+ * through (batch, head, seq) strides in elements, multiples of 8, or NULL for zeros.  workspace (only with grad_bias):
+ * wx_qkv_rope_bwd_workspace_bytes(). */
+size_t wx_qkv_rope_bwd_workspace_bytes(int n_q_heads, int n_kv_heads, int head_dim);
+int wx_qkv_rope_bwd(const void* grad_q, const void* grad_k, const void* grad_v, const uint32_t* table, int table_width,
+                    void* grad_out, void* grad_bias, int64_t batch, int64_t seq, int n_q_heads, int n_kv_heads, int head_dim,
+                    const int64_t q_strides[3], const int64_t k_strides[3], const int64_t v_strides[3], void* workspace,
+                    size_t workspace_bytes, wx_stream_t stream);
 int wx_qkv_rope_proj(const void* x, const void* weight, const void* bias, const uint32_t* rope_table,
                      int table_width, void* out, int64_t num_tokens, int64_t hidden, int n_q_heads, int n_kv_heads,
                      int head_dim, wx_stream_t stream);

@@ -210,3 +210,58 @@ def test_qkv_rope_projection_with_table_and_bias_at_any_element(dev, rows, layou
         assert t2.data_ptr() % 16 == 4 * off and b2.data_ptr() % 8 == 2 * off
         for got, ref in zip(ops.qkv_projection_with_rope(x, w, b2, t2, nq, nkv), want):
             assert torch.equal(got, ref)
+
+
+@pytest.mark.parametrize("layout", ["hf", "csrc"])
+@pytest.mark.parametrize("B,S,nq,nkv,order", [(1, 1, 1, 1, "bshd"), (1, 15, 4, 2, "bhsd"), (3, 17, 5, 1, "split"), (2, 2050, 16, 2, "bshd"),
+                                              (1, 4113, 3, 3, "mixed"), (2, 33, 2, 1, "none"), (2, 40, 4, 1, "expanded")])
+def test_gradient_of_the_projection_before_the_rotation(dev, B, S, nq, nkv, order, layout):
+    """wx_qkv_rope_bwd: the q and k heads as rope_from_table's adjoint gives them, the v heads as they are, bit for bit, and the
+    column sums against 64 bits: fp32 sums of T values (T 2^-24 of the sum of sizes bounds any order) and one rounding."""
+    g = torch.Generator(device=dev).manual_seed(S)
+    D, section = 128, list(wl.MROPE_SECTION)
+    pos = torch.randint(0, 500, (3, B, S), device=dev, generator=g)
+    table = native.mrope_table(pos, wl.text_inv_freq().to(dev), section, layout)
+
+    def grad(n, how):
+        if how == "bshd":
+            return torch.randn((B, S, n, D), device=dev, generator=g).to(torch.bfloat16).transpose(1, 2)
+        if how == "split":  # heads of a wider matrix, at an offset that is not a multiple of 16 bytes
+            return torch.randn((B, S, n * D + 12), device=dev, generator=g).to(torch.bfloat16)[..., 4:4 + n * D].view(B, S, n, D).transpose(1, 2)
+        if how == "expanded":
+            return torch.randn((1, n, 1, 1), device=dev, generator=g).to(torch.bfloat16).expand(B, n, S, D)
+        return torch.randn((B, n, S, D), device=dev, generator=g).to(torch.bfloat16)
+
+    hows = {"mixed": ("bhsd", "bshd", "float"), "none": ("bshd", None, "bhsd")}.get(order, (order,) * 3)
+    grads = [None if h is None else (grad(n, "bhsd").float() if h == "float" else grad(n, h)) for h, n in zip(hows, (nq, nkv, nkv))]
+    out, bias = native.qkv_rope_bwd(*grads, table, B, S, nq, nkv, True)
+    full = [torch.zeros((B, n, S, D), dtype=torch.bfloat16, device=dev) if t is None else t.to(torch.bfloat16).contiguous() for t, n in zip(grads, (nq, nkv, nkv))]
+    rq, rk = torch.empty_like(full[0]), torch.empty_like(full[1])
+    native.rope_from_table(full[0], full[1], table, rq, rk, [2 * v for v in section], backward=True, layout=layout)
+    want = torch.cat((rq, rk, full[2]), 1).transpose(1, 2).reshape(B * S, -1)
+    assert torch.equal(out, want)
+    exact, size = want.double().sum(0), want.double().abs().sum(0)
+    assert bool(((bias.double() - exact).abs() <= 2 ** -8 * exact.abs() + B * S * 2 ** -24 * size + 1e-30).all())
+    again, none = native.qkv_rope_bwd(*grads, table, B, S, nq, nkv, False)
+    assert none is None and torch.equal(again, out)
+
+
+def test_projection_backward_with_one_output_used_or_changed_in_place(dev):
+    g = torch.Generator(device=dev).manual_seed(5)
+    h = torch.randn((2, 24, 64), device=dev, generator=g).to(torch.bfloat16).requires_grad_()
+    w = (torch.randn((4 * 128, 64), device=dev, generator=g) * 0.1).to(torch.bfloat16).requires_grad_()
+    pos = torch.randint(0, 90, (3, 2, 24), device=dev, generator=g)
+    table = ops.multimodal_rope_table(pos, wl.text_inv_freq().to(dev), wl.MROPE_SECTION)
+    seed = torch.randn((2, 1, 24, 128), device=dev, generator=g).to(torch.bfloat16)
+    q, k, v = ops.qkv_projection_with_rope(h, w, None, table, 2, 1)
+    assert q.transpose(1, 2).stride() == (24 * 512, 512, 128, 1) and v.data_ptr() == q.data_ptr() + 3 * 256
+    dw = torch.autograd.grad(v, w, seed, retain_graph=True)[0]
+    assert not dw[:384].any() and dw[384:].any()
+    k.mul_(2)
+    (dk,) = torch.autograd.grad(k, w, seed)
+    q1, k1, v1 = ops.qkv_projection_with_rope(h, w, None, table, 2, 1)
+    (once,) = torch.autograd.grad(k1, w, seed)
+    assert torch.equal(dk, 2 * once)
+    with pytest.raises(RuntimeError, match="table must be"):
+        bad = ops.qkv_projection_with_rope(h, w, None, table, 2, 1, layout="csrc")
+        torch.autograd.grad(bad[0].sum(), w)

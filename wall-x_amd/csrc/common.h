@@ -121,4 +121,7 @@ int ffn_fused(const void* x_rows, void* x_tiled, void* out, const void* residual
               int64_t num_rows, int64_t hidden, int64_t inter0, int64_t inter1, const int64_t* host_rows_per_expert,
               const int32_t* out_row_id, void* workspace, void* split_scratch, wx_stream_t stream);
 
+// grad[c] = sum over p of partial[p][c] (n_partials x cols, fp32), rounded to bf16 (fused_movers.hip)
+int launch_column_sums(const float* partial, void* grad, int64_t n_partials, int64_t cols, hipStream_t stream);
+
 }  // namespace wx

@@ -406,6 +406,12 @@ __global__ __launch_bounds__(kSumCols* kSumGroups) void column_sums_kernel(const
 }
 
 }  // namespace
+
+int launch_column_sums(const float* partial, void* grad, int64_t n_partials, int64_t cols, hipStream_t stream) {
+  hipLaunchKernelGGL(column_sums_kernel, dim3(static_cast<unsigned>((cols + kSumCols - 1) / kSumCols)), dim3(kSumCols * kSumGroups), 0, stream,
+                     partial, static_cast<__bf16*>(grad), n_partials, cols);
+  return check_launch("column_sums_kernel");
+}
 }  // namespace wx
 
 using namespace wx;
@@ -589,9 +595,7 @@ extern "C" int wx_unpermute_rows_rmsnorm_bwd(const void* grad_sorted, const void
   }
 #undef WX_CASE
   if (int rc = check_launch("unpermute_rmsnorm_bwd_kernel")) return rc;
-  hipLaunchKernelGGL(column_sums_kernel, dim3(static_cast<unsigned>((num_cols + kSumCols - 1) / kSumCols)), dim3(kSumCols * kSumGroups), 0, s,
-                     static_cast<const float*>(workspace), static_cast<__bf16*>(grad_weight), blocks * 4, num_cols);
-  return check_launch("column_sums_kernel");
+  return launch_column_sums(static_cast<const float*>(workspace), grad_weight, blocks * 4, num_cols, s);
 }
 
 extern "C" int wx_moe_block_forward_split(const void* x, void* out, const int32_t* row_id_map, const int32_t* sorted_row_id,

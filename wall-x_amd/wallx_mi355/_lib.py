@@ -59,6 +59,8 @@ PROTOTYPES = {
     "wx_mrope_table": (_i32, [_vp, _vp, _i64, _i64, _i32, _c.POINTER(_i32), _i32, _vp, _vp]),
     "wx_mrope_apply_packed": (_i32, [_vp] * 5 + [_i64, _i64, _i32, _i32, _i32] + [_c.POINTER(_i64)] * 4
                               + [_c.POINTER(_i32), _i32, _i32, _i32, _vp]),
+    "wx_qkv_rope_bwd_workspace_bytes": (_sz, [_i32] * 3),
+    "wx_qkv_rope_bwd": (_i32, [_vp] * 4 + [_i32, _vp, _vp, _i64, _i64, _i32, _i32, _i32] + [_c.POINTER(_i64)] * 3 + [_vp, _sz, _vp]),
     "wx_qkv_rope_proj": (_i32, [_vp, _vp, _vp, _vp, _i32, _vp, _i64, _i64, _i32, _i32, _i32, _vp]),
     "wx_rope_index_workspace_bytes": (_sz, [_i64, _i64]),
     "wx_rope_index": (_i32, [_vp, _vp, _vp, _i64, _vp, _i64, _vp, _i64, _i64, _i32, _i64, _i64, _i64, _f32,

@@ -88,6 +88,16 @@ def qkv_rope_proj(x, weight, bias, table, n_q_heads, n_kv_heads, head_dim=128, o
     return native.qkv_rope_proj(x, weight, bias, table, n_q_heads, n_kv_heads, head_dim, out)
 
 
+def check_mrope_table(table, tokens, head_dim, mrope_section, layout):
+    """No counterpart in backend.py: raises for a table that rope_from_table would refuse."""
+    return native.check_mrope_table(table, tokens, head_dim, mrope_section, layout)
+
+
+def qkv_rope_bwd(grad_q, grad_k, grad_v, table, batch, seq, n_q_heads, n_kv_heads, want_bias):
+    """No counterpart in backend.py: the gradient of the projection's result before the rotation, and the bias's."""
+    return native.qkv_rope_bwd(grad_q, grad_k, grad_v, table, batch, seq, n_q_heads, n_kv_heads, want_bias)
+
+
 def get_rope_index(input_ids, image_grid_thw, video_grid_thw, second_per_grid_ts, attention_mask,
                    spatial_merge_size, image_token_id, video_token_id, vision_start_token_id, tokens_per_second):
     """backend.py:302-352 (forwards to the native op named rope_index)."""

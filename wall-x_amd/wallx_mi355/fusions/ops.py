@@ -399,50 +399,52 @@ def multimodal_rope_from_table(q, k, table, mrope_section, layout="hf"):
 
 
 class QkvProjectionWithRoPE(torch.autograd.Function):
-    """The fused projection under autograd.  Forward: one launch (backend.qkv_rope_proj).  Backward, for the gradient
-    `g` of the [B, S, (Hq + 2 Hkv) D] result: the adjoint rotation of g's q and k heads from the same packed table
-    (backend.rope_from_table(backward=True), what ops.py:463-493 gives the separate rope op) into a buffer of
-    g's shape, the v heads copied beside them; then d hidden = g W and d W = g^T hidden as dual-GEMM launches on the row-major operands (the transposition
-    happens inside the kernel) and d bias = the column sums of g (fp32 accumulation, like nn.Linear's)."""
+    """The fused projection under autograd.  Forward: one launch (backend.qkv_rope_proj), q, k and v as tensors over its one
+    buffer.  Backward: one launch (backend.qkv_rope_bwd) rotates the q and k heads' gradients back with the same packed
+    table (what ops.py:463-493 gives the separate rope op), sets the v heads' beside them and adds up the bias's
+    gradient (fp32, like nn.Linear's); then d hidden = g W and d W = g^T hidden as dual-GEMM launches on the row-major
+    operands (the transposition happens inside the kernel)."""
 
     @staticmethod
     def forward(ctx, hidden_states, qkv_weight, qkv_bias, rope_table, nq, nkv, D, mrope_section, layout):
         out = backend.qkv_rope_proj(hidden_states, qkv_weight, qkv_bias, rope_table, nq, nkv, D)
         ctx.save_for_backward(hidden_states, qkv_weight, rope_table)
         ctx.heads = (nq, nkv, D)
-        ctx.rope = ([2 * int(v) for v in mrope_section], layout)
+        ctx.rope = ([int(v) for v in mrope_section], layout)
         ctx.has_bias = qkv_bias is not None
-        return out
+        ctx.set_materialize_grads(False)
+        B, S, _ = hidden_states.shape
+        N, storage = (nq + 2 * nkv) * D, out.untyped_storage()
+
+        # (not views of `out` for autograd: what a caller writes into one of them in place stays that one's)
+        def heads(first, count):
+            return out.new_empty(0).set_(storage, out.storage_offset() + first * D, (B, count, S, D), (S * N, D, N, 1))
+
+        return heads(0, nq), heads(nq, nkv), heads(nq + nkv, nkv)
 
     @staticmethod
-    def backward(ctx, grad_out):
+    def backward(ctx, grad_q, grad_k, grad_v):
         hidden_states, weight, table = ctx.saved_tensors
+        if grad_q is None and grad_k is None and grad_v is None:
+            return (None,) * 9
         nq, nkv, D = ctx.heads
-        doubled, layout = ctx.rope
+        section, layout = ctx.rope
         B, S, H = hidden_states.shape
         N = (nq + 2 * nkv) * D
-        go = grad_out.to(torch.bfloat16).contiguous().view(B, S, N)
-        g = torch.empty_like(go)  # the gradient w.r.t. the projection's own output: q and k heads rotated back, v as is
-
-        def heads(t, first, count):
-            return t[..., first * D:(first + count) * D].view(B, S, count, D).transpose(1, 2)
-
-        backend.rope_from_table(heads(go, 0, nq), heads(go, nq, nkv), table, heads(g, 0, nq), heads(g, nq, nkv), doubled,
-                                backward=True, layout=layout)
-        g[..., (nq + nkv) * D:].copy_(go[..., (nq + nkv) * D:])
-        g2, x2 = g.view(B * S, N), hidden_states.reshape(B * S, H)
-        none = g2.new_empty((0, 0))
         want_x, want_w, want_b = ctx.needs_input_grad[0], ctx.needs_input_grad[1], ctx.needs_input_grad[2]
-        dx = dw = db = None
+        # the gradient w.r.t. the projection's own output
+        backend.check_mrope_table(table, B * S, D, section, layout)
+        g2, db = backend.qkv_rope_bwd(grad_q, grad_k, grad_v, table, B, S, nq, nkv, want_b and ctx.has_bias)
+        x2 = hidden_states.reshape(B * S, H)
+        none = g2.new_empty((0, 0))
+        dx = dw = None
         if want_x:  # [T, N] @ [N, H]: the weight is read as stored, K-major
-            dx = torch.empty(B * S, H, dtype=torch.bfloat16, device=g.device)
+            dx = torch.empty(B * S, H, dtype=torch.bfloat16, device=g2.device)
             backend.asym_dual_gmm_separated(g2, none, weight, g2.new_empty((0, H)), dx, g2.new_empty((0, H)), False, False)
             dx = dx.view(B, S, H)
         if want_w:  # [T, N]^T @ [T, H]: both operands K-major
-            dw = torch.empty(N, H, dtype=torch.bfloat16, device=g.device)
+            dw = torch.empty(N, H, dtype=torch.bfloat16, device=g2.device)
             backend.asym_dual_gmm_separated(g2, none, x2, g2.new_empty((0, H)), dw, g2.new_empty((0, H)), True, False)
-        if want_b and ctx.has_bias:
-            db = g2.sum(0, dtype=torch.float32).to(torch.bfloat16)
         return dx, dw, db, None, None, None, None, None, None
 
 
@@ -475,10 +477,9 @@ def qkv_projection_with_rope(hidden_states, qkv_weight, qkv_bias, rope_table, nu
             raise RuntimeError("[Error] The input `mrope_section` of multimodal_rope op must be a list of 3 integers!")
         if layout is None:
             layout = "hf" if rope_table.size(-1) == D // 2 else "csrc"
-        out = QkvProjectionWithRoPE.apply(hidden_states, qkv_weight, qkv_bias, rope_table, nq, nkv, D,
-                                          tuple(mrope_section), layout)
-    else:
-        out = backend.qkv_rope_proj(hidden_states, qkv_weight, qkv_bias, rope_table, nq, nkv, D)
+        return QkvProjectionWithRoPE.apply(hidden_states, qkv_weight, qkv_bias, rope_table, nq, nkv, D,
+                                           tuple(mrope_section), layout)
+    out = backend.qkv_rope_proj(hidden_states, qkv_weight, qkv_bias, rope_table, nq, nkv, D)
     q, k, v = out.split([nq * D, nkv * D, nkv * D], dim=-1)
     return (q.view(B, S, nq, D).transpose(1, 2), k.view(B, S, nkv, D).transpose(1, 2),
             v.view(B, S, nkv, D).transpose(1, 2))

@@ -464,6 +464,51 @@ def qkv_rope_proj(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Te
     return out.view(*x.shape[:-1], n)
 
 
+def check_mrope_table(table: torch.Tensor, tokens: int, head_dim: int, mrope_section, layout: str) -> None:
+    """Raises where rope_from_table would refuse the table for these sections and this layout."""
+    section = [int(v) for v in mrope_section]
+    width = _table_width(head_dim, _lib.i32x3(section), layout)
+    if tuple(table.shape) != (tokens, width) or table.dtype != torch.int32 or not table.is_contiguous():
+        raise RuntimeError(f"table must be a contiguous int32 [{tokens}, {width}] tensor from mrope_table with the same "
+                           f"mrope_section and layout ({layout!r})")
+    step = 1 if layout == "hf" else 2
+    if step * section[0] % 8 or step * (section[0] + section[1]) % 8:
+        raise RuntimeError("the packed table needs sections that end on chunks of 8 channels; build the cos/sin tables and call "
+                           "multimodal_rope instead")
+
+
+def qkv_rope_bwd(grad_q, grad_k, grad_v, table: torch.Tensor, B: int, S: int, n_q_heads: int, n_kv_heads: int, want_bias: bool):
+    """The gradient of `qkv_rope_proj`'s result before the rotation, [B * S, (n_q + 2 n_kv) * 128], and its column sums (the
+    bias's gradient) or None.  grad_q / grad_k / grad_v: [B, heads, S, 128] in any strides, or None for zeros."""
+    D, heads = 128, n_q_heads + 2 * n_kv_heads
+    grads, strides = [], []
+    for t, n in ((grad_q, n_q_heads), (grad_k, n_kv_heads), (grad_v, n_kv_heads)):
+        if t is None:
+            grads.append(None)
+            strides.append(_lib.i64x3((0, 0, 0)))
+            continue
+        _need_cuda("gradient", t)
+        if tuple(t.shape) != (B, n, S, D) or t.device != table.device:
+            raise RuntimeError(f"gradients must be [{B}, {n}, {S}, {D}] tensors on the table's device")
+        t = t.to(torch.bfloat16)
+        sb, sh, ss, sd = t.stride()
+        if sd != 1 or (sb | sh | ss) & 7 or t.data_ptr() & 15:
+            t = t.clone(memory_format=torch.contiguous_format)
+        grads.append(t)
+        strides.append(_bhsd_strides(t))
+    g = torch.empty((B * S, heads * D), dtype=torch.bfloat16, device=table.device)
+    bias = work = None
+    n_work = 0
+    if want_bias:
+        bias = torch.empty(heads * D, dtype=torch.bfloat16, device=table.device)
+        n_work = _lib.load().wx_qkv_rope_bwd_workspace_bytes(n_q_heads, n_kv_heads, D)
+        work = torch.empty(n_work, dtype=torch.uint8, device=table.device)
+    with _DeviceGuard(table):
+        _lib.call("wx_qkv_rope_bwd", _ptr(grads[0]), _ptr(grads[1]), _ptr(grads[2]), _ptr(table), int(table.size(1)), _ptr(g), _ptr(bias), B, S,
+                  n_q_heads, n_kv_heads, D, *strides, _ptr(work), n_work, _stream(table))
+    return g, bias
+
+
 # ----------------------------------------------------------------------------- index builders
 def rope_index(input_ids, image_grid_thw, video_grid_thw, second_per_grid_ts, attention_mask,
                spatial_merge_size: int, image_token_id: int, video_token_id: int, vision_start_token_id: int,
