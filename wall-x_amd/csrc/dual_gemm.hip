@@ -251,7 +251,7 @@ __host__ __device__ inline int tail_split_point(int tiles0, int tiles1, int k0, 
 // and 88 left over that take 37 us as small ones, where three whole row blocks and a strip are one round, two large tiles
 // and 172 small ones: us a layer 158 -> 146, 2310 to 2400 rows 318 to 323 -> 307 to 311, 1656 rows 240 -> 230.
 // The rounds are counted in kTailRound-ths of a round of large tiles: kTailOne for a launch of small tiles with one to a CU,
-// kTailTwo with two (contractions of 2048, us: 47 to 53, 20, 37).
+// kTailTwo with two (contractions of 2048, us: 47 to 56, 20 to 25, 37).
 struct TailPlan {
   int rows[2];  // row blocks of 256 of each expert that are large tiles
   int first;    // large tiles of the first launch
