@@ -121,3 +121,72 @@ def test_tensors_on_the_cpu_are_left_alone():
     assert host.unpermute(x, ids.view(-1), None, 4, 1) is None and host.unpermute_bwd(x, x, ids.view(-1)) is None
     with pytest.raises(TypeError):
         host.bind(1)
+
+
+@pytest.mark.gpu
+def test_recorded_into_a_graph_on_another_stream(dev):
+    """The native host side under capture: every replay on new contents equals the eager calls."""
+    q, k, c, s = _rope_inputs(dev, 0, torch.bfloat16, "hf", "bshd", rows=3, row_len=70)
+    g = torch.Generator(device=dev).manual_seed(9)
+    x = torch.randn((5000, 64), generator=g, device=dev).to(torch.bfloat16)
+    ids = torch.randint(0, 3, (5000, 1), generator=g, device=dev, dtype=torch.int32)
+
+    def work():
+        rq, rk = ops.multimodal_rope(q, k, c, s, SECTION)
+        permuted, rmap = ops.permute(x, ids)
+        return rq, rk, permuted, ops.unpermute(permuted, rmap)
+
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        work()
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = work()
+    for _ in range(3):
+        for t in (q, k, x):
+            t.copy_(torch.randn(t.shape, generator=g, device=dev).to(t.dtype))
+        ids.copy_(torch.randint(0, 3, ids.shape, generator=g, device=dev, dtype=torch.int32))
+        graph.replay()
+        got = [t.clone() for t in out]
+        torch.cuda.synchronize()
+        for a, b in zip(got, work()):
+            assert torch.equal(a, b)
+
+
+@pytest.mark.gpu
+def test_from_several_threads_with_streams_of_their_own(dev):
+    """Forward and backward from four threads at once, each on a stream of its own, equal the calls one after the other."""
+    import threading
+
+    inputs = [_rope_inputs(dev, 0, torch.bfloat16, "hf", "bshd", rows=1 + i, row_len=33 + i) for i in range(4)]
+
+    def one(i):
+        q, k, c, s = inputs[i]
+        q, k = q.detach().requires_grad_(), k.detach().requires_grad_()
+        out = ops.multimodal_rope(q, k, c, s, SECTION)
+        return [t.detach() for t in out] + list(torch.autograd.grad(out, (q, k), [t.detach() for t in out]))
+
+    want = [one(i) for i in range(4)]
+    got, errors = [None] * 4, []
+    torch.cuda.synchronize()
+
+    def thread(i):
+        try:
+            stream = torch.cuda.Stream()
+            with torch.cuda.stream(stream):
+                for _ in range(5):
+                    got[i] = one(i)
+            stream.synchronize()
+        except Exception as exc:  # noqa: BLE001 - reported below
+            errors.append(exc)
+
+    threads = [threading.Thread(target=thread, args=(i,)) for i in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not errors, errors
+    for a, b in zip(got, want):
+        assert all(torch.equal(x, y) for x, y in zip(a, b))
