@@ -95,8 +95,17 @@ def test_permute_and_unpermute_as_the_general_path(dev, tokens, topk, num_out, d
         assert host.unpermute(out, rmap.long(), None, tokens, topk) is None
     if topk == 1:
         grad = torch.randn((tokens, 72), generator=g, device=dev).to(dtype)
-        assert torch.equal(host.unpermute_bwd(grad, out, rmap), native.unpermute_rows_bwd(grad, out, rmap))
-        assert host.unpermute_bwd(grad, out[:, :40], rmap) is None
+        assert torch.equal(host.unpermute_bwd(grad, out, rmap, None), native.unpermute_rows_bwd(grad, out, rmap))
+        assert host.unpermute_bwd(grad, out[:, :40], rmap, None) is None
+        assert host.unpermute_bwd(grad, out, rmap, torch.ones((tokens, 1), device=dev)) is None  # a weight whose gradient is zeros
+    else:
+        grad = torch.randn((tokens, 72), generator=g, device=dev).to(dtype)
+        probs = torch.rand((tokens, topk), generator=g, device=dev)
+        got = host.unpermute_bwd(grad, out, rmap, probs)
+        for a, b in zip(got, native.unpermute_bwd(grad, out, rmap, probs)):
+            assert a.dtype == b.dtype and torch.equal(a, b)
+        assert host.unpermute_bwd(grad, out, rmap, probs.double()) is None and host.unpermute_bwd(grad, out, rmap[:-1], probs) is None
+        assert host.unpermute_bwd(grad, out, rmap, probs[:-1]) is None
 
 
 @pytest.mark.gpu
@@ -118,7 +127,7 @@ def test_tensors_on_the_cpu_are_left_alone():
     host = _lib.host()
     assert host.rope(0, q, k, c, c, SECTION, "hf", 0) is None
     assert host.permute(x, ids, 0, x, ids, 256) is None
-    assert host.unpermute(x, ids.view(-1), None, 4, 1) is None and host.unpermute_bwd(x, x, ids.view(-1)) is None
+    assert host.unpermute(x, ids.view(-1), None, 4, 1) is None and host.unpermute_bwd(x, x, ids.view(-1), None) is None
     with pytest.raises(TypeError):
         host.bind(1)
 

@@ -216,23 +216,32 @@ PyObject* unpermute(PyObject*, PyObject* const* args, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
-// unpermute_bwd(grad [T, H], input_fwd [R, H], row_id_map int32 [T]) -> act_grad [R, H] or None: one expert per token, no weights.
+// unpermute_bwd(grad [T, H], input_fwd [R, H], row_id_map int32, probs fp32 [T, K] or None) -> act_grad [R, H], or with probs
+// (act_grad, their gradient [T, K]), or None.  Without probs: one expert per token.  (A single weight per token, whose
+// gradient is zeros, is the general path's.)
 PyObject* unpermute_bwd(PyObject*, PyObject* const* args, Py_ssize_t n) {
   HANDLE_TH_ERRORS
-  if (n != 3 || !entry.unpermute_bwd) return none();
-  const at::Tensor *g = plain(args[0]), *x = plain(args[1]), *map = plain(args[2]);
-  if (!g || !x || !map || g->dim() != 2 || x->dim() != 2 || !g->is_contiguous() || !x->is_contiguous() || !map->is_contiguous()) return none();
+  if (n != 4 || !entry.unpermute_bwd) return none();
+  const at::Tensor *g = plain(args[0]), *x = plain(args[1]), *map = plain(args[2]), *probs = args[3] == Py_None ? nullptr : plain(args[3]);
+  if (!g || !x || !map || (args[3] != Py_None && !probs) || g->dim() != 2 || x->dim() != 2 || !g->is_contiguous() || !x->is_contiguous() ||
+      !map->is_contiguous())
+    return none();
+  const int64_t T = g->size(0), K = probs ? (probs->dim() == 2 ? probs->size(1) : 0) : 1;
+  if (probs && (K < 2 || K > 128 || probs->size(0) != T || !probs->is_contiguous() || probs->scalar_type() != at::kFloat || probs->device() != g->device()))
+    return none();
   const int code = dtype_code(g->scalar_type());
   if (code < 0 || x->scalar_type() != g->scalar_type() || map->scalar_type() != at::kInt || x->size(1) != g->size(1) || g->numel() == 0 || x->numel() == 0 ||
-      map->numel() < g->size(0) || x->device() != g->device() || map->device() != g->device())
+      map->numel() < T * K || x->device() != g->device() || map->device() != g->device())
     return none();
-  at::Tensor out;
+  at::Tensor out, prob_grad;
   const bool ok = run(*g, [&] {
     out = at::empty({x->size(0), g->size(1)}, g->options());
-    return entry.unpermute_bwd(ptr(*g), ptr(*x), ptr(out), out.size(0), nullptr, static_cast<const int32_t*>(ptr(*map)), nullptr, g->size(0), 1, g->size(1), code,
-                               stream_of(*g));
+    if (probs) prob_grad = at::empty({T, K}, probs->options());
+    return entry.unpermute_bwd(ptr(*g), ptr(*x), ptr(out), out.size(0), probs ? static_cast<float*>(ptr(prob_grad)) : nullptr,
+                               static_cast<const int32_t*>(ptr(*map)), probs ? static_cast<const float*>(ptr(*probs)) : nullptr, T, static_cast<int>(K),
+                               g->size(1), code, stream_of(*g));
   });
-  return ok ? wrap(out) : nullptr;
+  return !ok ? nullptr : (probs ? pair(out, prob_grad) : wrap(out));
   END_HANDLE_TH_ERRORS
 }
 

@@ -185,12 +185,13 @@ class UnpermuteMoE_topK(torch.autograd.Function):
         act_grad = prob_grad = None
         if ctx.needs_input_grad[0]:
             if probs is None:
-                act_grad = _lib.host().unpermute_bwd(unpermuted_act_grad, input_act, row_id_map)
+                act_grad = _lib.host().unpermute_bwd(unpermuted_act_grad, input_act, row_id_map, None)
                 if act_grad is None:
                     act_grad = backend.unpermute_rows_bwd(unpermuted_act_grad.contiguous(), input_act, row_id_map)
             else:
-                act_grad, prob_grad = backend.unpermute_bwd(unpermuted_act_grad.contiguous(), input_act, row_id_map,
-                                                            probs)
+                made = _lib.host().unpermute_bwd(unpermuted_act_grad, input_act, row_id_map, probs)
+                act_grad, prob_grad = made if made is not None else backend.unpermute_bwd(
+                    unpermuted_act_grad.contiguous(), input_act, row_id_map, probs)
         if not ctx.needs_input_grad[2]:
             prob_grad = None
         return act_grad, None, prob_grad
