@@ -1,5 +1,8 @@
 """The native host side of the row and rotary ops (csrc/host_ops.cpp) against the general path in native.py: what it takes
 gives the same bits, and whatever has to be warned of, copied or refused it leaves alone."""
+import threading
+import warnings
+
 import pytest
 import torch
 
@@ -199,3 +202,93 @@ def test_from_several_threads_with_streams_of_their_own(dev):
     assert not errors, errors
     for a, b in zip(got, want):
         assert all(torch.equal(x, y) for x, y in zip(a, b))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("ids_dtype", [torch.int32, torch.int64])
+def test_recorded_permute_is_its_own_beside_calls_of_other_sizes_and_types(dev, ids_dtype):
+    """More than 4096 keys: one launch writes histograms that the next reads.  A graph replayed after calls that need
+    larger scratch gives its own result, and writes nothing into memory allocated since."""
+    g = torch.Generator(device=dev).manual_seed(2)
+    x = torch.randn((5000, 64), generator=g, device=dev).to(torch.bfloat16)
+    ids = torch.randint(0, 3, (5000, 1), generator=g, device=dev, dtype=ids_dtype)
+    big, big_ids = torch.randn((40000, 64), generator=g, device=dev), torch.randint(0, 3, (40000, 1), generator=g, device=dev, dtype=ids_dtype)
+
+    def call(x, ids):
+        with warnings.catch_warnings():
+            warnings.simplefilter("ignore")
+            return ops.permute(x, ids)
+
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        call(x, ids)
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out, rmap = call(x, ids)
+    for _ in range(3):
+        call(big, big_ids)
+        since = [torch.full((n,), 7, dtype=torch.uint8, device=dev) for n in (1, 512, 1024, 10240, 20480, 40960, 1 << 20) for _ in range(8)]
+        ids.copy_(torch.randint(0, 3, ids.shape, generator=g, device=dev, dtype=ids_dtype))
+        graph.replay()
+        torch.cuda.synchronize()
+        want, want_map = call(x, ids)
+        assert torch.equal(rmap, want_map) and torch.equal(out, want)
+        assert all(bool((t == 7).all()) for t in since)
+
+
+@pytest.mark.gpu
+def test_permute_from_several_threads_with_streams_of_their_own(dev):
+    """Forward and backward of more than 4096 keys from four threads at once equal the calls one after the other."""
+    g = torch.Generator(device=dev).manual_seed(11)
+    cases = []
+    for i in range(4):
+        dtype = (torch.bfloat16, torch.float32)[i & 1]
+        cases.append((torch.randn((4500 + 1000 * i, 64), generator=g, device=dev).to(dtype),
+                      torch.randint(0, 2 + i, (4500 + 1000 * i, 1 + i % 2), generator=g, device=dev, dtype=torch.int32)))
+
+    def one(i):
+        x, ids = cases[i][0].detach().requires_grad_(), cases[i][1]
+        out, rmap = ops.permute(x, ids)
+        return [out.detach(), rmap, *torch.autograd.grad(out, x, out.detach())]
+
+    want = [one(i) for i in range(4)]
+    got, errors = [[] for _ in range(4)], []
+    torch.cuda.synchronize()
+
+    def thread(i):
+        try:
+            stream = torch.cuda.Stream()
+            with torch.cuda.stream(stream):
+                for _ in range(10):
+                    got[i].append(one(i))
+            stream.synchronize()
+        except Exception as exc:  # noqa: BLE001 - reported below
+            errors.append(exc)
+
+    threads = [threading.Thread(target=thread, args=(i,)) for i in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not errors, errors
+    for made, expect in zip(got, want):
+        assert len(made) == 10
+        for result in made:
+            assert all(torch.equal(a, b) for a, b in zip(result, expect))
+
+
+@pytest.mark.gpu
+def test_permute_keeps_the_status_word_of_a_workspace_and_nothing_else_of_it(dev):
+    x = torch.randn((5000, 64), device=dev)
+    ids = torch.zeros((5000, 1), dtype=torch.int32, device=dev)
+    _, _, ws = native.permute(x, ids, 0, [], 0)
+    before = ws[0].fill_(3).clone()
+    out, rmap, again = native.permute(x, ids, 0, ws, 0)
+    assert again is ws and torch.equal(ws[0], before) and not int(ws[1]) and torch.equal(out, x)
+    native.permute(x, ids.fill_(native.MAX_EXPERTS), 0, ws, 0)
+    assert int(ws[1]) == 1 and torch.equal(ws[0], before)
+    native.permute(x, ids.long(), 0, ws, 0)  # the general path
+    assert torch.equal(ws[0], before)
+    assert native.permute(x, ids.zero_(), 0, None, 0)[2] is None

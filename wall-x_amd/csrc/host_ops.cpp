@@ -167,29 +167,34 @@ PyObject* rope(PyObject*, PyObject* const* args, Py_ssize_t n) {
 }
 
 // permute(input [T, H], indices int32 [T, K], num_out_tokens, histograms, status, experts) -> (permuted, row_id_map) or None.
-// The scratch is the caller's, and large enough (else the general path makes another).
+// The scratch is the caller's, and large enough (else the general path makes another), or with None this call's own; no status
+// word with None.
 PyObject* permute(PyObject*, PyObject* const* args, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   int64_t num_out, experts;
   if (n != 6 || !entry.partition || !to_int(args[2], num_out) || !to_int(args[5], experts)) return none();
-  const at::Tensor *x = plain(args[0]), *ids = plain(args[1]), *hist = plain(args[3]), *status = plain(args[4]);
-  if (!x || !ids || !hist || !status || x->dim() != 2 || ids->dim() != 2 || !x->is_contiguous() || !ids->is_contiguous()) return none();
+  const at::Tensor *x = plain(args[0]), *ids = plain(args[1]), *hist = args[3] == Py_None ? nullptr : plain(args[3]),
+                   *status = args[4] == Py_None ? nullptr : plain(args[4]);
+  if (!x || !ids || (args[3] != Py_None && !hist) || (args[4] != Py_None && !status)) return none();
+  if (x->dim() != 2 || ids->dim() != 2 || !x->is_contiguous() || !ids->is_contiguous()) return none();
   const int64_t T = ids->size(0), K = ids->size(1), H = x->size(1);
   const int code = dtype_code(x->scalar_type());
   if (code < 0 || ids->scalar_type() != at::kInt || x->size(0) != T || T <= 0 || K <= 0 || K > 128 || H <= 0 || num_out < 0) return none();
   for (const at::Tensor* t : {ids, hist, status})
-    if (t->device() != x->device()) return none();
-  if (!hist->is_contiguous() || hist->numel() * hist->element_size() < static_cast<int64_t>(entry.partition_bytes(T * K)) || status->numel() < 1) return none();
+    if (t && t->device() != x->device()) return none();
+  const int64_t need = static_cast<int64_t>(entry.partition_bytes(T * K));
+  if ((hist && (!hist->is_contiguous() || hist->numel() * hist->element_size() < need)) || (status && status->numel() < 1)) return none();
   at::Tensor out, map;
   const bool ok = run(*x, [&] {
     const at::TensorOptions i32 = ids->options();
     map = at::empty({T * K}, i32);
     at::Tensor offsets = at::empty({experts + 1}, i32);
     out = at::empty({num_out > 0 ? num_out : T * K, H}, x->options());
+    const at::Tensor scratch = hist ? *hist : at::empty({need}, x->options().dtype(at::kByte));
     const wx_stream_t stream = stream_of(*x);
     const int rc = entry.partition(ptr(*ids), WX_I32, T, static_cast<int>(K), static_cast<int>(experts), num_out, static_cast<int32_t*>(ptr(map)), nullptr,
-                                   static_cast<int32_t*>(offsets.data_ptr()), static_cast<int32_t*>(status->data_ptr()), ptr(*hist),
-                                   static_cast<size_t>(hist->numel()) * hist->element_size(), stream);
+                                   static_cast<int32_t*>(offsets.data_ptr()), status ? static_cast<int32_t*>(status->data_ptr()) : nullptr, ptr(scratch),
+                                   static_cast<size_t>(scratch.numel()) * scratch.element_size(), stream);
     return rc != 0 ? rc : entry.permute(ptr(*x), ptr(out), static_cast<const int32_t*>(ptr(map)), T, static_cast<int>(K), H, code, stream);
   });
   return ok ? pair(out, map) : nullptr;

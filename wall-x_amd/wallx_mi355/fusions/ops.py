@@ -66,11 +66,7 @@ def asym_dual_gmm(input_expert0, input_expert1, weight_expert0, weight_expert1, 
 
 # ----------------------------------------------------------------------------- permute / unpermute
 class PermuteMoE_topK(torch.autograd.Function):
-    """ops.py:175-274.  The scratch workspace is cached on the class like the reference's."""
-
-    workspace_fw = None
-    dtype = None
-    max_expanded_token_num = 0
+    """ops.py:175-274.  The scratch is each call's own (the reference caches one on the class)."""
 
     @staticmethod
     def forward(ctx, input_act, indices, num_out_tokens, max_token_num):
@@ -98,17 +94,9 @@ class PermuteMoE_topK(torch.autograd.Function):
             warnings.warn("The input `indices` of permute_topK op is discontiguous!")
             indices = indices.contiguous()
 
-        cls = PermuteMoE_topK
         num_topK = indices.size(1)
-        want = max(max_token_num, input_act.size(0)) * num_topK
-        if cls.max_expanded_token_num < want:
-            cls.max_expanded_token_num = want
-            cls.workspace_fw = []
-        if cls.dtype != input_act.dtype:
-            cls.dtype = input_act.dtype
-            cls.workspace_fw = []
-        permuted_act, row_id_map, cls.workspace_fw = backend.permute(
-            input_act, indices, num_out_tokens, cls.workspace_fw, cls.max_expanded_token_num)
+        permuted_act, row_id_map, _ = backend.permute(input_act, indices, num_out_tokens, None,
+                                                      max(max_token_num, input_act.size(0)) * num_topK)
         ctx.set_materialize_grads(False)  # no zeros for row_id_map's gradient, which nothing reads
         ctx.permuted_like = (permuted_act.shape, permuted_act.dtype, permuted_act.device)
         ctx.row_id_map = row_id_map

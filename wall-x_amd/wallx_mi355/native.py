@@ -219,11 +219,15 @@ def permute_rows(input: torch.Tensor, row_id_map: torch.Tensor, num_topk: int, n
 MAX_EXPERTS = 256
 
 
-def permute(input: torch.Tensor, indices: torch.Tensor, num_out_tokens: int, workspace: List[torch.Tensor],
-            max_expanded_token_num: int) -> Tuple[torch.Tensor, torch.Tensor, List[torch.Tensor]]:
-    """csrc/permute.cu:450-630: (permuted [num_out, H], row_id_map int32 [T*K], workspace)."""
-    if workspace and not _checked:
-        made = _lib.host().permute(input, indices, num_out_tokens, workspace[0], workspace[1], MAX_EXPERTS)
+def permute(input: torch.Tensor, indices: torch.Tensor, num_out_tokens: int, workspace: Optional[List[torch.Tensor]],
+            max_expanded_token_num: int) -> Tuple[torch.Tensor, torch.Tensor, Optional[List[torch.Tensor]]]:
+    """csrc/permute.cu:450-630: (permuted [num_out, H], row_id_map int32 [T*K], workspace).
+
+    Of `workspace` ([] or what an earlier call returned) only the status word workspace[1] is used; None keeps none.  The
+    histograms, which one launch writes and the next reads, are every call's own: callers keep one list for all their
+    calls, and two streams, two threads or a graph and the calls beside it must not share them."""
+    if not _checked and (workspace or workspace is None):
+        made = _lib.host().permute(input, indices, num_out_tokens, None, workspace[1] if workspace else None, MAX_EXPERTS)
         if made is not None:
             return made[0], made[1], workspace
     _need_cuda("input", input)
@@ -237,7 +241,13 @@ def permute(input: torch.Tensor, indices: torch.Tensor, num_out_tokens: int, wor
     T, K = indices.shape
     if K > 128:
         raise RuntimeError("num_topK cannot exceed 128.")  # csrc/permute.cu:394
-    row_id_map, _, _, workspace = partition(indices, MAX_EXPERTS, num_out_tokens, workspace)
+    scratch = workspace
+    if workspace is None or (workspace and workspace[1].device == indices.device):
+        need = _lib.load().wx_partition_workspace_bytes(T * K)
+        buf = torch.empty(need + 4, dtype=torch.uint8, device=indices.device)
+        scratch = [buf, workspace[1] if workspace else buf[need:].view(torch.int32)]
+    row_id_map, _, _, scratch = partition(indices, MAX_EXPERTS, num_out_tokens, scratch)
+    workspace = workspace if workspace or workspace is None else scratch
     num_out = num_out_tokens if num_out_tokens and num_out_tokens > 0 else T * K
     permuted = permute_rows(input, row_id_map, K, num_out)
     return permuted, row_id_map, workspace
