@@ -125,6 +125,13 @@ struct Group {
   const __bf16* add;  // generic: optional [m, n] row-major (ldc) matrix added to the product (may be c itself)
 };
 
+// The two launches of a problem of more than one round of large tiles (tail_plan).
+struct TailPlan {
+  int rows[2];  // row blocks of 256 of each expert that are large tiles
+  int first;    // large tiles of the first launch
+  bool split;   // whether there is a second one
+};
+
 struct Params {
   Group g[2];
   const int32_t* offsets;  // device int32[3]: rows of expert e are [offsets[e], offsets[e+1]); null for kGeneric
@@ -135,8 +142,11 @@ struct Params {
   int gate, gate_tiles;
   // Tail split (see tail_plan): 0 = off; 1 = this launch does the whole rounds of 256 x 256 tiles and leaves
   // the ragged last round to a second launch; 2 = this is that second launch, with 128 x 128 tiles.
-  // split_cus = workgroups of the first launch (one per CU).
+  // split_cus = workgroups of the first launch (one per CU).  plan: the launches' plan where the host alone makes it (kGeneric,
+  // kQkvRope, kQkvRopeFull).  (Made again by every workgroup of both launches: 1656 rows of 11008 columns, contractions of 64
+  // to 4096, 0.6 us longer.)
   int split, split_cus;
+  TailPlan plan;
   // kDown only: when set (the partition's sorted_row_id), row r of the sorted result is stored to row scatter[r] of
   // the output instead of row r -- the unpermute folded into the store.
   const int32_t* scatter;
@@ -252,11 +262,6 @@ __host__ __device__ inline int tail_split_point(int tiles0, int tiles1, int k0, 
 // and 172 small ones: us a layer 158 -> 146, 2310 to 2400 rows 318 to 323 -> 307 to 311, 1656 rows 240 -> 230.
 // The rounds are counted in kTailRound-ths of a round of large tiles: kTailOne for a launch of small tiles with one to a CU,
 // kTailTwo with two (contractions of 2048, us: 47 to 56, 20 to 25, 37).
-struct TailPlan {
-  int rows[2];  // row blocks of 256 of each expert that are large tiles
-  int first;    // large tiles of the first launch
-  bool split;   // whether there is a second one
-};
 constexpr int kTailRound = 10, kTailOne = 4, kTailTwo = 8;
 __host__ __device__ inline TailPlan tail_plan(int m0, int m1, int cols0, int cols1, int k0, int k1, int cus, bool strips) {
   TailPlan p;
@@ -1121,7 +1126,11 @@ __device__ __forceinline__ void dual_gemm_body(const Params& p, const int wg, co
     big_n[0] = (g0.n + kBigN - 1) / kBigN;
     big_n[1] = (g1.n + kBigN - 1) / kBigN;
     const bool any0 = g0.m > 0 && g0.n > 0, any1 = g1.m > 0 && g1.n > 0;
-    const TailPlan plan = tail_plan(any0 ? g0.m : 0, any1 ? g1.m : 0, any0 ? big_n[0] : 0, any1 ? big_n[1] : 0, g0.k, g1.k, p.split_cus, MODE != kDown);
+    TailPlan plan;
+    if constexpr (MODE == kGateUp || MODE == kDown)
+      plan = tail_plan(any0 ? g0.m : 0, any1 ? g1.m : 0, any0 ? big_n[0] : 0, any1 ? big_n[1] : 0, g0.k, g1.k, p.split_cus, MODE != kDown);
+    else
+      plan = p.plan;
     if (!any0) big_n[0] = 0;
     if (!any1) big_n[1] = 0;
     big_m[0] = plan.rows[0];
@@ -2464,7 +2473,8 @@ int launch_mfma(Params p, int64_t tiles_lo, int64_t tiles_hi, hipStream_t s, con
         split = false;
       } else if (rows != nullptr) {
         auto cols = [&](int e) { return rows[e] > 0 ? static_cast<int>(tiles_by_expert[e] / ceil_div(rows[e], BigTile::BM)) : 0; };
-        split = tail_plan(static_cast<int>(rows[0]), static_cast<int>(rows[1]), cols(0), cols(1), p.g[0].k, p.g[1].k, cus, true).split;
+        p.plan = tail_plan(static_cast<int>(rows[0]), static_cast<int>(rows[1]), cols(0), cols(1), p.g[0].k, p.g[1].k, cus, true);
+        split = p.plan.split;
       } else {
         split = tail_split_point(static_cast<int>(tiles_by_expert[0]), static_cast<int>(tiles_by_expert[1]), p.g[0].k, p.g[1].k, cus) != all;
       }
@@ -2634,7 +2644,8 @@ extern "C" int wx_qkv_rope_proj(const void* x, const void* weight, const void* b
   // The table, this launch and the o projection at n 2560, k 2048: 32 rows 66 -> 45 us, 1024 rows 70 -> 48, 2048 rows
   // 73 -> 63, 3072 rows 83 -> 76; one more row of large tiles is past the line.
   const bool small = tiles <= cus / 2;
-  const bool split = !small && tiles < INT32_MAX && tail_plan(g.m, 0, static_cast<int>(ceil_div(g.n, Tile::BN)), 0, g.k, 0, cus, true).split;
+  if (!small && tiles < INT32_MAX) p.plan = tail_plan(g.m, 0, static_cast<int>(ceil_div(g.n, Tile::BN)), 0, g.k, 0, cus, true);
+  const bool split = p.plan.split;
   p.split = split ? 1 : 0;
   p.split_cus = cus;
   hipStream_t s = as_stream(stream);
