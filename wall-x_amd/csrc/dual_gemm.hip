@@ -141,7 +141,7 @@ struct Params {
   // 2 = run if more.
   int gate, gate_tiles;
   // Tail split (see tail_plan): 0 = off; 1 = this launch does the whole rounds of 256 x 256 tiles and leaves
-  // the ragged last round to a second launch; 2 = this is that second launch, with 128 x 128 tiles.
+  // the ragged last round to a second launch, with 128 x 128 tiles (ROLE 4).
   // split_cus = workgroups of the first launch (one per CU).  plan: the launches' plan where the host alone makes it (kGeneric,
   // kQkvRope, kQkvRopeFull).  (Made again by every workgroup of both launches: 1656 rows of 11008 columns, contractions of 64
   // to 4096, 0.6 us longer.)
@@ -980,7 +980,8 @@ __device__ __forceinline__ void few_rows_body(const Params& p, const int wg, con
 // launch below: some workgroups run the gate/up form, the others the down form).  `wg` of `n_wg` is the workgroup's
 // place among those that share this body's tile list (blockIdx.x of gridDim.x in a plain launch).
 // ROLE: 0 = a plain launch; 1 / 2 = producer / consumer of a fused launch (see FusedSync); 3 = the contraction in parts, as
-// `parts` says, with the scratch `split`.  AROWS (gate/up form of a fused launch): the A operand is read from the token rows themselves,
+// `parts` says, with the scratch `split`; 4 = the second launch of a tail split, an instantiation of its own (a launch of small
+// tiles alone that carries its code too runs 0.2 to 0.3 us longer: o projection of 512 rows, hidden 2048, 16.3 -> 15.95).  AROWS (gate/up form of a fused launch): the A operand is read from the token rows themselves,
 // fs.x through fs.gather, instead of from a K-tiled copy of them.
 template <int MODE, typename TS, bool KA, bool KB, int ROLE, bool AROWS = false>
 __device__ __forceinline__ void dual_gemm_body(const Params& p, const int wg, const int n_wg, const FusedSync& fs,
@@ -1118,10 +1119,11 @@ __device__ __forceinline__ void dual_gemm_body(const Params& p, const int wg, co
   int total = tiles_m[0] * tiles_n[0] + tiles_m[1] * tiles_n[1];  // the host bounds this below 2^31
   // tail split (tail_plan): the first launch (256 x 256 tiles) stops at `split_at`; the second (this shape: 128 x 128)
   // takes virtual tiles [split_at, all) of the 256 x 256 tiling, kSubM x kSubN pieces each, and then the strips
-  constexpr bool kIsTail = std::is_same_v<TS, TailTileFor<MODE>>, kIsBig = std::is_same_v<TS, BigTileFor<MODE>>;
+  constexpr bool kIsTail = ROLE == 4, kIsBig = ROLE == 0 && std::is_same_v<TS, BigTileFor<MODE>>;
+  static_assert(!kIsTail || std::is_same_v<TS, TailTileFor<MODE>>, "the second launch's tile");
   constexpr int kSubM = BigTile::BM / BM, kSubN = BigTile::BN / BN;
   int big_m[2], big_n[2], split_at = 0, pieces = 0, strip_cols[2] = {0, 0};
-  if (ROLE != 3 && ((kIsBig && p.split == 1) || (kIsTail && p.split == 2))) {
+  if (kIsTail || (kIsBig && p.split == 1)) {
     constexpr int kBigN = SWIGLU ? BigTile::BN / 2 : BigTile::BN;
     big_n[0] = (g0.n + kBigN - 1) / kBigN;
     big_n[1] = (g1.n + kBigN - 1) / kBigN;
@@ -2070,7 +2072,7 @@ __device__ __forceinline__ void dual_gemm_body(const Params& p, const int wg, co
   int next_t = wg;
   auto next_tile = [&](TileCoord& tc) {
     bool have = false;
-    if (kIsTail && p.split == 2) {
+    if constexpr (kIsTail) {
       for (; next_t < pieces && !have; next_t += n_wg) {
         const int piece = next_t % (kSubM * kSubN);
         tile_coords(split_at + next_t / (kSubM * kSubN), big_m, big_n, tc);
@@ -2251,9 +2253,9 @@ __device__ __forceinline__ void dual_gemm_body(const Params& p, const int wg, co
 #endif
 }
 
-template <int MODE, typename TS, bool KA = false, bool KB = false>
+template <int MODE, typename TS, bool KA = false, bool KB = false, int ROLE = 0>
 __global__ __launch_bounds__(TS::kThreads, TS::kWgPerCu) void dual_gemm_kernel(Params p) {
-  dual_gemm_body<MODE, TS, KA, KB, 0>(p, blockIdx.x, gridDim.x, FusedSync{});
+  dual_gemm_body<MODE, TS, KA, KB, ROLE>(p, blockIdx.x, gridDim.x, FusedSync{});
 }
 
 // The down launch whose contraction may be in parts: the plain form or the parts', by the row counts.  Rows that are not cut
@@ -2484,11 +2486,8 @@ int launch_mfma(Params p, int64_t tiles_lo, int64_t tiles_hi, hipStream_t s, con
       hipLaunchKernelGGL(down_split_kernel<BigTile>, dim3(cus), dim3(BigTile::kThreads), 0, s, p, *parts);
     else
       hipLaunchKernelGGL((dual_gemm_kernel<MODE, Big, KA, KB>), dim3(cus), dim3(Big::kThreads), 0, s, p);
-    if (split) {
-      p.split = 2;
-      hipLaunchKernelGGL((dual_gemm_kernel<MODE, TailTile, KA, KB>), dim3(cus * TailTile::kWgPerCu),
-                         dim3(TailTile::kThreads), 0, s, p);
-    }
+    if (split)
+      hipLaunchKernelGGL((dual_gemm_kernel<MODE, TailTile, KA, KB, 4>), dim3(cus * TailTile::kWgPerCu), dim3(TailTile::kThreads), 0, s, p);
   }
   return check_launch(who);
 }
@@ -2649,23 +2648,15 @@ extern "C" int wx_qkv_rope_proj(const void* x, const void* weight, const void* b
   p.split = split ? 1 : 0;
   p.split_cus = cus;
   hipStream_t s = as_stream(stream);
-  if (table_width == head_dim) {
-    if (!small)
-      hipLaunchKernelGGL((dual_gemm_kernel<kQkvRopeFull, Tile, false, false>), dim3(cus), dim3(Tile::kThreads), 0, s, p);
-    if (split || small) {
-      p.split = split ? 2 : 0;
-      hipLaunchKernelGGL((dual_gemm_kernel<kQkvRopeFull, Tail, false, false>), dim3(cus * Tail::kWgPerCu),
-                         dim3(Tail::kThreads), 0, s, p);
-    }
-  } else {
-    if (!small)
-      hipLaunchKernelGGL((dual_gemm_kernel<kQkvRope, Tile, false, false>), dim3(cus), dim3(Tile::kThreads), 0, s, p);
-    if (split || small) {
-      p.split = split ? 2 : 0;
-      hipLaunchKernelGGL((dual_gemm_kernel<kQkvRope, Tail, false, false>), dim3(cus * Tail::kWgPerCu),
-                         dim3(Tail::kThreads), 0, s, p);
-    }
-  }
+  auto launch = [&](auto large, auto alone, auto second) {
+    if (small) hipLaunchKernelGGL(alone, dim3(cus * Tail::kWgPerCu), dim3(Tail::kThreads), 0, s, p);
+    else hipLaunchKernelGGL(large, dim3(cus), dim3(Tile::kThreads), 0, s, p);
+    if (split) hipLaunchKernelGGL(second, dim3(cus * Tail::kWgPerCu), dim3(Tail::kThreads), 0, s, p);
+  };
+  if (table_width == head_dim)
+    launch(dual_gemm_kernel<kQkvRopeFull, Tile>, dual_gemm_kernel<kQkvRopeFull, Tail>, dual_gemm_kernel<kQkvRopeFull, Tail, false, false, 4>);
+  else
+    launch(dual_gemm_kernel<kQkvRope, Tile>, dual_gemm_kernel<kQkvRope, Tail>, dual_gemm_kernel<kQkvRope, Tail, false, false, 4>);
   return check_launch("dual_gemm_kernel<qkv_rope>");
 }
 
