@@ -289,6 +289,22 @@ def test_dual_gemm_with_a_strip_of_small_tiles(dev, trans_a, trans_b, m0, m1, n)
     assert torch.equal(add[0], summed[0]) and torch.equal(add[1], summed[1])
 
 
+@pytest.mark.parametrize("trans_b", [False, True])
+@pytest.mark.parametrize("m0,m1,n,k", [(2150, 0, 11008, 1272), (2150, 0, 11008, 1280), (2100, 40, 11008, 1280), (384, 0, 65792, 1280)])
+def test_dual_gemm_with_strips_two_to_a_cu(dev, trans_b, m0, m1, n, k):
+    """Strips and what the whole rounds leave are more small tiles than CUs: in a second launch from a contraction of 1280 on, as
+    large tiles below it, and as large tiles where they are more than two to a CU."""
+    g = torch.Generator(device=dev).manual_seed(k + n)
+    a = [torch.randn((m, k), device=dev, generator=g).to(torch.bfloat16) for m in (m0, m1)]
+    w = [torch.randn((c, k) if trans_b else (k, c), device=dev, generator=g).to(torch.bfloat16) for c in (n, 264)]
+    out = [torch.full((m, c), float("nan"), device=dev, dtype=torch.bfloat16) for m, c in ((m0, n), (m1, 264))]
+    native.asym_dual_gmm(a[0], a[1], w[0], w[1], out[0], out[1], False, trans_b)
+    for got, x, y in zip(out, a, w):
+        x, y = x.float(), (y.t() if trans_b else y).float()
+        # one rounding to bf16 (2^-9 of the value) and fp32 sums of k products
+        assert bool(((got.float() - x @ y).abs() <= 2 ** -8 * (x @ y).abs() + 1e-5 * (x.abs() @ y.abs())).all())
+
+
 @pytest.mark.parametrize("T,n_act,hidden,inters", [
     (8600, 300, 2048, (1056, 256)),   # gate/up: 301 large tiles, 45 left over, among them a ragged last column
     (8600, 8300, 2048, (256, 1056)),  # the action expert is the long one

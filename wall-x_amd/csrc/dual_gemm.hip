@@ -261,9 +261,16 @@ __host__ __device__ inline int tail_split_point(int tiles0, int tiles1, int k0, 
 // and 88 left over that take 37 us as small ones, where three whole row blocks and a strip are one round, two large tiles
 // and 172 small ones: us a layer 158 -> 146, 2310 to 2400 rows 318 to 323 -> 307 to 311, 1656 rows 240 -> 230.
 // The rounds are counted in kTailRound-ths of a round of large tiles: kTailOne for a launch of small tiles with one to a CU,
-// kTailTwo with two (contractions of 2048, us: 47 to 56, 20 to 25, 37).
-constexpr int kTailRound = 10, kTailOne = 4, kTailTwo = 8;
-__host__ __device__ inline TailPlan tail_plan(int m0, int m1, int cols0, int cols1, int k0, int k1, int cus, bool strips) {
+// kTailTwo with two (contractions of 2048, us: 47 to 56, 20 to 25, 37; row-major 45, 30, 41), none with more (384 rows of 76800
+// columns as 776 small tiles behind one round in place of 352 behind two: 147 -> 158).  What a launch costs beside its contraction, 10 us
+// with two to a CU against 4 of a round behind another, makes two the dearer below contractions of `length`: row-major, 3704
+// rows of 11008 columns, a round and 446 small tiles, us: K 256 31 and 36, 512 46 and 49, 1024 level, 1280 90.8 and 90.3, 2048 129
+// and 127; 2150 rows 23.2 and 25.3, 32.2 and 33.7, level, 58.1 and 57.3, 84 and 80; gate/up of the same tiles, us a layer, K 1280
+// 105.2 and 106.5, 1536 119.0 and 118.4, 2048 161 and 160.  (One to a CU in place of two pays at any: 880 rows of 22016 columns,
+// K 256, 24.0 -> 23.0.)
+constexpr int kTailRound = 10, kTailOne = 4, kTailTwo = 8, kTailNever = 1 << 28;
+constexpr int kTailLongRows = 1280, kTailLongTiled = 1536;  // `length` of the row-major and the K-tiled operands
+__host__ __device__ inline TailPlan tail_plan(int m0, int m1, int cols0, int cols1, int k0, int k1, int cus, bool strips, int length) {
   TailPlan p;
   p.rows[0] = (m0 + 255) >> 8;
   p.rows[1] = (m1 + 255) >> 8;
@@ -276,7 +283,8 @@ __host__ __device__ inline TailPlan tail_plan(int m0, int m1, int cols0, int col
   const int pieces = 2 * (strip0 * cols0 + strip1 * cols1);
   if (pieces == 0) return p;
   const int large = total - pieces / 2, full = large / cus, left = large - full * cus, whole = total / cus;
-  auto small = [&](int n) { return n <= 0 ? 0 : (n <= cus ? kTailOne : (n <= 2 * cus ? kTailTwo : 4 * kTailRound)); };
+  const int two = (tiles0 == 0 ? k1 : (tiles1 == 0 || k0 < k1 ? k0 : k1)) >= length ? kTailTwo : kTailRound + 2;
+  auto small = [&](int n) { return n <= 0 ? 0 : (n <= cus ? kTailOne : (n <= 2 * cus ? two : kTailNever)); };
   const int as_is = whole * kTailRound + (p.split ? small(4 * (total - p.first)) : (total > whole * cus ? kTailRound : 0));
   const int both = full > 0 ? full * kTailRound + small(4 * left + pieces) : as_is;  // strips and what the whole rounds leave
   const int alone = (full + (left > 0 ? 1 : 0)) * kTailRound + small(pieces);       // strips alone
@@ -1130,7 +1138,7 @@ __device__ __forceinline__ void dual_gemm_body(const Params& p, const int wg, co
     const bool any0 = g0.m > 0 && g0.n > 0, any1 = g1.m > 0 && g1.n > 0;
     TailPlan plan;
     if constexpr (MODE == kGateUp || MODE == kDown)
-      plan = tail_plan(any0 ? g0.m : 0, any1 ? g1.m : 0, any0 ? big_n[0] : 0, any1 ? big_n[1] : 0, g0.k, g1.k, p.split_cus, MODE != kDown);
+      plan = tail_plan(any0 ? g0.m : 0, any1 ? g1.m : 0, any0 ? big_n[0] : 0, any1 ? big_n[1] : 0, g0.k, g1.k, p.split_cus, MODE != kDown, kTailLongTiled);
     else
       plan = p.plan;
     if (!any0) big_n[0] = 0;
@@ -2475,7 +2483,7 @@ int launch_mfma(Params p, int64_t tiles_lo, int64_t tiles_hi, hipStream_t s, con
         split = false;
       } else if (rows != nullptr) {
         auto cols = [&](int e) { return rows[e] > 0 ? static_cast<int>(tiles_by_expert[e] / ceil_div(rows[e], BigTile::BM)) : 0; };
-        p.plan = tail_plan(static_cast<int>(rows[0]), static_cast<int>(rows[1]), cols(0), cols(1), p.g[0].k, p.g[1].k, cus, true);
+        p.plan = tail_plan(static_cast<int>(rows[0]), static_cast<int>(rows[1]), cols(0), cols(1), p.g[0].k, p.g[1].k, cus, true, MODE == kGateUp ? kTailLongTiled : kTailLongRows);
         split = p.plan.split;
       } else {
         split = tail_split_point(static_cast<int>(tiles_by_expert[0]), static_cast<int>(tiles_by_expert[1]), p.g[0].k, p.g[1].k, cus) != all;
@@ -2643,7 +2651,7 @@ extern "C" int wx_qkv_rope_proj(const void* x, const void* weight, const void* b
   // The table, this launch and the o projection at n 2560, k 2048: 32 rows 66 -> 45 us, 1024 rows 70 -> 48, 2048 rows
   // 73 -> 63, 3072 rows 83 -> 76; one more row of large tiles is past the line.
   const bool small = tiles <= cus / 2;
-  if (!small && tiles < INT32_MAX) p.plan = tail_plan(g.m, 0, static_cast<int>(ceil_div(g.n, Tile::BN)), 0, g.k, 0, cus, true);
+  if (!small && tiles < INT32_MAX) p.plan = tail_plan(g.m, 0, static_cast<int>(ceil_div(g.n, Tile::BN)), 0, g.k, 0, cus, true, kTailLongRows);
   const bool split = p.plan.split;
   p.split = split ? 1 : 0;
   p.split_cus = cus;
