@@ -2422,6 +2422,8 @@ int check_dims(const char* who, int64_t m, int64_t n, int64_t k, bool k_in_rows 
   return WX_OK;
 }
 
+int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
+
 // The problem has between `tiles_lo` and `tiles_hi` 256 x 256 tiles (equal when the host knows the row counts).
 // When they would occupy at most half of the CUs, the 128 x 128 tile gives four times as many workgroups to spread
 // over the chip.  If the bounds fall on both sides of that threshold the choice is made on the device: both
@@ -2434,8 +2436,7 @@ int check_dims(const char* who, int64_t m, int64_t n, int64_t k, bool k_in_rows 
 // second returns at once if there is nothing to split).
 // few: the few-rows form takes the problem; its number of rows, or 0.
 // parts: the down launch's contraction may be in parts (PartsRule), with this scratch.
-int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
-
+// rows: with tiles_by_expert, the rows of each expert (0 for one without columns), for the plan with strips (always for kGeneric).
 template <int MODE, bool KA = false, bool KB = false>
 int launch_mfma(Params p, int64_t tiles_lo, int64_t tiles_hi, hipStream_t s, const char* who,
                 const int64_t* tiles_by_expert = nullptr, int64_t few = 0, const DownSplit* parts = nullptr,
