@@ -61,8 +61,7 @@ def _newer(target: str, deps) -> bool:
 # memory, which costs a factor of three and shows in no test of results.  Their compile prints the resource-usage remarks
 # and this limit on "ScratchSize [bytes/lane]" of any kernel of the file turns a spill into a loud warning.
 # (Values that are only live outside the K loop do spill: 56 bytes in the few-rows kernel with the norm and 64-row B tiles, 8 in
-# the large tile with a K-major A, 24 in the down launch's parts of large tiles;
-# tests/test_k_loop_assembly.py shows that none is inside a loop.)
+# the large tile with a K-major A; tests/test_k_loop_assembly.py shows that none is inside a loop.)
 RESOURCE_CHECKED = {"dual_gemm.hip": 96}
 
 

@@ -1796,9 +1796,10 @@ __device__ __forceinline__ void dual_gemm_body(const Params& p, const int wg, co
     // chunks kAhead row blocks in front of their use.  (Asked for row block by row block, a tile of 256 rows waited for eight
     // memory latencies one after the other, twice over with row ids and an addend: q / k / v and o projections of 14592 rows with
     // the rotary table's loads a row block ahead as well 291.6 -> 283.9 us, a layer of 912 rows 157 -> 155, training on 29184 rows
-    // 9630 -> 9600.)  Three row blocks where the row ids take registers: with four the kernel with the parts spills 56 bytes.
+    // 9630 -> 9600.)  Three row blocks where the row ids take registers, two in the kernel with the
+    // parts, which spills 24 bytes with three (56 with four): layers of 2049 to 3500 rows on device-side counts 0.6 % longer.
     // Rows past the tile's end read a row that is there.
-    constexpr int kMost = MODE == kDown ? 3 : 4, kAhead = FM < kMost ? FM : kMost;
+    constexpr int kMost = ROLE == 3 ? 2 : (MODE == kDown ? 3 : 4), kAhead = FM < kMost ? FM : kMost;
     auto row_of = [&](int i, int q) { return (wm * FM + i) * 16 + q * kRowsPerStore + rl; };
     // (a wavefront's ids: a lane has those of rows lane, lane + 64, .. of its share, and hands them out)
     constexpr int kIds = MODE == kDown ? (FM * 16 + 63) / 64 : 1;
