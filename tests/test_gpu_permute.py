@@ -242,3 +242,17 @@ def test_partition_of_ragged_segments(dev, T, E):
     _, ref_map, ref_sorted = oracle.permute_ref(torch.zeros(T, 8), ids)
     assert torch.equal(rmap.cpu(), ref_map) and torch.equal(srt.cpu(), ref_sorted)
     assert torch.equal(off.cpu(), oracle.expert_offsets_ref(ids, E))
+
+
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 1023, 1024, 1025, 2049, 3072, 3073, 4095, 4096, 4097])
+@pytest.mark.parametrize("dtype,experts", [(torch.bool, 2), (torch.int32, 5), (torch.int64, 256)])
+def test_partition_at_the_edges_of_its_groups_of_keys(dev, n, dtype, experts):
+    """One to four groups of 64 keys a wavefront in the one-launch form (up to 4096 keys), and the two launches behind it."""
+    g = torch.Generator(device=dev).manual_seed(n)
+    ids = torch.randint(0, experts, (n, 1), generator=g, device=dev).to(dtype)
+    rmap, offsets, inverse, _ = native.partition(ids, experts, 0, want_sorted=True)
+    order = ids.view(-1).to(torch.int64).sort(stable=True).indices
+    assert torch.equal(inverse.long(), order)
+    assert torch.equal(rmap.long()[order], torch.arange(n, device=dev))
+    counts = torch.bincount(ids.view(-1).to(torch.int64), minlength=experts)
+    assert torch.equal(offsets.long(), torch.cat((counts.new_zeros(1), counts.cumsum(0))))

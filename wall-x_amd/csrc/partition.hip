@@ -35,8 +35,7 @@ __device__ __forceinline__ int load_key(const void* ids, int itype, int64_t i, i
 }
 
 // The keys of kAhead groups of 64 from `base` on (a lane past `end` holds 0).  They are asked for together: a wavefront that
-// loads one group at a time waits out a memory latency per group: partition_count of 14593 int32 keys 7.6 -> 5.6 us.  (Not in
-// partition_small_kernel: its wavefronts have a few groups only and lost 4 us on 1424 keys.)
+// loads one group at a time waits out a memory latency per group: partition_count of 14593 int32 keys 7.6 -> 5.6 us.
 constexpr int kAhead = 8;
 constexpr int kHistAhead = 32;  // histograms
 static_assert(kHistAhead % kWavesPerBlock == 0, "a block's segments lie in one trip");
@@ -177,6 +176,10 @@ __global__ __launch_bounds__(kBlock) void partition_scatter(
 // two launches over many CUs (36 us against 15 at 29184 keys).
 constexpr int kSmallWaves = 16;
 constexpr int64_t kSmallKeys = 4096;
+// Groups of 64 keys of a wavefront at most.  All of them are read at once and kept for both passes: with a read per group and
+// pass, each waited for ahead of the counts' own barriers, 2304 two-valued keys took 6.45 us, now 5.86, 4096 8.3 and 7.3 (8.1 with the
+// reads one by one and the counts key by key), 2000 tokens' two copies among eight experts 11.5 and 10.8.
+constexpr int kSmallGroups = static_cast<int>(kSmallKeys / kSmallWaves / kWave);
 
 __global__ __launch_bounds__(kSmallWaves* kWave) void partition_small_kernel(
     const void* __restrict__ ids, int itype, int64_t num_tokens, int num_topk, int num_experts, int64_t num_out,
@@ -193,12 +196,15 @@ __global__ __launch_bounds__(kSmallWaves* kWave) void partition_small_kernel(
   const int64_t end = begin + chunk < n ? begin + chunk : n;
   bool bad = false;
   __builtin_amdgcn_wave_barrier();
-  for (int64_t base = begin; base < end; base += kWave) {
-    const int64_t i = base + lane;
-    const bool active = i < end;
-    const int key = active ? load_key(ids, itype, i, num_experts, bad) : 0;
-    count_keys(s_run[w], key, active);
+  int key[kSmallGroups];
+#pragma unroll
+  for (int u = 0; u < kSmallGroups; ++u) {
+    const int64_t i = begin + u * kWave + lane;
+    key[u] = i < end ? load_key(ids, itype, i, num_experts, bad) : 0;
   }
+#pragma unroll
+  for (int u = 0; u < kSmallGroups; ++u)
+    if (begin + u * kWave < end) count_keys(s_run[w], key[u], begin + u * kWave + lane < end);
   if (status != nullptr && __ballot(bad) != 0 && lane == 0) *status = 1;
   __syncthreads();
   // bin `tid` (tid < 256): exclusive prefix over the bins of the totals, then running starts per wavefront
@@ -228,11 +234,12 @@ __global__ __launch_bounds__(kSmallWaves* kWave) void partition_small_kernel(
     }
   }
   __syncthreads();
-  for (int64_t base = begin; base < end; base += kWave) {
-    const int64_t i = base + lane;
+#pragma unroll
+  for (int u = 0; u < kSmallGroups; ++u) {
+    if (begin + u * kWave >= end) break;
+    const int64_t i = begin + u * kWave + lane;
     const bool active = i < end;
-    const int key = active ? load_key(ids, itype, i, num_experts, bad) : 0;
-    const int32_t pos = count_keys(s_run[w], key, active);
+    const int32_t pos = count_keys(s_run[w], key[u], active);
     if (active) {
       const int64_t t = i / num_topk, k = i - t * num_topk;
       row_id_map[k * num_tokens + t] = pos < num_out ? pos : -1;
