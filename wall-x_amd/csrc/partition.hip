@@ -250,7 +250,10 @@ __global__ __launch_bounds__(kSmallWaves* kWave) void partition_small_kernel(
 
 // ---- row movers ---------------------------------------------------------------------------------
 constexpr int kMoverWaves = 4;
-constexpr int kMoverPlaces = 8;  // wavefronts per SIMD that the grids count on
+// Workgroups per CU that the grids ask for.  The weighted kernels have registers for four to seven at once; the others start as
+// places come free, which keeps the chip fuller than as many as it holds, each with a row more: weighted backward of 6000 tokens, five
+// or four to a CU -> eight, us: two copies in fp32 41.4 -> 39.4, three in bf16 33.1 -> 31.5, four in fp32 73 -> 69 (forward level).
+constexpr int kMoverGrid = 8;
 
 __device__ __forceinline__ u32x4 ld16(const u32x4* p) { return __builtin_nontemporal_load(p); }
 __device__ __forceinline__ void st16(u32x4* p, const u32x4& v) { __builtin_nontemporal_store(v, p); }
@@ -507,7 +510,7 @@ __global__ __launch_bounds__(kMoverWaves* kWave) void combine_rows_kernel(
 }
 
 // Backward of the weighted combine; one wavefront per token.  (With the copies one after the other and their gradient's row read
-// for each: 8000 tokens of 2048, us, two copies in bf16 39.0 -> 32.8, three in fp32 110 -> 90.)  The rows of act_grad that no token maps to are zeros: the
+// for each, and a chunk at a time: 8000 tokens of 2048, us, two copies in bf16 42 -> 30, three in fp32 110 -> 72.)  The rows of act_grad that no token maps to are zeros: the
 // first `clearers` workgroups find them in their share of the num_rows rows by reading the whole map into a bitmap in LDS, and
 // clear them, beside the workgroups that move rows.  (Clearing all of act_grad in a launch of its own ahead of this one
 // writes every row twice: 14593 rows of 4 KiB 10.4 us + 25.5.)  The search must not take longer than the moving: with 64-bit
@@ -517,7 +520,7 @@ typedef int32_t i32x4_word __attribute__((ext_vector_type(4), aligned(4)));  // 
 constexpr int kClearRows = 65536;  // rows of act_grad one workgroup looks after at a time: 8 KiB of bits
 // COPIES: copies of a token handled together (its gradient's row is read once for all of them); 0 = rows without weights.
 template <int DT, int COPIES>
-__global__ __launch_bounds__(kMoverWaves* kWave, COPIES == 0 ? kMoverPlaces : 5) void combine_rows_bwd_kernel(
+__global__ __launch_bounds__(kMoverWaves* kWave, COPIES == 0 ? 8 : (COPIES == 2 ? 5 : 4)) void combine_rows_bwd_kernel(
     const u32x4* __restrict__ grad_out, const u32x4* __restrict__ y_fwd, u32x4* __restrict__ act_grad,
     float* __restrict__ prob_grad, const int32_t* __restrict__ row_id_map, const float* __restrict__ probs,
     int64_t num_tokens, int num_topk, int64_t vec_per_row, int64_t num_rows, int clearers) {
@@ -599,27 +602,39 @@ __global__ __launch_bounds__(kMoverWaves* kWave, COPIES == 0 ? kMoverPlaces : 5)
           p[c] = Elem<DT>::round(probs[t * num_topk + k]);
           dot[c] = 0.f;
         }
-        for (int64_t v = lane; v < vec_per_row; v += kWave) {
-          const u32x4 graw = ld16(src + v);
-          u32x4 yraw[kCopies];
+        // Two chunks at a time.  (A copy may be missing, so its loads are under a branch, behind which the compiler does not know
+        // how many are in flight and waits for all of them, and for the stores: with a chunk at a time that is a memory latency per
+        // chunk.)  The forward's rows were written a moment ago and are read with plain loads, which find them in the last-level cache.
+        // us, a chunk at a time and non-temporal loads -> now: 668 tokens of 2048, two copies in fp32 14.9 -> 9.6, three 14.3 -> 9.5,
+        // three in fp16 10.2 -> 7.3; 9728 tokens, two copies in bf16 39 -> 35, in fp32 84 -> 62.
+        chunks_of_a_row<2>(lane, vec_per_row, [&](int64_t v, auto n) {
+          constexpr int N = decltype(n)::value;
+          u32x4 graw[N], yraw[kCopies][N];
+#pragma unroll
+          for (int u = 0; u < N; ++u) graw[u] = ld16(src + v + u * kWave);
 #pragma unroll
           for (int c = 0; c < kCopies; ++c)
-            if (r[c] >= 0) yraw[c] = ld16(y_fwd + static_cast<int64_t>(r[c]) * vec_per_row + v);
-          float g[E];
-          unpack16<DT>(graw, g);
 #pragma unroll
-          for (int c = 0; c < kCopies; ++c) {
-            if (r[c] < 0) continue;
-            float yv[E], o[E];
-            unpack16<DT>(yraw[c], yv);
+            for (int u = 0; u < N; ++u)
+              if (r[c] >= 0) yraw[c][u] = y_fwd[static_cast<int64_t>(r[c]) * vec_per_row + v + u * kWave];
 #pragma unroll
-            for (int e = 0; e < E; ++e) {
-              o[e] = Elem<DT>::round(g[e] * p[c]);
-              dot[c] += Elem<DT>::round(g[e] * yv[e]);
+          for (int u = 0; u < N; ++u) {
+            float g[E];
+            unpack16<DT>(graw[u], g);
+#pragma unroll
+            for (int c = 0; c < kCopies; ++c) {
+              if (r[c] < 0) continue;
+              float yv[E], o[E];
+              unpack16<DT>(yraw[c][u], yv);
+#pragma unroll
+              for (int e = 0; e < E; ++e) {
+                o[e] = Elem<DT>::round(g[e] * p[c]);
+                dot[c] += Elem<DT>::round(g[e] * yv[e]);
+              }
+              st16(act_grad + static_cast<int64_t>(r[c]) * vec_per_row + v + u * kWave, pack16<DT>(o));
             }
-            st16(act_grad + static_cast<int64_t>(r[c]) * vec_per_row + v, pack16<DT>(o));
           }
-        }
+        });
 #pragma unroll
         for (int c = 0; c < kCopies; ++c) {
           if (k0 + c >= num_topk) continue;
@@ -642,8 +657,8 @@ int elem_bytes(int dtype) {
 }
 
 int mover_grid(int64_t rows) {
-  // enough resident wavefronts to cover HBM latency: 8 blocks of 4 waves per CU, capped by the row count
-  const int64_t want = static_cast<int64_t>(device_cu_count()) * 8;
+  // enough wavefronts to cover HBM latency: kMoverGrid blocks of 4 per CU, capped by the row count
+  const int64_t want = static_cast<int64_t>(device_cu_count()) * kMoverGrid;
   const int64_t need = (rows + kMoverWaves - 1) / kMoverWaves;
   return static_cast<int>(need < want ? (need < 1 ? 1 : need) : want);
 }
@@ -897,7 +912,7 @@ int unpermute_rows_bwd(const char* who, const void* grad_out, const void* y_fwd,
   // (a workgroup's share of the rows: what it reads is the whole map, so few of them, but enough to clear many rows quickly)
   const int64_t shares = (num_rows + 127) / 128;
   const int clearers = static_cast<int>(shares < 64 ? shares : 64);
-  const int movers = mover_grid(num_tokens), places = device_cu_count() * 8 - clearers;  // (all of them have a place at once)
+  const int movers = mover_grid(num_tokens), places = device_cu_count() * kMoverGrid - clearers;
   const dim3 grid(static_cast<unsigned>((movers < places ? movers : places) + clearers)), block(kMoverWaves * kWave);
   const u32x4* g = static_cast<const u32x4*>(grad_out);
   const u32x4* yf = static_cast<const u32x4*>(y_fwd);
