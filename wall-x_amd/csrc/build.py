@@ -5,7 +5,7 @@
 Sources are compiled one by one (objects under csrc/build/) and linked into
 wall-x_amd/wallx_mi355/libwallx_mi355.so, next to the Python package that loads it.  The benchmark's MFMA rate
 probe (probe.hip) goes into a library of its own, libwallx_probe.so, beside it, and the host side of the row and rotary
-ops (host_ops.cpp) into the Python module _wallx_host.so.
+ops (host_ops.cpp) into a Python module, which carries the torch and the Python that it was built for in its name.
 """
 
 import os
@@ -30,7 +30,6 @@ PROBE_LIB = os.path.join(OUT_DIR, "libwallx_probe.so")
 
 # the ops' host side, a Python module against torch's headers (no GPU code, and no HIP runtime of its own)
 HOST_SOURCE = "host_ops.cpp"
-HOST_LIB = os.path.join(OUT_DIR, "_wallx_host.so")
 
 FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-fno-gpu-rdc",
@@ -101,21 +100,30 @@ def build_probe(force: bool = False, verbose: bool = True) -> str:
     return PROBE_LIB
 
 
+def host_lib() -> str:
+    """The host module's file: of another torch or Python it is another file, and never taken for this one's."""
+    import sysconfig
+
+    import torch
+
+    return os.path.join(OUT_DIR, f"_wallx_host.torch-{torch.__version__}{sysconfig.get_config_var('EXT_SUFFIX')}")
+
+
 def build_host(force: bool = False, verbose: bool = True) -> str:
     import sysconfig
 
-    path = os.path.join(HERE, HOST_SOURCE)
-    if force or not _newer(HOST_LIB, [path, os.path.join(INCLUDE, "wallx_mi355.h")]):
-        import torch
+    import torch
 
+    path, lib = os.path.join(HERE, HOST_SOURCE), host_lib()
+    if force or not _newer(lib, [path, os.path.join(INCLUDE, "wallx_mi355.h"), os.path.abspath(__file__)]):
         root = os.path.dirname(torch.__file__)
         _run([_hipcc(), "-x", "c++", "-std=c++17", "-O2", "-fPIC", "-shared", "-no-hip-rt", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
               f"-I{root}/include", f"-I{root}/include/torch/csrc/api/include", f"-I{sysconfig.get_paths()['include']}",
               f"-I{os.path.dirname(os.path.dirname(os.path.realpath(_hipcc())))}/include", f"-I{INCLUDE}", f"-L{root}/lib",
-              "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_python", path, "-o", HOST_LIB])
+              "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_python", path, "-o", lib])
         if verbose:
-            print(f"[wallx_mi355] built {HOST_LIB}", flush=True)
-    return HOST_LIB
+            print(f"[wallx_mi355] built {lib}", flush=True)
+    return lib
 
 
 def build(force: bool = False, verbose: bool = True, probe: bool = True) -> str:

@@ -7,11 +7,12 @@ missing, loading raises.
 import ctypes
 import importlib.util
 import os
+import sysconfig
 import threading
+import warnings
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 # WALLX_MI355_LIB points at an alternative build of the same library (e.g. one compiled with other tuning flags)
-HOST_PATH = os.path.join(_HERE, "_wallx_host.so")
 LIB_PATH = os.environ.get("WALLX_MI355_LIB") or os.path.join(_HERE, "libwallx_mi355.so")
 
 WX_F32, WX_F16, WX_BF16 = 0, 1, 2
@@ -112,6 +113,19 @@ def load():
     return _lib
 
 
+def host_path() -> str:
+    """The host module for the running torch and Python, whose binary interfaces it is built against (csrc/build.py: host_lib)."""
+    import torch
+
+    return os.path.join(_HERE, f"_wallx_host.torch-{torch.__version__}{sysconfig.get_config_var('EXT_SUFFIX')}")
+
+
+class _NoHost:
+    """In the place of the host module where it is not built: every call goes on in the general path."""
+
+    rope = permute = unpermute = unpermute_bwd = staticmethod(lambda *args: None)
+
+
 def host():
     """The module of csrc/host_ops.cpp (a call's checks, outputs and launches in native code), bound to the loaded library."""
     global _host
@@ -119,15 +133,17 @@ def host():
         lib = load()
         with _lock:
             if _host is None:
-                if not os.path.exists(HOST_PATH):
-                    raise WallxLibraryError(f"{HOST_PATH} is missing: build it with `python wall-x_amd/csrc/build.py`.")
-                import torch  # noqa: F401  (its libraries, which the module is linked against)
-
-                spec = importlib.util.spec_from_file_location("_wallx_host", HOST_PATH)
-                mod = importlib.util.module_from_spec(spec)
-                spec.loader.exec_module(mod)
-                mod.bind(*(ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in mod.names()))
-                _host = mod
+                path = host_path()
+                if os.path.exists(path):
+                    spec = importlib.util.spec_from_file_location("_wallx_host", path)
+                    mod = importlib.util.module_from_spec(spec)
+                    spec.loader.exec_module(mod)
+                    mod.bind(*(ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in mod.names()))
+                    _host = mod
+                else:
+                    warnings.warn(f"{path} is missing (build it with `python wall-x_amd/csrc/build.py`): the row and rotary ops' calls "
+                                  "take up to 60 us longer on the host")
+                    _host = _NoHost
     return _host
 
 
