@@ -292,3 +292,72 @@ def test_permute_keeps_the_status_word_of_a_workspace_and_nothing_else_of_it(dev
     native.permute(x, ids.long(), 0, ws, 0)  # the general path
     assert torch.equal(ws[0], before)
     assert native.permute(x, ids.zero_(), 0, None, 0)[2] is None
+
+
+@pytest.mark.gpu
+def test_wrappers_of_the_transforms_are_left_alone(dev):
+    """vmap's, grad's and functionalization's tensors are exact torch.Tensors that are none inside; a fake one is a subclass."""
+    q, k, c, s = _rope_inputs(dev, 0, torch.bfloat16, "hf", "bshd")
+    x, ids = torch.randn((6, 64), device=dev), torch.zeros((6, 1), dtype=torch.int32, device=dev)
+    rmap = torch.arange(6, dtype=torch.int32, device=dev)
+    host, seen = _lib.host(), []
+
+    def calls(q, x):
+        seen.append([host.rope(0, q, k, c, s, SECTION, "hf", 0), host.permute(x, ids, 0, None, None, 256), host.unpermute(x, rmap, None, 6, 1),
+                     host.unpermute_bwd(x, x, rmap, None)])
+        return q
+
+    calls(q, x)
+    assert all(r is not None for r in seen.pop())
+    torch.func.vmap(calls)(q[None], x[None])
+    torch.func.grad(lambda q, x: calls(q, x).float().sum())(q.contiguous(), x)
+    torch.func.functionalize(calls)(q, x)
+    torch.func.jvp(lambda t: calls(q, t), (x,), (x,))
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    with FakeTensorMode(allow_non_fake_inputs=True) as mode:
+        calls(mode.from_tensor(q), mode.from_tensor(x))
+    half = torch.randn((6, 64, 2), device=dev)
+    calls(torch.view_as_complex(torch.randn((*q.shape, 2), device=dev)).conj().imag, torch.view_as_complex(half).conj().imag)  # negation pending
+    assert len(seen) == 6 and all(r is None for results in seen for r in results), seen
+
+
+@pytest.mark.gpu
+def test_backwards_and_the_other_forms_recorded_into_a_graph(dev):
+    """Forward and backward of all three forms of the rotary op, and of permute and unpermute with and without weights."""
+    q, k, c, s = _rope_inputs(dev, 0, torch.bfloat16, "hf", "bshd", rows=2, row_len=70)
+    pos, freq = _rope_inputs(dev, 1, torch.bfloat16, "hf", "bshd", rows=2, row_len=70)[2:]
+    table = native.mrope_table(pos, freq, SECTION)
+    g = torch.Generator(device=dev).manual_seed(9)
+    q, k = q.requires_grad_(), k.requires_grad_()
+    x = torch.randn((5000, 64), generator=g, device=dev).to(torch.bfloat16).requires_grad_()
+    probs = torch.rand((5000, 2), generator=g, device=dev).requires_grad_()
+    ids = torch.rand((5000, 4), generator=g, device=dev).argsort(1)[:, :2].to(torch.int32).contiguous()
+    dq, dk, dx = (torch.randn(t.shape, generator=g, device=dev).to(t.dtype) for t in (q, k, x))
+
+    def work():
+        out = []
+        for rotated in (ops.multimodal_rope(q, k, c, s, SECTION), ops.multimodal_rope_from_positions(q, k, pos, freq, SECTION),
+                        ops.multimodal_rope_from_table(q, k, table, SECTION)):
+            out += [t.detach() for t in rotated] + list(torch.autograd.grad(rotated, (q, k), (dq, dk)))
+        permuted, rmap = ops.permute(x, ids)
+        out += [permuted.detach(), rmap, *torch.autograd.grad(ops.unpermute(permuted, rmap, probs), (x, probs), dx)]
+        one, one_map = ops.permute(x, ids[:, :1].contiguous())
+        return out + [one.detach(), *torch.autograd.grad(ops.unpermute(one, one_map), x, dx)]
+
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        work()
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = work()
+    for _ in range(3):
+        with torch.no_grad():
+            for t in (q, k, x, probs, dq, dk, dx):
+                t.copy_(torch.randn(t.shape, generator=g, device=dev).to(t.dtype))
+            ids.copy_(torch.rand((5000, 4), generator=g, device=dev).argsort(1)[:, :2])
+        graph.replay()
+        got = [t.clone() for t in out]
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(got, work()))

@@ -10,6 +10,7 @@
 
 #include <ATen/ATen.h>
 #include <c10/core/DeviceGuard.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/hip/HIPStream.h>
 #include <pybind11/pybind11.h>
 #include <torch/csrc/Exceptions.h>
@@ -43,9 +44,12 @@ const char* const kNames[] = {"wx_last_error_string", "wx_mrope_apply", "wx_mrop
 constexpr int kEntries = sizeof(kNames) / sizeof(kNames[0]);
 static_assert(sizeof(Entry) == kEntries * sizeof(void*), "a name per entry point");
 
-// A tensor that is what it looks like: strided CUDA memory, no wrapper, no pending conjugation or negation.
+// A tensor that is what it looks like: strided CUDA memory, no wrapper, no pending conjugation or negation -- and, as what is
+// allocated inside a transform is a wrapper whatever the inputs are, outside of all transforms.
 const at::Tensor* plain(PyObject* o) {
   if (!THPVariable_CheckExact(o)) return nullptr;
+  for (const c10::DispatchKey transform : {c10::DispatchKey::FuncTorchDynamicLayerFrontMode, c10::DispatchKey::Functionalize})
+    if (c10::impl::tls_is_dispatch_key_included(transform)) return nullptr;
   const at::Tensor& t = THPVariable_Unpack(o);
   if (!t.defined() || !t.is_cuda() || t.layout() != at::kStrided || t.is_conj() || t.is_neg()) return nullptr;
   constexpr c10::DispatchKeySet wrappers({c10::DispatchKey::Python, c10::DispatchKey::PythonTLSSnapshot, c10::DispatchKey::FuncTorchBatched,
