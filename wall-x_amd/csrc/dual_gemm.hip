@@ -142,11 +142,8 @@ struct Params {
   int gate, gate_tiles;
   // Tail split (see tail_plan): 0 = off; 1 = this launch does the whole rounds of 256 x 256 tiles and leaves
   // the ragged last round to a second launch, with 128 x 128 tiles (ROLE 4).
-  // split_cus = workgroups of the first launch (one per CU).  plan: the launches' plan where the host alone makes it (kGeneric,
-  // kQkvRope, kQkvRopeFull).  (Made again by every workgroup of both launches: 1656 rows of 11008 columns, contractions of 64
-  // to 4096, 0.6 us longer.)
+  // split_cus = workgroups of the first launch (one per CU).
   int split, split_cus;
-  TailPlan plan;
   // kDown only: when set (the partition's sorted_row_id), row r of the sorted result is stored to row scatter[r] of
   // the output instead of row r -- the unpermute folded into the store.
   const int32_t* scatter;
@@ -161,10 +158,16 @@ struct Params {
   const __bf16* bias;
   const uint32_t* rope_table;
   int rope_cols, rope_width;
-  // kGateUp only (training): when set, the two projections themselves (rounded to bf16, before the SwiGLU) are
-  // stored as well, K-tiled with the geometry of the intermediate, so that a backward pass need not recompute them.
-  __bf16* keep_gate;
-  __bf16* keep_up;
+  // One place for what only one kind of launch has (the one launch of both GEMMs on few rows takes two of these structs: 16 bytes
+  // more in each cost a denoise step of 36 layers 10 us of 564).
+  union {
+    // kGateUp only (training): when set, the two projections themselves (gate and up, rounded to bf16, before the SwiGLU) are
+    // stored as well, K-tiled with the geometry of the intermediate, so that a backward pass need not recompute them.
+    __bf16* keep[2];
+    // kGeneric, kQkvRope, kQkvRopeFull: the plan of the two launches, which the host alone makes there.  (Made again by every
+    // workgroup of both launches: 1656 rows of 11008 columns, contractions of 64 to 4096, 0.6 us longer.)
+    TailPlan plan;
+  };
 };
 
 #define LDS_PTR(p) ((__attribute__((address_space(3))) void*)(p))
@@ -950,9 +953,9 @@ __device__ __forceinline__ void few_rows_body(const Params& p, const int wg, con
           if constexpr (ROLE == 1) __builtin_amdgcn_raw_buffer_store_b64(v, make_rsrc(dst, kBlkBytes), in_block, 0, 16 /* sc1 */);
           else *reinterpret_cast<u32x2*>(dst + in_block) = v;
           if constexpr (ROLE == 0) {  // the projections themselves, for a backward pass
-            if (p.keep_gate != nullptr) {
-              *reinterpret_cast<u32x2*>(reinterpret_cast<unsigned char*>(p.keep_gate) + block + in_block) = u32x2{pack_bf16x2(g[0], g[1]), pack_bf16x2(g[2], g[3])};
-              *reinterpret_cast<u32x2*>(reinterpret_cast<unsigned char*>(p.keep_up) + block + in_block) = u32x2{pack_bf16x2(u[0], u[1]), pack_bf16x2(u[2], u[3])};
+            if (p.keep[0] != nullptr) {
+              *reinterpret_cast<u32x2*>(reinterpret_cast<unsigned char*>(p.keep[0]) + block + in_block) = u32x2{pack_bf16x2(g[0], g[1]), pack_bf16x2(g[2], g[3])};
+              *reinterpret_cast<u32x2*>(reinterpret_cast<unsigned char*>(p.keep[1]) + block + in_block) = u32x2{pack_bf16x2(u[0], u[1]), pack_bf16x2(u[2], u[3])};
             }
           }
         }
@@ -1885,9 +1888,9 @@ __device__ __forceinline__ void dual_gemm_body(const Params& p, const int wg, co
       constexpr int kRound = kStageBytes / (kColBlocks * kBlkBytes);
       static_assert(FN % 4 == 0 && kRound >= 1 && FM % kRound == 0, "staging holds whole rounds of blocks");
       // what == 0: the intermediate h; 1 / 2: the gate / up projections themselves, when the caller keeps them
-      const int n_what = p.keep_gate != nullptr ? 3 : 1;
-      const int64_t keep_off[3] = {0, reinterpret_cast<unsigned char*>(p.keep_gate) - reinterpret_cast<unsigned char*>(p.g[0].c),
-                                   reinterpret_cast<unsigned char*>(p.keep_up) - reinterpret_cast<unsigned char*>(p.g[0].c)};
+      const int n_what = p.keep[0] != nullptr ? 3 : 1;
+      const int64_t keep_off[3] = {0, reinterpret_cast<unsigned char*>(p.keep[0]) - reinterpret_cast<unsigned char*>(p.g[0].c),
+                                   reinterpret_cast<unsigned char*>(p.keep[1]) - reinterpret_cast<unsigned char*>(p.g[0].c)};
 #pragma unroll
       for (int round = 0; round < FM / kRound; ++round) {
         for (int what = 0; what < n_what; ++what) {
@@ -2485,8 +2488,9 @@ int launch_mfma(Params p, int64_t tiles_lo, int64_t tiles_hi, hipStream_t s, con
         split = false;
       } else if (rows != nullptr) {
         auto cols = [&](int e) { return rows[e] > 0 ? static_cast<int>(tiles_by_expert[e] / ceil_div(rows[e], BigTile::BM)) : 0; };
-        p.plan = tail_plan(static_cast<int>(rows[0]), static_cast<int>(rows[1]), cols(0), cols(1), p.g[0].k, p.g[1].k, cus, true, MODE == kGateUp ? kTailLongTiled : kTailLongRows);
-        split = p.plan.split;
+        const TailPlan plan = tail_plan(static_cast<int>(rows[0]), static_cast<int>(rows[1]), cols(0), cols(1), p.g[0].k, p.g[1].k, cus, true, MODE == kGateUp ? kTailLongTiled : kTailLongRows);
+        split = plan.split;
+        if (MODE == kGeneric) p.plan = plan;
       } else {
         split = tail_split_point(static_cast<int>(tiles_by_expert[0]), static_cast<int>(tiles_by_expert[1]), p.g[0].k, p.g[1].k, cus) != all;
       }
@@ -2653,6 +2657,7 @@ extern "C" int wx_qkv_rope_proj(const void* x, const void* weight, const void* b
   // The table, this launch and the o projection at n 2560, k 2048: 32 rows 66 -> 45 us, 1024 rows 70 -> 48, 2048 rows
   // 73 -> 63, 3072 rows 83 -> 76; one more row of large tiles is past the line.
   const bool small = tiles <= cus / 2;
+  p.plan = TailPlan{};
   if (!small && tiles < INT32_MAX) p.plan = tail_plan(g.m, 0, static_cast<int>(ceil_div(g.n, Tile::BN)), 0, g.k, 0, cus, true, kTailLongRows);
   const bool split = p.plan.split;
   p.split = split ? 1 : 0;
@@ -2749,8 +2754,8 @@ Params gate_up_params(const FfnArgs& a) {
     g.a_row0 = 0;
   }
   p.offsets = a.offsets;
-  p.keep_gate = static_cast<__bf16*>(a.keep_gate);
-  p.keep_up = static_cast<__bf16*>(a.keep_up);
+  p.keep[0] = static_cast<__bf16*>(a.keep_gate);
+  p.keep[1] = static_cast<__bf16*>(a.keep_up);
   return p;
 }
 
