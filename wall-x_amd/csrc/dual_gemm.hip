@@ -1798,8 +1798,8 @@ __device__ __forceinline__ void dual_gemm_body(const Params& p, const int wg, co
     // What the stores need from memory is asked for ahead of the first of them: the row ids of the whole tile, and the addend's
     // chunks kAhead row blocks in front of their use.  (Asked for row block by row block, a tile of 256 rows waited for eight
     // memory latencies one after the other, twice over with row ids and an addend: q / k / v and o projections of 14592 rows with
-    // the rotary table's loads a row block ahead as well 291.6 -> 283.9 us, a layer of 912 rows 157 -> 155, training on 29184 rows
-    // 9630 -> 9600.)  Three row blocks where the row ids take registers, two in the kernel with the
+    // the rotary table's loads a row block ahead as well 291.6 -> 283.9 us, four layers of 912 rows 627 -> 618; training and a
+    // prefill of 29184 rows level.)  Three row blocks where the row ids take registers, two in the kernel with the
     // parts, which spills 24 bytes with three (56 with four): layers of 2049 to 3500 rows on device-side counts 0.6 % longer.
     // Rows past the tile's end read a row that is there.
     constexpr int kMost = ROLE == 3 ? 2 : (MODE == kDown ? 3 : 4), kAhead = FM < kMost ? FM : kMost;

@@ -1,7 +1,8 @@
 // The host side of the row and rotary ops in native code: the checks, the outputs and the launches of one call.
 //
 // What such a pass costs is the host's work: the rotary op forward and backward on 16 tokens took 135 us of Python, where the
-// kernels of 14336 tokens take 58, and takes 77 this way; permute and unpermute forward and backward 140 and 88.  Each function here takes the call as the op got it, and either makes it whole --
+// kernels of 14336 tokens take 58, and takes 70 to 83 this way; permute and unpermute of 14593 tokens forward and backward took
+// 140 and take 100, which is what their kernels take.  Each function here takes the call as the op got it, and either makes it whole --
 // allocates, launches, returns the outputs -- or returns None and has touched nothing: anything but plain CUDA tensors of one device
 // with the shapes, types and strides that the kernels read in place (a subclass, a transform's wrapper, a tensor that would
 // first be copied or moved, anything to be refused) is the general path's, in native.py, which warns, copies and raises.

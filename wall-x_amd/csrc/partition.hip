@@ -510,7 +510,7 @@ __global__ __launch_bounds__(kMoverWaves* kWave) void combine_rows_kernel(
 }
 
 // Backward of the weighted combine; one wavefront per token.  (With the copies one after the other and their gradient's row read
-// for each, and a chunk at a time: 8000 tokens of 2048, us, two copies in bf16 42 -> 30, three in fp32 110 -> 72.)  The rows of act_grad that no token maps to are zeros: the
+// for each, and a chunk at a time: 8000 tokens of 2048, us, two copies in bf16 41.9 -> 34.4, three in fp32 113 -> 85.)  The rows of act_grad that no token maps to are zeros: the
 // first `clearers` workgroups find them in their share of the num_rows rows by reading the whole map into a bitmap in LDS, and
 // clear them, beside the workgroups that move rows.  (Clearing all of act_grad in a launch of its own ahead of this one
 // writes every row twice: 14593 rows of 4 KiB 10.4 us + 25.5.)  The search must not take longer than the moving: with 64-bit
@@ -605,8 +605,9 @@ __global__ __launch_bounds__(kMoverWaves* kWave, COPIES == 0 ? 8 : (COPIES == 2 
         // Two chunks at a time.  (A copy may be missing, so its loads are under a branch, behind which the compiler does not know
         // how many are in flight and waits for all of them, and for the stores: with a chunk at a time that is a memory latency per
         // chunk.)  The forward's rows were written a moment ago and are read with plain loads, which find them in the last-level cache.
-        // us, a chunk at a time and non-temporal loads -> now: 668 tokens of 2048, two copies in fp32 14.9 -> 9.6, three 14.3 -> 9.5,
-        // three in fp16 10.2 -> 7.3; 9728 tokens, two copies in bf16 39 -> 35, in fp32 84 -> 62.
+        // us inside a pass, copies one by one / a chunk at a time and non-temporal loads / now: 1500 tokens of 2048, two copies in fp32
+        // 17.2 / 19.7 / 12.9; 668 tokens, three in fp16 10.2 / 8.7 / 6.4; 8000 tokens, two in bf16 41.9 / 34.3 / 34.4, three in fp32
+        // 113 / 91 / 85.  (The same launch again and again on one set of buffers: 9728 tokens, two copies in bf16 39 -> 35, in fp32 84 -> 62.)
         chunks_of_a_row<2>(lane, vec_per_row, [&](int64_t v, auto n) {
           constexpr int N = decltype(n)::value;
           u32x4 graw[N], yraw[kCopies][N];
